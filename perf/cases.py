@@ -390,3 +390,115 @@ def prepare(case, seed):
 def run(state):
     gpu.check(state.fn(*state.args), "call")
     return state.outputs
+
+
+# ------------------------------------------------------------------------------------------------ the same in 64 bits
+
+def _q4_rows(blob, R, Cc):
+    """One matrix of _q4_blobs as float64 [R][Cc]."""
+    n = R * Cc
+    v = blob[:n // 2]
+    q = torch.stack((v & 15, v >> 4), 1).view(R, Cc // GROUP, GROUP).double()
+    s, b = (blob[n // 2 + 2 * k * (n // GROUP):][:2 * (n // GROUP)].clone().view(torch.bfloat16).double().view(R, -1, 1)
+            for k in (0, 1))
+    return q.mul_(s).add_(b).view(R, Cc)
+
+
+def _q4_product(blob, R, Cc, xs):
+    """xs [B][Cc] (float64) times the matrix, in slabs of rows."""
+    n, slab, outs = R * Cc, 4096, []
+    groups = Cc // GROUP
+    for r in range(0, R, slab):
+        m = min(slab, R - r)
+        part = torch.cat((blob[r * Cc // 2:(r + m) * Cc // 2], blob[n // 2 + 2 * r * groups:n // 2 + 2 * (r + m) * groups],
+                          blob[n // 2 + 2 * (R + r) * groups:n // 2 + 2 * (R + r + m) * groups]))
+        outs.append(xs @ _q4_rows(part, m, Cc).T.contiguous())
+    return torch.cat(outs, 1)
+
+
+def _e2m1(codes):
+    table = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], device="cuda", dtype=torch.float64)
+    mag = table[(codes & 7).long()]
+    return torch.where(codes > 7, -mag, mag)
+
+
+def _fp4_values(w, s):
+    R, half = w.shape
+    v = torch.stack((w & 15, w >> 4), 2).view(R, half // 8, 16)
+    return (_e2m1(v) * s.view(torch.float8_e4m3fn).double().unsqueeze(2)).view(R, 2 * half) / DIVISOR
+
+
+def _fp4_activations(xs):
+    """The NVFP4 image of the activations: which code an element gets is decided in 32 bits, as the format's quantiser does."""
+    v = xs.view(xs.shape[0], -1, 16)
+    raw = (INPUT_SCALE * (v.abs().amax(2, keepdim=True) * torch.tensor(1 / 6, device="cuda"))).clamp(max=448.0)
+    scale = raw.to(torch.float8_e4m3fn).float()
+    to_code = torch.where(scale == 0, torch.zeros_like(scale), INPUT_SCALE / scale)
+    m = (v * to_code).clamp(-6.0, 6.0)
+    a = m.abs()
+    code = sum((test.to(torch.uint8) for test in (a > 0.25, a >= 0.75, a > 1.25, a >= 1.75, a > 2.5, a >= 3.5, a > 5.0)))
+    return (_e2m1(code) * torch.sign(m).double() * (scale / INPUT_SCALE).double()).view(xs.shape)
+
+
+def _fp4_product(w, s, xs, slab=2048):
+    return torch.cat([xs @ _fp4_values(w[r:r + slab], s[r:r + slab]).T.contiguous() for r in range(0, w.shape[0], slab)], 1)
+
+
+def _gelu(v):
+    return 0.5 * v * (1.0 + torch.tanh(math.sqrt(2.0 / math.pi) * (v + 0.044715 * v ** 3)))
+
+
+def _expert(blobs, H, F, xs):
+    """Output of the expert with the three matrices blobs for the rows xs (float64)."""
+    gate, up, down = blobs.view(3, -1)
+    return _q4_product(down, H, F, _gelu(_q4_product(gate, F, H, xs)) * _q4_product(up, F, H, xs))
+
+
+def exact(case, seed):
+    kind, g = case["kind"], _generator(seed)
+    status = torch.zeros(1, device="cuda", dtype=torch.int32)
+    if kind in ("q4", "q4_matmul"):
+        R, Cc, B, n = case["R"], case["C"], case["B"], case.get("mats", 1)
+        w, xs = _q4_blobs(g, n, R * Cc), _normal(g, B, Cc).double()
+        ys = torch.stack([_q4_product(w[j], R, Cc, xs) for j in range(n)])
+        return ys if kind == "q4" else ys[0]
+    if kind in ("nvfp4", "nvfp4_matmul"):
+        R, Cc, B, n = case["R"], case["C"], case.get("B", 1), case.get("mats", 1)
+        (w, s), xs = _nvfp4(g, n, R, Cc), _normal(g, B, Cc)
+        xs = _fp4_activations(xs)
+        ys = torch.stack([_fp4_product(w[j], s[j], xs) for j in range(n)])
+        return [ys if kind == "nvfp4" else ys[0], status]
+    if kind == "head":
+        R, Cc, B = case["R"], case["C"], case["B"]
+        w, xs = (0.02 * _normal(g, R, Cc)).bfloat16(), _normal(g, B, Cc).double()
+        return torch.cat([xs @ w[r:r + 16384].double().T.contiguous() for r in range(0, R, 16384)], 1)
+    if kind == "abi_matvec":
+        R, Cc = case["R"], case["C"]
+        blob, x = _q4_blobs(g, 1, R * Cc), _normal(g, Cc).double()
+        return _host(_q4_product(blob[0], R, Cc, x[None])[0])
+    if kind == "ffn_block":             # a router's choice between near-equal gates is not a number to compare
+        return None
+    E, K, H, F = case["E"], case["K"], case["H"], case["F"]
+    pool = _pool(g, E, H, F)
+    if kind == "abi_chain":
+        chosen = sorted(torch.randperm(E, generator=g, device="cuda")[:K].tolist())
+        x = _normal(g, H).double()[None]
+        return _host(torch.cat([_expert(pool[e], H, F, x) for e in chosen]))
+    if kind == "moe_decode":
+        logits, scale, x = _normal(g, E), _uniform(g, 0.5, 2.0, E), _normal(g, H).double()[None]
+        sel = logits.topk(K).indices.sort().values
+        wts = torch.softmax(logits[sel].double(), 0) * scale[sel].double()
+        eo = torch.cat([_expert(pool[e], H, F, x) for e in sel.tolist()])
+        return [sel.int(), wts, eo, wts @ eo]
+    T = case["T"]
+    xs = _normal(g, T, H).double()
+    rank = torch.randperm(E, generator=g, device="cuda") + 1
+    keys = -1.1 * torch.log(rank.float()) - torch.log(-torch.log(_uniform(g, 1e-7, 1 - 1e-7, T, E)))
+    sel = keys.topk(K, dim=1).indices.sort(dim=1).values
+    wts = torch.softmax(_normal(g, T, K), dim=1).double()
+    out = torch.zeros(T, H, device="cuda", dtype=torch.float64)
+    for e in range(E):
+        token, k = (sel == e).nonzero(as_tuple=True)
+        if token.numel():
+            out.index_add_(0, token, _expert(pool[e], H, F, xs[token]) * wts[token, k][:, None])
+    return [out, torch.bincount(sel.flatten(), minlength=E).int(), sel.flatten().argsort(stable=True).int(), status]
