@@ -12,7 +12,7 @@ extern "C" {
 
 size_t salt_mi355_q4_matmul_workspace_bytes(int C, int B) {
     if (C < 64 || (C & 63) || B < 1) return 0;
-    return 3 * (size_t)B * C * 2 + (((size_t)B * (C / 64) * 4 + 255) & ~(size_t)255) + 256;
+    return 3 * (size_t)B * C * 2;                // three planes of 16 bits per activation
 }
 
 int salt_mi355_q4_matmul_dev(const void *vals, const void *scales, const void *biases, int R, int C, int B,
@@ -26,8 +26,7 @@ int salt_mi355_q4_matmul_dev(const void *vals, const void *scales, const void *b
     }
     uint16_t *planes = (uint16_t *)workspace;
     const size_t plane_stride = (size_t)B * C;
-    float *xsum = (float *)((uint8_t *)workspace + ((3 * plane_stride * 2 + 255) & ~(size_t)255));
-    if (x_split_launch(xs, nullptr, nullptr, 1, C, B, C, planes, plane_stride, xsum, (hipStream_t)stream) != 0) {
+    if (x_split_launch(xs, nullptr, nullptr, 1, C, B, C, planes, plane_stride, (hipStream_t)stream) != 0) {
         set_error("q4 matmul: activation split launch failed");
         return -1;
     }
@@ -35,10 +34,9 @@ int salt_mi355_q4_matmul_dev(const void *vals, const void *scales, const void *b
     memset(&launch, 0, sizeof launch);
     launch.one.vals = (const uint8_t *)vals; launch.one.scales = (const uint8_t *)scales;
     launch.one.biases = (const uint8_t *)biases;
-    launch.one.planes = planes; launch.one.xsum = xsum; launch.one.y = ys;
+    launch.one.planes = planes; launch.one.y = ys;
     launch.one.tokens = B; launch.one.rows = R;
     launch.njobs = 1; launch.cols = C; launch.plane_stride = plane_stride;
-    launch.blocks_per_wave = 0;                  // the launcher picks the tile width and counts the tiles
     if (q4_mfma_launch(launch, (hipStream_t)stream) != 0) { set_error("q4 matmul: launch failed"); return -1; }
     return 0;
 }

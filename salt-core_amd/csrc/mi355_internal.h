@@ -150,7 +150,6 @@ constexpr int MFMA_TM = 64;   // tokens per workgroup of the matrix-core kernel;
 struct MfmaJob {
     const uint8_t *vals, *scales, *biases;   // biases may be null
     const uint16_t *planes;   // plane 0 of this job's first token; plane p lies p * plane_stride elements further
-    const float *xsum;        // [tokens][C/64]
     float *y;                 // [tokens][rows]
     int tokens;
     int rows;
@@ -169,17 +168,17 @@ struct MfmaLaunch {
     const int *total_tiles_dev;   // workgroups past *total_tiles_dev exit at once
     const int *row_map;       // optional gather: token t of a job reads plane row row_map[row_base + t] / map_divisor
     int map_divisor;
-    int blocks_per_wave;      // the tile is 64 tokens x 64 * blocks_per_wave rows (mfma_blocks_per_wave()); 0 = choose (single job only)
+    int column_parts;         // the tile is tile_tokens (64 or 32) x 256 / column_parts rows (mfma_column_parts());
+    int tile_tokens;          // the launcher chooses both for a single job
 };
 
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream);
-int mfma_tile_rows(int blocks_per_wave);
-int mfma_tiles(int tokens, int rows, int blocks_per_wave);
-int mfma_blocks_per_wave(long long wide_tiles);
+int mfma_tile_rows(int column_parts);
+int mfma_column_parts(long long wide_tiles, int ngrp);
 // rows of fp32 -> bf16 planes + group sums; output row r reads input row row_map[r] / map_divisor when a map is
 // given; with a gate the value split is gelu_tanh(gate) * x (gate has the layout of x)
 int x_split_launch(const float *x, const float *gate, const int *row_map, int map_divisor, int x_stride, int rows,
-                   int cols, uint16_t *planes, size_t plane_stride, float *xsum, hipStream_t stream);
+                   int cols, uint16_t *planes, size_t plane_stride, hipStream_t stream);
 
 // ---------------------------------------------------------------- NVFP4
 

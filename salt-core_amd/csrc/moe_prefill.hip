@@ -83,8 +83,8 @@ struct ScanArgs {
     PrefillPlan *plan;
     int *status_out;                     // optional
     MfmaJob *gate_up_jobs, *down_jobs;
-    const uint16_t *planes_in;  const float *xsum_in;      // split of the inputs, one row per token  [tokens][hidden]
-    const uint16_t *planes_act; const float *xsum_act;     // split of the activations, grouped rows   [rows][routed]
+    const uint16_t *planes_in;           // split of the inputs, one row per token  [tokens][hidden]
+    const uint16_t *planes_act;          // split of the activations, grouped rows   [rows][routed]
     float *gate, *up, *down;
 };
 
@@ -120,7 +120,6 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
             MfmaJob j;
             j.vals = slot + p * proj; j.scales = j.vals + vals_bytes; j.biases = j.scales + meta_bytes;
             j.planes = a.planes_in;                           // gathered through the row map
-            j.xsum = a.xsum_in;
             j.y = (p == 0 ? a.gate : a.up) + (size_t)row0 * a.routed;
             j.tokens = n; j.rows = a.routed;
             j.tile0 = (2 * mt0 + p * mt) * nt_up;
@@ -130,7 +129,6 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
         MfmaJob d;
         d.vals = slot + 2 * proj; d.scales = d.vals + vals_bytes; d.biases = d.scales + meta_bytes;
         d.planes = a.planes_act + (size_t)row0 * a.routed;
-        d.xsum = a.xsum_act + (size_t)row0 * (a.routed >> 6);
         d.y = a.down + (size_t)row0 * a.hidden;
         d.tokens = n; d.rows = a.hidden;
         d.tile0 = mt0 * nt_down;
@@ -213,7 +211,7 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 struct PrefillWorkspace {
     PrefillPlan *plan; int *counts, *offsets, *pair_rows, *row_pairs;
     MfmaJob *gate_up_jobs, *down_jobs;
-    uint16_t *planes_in; float *xsum_in; uint16_t *planes_act; float *xsum_act;
+    uint16_t *planes_in, *planes_act;
     float *gate, *up, *down;
     size_t bytes;
 };
@@ -231,9 +229,7 @@ PrefillWorkspace carve(const MoeGeometry &g, int tokens, void *base) {
     w.gate_up_jobs = (MfmaJob *)take(2 * E * sizeof(MfmaJob));
     w.down_jobs = (MfmaJob *)take(E * sizeof(MfmaJob));
     w.planes_in = (uint16_t *)take(3 * (size_t)tokens * g.hidden * 2);
-    w.xsum_in = (float *)take((size_t)tokens * (g.hidden / 64) * 4);
     w.planes_act = (uint16_t *)take(3 * rows * g.routed * 2);
-    w.xsum_act = (float *)take(rows * (g.routed / 64) * 4);
     w.gate = (float *)take(rows * g.routed * 4);
     w.up = (float *)take(rows * g.routed * 4);
     w.down = (float *)take(rows * g.hidden * 4);
@@ -254,11 +250,11 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
         return -1;
     const PrefillWorkspace w = carve(g, tokens, workspace);
     const int rows = tokens * g.topk;
-    // Tile widths: the wide tile when the upper bound of the grid fills the device twice.
+    // Column parts from the upper bound of the tiles: an expert's token count is known only on the device.
     const int m_upper = rows / MFMA_TM + (g.n_experts < rows ? g.n_experts : rows);
-    const int bpw_up = mfma_blocks_per_wave(2LL * m_upper * ((g.routed + 255) / 256));
-    const int bpw_down = mfma_blocks_per_wave((long long)m_upper * ((g.hidden + 255) / 256));
-    const int tn_up = mfma_tile_rows(bpw_up), tn_down = mfma_tile_rows(bpw_down);
+    const int parts_up = mfma_column_parts(2LL * m_upper * ((g.routed + 255) / 256), g.hidden >> 6);
+    const int parts_down = mfma_column_parts((long long)m_upper * ((g.hidden + 255) / 256), g.routed >> 6);
+    const int tn_up = mfma_tile_rows(parts_up), tn_down = mfma_tile_rows(parts_down);
     const int nt_up = (g.routed + tn_up - 1) / tn_up, nt_down = (g.hidden + tn_down - 1) / tn_down;
     // plan and counts are adjacent 256-byte aligned pieces of the workspace: one clear covers both
     static_assert(sizeof(PrefillPlan) <= 256, "the plan fits the first aligned piece");
@@ -271,7 +267,7 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
     a.tn_up = tn_up; a.tn_down = tn_down;
     a.counts = w.counts; a.offsets = w.offsets; a.group_rows = group_rows; a.plan = w.plan; a.status_out = status_dev;
     a.gate_up_jobs = w.gate_up_jobs; a.down_jobs = w.down_jobs;
-    a.planes_in = w.planes_in; a.xsum_in = w.xsum_in; a.planes_act = w.planes_act; a.xsum_act = w.xsum_act;
+    a.planes_in = w.planes_in; a.planes_act = w.planes_act;
     a.gate = w.gate; a.up = w.up; a.down = w.down;
     hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(MAX_EXPERTS), 0, stream, a);
     int *rp = row_pairs ? row_pairs : w.row_pairs;
@@ -285,24 +281,24 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
     // bound (sum over experts of ceil(n_e / 64) <= rows / 64 + experts) and
     // surplus workgroups leave at once.
     if (x_split_launch(inputs, nullptr, nullptr, 1, g.hidden, tokens, g.hidden, w.planes_in, (size_t)tokens * g.hidden,
-                       w.xsum_in, stream) != 0)
+                       stream) != 0)
         return -1;
     MfmaLaunch gu;
     memset(&gu, 0, sizeof gu);
     gu.table = w.gate_up_jobs; gu.cols = g.hidden; gu.total_tiles = 2 * m_upper * nt_up;
     gu.plane_stride = (size_t)tokens * g.hidden;
-    gu.row_map = rp; gu.map_divisor = g.topk; gu.blocks_per_wave = bpw_up;
+    gu.row_map = rp; gu.map_divisor = g.topk; gu.column_parts = parts_up; gu.tile_tokens = MFMA_TM;
     gu.njobs_dev = &w.plan->gate_up_jobs; gu.total_tiles_dev = &w.plan->gate_up_tiles;
     if (q4_mfma_launch(gu, stream) != 0) return -1;
     // gelu(gate) * up, split for the down projection
     if (x_split_launch(w.up, w.gate, nullptr, 1, g.routed, rows, g.routed, w.planes_act, (size_t)rows * g.routed,
-                       w.xsum_act, stream) != 0)
+                       stream) != 0)
         return -1;
     MfmaLaunch dn;
     memset(&dn, 0, sizeof dn);
     dn.table = w.down_jobs; dn.cols = g.routed; dn.total_tiles = m_upper * nt_down;
     dn.plane_stride = (size_t)rows * g.routed;
-    dn.blocks_per_wave = bpw_down;
+    dn.column_parts = parts_down; dn.tile_tokens = MFMA_TM;
     dn.njobs_dev = &w.plan->down_jobs; dn.total_tiles_dev = &w.plan->down_tiles;
     if (q4_mfma_launch(dn, stream) != 0) return -1;
     hipLaunchKernelGGL(prefill_reduce_kernel, dim3(tokens, (g.hidden + 1023) / 1024), dim3(256), 0, stream, w.down,

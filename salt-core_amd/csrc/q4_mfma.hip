@@ -7,67 +7,127 @@
 // and are told so (the engine's bit-exact path remains the tiled kernels).
 //
 // How the affine weights reach the matrix cores without losing bits:
-//  * per 64-column scale group,  sum_c (q s + b) x = s * sum_c q x + b * sum_c x.
-//    The integer codes are exact in bf16, so only sum_c q x goes through MFMA
-//    per group; the scale is applied per group in fp32 on the VALU.
-//  * a nibble becomes the fp16 value 16 + q with two bit operations per pair
-//    ((w shifted) & 0x03C003C0 | 0x4C004C00); the surplus 16 * s * sum_c x joins
-//    the bias term.
+//  * q s + b = s (q - 8) + (b + 8 s).  q - 8 lies in -8..7: three significant
+//    bits, or a power of two.  Times the eight of a bf16 scale that is at most
+//    eleven, an fp16 significand, so s (q - 8) is an exact fp16 operand and the
+//    whole row accumulates in the matrix cores with no work per scale group.
+//  * fp16's exponents are the limit: a row's scales are brought to the top of
+//    its range by a power of two 2^(11 - E) (E from the row's largest |s| and
+//    |b| / 8), below which 28 binades are exact.  A tile with scales further
+//    apart walks its columns once per 28 binades ("window"), each time with the
+//    other scales taken as zero, and adds the results in the output.  Weights in
+//    earnest span a few binades: one window.
+//  * a nibble becomes the fp16 value 16 + q with two bit operations per pair,
+//    and fma(16 + q, s, -24 s) is s (q - 8), exact at every step.
 //  * the activation row is scaled by a power of two that puts its largest
 //    magnitude in [2^13, 2^14) and split into two fp16 planes, x * 2^k = hi + lo
 //    (each rounded to nearest: 23 significant bits, |x 2^k - hi - lo| <= 2^-22
 //    of the element's own magnitude, or 2^-25 of the scaled row for elements so
 //    small that lo is subnormal); each plane is an exact MFMA operand,
-//    accumulation is fp32, and the power of two leaves with the store.
-//  * the bias term sum_g (b_g - 16 s_g) * X_g (X_g = the group sums of x) is
+//    accumulation is fp32, and the powers of two leave with the store.
+//  * the bias term sum_g (b_g + 8 s_g) * X_g (X_g = the group sums of x) is
 //    itself a small contraction over the groups; b and s are bf16, so it runs
 //    on the matrix cores once per tile before the main loop, with X_g split
 //    into three bf16 planes (v = hi + mid + lo to 2^-24).
 //
-// Tiling: a workgroup of four waves computes 64 tokens x 128 weight rows, each
-// wave 32 tokens x 64 rows as two 32 x 32 blocks of v_mfma_f32_32x32x16_f16
-// that share the token operand (tokens are the M rows, weight rows the N
-// columns, so a lane owns one weight row per block and needs one scale per
-// group).  Per group the planes, the packed codes and the scales are staged in
-// one of two LDS stages, the next group's loads in flight during the matrix
-// work, one barrier per group.  Inside every aligned run of eight columns the
-// planes are stored in the order 0,4,1,5,2,6,3,7, which is the order the pair
-// extraction above yields the codes in.
+// Tiling.  A wave computes 64 tokens x 64 weight rows as 2 x 2 blocks of
+// v_mfma_f32_32x32x16_f16 (tokens are the M rows, weight rows the N columns).
+// The codes of its rows go from memory to its registers and are converted
+// there, once per 64 tokens; the token planes are staged in LDS for the
+// workgroup, two stages, the next one's loads in flight during the matrix work,
+// one barrier per stage.  Per 16 columns a wave reads 4 KB of LDS for eight
+// matrix instructions, 64 bytes per clock of the 128 a compute unit has, and
+// issues 24 other vector instructions in their shadow.  The four waves of a
+// workgroup are four row blocks (64 x 256 tile, 128 columns per stage) or, in
+// launches too small for that, also two or four parts of the columns, which
+// meet in LDS in part order.
+//
+// Bound: the matrix cores, which execute twice the useful operations, at the
+// clock that their power leaves them: 44 % busy at 1.6 to 2.1 GHz in the grouped
+// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 602 us a layer);
+// one 16384 x 2816 matrix, 333 tokens: 101 -> 82 us, 384 tiles on 256 compute
+// units.  Before, every scale group cost 16 multiply-adds per block and a
+// conversion in each of two waves, and each 32 bytes of codes and each scale
+// fetched a cache line of its own.
+//
+// Inside every aligned run of eight columns the planes are stored in the order
+// 0,4,1,5,2,6,3,7, which is the order the pair extraction yields the codes in;
+// the two lane halves of an instruction take columns 32 h + 8 k .. + 7 of a
+// scale group, so that a lane's codes of a group are 16 consecutive bytes.
 #include "device_math.h"
 #include "mi355_internal.h"
 
 #include <stddef.h>
+
 #include <type_traits>
 
 namespace mi355 {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-constexpr int X_PLANES = 2;                // fp16 planes of the scaled activation
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;                 // rows of scales start on any even address
 typedef const uint64_t __attribute__((address_space(4))) *uniform_u64_ptr;
 typedef const u32x4 __attribute__((address_space(1))) *global_u128_ptr;
+typedef const u32x4_any __attribute__((address_space(1))) *global_u128_any_ptr;
 typedef const uint16_t __attribute__((address_space(1))) *global_u16_ptr;
-typedef const float __attribute__((address_space(1))) *global_f32_ptr;
+typedef const uint8_t __attribute__((address_space(1))) *global_u8_ptr;
+typedef const void __attribute__((address_space(1))) *global_void_ptr;
+typedef void __attribute__((address_space(3))) *lds_void_ptr;
+typedef const int __attribute__((address_space(1))) *global_i32_ptr;
+typedef float __attribute__((address_space(1))) *global_f32_out;
 
-constexpr int TM = MFMA_TM;                 // tokens per workgroup; weight rows per workgroup: 64 * NBW
-constexpr int X_PITCH = 144;               // bytes per staged token row of one plane: 64 halves + 16 pad
-constexpr int W_PITCH = 36;                // bytes per staged weight row of one group: 32 + 4 pad
-constexpr int XS_BYTES = X_PLANES * TM * X_PITCH;
-constexpr int G_PITCH = 48;                // bias pass: bytes per staged row of 16 bf16: 32 + 16 pad
-constexpr int XG_BYTES = 3 * TM * G_PITCH;
+constexpr int TM = MFMA_TM;                 // tokens per workgroup
+constexpr int X_PLANES = 2;                 // fp16 planes of the scaled activation
+constexpr int WINDOW = 28;                  // binades of scale that are exact fp16 operands at a time
+constexpr int MAX_WINDOWS = 10;             // all of a bf16's binades
+constexpr int WEIGHT_TOP = 11;              // scales are brought below 2^WEIGHT_TOP: 24 * 2^11 is inside fp16
 
-// LDS layout of one stage for a tile of TN weight rows
-template <int TN> struct Stage {
-    static constexpr int WS_OFF = XS_BYTES;                        // codes [TN][W_PITCH]
-    static constexpr int SC_OFF = WS_OFF + TN * W_PITCH;           // float scale[TN]
-    static constexpr int BYTES = (SC_OFF + TN * 4 + 15) & ~15;
-    static_assert(XG_BYTES + 2 * TN * G_PITCH <= 2 * BYTES, "the bias pass reuses the staging memory");
+// A row of the third plane holds what the split has to say about its row of x: at byte 0 the exponent k of the power
+// of two 2^-k that undoes its scaling, from byte 16 on the group sums as three bf16 planes of padded_groups() entries.
+// The bias pass reads scales, biases and sums eight groups at a time, the last eight of a row from its end backwards,
+// so that it never reads past the row: entry j of eight c stands for group eight_start(c) + j, and is zero where an
+// earlier eight already holds that group.  16 + 6 * padded_groups(C / 64) bytes fit the 2 * C of the row for every C.
+__host__ __device__ constexpr int padded_groups(int ngrp) { return (ngrp + 15) & ~15; }
+__device__ __forceinline__ int eight_start(int c, int ngrp) {
+    const int last = ngrp > 8 ? ngrp - 8 : 0;
+    return 8 * c < last ? 8 * c : last;
+}
+
+// KP parts of the columns per workgroup: the tile is 64 tokens x 256 / KP rows.  LDS holds two stages of the token
+// planes, one scale group of each part, and for every wave one chunk, CH groups, of the codes and the scale bits of its
+// own 64 rows: 128 bytes of a row at a time, because a cache line that is fetched again for each of its quarters
+// costs as much as four lines.
+template <int KP> struct Shape {
+    static constexpr int ROW_WAVES = 4 / KP;
+    static constexpr int TN = 64 * ROW_WAVES;
+    static constexpr int CH = KP == 4 ? 2 : 4;
+    static constexpr int X_BYTES = X_PLANES * TM * 128;              // of one part
+    static constexpr int STAGE_BYTES = KP * X_BYTES;
+    static constexpr int W_OFF = 2 * STAGE_BYTES, W_BYTES = 64 * 32 * CH;        // of one wave
+    static constexpr int S_OFF = W_OFF + 4 * W_BYTES, S_BYTES = 64 * 4 * CH;
+    static constexpr int LDS_BYTES = S_OFF + 4 * S_BYTES;
+    static constexpr int XT = TM / (8 * ROW_WAVES);                  // loads per wave and plane: eight token rows each
+    static constexpr int PIECES = 2 * CH;                            // 16-byte pieces of a row's chunk
+    static constexpr int WT = PIECES;                                // loads per wave and chunk: 64 / PIECES rows each
+    static_assert((KP - 1) * ROW_WAVES * 64 * 64 * 4 <= 2 * STAGE_BYTES, "the parts' sums reuse the staging memory");
 };
 
-static_assert(sizeof(MfmaJob) == 64, "find_job reads a job record as eight 64-bit words");
+// Planes arrive in LDS by loads that write 64 consecutive 16-byte pieces, so rows cannot be padded: piece p of token
+// row r lies at place p ^ place_mask(r), which spreads the sixteen rows of an LDS read phase over all banks.  The
+// same for the codes; chunks of four pieces per row have four rows to a turn of the banks instead of two.
+template <int PIECES> __device__ __forceinline__ int place_mask(int row) {
+    return PIECES == 8 ? (row >> 1) & 7 : (row >> 2) & 3;
+}
+
+template <int N> __device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+static_assert(sizeof(MfmaJob) == 56, "find_job reads a job record as seven 64-bit words");
 
 __device__ __forceinline__ MfmaJob find_job(const MfmaLaunch &L, int tile) {
     if (L.table == nullptr) return L.one;
@@ -76,46 +136,32 @@ __device__ __forceinline__ MfmaJob find_job(const MfmaLaunch &L, int tile) {
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if ((int)(uint32_t)words[8 * mid + 7] <= tile) lo = mid; else hi = mid - 1;
+        if ((int)(uint32_t)words[7 * mid + 6] <= tile) lo = mid; else hi = mid - 1;
     }
-    const uniform_u64_ptr rec = words + 8 * lo;
+    const uniform_u64_ptr rec = words + 7 * lo;
     MfmaJob job;
     job.vals = (const uint8_t *)rec[0];
     job.scales = (const uint8_t *)rec[1];
     job.biases = (const uint8_t *)rec[2];
     job.planes = (const uint16_t *)rec[3];
-    job.xsum = (const float *)rec[4];
-    job.y = (float *)rec[5];
-    job.tokens = (int)(uint32_t)rec[6];
-    job.rows = (int)(rec[6] >> 32);
-    job.tile0 = (int)(uint32_t)rec[7];
-    job.row_base = (int)(rec[7] >> 32);
+    job.y = (float *)rec[4];
+    job.tokens = (int)(uint32_t)rec[5];
+    job.rows = (int)(rec[5] >> 32);
+    job.tile0 = (int)(uint32_t)rec[6];
+    job.row_base = (int)(rec[6] >> 32);
     return job;
 }
 
 __device__ __forceinline__ float bf16_to_f32(uint32_t half) { return __uint_as_float(half << 16); }
 
-// Eight nibbles -> eight fp16 values 16 + q, in the column order 0,4,1,5,2,6,3,7.
-// (a & mask) | bits in one instruction; the three-operand form takes no
-// literals, so the mask travels in a scalar register and the bits in a vector one.
-__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t bits) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(bits));
-    return r;
-}
-
-__device__ __forceinline__ f16x8 codes_to_f16(uint32_t w, uint32_t mask, uint32_t sixteen) {
-    u32x4 r;                                             // a code's four bits land on mantissa bits 6..9 of 16.0
-    r.x = and_or((w << 6), mask, sixteen);               // columns 0 and 4
-    r.y = and_or((w << 2), mask, sixteen);               // 1 and 5
-    r.z = and_or((w >> 2), mask, sixteen);               // 2 and 6
-    r.w = and_or((w >> 6), mask, sixteen);               // 3 and 7
+// Eight nibbles -> eight fp16 values s (q - 8), in the column order 0,4,1,5,2,6,3,7.  A code's four bits land on
+// mantissa bits 6..9 of 16.0, which makes 16 + q; `less` is -24 s.
+__device__ __forceinline__ f16x8 weights_to_f16(uint32_t w, uint32_t mask, uint32_t sixteen, f16x2 s, f16x2 less) {
+    auto pair = [&](uint32_t shifted) {
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, (shifted & mask) | sixteen), s, less));
+    };
+    const u32x4 r = {pair(w << 6), pair(w << 2), pair(w >> 2), pair(w >> 6)};
     return __builtin_bit_cast(f16x8, r);
-}
-
-// 2^-k <-> 2^k for a float that is a power of two (normal range)
-__device__ __forceinline__ float reciprocal_power_of_two(float p) {
-    return __uint_as_float((254u - ((__float_as_uint(p) >> 23) & 0xffu)) << 23);
 }
 
 __device__ __forceinline__ uint32_t f32_to_bf16_rne(float v) {
@@ -132,292 +178,484 @@ __device__ __forceinline__ void split3(float v, uint32_t &h, uint32_t &m, uint32
     l = f32_to_bf16_rne(r2);
 }
 
-// One scale group of one wave: NB blocks of 32 rows against the wave's 32 tokens.
-template <int NB, int NBW>
-__device__ __forceinline__ void group_product(const uint8_t *cur, int wm, int wn, int l32, int half,
-                                              f32x16 (&acc)[NBW]) {
-    using S = Stage<64 * NBW>;
-    const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    uint32_t sixteen;                                   // two fp16 values 16.0, kept in a vector register
-    asm("v_mov_b32 %0, 0x4C004C00" : "=v"(sixteen));
-    const uint8_t *wrow = cur + S::WS_OFF + (wn * 32 * NBW + l32) * W_PITCH + half * 4;
-    const uint8_t *xrow = cur + (wm * 32 + l32) * X_PITCH + half * 16;
-    const float *sc = reinterpret_cast<const float *>(cur + S::SC_OFF) + wn * 32 * NBW + l32;
-    // The token operand of the whole group stays in registers; the row blocks
-    // then run two at a time so that only two partial products are live.
-    f16x8 a[4][X_PLANES];
+// The first eight bf16 of a row of fewer than eight, zeros past its end.
+__device__ __forceinline__ u32x4 load_short(global_u16_ptr row, int ngrp) {
+    u32x4 v = {0, 0, 0, 0};
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-        for (int plane = 0; plane < X_PLANES; ++plane)
-            a[ks][plane] = __builtin_bit_cast(
-                f16x8, *reinterpret_cast<const u32x4 *>(xrow + plane * (TM * X_PITCH) + ks * 32));
-#pragma unroll
-    for (int nb0 = 0; nb0 < NB; nb0 += 2) {
-        constexpr int PAIR_MAX = 2;
-        const int pair = NB - nb0 < PAIR_MAX ? NB - nb0 : PAIR_MAX;
-        f32x16 part[PAIR_MAX];
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            f16x8 b[PAIR_MAX];
-#pragma unroll
-            for (int k = 0; k < PAIR_MAX; ++k)
-                if (k < pair)
-                    b[k] = codes_to_f16(*reinterpret_cast<const uint32_t *>(wrow + (nb0 + k) * 32 * W_PITCH + ks * 8),
-                                        0x03C003C0u, sixteen);
-#pragma unroll
-            for (int plane = 0; plane < X_PLANES; ++plane)
-#pragma unroll
-                for (int k = 0; k < PAIR_MAX; ++k)
-                    if (k < pair)
-                        part[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks][plane], b[k],
-                                                                         (ks | plane) ? part[k] : zero, 0, 0, 0);
-        }
-#pragma unroll
-        for (int k = 0; k < PAIR_MAX; ++k)
-            if (k < pair) {
-                const float s = sc[(nb0 + k) * 32];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) acc[nb0 + k][i] = __builtin_fmaf(s, part[k][i], acc[nb0 + k][i]);
-            }
-    }
+    for (int j = 0; j < 8; ++j)
+        if (j < ngrp) v[j >> 1] |= (uint32_t)row[j] << (16 * (j & 1));
+    return v;
 }
 
-// NBW = 32-row blocks per wave: the workgroup's tile is 64 tokens x 64 * NBW rows.
-template <int NBW>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t pk_less_one(uint32_t a) {            // zeros wrap to 0xffff
+    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) - (u16x2){1, 1}));
+}
+
+// The codes and the scale bits of a lane's two rows for one chunk of scale groups.
+template <int CH> struct Weights { u32x4 w[CH][2]; uint32_t s[CH][2]; };
+
+template <int KP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KP == 1 ? 2 : 1), amdgpu_num_vgpr(256)))
 void q4_mfma_kernel(const MfmaLaunch L) {
-    constexpr int TN = 64 * NBW;
-    using S = Stage<TN>;
-    constexpr int STAGE_BYTES = S::BYTES;
-    // two stages of { planes [2][64 tokens], codes [TN rows], scales [TN] }
-    __shared__ __attribute__((aligned(16))) uint8_t stage[2 * STAGE_BYTES];
+    using S = Shape<KP>;
+    __shared__ __attribute__((aligned(16))) uint8_t stage[S::LDS_BYTES];
+    __shared__ int s_down[TM];                     // per token: exponent of the power of two that undoes the split's scaling
+    __shared__ int s_windows[4];
+    __shared__ uint32_t s_row[TM];                 // per token: its row of the planes
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;       // wave tile: tokens wm*32.., rows wn*32*NBW.. (NBW 32-row blocks)
+    const int part = wave / S::ROW_WAVES, wn = wave % S::ROW_WAVES;
     const int l32 = lane & 31, half = lane >> 5;
 
-    if (L.total_tiles_dev &&
-        (int)blockIdx.x >= *(const int __attribute__((address_space(4))) *)(uintptr_t)L.total_tiles_dev)
-        return;                                     // uniform: the whole workgroup leaves
-    const MfmaJob job = find_job(L, blockIdx.x);
+    // Workgroups go round the eight partitions of the device in turn; a partition takes one run of consecutive tiles,
+    // so that the tiles of one weight matrix, or of one expert, meet in one partition's cache.
+    const int total = L.total_tiles_dev ? *(const int __attribute__((address_space(4))) *)(uintptr_t)L.total_tiles_dev
+                                        : L.total_tiles;
+    const int run = (total + 7) >> 3;
+    const int tile = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= run || tile >= total) return;      // uniform: the whole workgroup leaves
+    const MfmaJob job = find_job(L, tile);
     const int C = L.cols, ngrp = C >> 6;
-    const int ntiles = (job.rows + TN - 1) / TN;
-    const int t = blockIdx.x - job.tile0;
-    const int tok0 = (t / ntiles) * TM, row0 = (t % ntiles) * TN;
-    const int toks_here = job.tokens - tok0 < TM ? job.tokens - tok0 : TM;
-    const int rows_here = job.rows - row0 < TN ? job.rows - row0 : TN;
+    const int tm = L.tile_tokens;                   // TM, or half of it
+    const int mtiles = (job.tokens + tm - 1) / tm;
+    const int t = tile - job.tile0;
+    const int tok0 = (t % mtiles) * tm, row0 = (t / mtiles) * S::TN + wn * 64;
+    const int toks_here = job.tokens - tok0 < tm ? job.tokens - tok0 : tm;
+    const bool wide = toks_here > 32;               // both token blocks hold tokens
+    const bool live = row0 < job.rows;              // this wave has rows; the others only help to stage
 
     // Token t of the job is row (tok0 + t) of the planes, or, with a map, row
-    // row_map[row_base + tok0 + t] / map_divisor (the grouped MoE gather).
-    const int *row_map = L.row_map;
-    auto source_row = [&](int tok) -> uint32_t {
-        const int tc = tok < toks_here ? tok : toks_here - 1;
-        return row_map ? (uint32_t)(row_map[job.row_base + tok0 + tc] / L.map_divisor) : (uint32_t)(tok0 + tc);
-    };
-
-    // staging geometry of this thread
-    // planes: 2 * 64 tokens * 8 segments of 16 bytes = 1024 pieces, 4 per thread
-    constexpr int XP = X_PLANES * TM * 8 / 256;
-    const global_u16_ptr planes = (global_u16_ptr)(uintptr_t)job.planes;
-    uint32_t x_src[XP], x_dst[XP];                  // element offsets: the planes of one launch stay below 2^32 elements
-#pragma unroll
-    for (int i = 0; i < XP; ++i) {
-        const int p = tid + i * 256;
-        const int plane = p >> 9, tok = (p >> 3) & 63, seg = p & 7;
-        x_src[i] = (uint32_t)plane * (uint32_t)L.plane_stride + source_row(tok) * (uint32_t)C + seg * 8;
-        x_dst[i] = plane * (TM * X_PITCH) + tok * X_PITCH + seg * 16;
+    // row_map[row_base + tok0 + t] / map_divisor (the grouped MoE gather); tokens past the end repeat the last one.
+    if (tid < TM) {
+        const int tc = tid < toks_here ? tid : toks_here - 1;
+        s_row[tid] = L.row_map ? (uint32_t)(L.row_map[job.row_base + tok0 + tc] / L.map_divisor) : (uint32_t)(tok0 + tc);
     }
-    // codes: TN rows * 2 pieces of 16 bytes, NBW / 2 per thread
-    constexpr int WP = NBW / 2;
-    const int w_half = tid & 1;
-    global_u128_ptr w_src[WP];
-    uint32_t w_dst[WP];
-#pragma unroll
-    for (int i = 0; i < WP; ++i) {
-        const int row = (tid >> 1) + i * 128;
-        const int rc = row < rows_here ? row : rows_here - 1;
-        w_src[i] = (global_u128_ptr)((uintptr_t)job.vals + (size_t)(row0 + rc) * (C >> 1) + w_half * 16);
-        w_dst[i] = S::WS_OFF + row * W_PITCH + w_half * 16;
-    }
-    // scales: threads 0..TN-1
-    const int m_row = tid & (TN - 1);
-    const int m_rc = m_row < rows_here ? m_row : rows_here - 1;
-    const global_u16_ptr scales = (global_u16_ptr)(uintptr_t)job.scales + (size_t)(row0 + m_rc) * ngrp;
+    __syncthreads();
+    const global_u8_ptr plane0 = (global_u8_ptr)(uintptr_t)job.planes;
+    const global_u8_ptr plane1 = plane0 + 2 * L.plane_stride, notes = plane0 + 4 * L.plane_stride;
 
-    // Loads travel through registers; two sets are in flight so that a load has
-    // two groups of matrix work (of both workgroups on the compute unit) to land.
-    struct Loads { u32x4 x[XP], w[WP]; uint32_t s; };
-    auto issue = [&](int g, Loads &r) {
+    // The part's columns: `iterations` groups from g_first on, those from g_end on staged from inside the row and
+    // unused.  Whole chunks, for the sake of whole cache lines, where that leaves the parts about equal.
+    const int even = (ngrp + KP - 1) / KP;
+    const int per_part = even >= 4 * S::CH ? (even + S::CH - 1) / S::CH * S::CH : even;
+    const int iterations = per_part < ngrp ? per_part : ngrp;
+    const int g_first = part * per_part;
+    const int g_end = g_first + per_part < ngrp ? g_first + per_part : ngrp;
+
+    // Staging geometry of this lane: load i of a wave brings the eight token rows from (i * ROW_WAVES + wn) * 8 on;
+    // which piece of its row a lane fetches follows from the place that the load will put it in.
+    uint32_t x_src[S::XT];                          // byte offsets below 2^32
 #pragma unroll
-        for (int i = 0; i < XP; ++i) r.x[i] = *(global_u128_ptr)(planes + x_src[i] + (uint32_t)g * 64u);
+    for (int i = 0; i < S::XT; ++i) {
+        const int r = (i * S::ROW_WAVES + wn) * 8 + (lane >> 3);
+        const int piece = (lane & 7) ^ place_mask<8>(r);
+        x_src[i] = s_row[r] * (uint32_t)(2 * C) + (uint32_t)piece * 16u;
+    }
+
+    // rows of this lane, clamped to the matrix
+    uint32_t row[2];
+    global_u16_ptr scales[2];
 #pragma unroll
-        for (int i = 0; i < WP; ++i) r.w[i] = w_src[i][g * 2];
-        if (tid < TN) r.s = scales[g];
-    };
-    auto commit = [&](uint8_t *base, const Loads &r) {
+    for (int nb = 0; nb < 2; ++nb) {
+        const int r = row0 + nb * 32 + l32;
+        row[nb] = (uint32_t)(r < job.rows ? r : job.rows - 1);
+        scales[nb] = (global_u16_ptr)(uintptr_t)job.scales + (size_t)row[nb] * (size_t)ngrp;
+    }
+    // codes of the wave's rows: load j of a chunk brings rows j * 64 / PIECES .., clamped to the matrix
+    const int rows_left = live ? job.rows - row0 : 1;
+    const int row_base = live ? row0 : 0;           // waves without rows fetch the first row and use nothing
+    const global_u8_ptr codes = (global_u8_ptr)(uintptr_t)job.vals + (size_t)row_base * (size_t)(C >> 1);
+    const global_u8_ptr scale_rows = (global_u8_ptr)(uintptr_t)job.scales + (size_t)row_base * (size_t)(2 * ngrp);
+
+    // Everything staged goes from memory into LDS without passing through registers, so that a wave's loads complete
+    // in the order they were sent in and a wait can leave the younger ones in flight.
+    auto issue_x = [&](int it) {
+        const int g = g_first + it < ngrp ? g_first + it : ngrp - 1;
+        uint8_t *const x = stage + (it & 1) * S::STAGE_BYTES + part * S::X_BYTES + wn * 1024;
+        uint32_t at = (uint32_t)g * 128u;
+        asm volatile("" : "+s"(at));                 // addresses are made here, not kept in registers through the loops
 #pragma unroll
-        for (int i = 0; i < XP; ++i) *reinterpret_cast<u32x4 *>(base + x_dst[i]) = r.x[i];
-#pragma unroll
-        for (int i = 0; i < WP; ++i) {
-            uint32_t *dst = reinterpret_cast<uint32_t *>(base + w_dst[i]);
-            dst[0] = r.w[i].x; dst[1] = r.w[i].y; dst[2] = r.w[i].z; dst[3] = r.w[i].w;
+        for (int i = 0; i < S::XT; ++i) {
+            if (i * S::ROW_WAVES * 8 >= 32 && !wide) break;
+            uint8_t *const to = x + i * (S::ROW_WAVES * 1024);
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(plane0 + (x_src[i] + at)), (lds_void_ptr)to, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(plane1 + (x_src[i] + at)), (lds_void_ptr)(to + TM * 128),
+                                             16, 0, 0);
         }
-        if (tid < TN) reinterpret_cast<float *>(base + S::SC_OFF)[m_row] = bf16_to_f32(r.s);
+    };
+    constexpr int CHUNK_LOADS = S::WT + S::CH;
+    auto issue_weights = [&](int it) {               // the chunk that starts with group `it` of the part
+        const uint32_t at = (uint32_t)(g_first + it) * 32u, last = (uint32_t)ngrp * 32u - 16u;
+        uint32_t lane_row = (uint32_t)lane / S::PIECES;
+        uint32_t scale_at = (uint32_t)(lane < rows_left ? lane : rows_left - 1) * (uint32_t)(2 * ngrp);
+        asm volatile("" : "+v"(lane_row), "+v"(scale_at));
+#pragma unroll
+        for (int j = 0; j < S::WT; ++j) {
+            uint32_t r = j * (64 / S::PIECES) + lane_row;
+            const uint32_t piece = ((uint32_t)lane & (S::PIECES - 1)) ^ (uint32_t)place_mask<S::PIECES>((int)r);
+            uint32_t byte = at + piece * 16u;
+            byte = byte < last ? byte : last;
+            r = r < (uint32_t)rows_left ? r : (uint32_t)rows_left - 1u;
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(codes + (__umul24(r, (uint32_t)(C >> 1)) + byte)),
+                                             (lds_void_ptr)(stage + S::W_OFF + wave * S::W_BYTES + j * 1024), 16, 0, 0);
+        }
+#pragma unroll
+        for (int gi = 0; gi < S::CH; ++gi) {
+            const int g = g_first + it + gi;
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(scale_rows + (scale_at + 2u * (uint32_t)(g < ngrp ? g : ngrp - 1))),
+                                             (lds_void_ptr)(stage + S::S_OFF + wave * S::S_BYTES + gi * 256), 2, 0, 0);
+        }
+    };
+    typedef const u32x4 __attribute__((address_space(3))) *lds_u128_ptr;
+    typedef const uint32_t __attribute__((address_space(3))) *lds_u32_ptr;
+    auto take_weights = [&](Weights<S::CH> &r) {     // and leave their place to the next chunk
+        const lds_u128_ptr w = (lds_u128_ptr)(stage + S::W_OFF + wave * S::W_BYTES);
+        const lds_u32_ptr sc = (lds_u32_ptr)(stage + S::S_OFF + wave * S::S_BYTES);
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+            const int at = (nb * 32 + l32) * S::PIECES, turn = place_mask<S::PIECES>(nb * 32 + l32);
+#pragma unroll
+            for (int gi = 0; gi < S::CH; ++gi) {
+                r.w[gi][nb] = w[at + ((gi * 2 + half) ^ turn)];
+                r.s[gi][nb] = sc[gi * 64 + nb * 32 + l32];
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
 
-    const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    f32x16 acc[NBW];
-#pragma unroll
-    for (int nb = 0; nb < NBW; ++nb) acc[nb] = zero;
+    issue_weights(0);
+    issue_x(0);
+    if (tid < TM) s_down[tid] = *(global_i32_ptr)(notes + (size_t)s_row[tid] * (size_t)(2 * C));
 
-    // ---- bias pass: acc[tok][row] = sum_g (b[row][g] - 16 s[row][g]) * X[tok][g]
-    {
-        const global_f32_ptr xsum = (global_f32_ptr)(uintptr_t)job.xsum;
-        const int xg_tok = tid >> 2, xg_g = (tid & 3) * 4;
-        const size_t xg_row = (size_t)source_row(xg_tok) * ngrp;
-        const global_u16_ptr all_scales = (global_u16_ptr)(uintptr_t)job.scales;
-        const global_u16_ptr all_biases = (global_u16_ptr)(uintptr_t)job.biases;
-        // Two 32-row blocks per pass keep the four partial products in registers.
-#pragma unroll 1
-        for (int pass = 0; pass < NBW / 2; ++pass) {
-            f32x16 tb[2] = {zero, zero}, ts[2] = {zero, zero};
-            for (int g0 = 0; g0 < ngrp; g0 += 16) {
-                uint32_t h[4], m[4], l[4];
+    // ---- bias term of the tile, acc[tok][row] = sum_g (b[row][g] + 8 s[row][g]) * X[tok][g], and the rows' exponents
+    const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    f32x16 acc[2][2] = {{zero, zero}, {zero, zero}};
+    int top[2] = {0, 0};                            // row block nb: the scales of this lane's row are below 2^top[nb]
+    int windows = 1;
+    if (live) {
+        const int padded = padded_groups(ngrp);
+        global_u8_ptr sums[2];
+        global_u16_ptr biases[2];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int g = g0 + xg_g + j;
-                    const float v = g < ngrp ? xsum[xg_row + g] : 0.0f;
-                    split3(v, h[j], m[j], l[j]);
+        for (int k = 0; k < 2; ++k) {
+            sums[k] = notes + (size_t)s_row[k * 32 + l32] * (size_t)(2 * C) + 16 + half * 16;
+            biases[k] = (global_u16_ptr)(uintptr_t)(job.biases ? job.biases : job.scales) + (size_t)row[k] * (size_t)ngrp;
+        }
+        struct Eights { u32x4 s[2], b[2]; };
+        const uint32_t keep = job.biases ? 0xffffffffu : 0u;        // without biases the scales stand in, masked
+        auto fetch = [&](int g0, bool whole, Eights &e) {           // sixteen groups, eight per lane half
+            const int first = eight_start((g0 >> 3) + half, ngrp);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                if (whole) {
+                    e.s[k] = *(global_u128_any_ptr)(scales[k] + first);
+                    e.b[k] = *(global_u128_any_ptr)(biases[k] + first);
+                } else {
+                    e.s[k] = load_short(scales[k], ngrp);
+                    e.b[k] = load_short(biases[k], ngrp);
                 }
-                __syncthreads();                                // the previous step's operands have been read
-                uint8_t *xgp = stage + xg_tok * G_PITCH + xg_g * 2;
-                *reinterpret_cast<uint2 *>(xgp) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
-                *reinterpret_cast<uint2 *>(xgp + TM * G_PITCH) = make_uint2(m[0] | m[1] << 16, m[2] | m[3] << 16);
-                *reinterpret_cast<uint2 *>(xgp + 2 * TM * G_PITCH) = make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16);
-                // (bias, scale) bits of 16 groups for every row of the tile: item = array * TN + row
-                for (int item = tid; item < 2 * TN; item += 256) {
-                    const int arr = item / TN, row = item % TN;
-                    const int rc = row < rows_here ? row : rows_here - 1;
-                    const global_u16_ptr src = (arr ? all_scales : all_biases) + (size_t)(row0 + rc) * ngrp;
-                    const bool present = arr || job.biases;
-                    uint32_t *bsp = reinterpret_cast<uint32_t *>(stage + XG_BYTES + item * G_PITCH);
+            }
+        };
+        f32x16 tb[2][2] = {{zero, zero}, {zero, zero}}, ts[2][2] = {{zero, zero}, {zero, zero}};
+        uint32_t s_max[2] = {0, 0}, b_max[2] = {0, 0}, s_min[2] = {0xffffffffu, 0xffffffffu};
+        Eights e;
+        if (ngrp >= 8) fetch(0, true, e); else fetch(0, false, e);
+        for (int g0 = 0; g0 < ngrp; g0 += 16) {
+            Eights c = e;
+            u32x4 x[3][2];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int g = g0 + 2 * j;
-                        const uint32_t lo = (present && g < ngrp) ? (uint32_t)src[g] : 0u;
-                        const uint32_t hi = (present && g + 1 < ngrp) ? (uint32_t)src[g + 1] : 0u;
-                        bsp[j] = lo | hi << 16;
-                    }
-                }
-                __syncthreads();
-                {
-                    const uint8_t *arow = stage + (wm * 32 + l32) * G_PITCH + half * 16;
-                    const uint8_t *brow = stage + XG_BYTES + (wn * 32 * NBW + pass * 64 + l32) * G_PITCH + half * 16;
+            for (int plane = 0; plane < 3; ++plane)
 #pragma unroll
-                    for (int plane = 0; plane < 3; ++plane) {
-                        const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(arow + plane * TM * G_PITCH));
+                for (int mb = 0; mb < 2; ++mb) x[plane][mb] = *(global_u128_ptr)(sums[mb] + (plane * padded + g0) * 2);
+            if (g0 + 16 < ngrp) fetch(g0 + 16, true, e);
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) c.b[nb][j] &= keep;
+            if (KP == 1 || part == 0) {
+#pragma unroll
+                for (int plane = 0; plane < 3; ++plane)
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
                         for (int nb = 0; nb < 2; ++nb) {
-                            const bf16x8 bb = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(brow + nb * 32 * G_PITCH));
-                            const bf16x8 sb = __builtin_bit_cast(
-                                bf16x8, *reinterpret_cast<const u32x4 *>(brow + (TN + nb * 32) * G_PITCH));
-                            tb[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bb, tb[nb], 0, 0, 0);
-                            ts[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, sb, ts[nb], 0, 0, 0);
+                            const bf16x8 a = __builtin_bit_cast(bf16x8, x[plane][mb]);
+                            tb[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, c.b[nb]),
+                                                                                 tb[mb][nb], 0, 0, 0);
+                            ts[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, c.s[nb]),
+                                                                                 ts[mb][nb], 0, 0, 0);
                         }
-                    }
-                }
             }
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const float v = __builtin_fmaf(-16.0f, ts[nb][i], tb[nb][i]);
-                    if (NBW == 2 || pass == 0) acc[nb][i] = v; else acc[(NBW > 2 ? 2 : 0) + nb][i] = v;
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t sa = c.s[nb][j] & 0x7fff7fffu;
+                    s_max[nb] = pk_max(s_max[nb], sa);
+                    s_min[nb] = pk_min(s_min[nb], pk_less_one(sa));
+                    b_max[nb] = pk_max(b_max[nb], c.b[nb][j] & 0x7fff7fffu);
                 }
         }
-        __syncthreads();
-    }
-
-    // The main loop works on x * 2^k (k per token, chosen by the split): the bias term joins it at that scale and
-    // the power of two leaves at the store.  A token's 2^-k lies at the head of its row of the third plane.
-    auto token_scale = [&](int i) -> float {
-        const int tok = wm * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-        return *(const float __attribute__((address_space(1))) *)(uintptr_t)(
-            job.planes + 2 * (size_t)L.plane_stride + (size_t)source_row(tok) * (size_t)C);
-    };
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const float up = reciprocal_power_of_two(token_scale(i));
+        for (int nb = 0; nb < 2; ++nb) {
+            const uint32_t s2 = pk_max(s_max[nb], (uint32_t)__shfl_xor((int)s_max[nb], 32, 64));
+            const uint32_t b2 = pk_max(b_max[nb], (uint32_t)__shfl_xor((int)b_max[nb], 32, 64));
+            const uint32_t m2 = pk_min(s_min[nb], (uint32_t)__shfl_xor((int)s_min[nb], 32, 64));
+            const uint32_t sm = (s2 & 0xffffu) > (s2 >> 16) ? (s2 & 0xffffu) : (s2 >> 16);
+            const uint32_t bm = (b2 & 0xffffu) > (b2 >> 16) ? (b2 & 0xffffu) : (b2 >> 16);
+            const uint32_t lowest = ((m2 & 0xffffu) < (m2 >> 16) ? (m2 & 0xffffu) : (m2 >> 16)) + 1u;
+            const float big_s = bf16_to_f32(sm), big_b = bf16_to_f32(bm) * 0.125f;
+            top[nb] = __builtin_amdgcn_frexp_expf(big_s > big_b ? big_s : big_b);      // 0 for 0, infinities and NaN
+            if (lowest <= 0x7f7fu) {
+                const int span = top[nb] - __builtin_amdgcn_frexp_expf(bf16_to_f32(lowest));
+                const int need = span < 0 ? 1 : span / WINDOW + 1;
+                windows = need > windows ? need : windows;
+            }
 #pragma unroll
-        for (int nb = 0; nb < NBW; ++nb) acc[nb][i] = acc[nb][i] * up;
-    }
-
-    // ---- main loop: acc += s[row][g] * sum_{c in g} (16 + q[row][c]) * x[tok][c] * 2^k
-    // Row blocks past the end of the matrix are computed on clamped rows and
-    // dropped at the store: one instantiation of the loop keeps the
-    // accumulators in place and the register count inside the budget.
-    {
-        Loads even, odd;
-        even.s = 0; odd.s = 0;
-        uint8_t *stage0 = stage, *stage1 = stage + STAGE_BYTES;
-        issue(0, even);
-        if (ngrp > 1) issue(1, odd);
-        commit(stage0, even);
-        __syncthreads();
-        for (int g = 0; g < ngrp; g += 2) {
-            if (g + 2 < ngrp) issue(g + 2, even);
-            group_product<NBW, NBW>(stage0, wm, wn, l32, half, acc);
-            if (g + 1 < ngrp) commit(stage1, odd);
-            __syncthreads();
-            if (g + 1 >= ngrp) break;
-            if (g + 3 < ngrp) issue(g + 3, odd);
-            group_product<NBW, NBW>(stage1, wm, wn, l32, half, acc);
-            if (g + 2 < ngrp) commit(stage0, even);
-            __syncthreads();
+            for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[mb][nb][i] = __builtin_fmaf(8.0f, ts[mb][nb][i], tb[mb][nb][i]);
         }
-    }
-
-    float __attribute__((address_space(1))) *y = (float __attribute__((address_space(1))) *)(uintptr_t)job.y;
-    float down[16];
+        windows = windows > MAX_WINDOWS ? MAX_WINDOWS : windows;
+        if (__ballot(windows > 1)) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) down[i] = token_scale(i);
-#pragma unroll
-    for (int nb = 0; nb < NBW; ++nb) {
-        const int row = wn * 32 * NBW + nb * 32 + l32;
-        if (row < rows_here) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int tok = wm * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                if (tok < toks_here) y[(size_t)(tok0 + tok) * job.rows + row0 + row] = acc[nb][i] * down[i];
+            for (int d = 1; d < 64; d <<= 1) {
+                const int other = __shfl_xor(windows, d, 64);
+                windows = windows > other ? windows : other;
             }
         }
+    }
+    if (lane == 0) s_windows[wave] = windows;
+    wait_loads<0>();
+    __syncthreads();                                // the first stage and chunk are there as well
+    windows = s_windows[0];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) windows = windows > s_windows[w] ? windows : s_windows[w];
+    windows = __builtin_amdgcn_readfirstlane(windows);
+    // the main loop works on s 2^(11 - top) and x 2^-down: the bias term joins it at that scale
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int down = s_down[mb * 32 + (i >> 2) * 8 + half * 4 + (i & 3)];
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+                acc[mb][nb][i] = __builtin_amdgcn_ldexpf(acc[mb][nb][i], WEIGHT_TOP - top[nb] - down);
+        }
+
+    const int mix = place_mask<8>(l32);             // rows 32 apart share it
+    uint32_t code_mask, sixteen;                    // opaque, so that (w & mask) | 16.0 stays one instruction
+    asm("s_mov_b32 %0, 0x03C003C0" : "=s"(code_mask));
+    asm("v_mov_b32 %0, 0x4C004C00" : "=v"(sixteen));
+    int raise[2];                                   // row block nb: the power of two that its scales are brought up by
+
+    // The wave's walk over its part's columns for MB blocks of 32 tokens, in steps of 16 columns: while the matrix
+    // cores work on a step, the operands of the next one are read and converted (left to itself the compiler reads
+    // a whole group ahead and spills).  The workgroup meets before the last step of a group: its planes are then in
+    // everybody's registers, so their place takes the group after the next one.
+    auto walk = [&](auto blocks) {
+        constexpr int MB = decltype(blocks)::value;
+        constexpr int LAST = S::CH - 1;
+        Weights<S::CH> now;
+        f16x8 a[2][MB][X_PLANES], b[2][2];
+        f16x2 s[2], less[2], s_next[2], less_next[2];
+        auto read = [&](int it, int step, f16x8 (&to)[MB][X_PLANES]) {
+            const lds_u128_ptr x = (lds_u128_ptr)(stage + (it & 1) * S::STAGE_BYTES + part * S::X_BYTES + l32 * 128);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int plane = 0; plane < X_PLANES; ++plane)
+                    to[mb][plane] = __builtin_bit_cast(
+                        f16x8, x[plane * (TM * 8) + mb * (32 * 8) + ((half * 4 + step) ^ mix)]);
+        };
+        // Scales that the window does not bring into the WINDOW binades below 2^WEIGHT_TOP count as zero, and so do
+        // groups past the part's end.
+        auto scale = [&](const uint32_t (&bits)[2], bool inside, f16x2 (&s)[2], f16x2 (&less)[2]) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                const float value = bf16_to_f32(inside ? bits[nb] : 0u);
+                const int place = __builtin_amdgcn_frexp_expf(value) + raise[nb];  // at most WEIGHT_TOP in this window
+                float raised = __builtin_amdgcn_ldexpf(value, raise[nb]);
+                const bool finite = __builtin_fabsf(value) < __builtin_inff();
+                if (finite && (unsigned)(WEIGHT_TOP - place) >= (unsigned)WINDOW) raised = 0.0f;
+                const _Float16 h = (_Float16)raised;
+                const _Float16 l = (_Float16)-24.0f * h;
+                s[nb] = f16x2{h, h};
+                less[nb] = f16x2{l, l};
+            }
+        };
+        auto convert = [&](const u32x4 (&w)[2], int step, f16x8 (&to)[2]) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) to[nb] = weights_to_f16(w[nb][step], code_mask, sixteen, s[nb], less[nb]);
+        };
+        auto multiply = [&](const f16x8 (&x)[MB][X_PLANES], const f16x8 (&w)[2]) {
+#pragma unroll
+            for (int plane = 0; plane < X_PLANES; ++plane)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int nb = 0; nb < 2; ++nb)
+                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[mb][plane], w[nb], acc[mb][nb], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, MB * X_PLANES, 0);      // LDS reads first, then one matrix
+#pragma unroll
+            for (int k = 0; k < 4 * MB; ++k) {                                  // instruction and its share of the rest
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 24 / (4 * MB) + 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // made here and not sunk to the use behind the workgroup's meeting, where nothing covers it
+        auto pin = [](auto (&values)[2]) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) asm volatile("" : "+v"(values[k]));
+        };
+        take_weights(now);
+        if (S::CH < iterations) issue_weights(S::CH);
+        read(0, 0, a[0]);
+        scale(now.s[0], g_first < g_end, s, less);
+        convert(now.w[0], 0, b[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int it0 = 0; it0 < iterations; it0 += S::CH) {
+#pragma unroll
+            for (int gi = 0; gi < S::CH; ++gi) {
+                const int it = it0 + gi;
+#pragma unroll
+                for (int step = 0; step < 3; ++step) {
+                    read(it, step + 1, a[(step + 1) & 1]);
+                    convert(now.w[gi], step + 1, b[(step + 1) & 1]);
+                    if (step == 1 && gi < LAST) {
+                        scale(now.s[gi < LAST ? gi + 1 : 0], g_first + it + 1 < g_end, s_next, less_next);
+                        pin(s_next); pin(less_next);
+                    }
+                    multiply(a[step & 1], b[step & 1]);
+                }
+                pin(b[1]);
+                // the next planes were sent for before the chunk that may still be on its way
+                if (gi == 0 && it0 + S::CH < iterations) wait_loads<CHUNK_LOADS>(); else wait_loads<0>();
+                __syncthreads();
+                if (it + 2 < iterations) issue_x(it + 2);
+                if (gi == S::CH - 1) {
+                    take_weights(now);
+                    if (it + 1 + S::CH < iterations) issue_weights(it + 1 + S::CH);
+                }
+                // after the last group these are stale and unused
+                if (gi == LAST) scale(now.s[0], g_first + it + 1 < g_end, s_next, less_next);
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) { s[nb] = s_next[nb]; less[nb] = less_next[nb]; }
+                read(it + 1, 0, a[0]);
+                convert(now.w[gi == LAST ? 0 : gi + 1], 0, b[0]);
+                multiply(a[1], b[1]);
+                if (it + 1 >= iterations) break;
+            }
+        }
+    };
+    // A wave without rows helps to stage.
+    auto stage_only = [&]() {
+        for (int it = 0; it < iterations; ++it) {
+            wait_loads<0>();
+            __syncthreads();
+            if (it + 2 < iterations) issue_x(it + 2);
+        }
+    };
+    for (int window = 0;;) {
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) raise[nb] = WEIGHT_TOP - top[nb] + WINDOW * window;
+        // ---- main loop: acc += s (q - 8) x over the part's columns
+        if (iterations > 1) issue_x(1);
+        if (!live) stage_only();
+        else if (wide) walk(std::integral_constant<int, 2>{});
+        else walk(std::integral_constant<int, 1>{});
+
+        // ---- the parts meet in part order
+        if (KP > 1) {
+            float *sums = reinterpret_cast<float *>(stage);
+            if (part > 0) {
+                float *mine = sums + ((part - 1) * S::ROW_WAVES + wn) * 4096 + lane;
+#pragma unroll
+                for (int k = 0; k < 64; ++k) mine[k * 64] = acc[k >> 5][(k >> 4) & 1][k & 15];
+            }
+            __syncthreads();
+            if (part == 0) {
+#pragma unroll
+                for (int p = 1; p < KP; ++p) {
+                    const float *theirs = sums + ((p - 1) * S::ROW_WAVES + wn) * 4096 + lane;
+#pragma unroll
+                    for (int k = 0; k < 64; ++k) acc[k >> 5][(k >> 4) & 1][k & 15] += theirs[k * 64];
+                }
+            }
+        }
+
+        if (live && part == 0) {
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) {
+                if (mb == 1 && !wide) break;
+                int tok_base = mb * 32 + half * 4;
+                asm volatile("" : "+v"(tok_base));      // the output addresses are made here, not kept through the loop
+                global_f32_out line = (global_f32_out)(uintptr_t)job.y + (size_t)(tok0 + tok_base) * job.rows + row0 + l32;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int tok = tok_base + (i >> 2) * 8 + (i & 3);
+                    const int down = s_down[tok];
+#pragma unroll
+                    for (int nb = 0; nb < 2; ++nb) {
+                        if (tok < toks_here && row0 + nb * 32 + l32 < job.rows) {
+                            float v = __builtin_amdgcn_ldexpf(acc[mb][nb][i], down - raise[nb]);
+                            if (window != 0) v = line[nb * 32] + v;
+                            line[nb * 32] = v;
+                        }
+                    }
+                    line += (size_t)job.rows * ((i & 3) == 3 ? 5 : 1);
+                }
+            }
+        }
+        if (++window >= windows) break;             // uniform over the workgroup
+        __syncthreads();                            // the parts' sums have been read
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = zero;
+        wait_loads<0>();
+        issue_weights(0);
+        issue_x(0);
+        wait_loads<0>();
+        __syncthreads();
     }
 }
 
 // fp32 rows -> two fp16 planes of the row scaled by a power of two (columns permuted inside every run of eight, see
-// the top of the file), the row's 2^-k at the head of its row of a third plane, and the per-64-column sums of the
-// unscaled values.  Row r of the output is row row_map[r] / map_divisor of the input when a map is given (the
-// grouped MoE gather).  One workgroup per row: the scale needs the row's largest magnitude.
+// the top of the file) and the row's notes in a third plane: the exponent that undoes the scaling and the
+// per-64-column sums of the unscaled values in three bf16 planes.  Row r of the output is row row_map[r] /
+// map_divisor of the input when a map is given (the grouped MoE gather).  ROW_WAVES waves per row, because the scale
+// needs the row's largest magnitude: a whole workgroup, or one wave where a row is short enough for that.
 // With GATED the value split is gelu_tanh(gate) * x (the expert activation, reference gemma4_text.c:8749-9137
 // "down input"), so the activations never make a round trip through memory in fp32.
-constexpr int SPLIT_MAX_ITEMS = 4;          // eight columns per item and thread: rows of up to 8192 columns
+constexpr int SPLIT_MAX_ITEMS = 4;          // eight columns per item and thread: rows of up to 2048 columns per wave
 
-template <bool GATED>
+template <bool GATED, int ROW_WAVES>
 __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ x, const float *__restrict__ gate,
                                                       const int *__restrict__ row_map, int map_divisor, int x_stride,
                                                       int rows, int cols, uint16_t *__restrict__ planes,
-                                                      size_t plane_stride, float *__restrict__ xsum) {
+                                                      size_t plane_stride) {
     __shared__ uint32_t wave_top[4];
-    const int row = blockIdx.x;
+    constexpr int THREADS = 64 * ROW_WAVES;
+    const int tid = threadIdx.x & (THREADS - 1);
+    const int row = ROW_WAVES == 4 ? (int)blockIdx.x : (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (row >= rows) return;                        // whole waves, and only where no barrier follows
     const int src_row = row_map ? row_map[row] / map_divisor : row;
     float v[SPLIT_MAX_ITEMS][8];
     uint32_t top = 0u;                              // largest magnitude as a bit pattern: a NaN or an infinity wins it
 #pragma unroll
     for (int it = 0; it < SPLIT_MAX_ITEMS; ++it) {
-        const int c0 = (it * 256 + (int)threadIdx.x) * 8;
+        const int c0 = (it * THREADS + tid) * 8;
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[it][j] = 0.0f;
         if (c0 < cols) {
@@ -444,21 +682,30 @@ __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ 
         const uint32_t other = (uint32_t)__shfl_xor((int)top, d, 64);
         top = top > other ? top : other;
     }
-    if ((threadIdx.x & 63) == 0) wave_top[threadIdx.x >> 6] = top;
-    __syncthreads();
-    top = wave_top[0];
+    if (ROW_WAVES == 4) {
+        if ((threadIdx.x & 63) == 0) wave_top[threadIdx.x >> 6] = top;
+        __syncthreads();
+        top = wave_top[0];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) top = top > wave_top[w] ? top : wave_top[w];
+        for (int w = 1; w < 4; ++w) top = top > wave_top[w] ? top : wave_top[w];
+    }
     // top in [2^E, 2^(E+1)) -> x * 2^(13 - E) in [2^13, 2^14); rows of zeros or tiny values are pinned
     int eb = (int)(top >> 23);
     eb = eb < 14 ? 14 : (eb > 253 ? 253 : eb);
     const float up = __uint_as_float((uint32_t)(267 - eb) << 23);          // 2^(13 - E)
-    const float down = __uint_as_float((uint32_t)(eb - 13) << 23);         // 2^(E - 13)
-    if (threadIdx.x == 0) *reinterpret_cast<float *>(planes + 2 * plane_stride + (size_t)row * cols) = down;
+    uint16_t *const notes = planes + 2 * plane_stride + (size_t)row * cols;
+    const int ngrp = cols >> 6, padded = padded_groups(ngrp);
+    if (tid == 0) *reinterpret_cast<int *>(notes) = eb - 140;              // E - 13
+    // the last eight groups sit at the end of theirs (eight_start): entries that stand for no group of their own are zero
+    const int tail = ((ngrp + 7) >> 3) - 1, shift = ngrp > 8 ? 8 * tail - (ngrp - 8) : 0;
+    for (int at = 8 * tail + tid; at < padded; at += THREADS)
+        if (at < 8 * tail + shift || at >= ngrp + shift)
+#pragma unroll
+            for (int plane = 0; plane < 3; ++plane) notes[8 + plane * padded + at] = 0;
 #pragma unroll
     for (int it = 0; it < SPLIT_MAX_ITEMS; ++it) {
-        const int c0 = (it * 256 + (int)threadIdx.x) * 8;
-        const bool live = c0 < cols;
+        const int c0 = (it * THREADS + tid) * 8;
+        const bool inside = c0 < cols;
         uint32_t hi[4], lo[4];
         float sum = 0.0f;
 #pragma unroll
@@ -476,60 +723,77 @@ __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ 
         sum += __shfl_xor(sum, 1, 64);
         sum += __shfl_xor(sum, 2, 64);
         sum += __shfl_xor(sum, 4, 64);
-        if (live) {
+        if (inside) {
             uint16_t *dst = planes + (size_t)row * cols + c0;
             *reinterpret_cast<uint4 *>(dst) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
             *reinterpret_cast<uint4 *>(dst + plane_stride) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-            if ((threadIdx.x & 7) == 0) xsum[(size_t)row * (cols >> 6) + (c0 >> 6)] = sum;
+            if ((tid & 7) == 0) {
+                uint32_t h, m, l;
+                split3(sum, h, m, l);
+                const int g = c0 >> 6;
+                uint16_t *at = notes + 8 + (g < 8 * tail ? g : g + shift);
+                at[0] = (uint16_t)h; at[padded] = (uint16_t)m; at[2 * padded] = (uint16_t)l;
+            }
         }
     }
 }
 
 }  // namespace
 
-int mfma_tile_rows(int blocks_per_wave) { return 64 * blocks_per_wave; }
+int mfma_tile_rows(int column_parts) { return 256 / column_parts; }
 
-int mfma_tiles(int tokens, int rows, int blocks_per_wave) {
-    const int tn = mfma_tile_rows(blocks_per_wave);
-    return ((tokens + TM - 1) / TM) * ((rows + tn - 1) / tn);
+namespace {
+int mfma_tiles(int tokens, int tile_tokens, int rows, int column_parts) {
+    const int tn = mfma_tile_rows(column_parts);
+    return ((tokens + tile_tokens - 1) / tile_tokens) * ((rows + tn - 1) / tn);
 }
+}  // namespace
 
-// Blocks of 32 rows per wave.  Four (a 64 x 256 tile) halves the LDS and cache
-// traffic per matrix instruction but measured no faster than two: on this
-// device the matrix instructions and the other vector instructions of a SIMD
-// do not overlap, so the kernel is bound by their sum, not by data movement.
-int mfma_blocks_per_wave(long long wide_tiles) {
-    (void)wide_tiles;
-    return 2;
+// Column parts for a launch of `wide_tiles` tiles of 64 x 256 over `ngrp` scale groups: as many as still leave every
+// workgroup a compute unit of its own.  A part shortens the walk of a workgroup that has its compute unit to itself;
+// beyond that it only adds rounds, and a workgroup of several parts fills a compute unit's LDS alone where two of one
+// part share it and hide each other's waits (16384 x 2816, 333 tokens, 384 tiles: 84 us in one part, 114 in two).
+int mfma_column_parts(long long wide_tiles, int ngrp) {
+    int parts = 1;
+    while (parts < 4 && wide_tiles * (2 * parts) <= 256 && ngrp >= 8 * parts) parts *= 2;
+    return parts;
 }
 
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream) {
     MfmaLaunch L = launch;
     if (L.cols < 64 || (L.cols & 63)) return -1;
     if (L.table == nullptr) {                   // one job: the tiling is chosen here
-        if (L.blocks_per_wave == 0) L.blocks_per_wave = mfma_blocks_per_wave(mfma_tiles(L.one.tokens, L.one.rows, 4));
+        L.column_parts = mfma_column_parts(mfma_tiles(L.one.tokens, TM, L.one.rows, 1), L.cols >> 6);
+        // Tiles of half the tokens where each still finds a compute unit of its own: half the matrix work per step of a
+        // walk that is bound by its waits (4096 x 4096, 64 tokens: 41 us in 64-token tiles, 32 in these).
+        const int halves = mfma_tiles(L.one.tokens, TM / 2, L.one.rows, L.column_parts);
+        L.tile_tokens = halves <= 256 ? TM / 2 : TM;
         L.one.tile0 = 0;
-        L.total_tiles = mfma_tiles(L.one.tokens, L.one.rows, L.blocks_per_wave);
+        L.total_tiles = mfma_tiles(L.one.tokens, L.tile_tokens, L.one.rows, L.column_parts);
     }
-    if (3 * (unsigned long long)L.plane_stride >= (1ull << 32)) return -1;      // 32-bit element offsets in the kernel
-    if (L.total_tiles < 1 || L.blocks_per_wave != 2 || (L.row_map && L.map_divisor < 1))
-        return -1;
-    hipLaunchKernelGGL(q4_mfma_kernel<2>, dim3(L.total_tiles), dim3(256), 0, stream, L);
+    if (3 * (unsigned long long)L.plane_stride >= (1ull << 32)) return -1;      // 32-bit byte offsets inside a plane
+    if (L.total_tiles < 1 || (L.tile_tokens != TM && L.tile_tokens != TM / 2) || (L.row_map && L.map_divisor < 1)) return -1;
+    switch (L.column_parts) {
+        case 1: hipLaunchKernelGGL(q4_mfma_kernel<1>, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L); break;
+        case 2: hipLaunchKernelGGL(q4_mfma_kernel<2>, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L); break;
+        case 4: hipLaunchKernelGGL(q4_mfma_kernel<4>, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L); break;
+        default: return -1;
+    }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int x_split_launch(const float *x, const float *gate, const int *row_map, int map_divisor, int x_stride, int rows,
-                   int cols, uint16_t *planes, size_t plane_stride, float *xsum, hipStream_t stream) {
+                   int cols, uint16_t *planes, size_t plane_stride, hipStream_t stream) {
     if (rows < 1 || cols < 64 || (cols & 63) || cols > SPLIT_MAX_ITEMS * 256 * 8) return -1;
-    const dim3 grid(rows);
-    if (gate)
-        hipLaunchKernelGGL(x_split_kernel<true>, grid, dim3(256), 0, stream, x, gate, row_map, map_divisor, x_stride,
-                           rows, cols, planes, plane_stride, xsum);
-    else
-        hipLaunchKernelGGL(x_split_kernel<false>, grid, dim3(256), 0, stream, x, gate, row_map, map_divisor, x_stride,
-                           rows, cols, planes, plane_stride, xsum);
+    // A wave per row leaves no thread of a short row idle (gelu_tanh(gate) * up, 16384 rows of 704: 50 -> 41 us), a
+    // workgroup per row shortens the chain of a call with few rows (900 rows of 704: 5.9 against 7.2 us).
+    const bool one_wave = cols <= SPLIT_MAX_ITEMS * 64 * 8 && rows >= 4096;
+    const dim3 grid(one_wave ? (rows + 3) / 4 : rows);
+    auto kernel = gate ? (one_wave ? x_split_kernel<true, 1> : x_split_kernel<true, 4>)
+                       : (one_wave ? x_split_kernel<false, 1> : x_split_kernel<false, 4>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, gate, row_map, map_divisor, x_stride, rows, cols, planes,
+                       plane_stride);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
-
 
 }  // namespace mi355
