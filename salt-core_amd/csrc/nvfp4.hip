@@ -40,8 +40,6 @@ constexpr int TILE_ROWS = 64;
 constexpr int CHUNK_BLOCKS = 16;                       // 32-column blocks per staged step
 constexpr int W_PITCH = 16 * CHUNK_BLOCKS + 4;         // bytes per staged row of codes
 constexpr int M_PITCH = 2 * CHUNK_BLOCKS + 1;          // floats per staged row of `scaled` factors (odd)
-constexpr int W_STAGE = TILE_ROWS * W_PITCH;
-constexpr int M_STAGE = TILE_ROWS * M_PITCH;
 constexpr int FOLD_PITCH = 33;
 
 static_assert(sizeof(Fp4Job) == 48 && offsetof(Fp4Job, weight_global_scale) == 32 && offsetof(Fp4Job, rows) == 36 &&
@@ -116,17 +114,24 @@ constexpr int x_batch_blocks(int S, int NB) {
 // nvfp4.c:228-256) into LDS, and the rows read it from there into vector
 // registers (every lane the same words); workgroup 0 reports a non-finite activation (-1 into a
 // status word the caller cleared) and nothing is published then.
-template <int S, int NB, bool QDQ = false>
-__global__ __launch_bounds__((32 / S) * 64) void fp4_tile_kernel(const Fp4Launch L) {
-    constexpr int WAVES = 32 / S;
+//
+// SPLIT (with QDQ): the tile is cut into SPLIT workgroups of 64 / SPLIT rows, as in the affine-Q4 kernel, for launches
+// that would leave compute units idle; lane l of a wave holds row l % ROWS of chain slice SPLIT * wave + l / ROWS.
+// 8192 x 8192, one token (128 tiles): 27.0 -> 18.5 us.
+template <int S, int NB, bool QDQ = false, int SPLIT = 1>
+__global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void fp4_tile_kernel(const Fp4Launch L) {
+    constexpr int ROWS = TILE_ROWS / SPLIT;
+    constexpr int W_STAGE = ROWS * W_PITCH, M_STAGE = ROWS * M_PITCH;
+    constexpr int WAVES = 32 / (S * SPLIT);
     constexpr int THREADS = WAVES * 64;
-    constexpr int PIECES = (TILE_ROWS * CHUNK_BLOCKS) / THREADS;     // 16-byte pieces == (row, block) items
-    constexpr int FOLD_BYTES = NB * TILE_ROWS * FOLD_PITCH * 4;
+    constexpr int PIECES = (ROWS * CHUNK_BLOCKS) / THREADS;          // 16-byte pieces == (row, block) items
+    constexpr int FOLD_BYTES = NB * ROWS * FOLD_PITCH * 4;
     constexpr int W_BYTES = 2 * W_STAGE > FOLD_BYTES ? 2 * W_STAGE : FOLD_BYTES;
     constexpr int XB = QDQ ? 2 : x_batch_blocks(S, NB);      // LDS-fed activations sit in vector registers: short batches
     constexpr int XN = XB * S;
     constexpr int W_ROW_STEP = THREADS / 16;
-    static_assert(THREADS >= NB * TILE_ROWS, "fold needs one thread per (token, row)");
+    static_assert(THREADS >= NB * ROWS, "fold needs one thread per (token, row)");
+    static_assert(SPLIT == 1 || QDQ, "split tiles take their activations from LDS");
 
     __shared__ __attribute__((aligned(16))) uint8_t w_lds[W_BYTES];
     __shared__ float m_lds[2 * M_STAGE];
@@ -138,7 +143,11 @@ __global__ __launch_bounds__((32 / S) * 64) void fp4_tile_kernel(const Fp4Launch
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    const Fp4Job job = find_job(L, blockIdx.x);
+    // lane's row of the tile and its slice of the chains
+    const int lane_row = lane & (ROWS - 1);
+    const int slice = SPLIT == 1 ? wave : wave * SPLIT + lane / ROWS;
+    const int tile = SPLIT == 1 ? (int)blockIdx.x : (int)blockIdx.x / SPLIT;
+    const Fp4Job job = find_job(L, tile);
     if (QDQ) {
         if (tid == 0) x_bad = 0;
         __syncthreads();
@@ -162,8 +171,9 @@ __global__ __launch_bounds__((32 / S) * 64) void fp4_tile_kernel(const Fp4Launch
         if (bad && blockIdx.x == 0 && tid == 0) *L.status = -1;        // like fp4_qdq_kernel: the caller cleared it
         if (bad) return;                                   // uniform
     }
-    const int row0 = (blockIdx.x - job.tile0) * TILE_ROWS;
-    const int rows_here = job.rows - row0 < TILE_ROWS ? job.rows - row0 : TILE_ROWS;
+    const int row0 = (tile - job.tile0) * TILE_ROWS + (SPLIT == 1 ? 0 : ((int)blockIdx.x % SPLIT) * ROWS);
+    if (SPLIT > 1 && row0 >= job.rows) return;             // uniform: the rest of the last tile
+    const int rows_here = job.rows - row0 < ROWS ? job.rows - row0 : ROWS;
     const int nblk = L.cols >> 5;
     const int nchunk = (nblk + CHUNK_BLOCKS - 1) / CHUNK_BLOCKS;
     const uint32_t row_bytes = (uint32_t)(L.cols >> 1);
@@ -219,7 +229,7 @@ __global__ __launch_bounds__((32 / S) * 64) void fp4_tile_kernel(const Fp4Launch
 
     auto load_x = [&](int blk0, float (&xq)[NB][XN], int blocks) {
         if (QDQ) {                        // every lane reads the same LDS words: the activations travel in vector registers
-            const float *xl = x_lds + blk0 * 32 + S * wave;
+            const float *xl = x_lds + blk0 * 32 + S * slice;
 #pragma unroll
             for (int k = 0; k < XN; ++k)
                 if (k < blocks * S) xq[0][k] = xl[(k / S) * 32 + (k % S)];
@@ -268,9 +278,9 @@ __global__ __launch_bounds__((32 / S) * 64) void fp4_tile_kernel(const Fp4Launch
         __syncthreads();
         if (ck + 1 < nchunk) issue(ck + 1);
 
-        const uint8_t *wrow = w_lds + stage * W_STAGE + lane * W_PITCH + wave * (S / 2);
-        // the wave's chains lie in the first (columns 0..15) or second half of a block
-        const float *mrow = m_lds + stage * M_STAGE + lane * M_PITCH + ((S * wave) >> 4);
+        const uint8_t *wrow = w_lds + stage * W_STAGE + lane_row * W_PITCH + slice * (S / 2);
+        // the slice's chains lie in the first (columns 0..15) or second half of a block
+        const float *mrow = m_lds + stage * M_STAGE + lane_row * M_PITCH + ((S * slice) >> 4);
 
         auto fetch = [&](int blk, uint32_t &w, float &scaled) {
             scaled = mrow[2 * blk];
@@ -307,11 +317,11 @@ __global__ __launch_bounds__((32 / S) * 64) void fp4_tile_kernel(const Fp4Launch
 #pragma unroll
     for (int t = 0; t < NB; ++t)
 #pragma unroll
-        for (int c = 0; c < S; ++c) fold[(t * TILE_ROWS + lane) * FOLD_PITCH + S * wave + c] = acc[t][c];
+        for (int c = 0; c < S; ++c) fold[(t * ROWS + lane_row) * FOLD_PITCH + S * slice + c] = acc[t][c];
     __syncthreads();
-    if (tid < NB * TILE_ROWS) {
-        const int t = tid >> 6;
-        const float *f = fold + (t * TILE_ROWS + lane) * FOLD_PITCH;
+    if (tid < NB * ROWS) {
+        const int t = tid / ROWS;
+        const float *f = fold + (t * ROWS + lane_row) * FOLD_PITCH;
         float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int a = 0; a < 8; ++a)
@@ -319,7 +329,7 @@ __global__ __launch_bounds__((32 / S) * 64) void fp4_tile_kernel(const Fp4Launch
             for (int j = 0; j < 4; ++j) part[j] = part[j] + f[4 * a + j];
         const float even = part[0] + part[2];
         const float odd = part[1] + part[3];
-        if (lane < rows_here) y[(size_t)t * job.rows + row0 + lane] = even + odd;
+        if (lane_row < rows_here) y[(size_t)t * job.rows + row0 + lane_row] = even + odd;
     }
 }
 
@@ -328,6 +338,16 @@ int launch_tiles(const Fp4Launch &L, hipStream_t stream) {
     const dim3 grid(L.total_tiles), block((32 / S) * 64);
     if (L.qdq) {
         if (L.tokens != 1 || L.table || L.cols > FP4_FUSED_MAX_COLS || !L.status || ((uintptr_t)L.one.x & 15)) return -1;
+        // sixteen-row workgroups while they find room at once, thirty-two-row ones up to one per compute unit
+        // (64 tiles of 8192 columns 26.2 -> 18.1 us, 128 27.0 -> 18.5)
+        if (S == 2 && L.total_tiles <= 64) {
+            hipLaunchKernelGGL((fp4_tile_kernel<2, 1, true, 4>), dim3(4 * L.total_tiles), dim3(256), 0, stream, L);
+            return hipGetLastError() == hipSuccess ? 0 : -1;
+        }
+        if (S == 2 && L.total_tiles <= 128) {
+            hipLaunchKernelGGL((fp4_tile_kernel<2, 1, true, 2>), dim3(2 * L.total_tiles), dim3(512), 0, stream, L);
+            return hipGetLastError() == hipSuccess ? 0 : -1;
+        }
         hipLaunchKernelGGL((fp4_tile_kernel<S, 1, true>), grid, block, 0, stream, L);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }

@@ -47,6 +47,7 @@ __device__ __forceinline__ uniform_f32_ptr as_uniform(const float *p) {
 
 constexpr int TILE_ROWS = 64;
 constexpr int FOLD_PITCH = 33;
+constexpr int SPLIT_MAX_COLS = 8192;          // activations that split tiles keep in LDS
 constexpr float BIG_SCALE = 0x1p118f;
 
 __device__ __forceinline__ float bf16_to_f32(uint32_t half) { return __uint_as_float(half << 16); }
@@ -157,27 +158,37 @@ constexpr int x_batch_groups(int S, int NB) {
 // gelu_tanh(gate) * up are computed into LDS and reach the VALU in vector
 // registers (every lane reads the same words) instead of through scalar loads;
 // 3 = the same activation prologue for jobs of the launch (one token each).
-template <int S, int NB, int CB, int PRO = 0>
-__global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L) {
+//
+// SPLIT cuts a tile into SPLIT workgroups of ROWS = 64 / SPLIT rows for launches that would leave compute units idle:
+// a wave then holds SPLIT chain slices of ROWS rows, lane l row l % ROWS of slice SPLIT * wave + l / ROWS, so a
+// workgroup has 1 / SPLIT of the waves and a wave the same work.  The chain order leaves rows as the only axis to cut
+// along, and a wave's instruction count does not shrink with idle lanes.  The slice differs inside a wave, so the
+// activations come from LDS as in the prologues above.
+// One token: 2816 x 2816 (44 tiles) 10.8 -> 6.8 us.
+template <int S, int NB, int CB, int PRO = 0, int SPLIT = 1>
+__global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const Q4Launch L) {
     constexpr int CHUNK_BLOCKS = CB;
+    constexpr int ROWS = TILE_ROWS / SPLIT;
+    constexpr bool LDS_X = PRO >= 2 || SPLIT > 1;
     constexpr int CHUNK_GROUPS = CB / 2;                   // 64-column scale groups per step
     constexpr int W_PITCH = 16 * CB + 4;                   // bytes per staged row: odd dword pitch
     constexpr int M_PITCH = 2 * CHUNK_GROUPS + 2;          // floats per staged row of (scale, bias)
-    constexpr int W_STAGE = TILE_ROWS * W_PITCH;
-    constexpr int M_STAGE = TILE_ROWS * M_PITCH;
-    constexpr int WAVES = 32 / S;
+    constexpr int W_STAGE = ROWS * W_PITCH;
+    constexpr int M_STAGE = ROWS * M_PITCH;
+    constexpr int WAVES = 32 / (S * SPLIT);
     constexpr int THREADS = WAVES * 64;
     // A staging item is one scale group of one row: 32 bytes of codes (two blocks) and its (scale, bias).
-    constexpr int ITEMS = (TILE_ROWS * CHUNK_GROUPS + THREADS - 1) / THREADS;
-    constexpr int FOLD_BYTES = NB * TILE_ROWS * FOLD_PITCH * 4;
+    constexpr int ITEMS = (ROWS * CHUNK_GROUPS + THREADS - 1) / THREADS;
+    constexpr int FOLD_BYTES = NB * ROWS * FOLD_PITCH * 4;
     constexpr int W_BYTES = 2 * W_STAGE > FOLD_BYTES ? 2 * W_STAGE : FOLD_BYTES;
-    constexpr int XG = PRO >= 2 ? 2 : x_batch_groups(S, NB);        // LDS-fed activations sit in vector registers: short batches
+    constexpr int XG = LDS_X ? 2 : x_batch_groups(S, NB);        // LDS-fed activations sit in vector registers: short batches
     constexpr int XN = XG * 2 * S;
-    static_assert(THREADS >= NB * TILE_ROWS, "fold needs one thread per (token, row)");
+    static_assert(THREADS >= NB * ROWS, "fold needs one thread per (token, row)");
+    static_assert(SPLIT == 1 || (NB == 1 && PRO != 2), "split tiles serve single tokens; the down launch counts whole tiles");
 
     __shared__ __attribute__((aligned(16))) uint8_t w_lds[W_BYTES];
     __shared__ __attribute__((aligned(16))) float m_lds[2 * M_STAGE];
-    __shared__ __attribute__((aligned(16))) float x_lds[PRO >= 2 ? MOE_FUSE_MAX_ROUTED : 4];
+    __shared__ __attribute__((aligned(16))) float x_lds[PRO >= 2 ? MOE_FUSE_MAX_ROUTED : SPLIT > 1 ? SPLIT_MAX_COLS : 4];
     __shared__ int slow_flag;
     static_assert(PRO == 0 || NB == 1, "the MoE prologues serve the single-token kernel");
     static_assert(PRO != 1 || (sizeof(RouterShared) <= W_BYTES && THREADS >= MOE_FUSE_MAX_EXPERTS),
@@ -187,13 +198,18 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
+    // lane's row of the tile and its slice of the chains
+    const int lane_row = lane & (ROWS - 1);
+    const int slice = SPLIT == 1 ? wave : wave * SPLIT + lane / ROWS;
+    const int tile = SPLIT == 1 ? (int)blockIdx.x : (int)blockIdx.x / SPLIT;
+
     Q4Job job;
     const float *act_gate = nullptr, *act_up = nullptr;     // PRO >= 2: the activation row is gelu_tanh(gate) * up
     if (PRO == 0) {
-        job = find_job(L, blockIdx.x);
+        job = find_job(L, tile);
     } else if (PRO == 3) {
         // the job's activation row is gelu_tanh(gate) * up of the two rows its x names: x[i] and x[i + act_delta]
-        job = find_job(L, blockIdx.x);
+        job = find_job(L, tile);
         act_gate = job.x; act_up = job.x + L.act_delta;
     } else {
         const MoeFuse &m = L.moe;
@@ -201,9 +217,9 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
         const size_t vals_bytes = n / 2, meta_bytes = (n / 64) * 2, proj_bytes = vals_bytes + 2 * meta_bytes;
         if (PRO == 1) {
             RouterShared &sh = *reinterpret_cast<RouterShared *>(w_lds);
-            const bool publisher = (int)blockIdx.x == L.total_tiles;       // one workgroup past the tiles
+            const bool publisher = tile == L.total_tiles;                  // one workgroup past the tiles
             const int up_tiles = (m.routed + TILE_ROWS - 1) / TILE_ROWS;
-            const int slot_index = (int)blockIdx.x / up_tiles;             // 2 * place + (0 gate | 1 up)
+            const int slot_index = tile / up_tiles;                        // 2 * place + (0 gate | 1 up)
             const int place = slot_index >> 1, proj = slot_index & 1;
             int expert;
             if (!publisher && m.n_experts <= ROUTER_WAVE_MAX_EXPERTS) {
@@ -249,9 +265,10 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
         job.scales = job.vals + vals_bytes;
         job.biases = job.scales + meta_bytes;
     }
-    const int row0 = (blockIdx.x - job.tile0) * TILE_ROWS;
+    const int row0 = (tile - job.tile0) * TILE_ROWS + (SPLIT == 1 ? 0 : ((int)blockIdx.x % SPLIT) * ROWS);
     const int R = job.rows;
-    const int rows_here = R - row0 < TILE_ROWS ? R - row0 : TILE_ROWS;
+    if (SPLIT > 1 && row0 >= R) return;             // uniform: the rest of a job's last tile
+    const int rows_here = R - row0 < ROWS ? R - row0 : ROWS;
     const int nblk = L.cols >> 5;
     const int ngrp = L.cols >> 6;
     const int nchunk = (nblk + CHUNK_BLOCKS - 1) / CHUNK_BLOCKS;
@@ -271,14 +288,14 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
     // group holds bytes 2t, 2t+1 of the first block and of the second, which is
     // exactly the pair of two-byte slices a four-chain wave consumes.
     constexpr int ROW_STEP = THREADS / CHUNK_GROUPS;
-    const bool has_item = tid < TILE_ROWS * CHUNK_GROUPS;    // only narrower than the block when THREADS == 1024
+    const bool has_item = tid < ROWS * CHUNK_GROUPS;    // only narrower than the block when THREADS == 1024
     const uint32_t it_grp = tid % CHUNK_GROUPS;
-    const uint32_t w_dst0 = ((tid / CHUNK_GROUPS) & (TILE_ROWS - 1)) * W_PITCH + it_grp * 32;
-    const uint32_t m_dst0 = ((tid / CHUNK_GROUPS) & (TILE_ROWS - 1)) * M_PITCH + 2 * it_grp;
+    const uint32_t w_dst0 = ((tid / CHUNK_GROUPS) & (ROWS - 1)) * W_PITCH + it_grp * 32;
+    const uint32_t m_dst0 = ((tid / CHUNK_GROUPS) & (ROWS - 1)) * M_PITCH + 2 * it_grp;
     uint32_t w_off[ITEMS], m_off[ITEMS];                     // source offsets of the item in step 0
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
-        const int row = ((tid / CHUNK_GROUPS) + i * ROW_STEP) & (TILE_ROWS - 1);
+        const int row = ((tid / CHUNK_GROUPS) + i * ROW_STEP) & (ROWS - 1);
         const uint32_t rc = (uint32_t)(row < rows_here ? row : rows_here - 1);
         w_off[i] = rc * row_bytes + it_grp * 32;
         m_off[i] = rc * ngrp + it_grp;
@@ -358,15 +375,19 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
     if (PRO >= 2) {
         // after the first weights have been sent for: they are on their way while the activation is computed
         for (int i = tid; i < L.cols; i += THREADS) x_lds[i] = det_gelu_tanh(act_gate[i]) * act_up[i];
+    } else if (SPLIT > 1) {
+        const float __attribute__((address_space(1))) *src = (const float __attribute__((address_space(1))) *)(uintptr_t)job.x;
+#pragma unroll 4
+        for (int i = tid; i < L.cols; i += THREADS) x_lds[i] = src[i];
     }
     __syncthreads();
 
-    const int my_row = lane < rows_here ? lane : rows_here - 1;
+    const int my_row = lane_row < rows_here ? lane_row : rows_here - 1;
 
     // x of `groups` consecutive scale groups starting at group g0 of the row
     auto load_x = [&](int g0, float (&xq)[NB][XN], int groups) {
-        if (PRO >= 2) {                   // every lane reads the same LDS words: the activations travel in vector registers
-            const float *xl = x_lds + g0 * 64 + S * wave;
+        if (LDS_X) {                      // every lane of a slice reads the same LDS words: the activations travel in vector registers
+            const float *xl = x_lds + g0 * 64 + S * slice;
 #pragma unroll
             for (int k = 0; k < XN; ++k)
                 if (k < groups * 2 * S) xq[0][k] = xl[(k / S) * 32 + (k % S)];
@@ -397,9 +418,9 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
 
         const int slow = __builtin_amdgcn_readfirstlane(slow_flag);
         // wave t reads dword t (S == 4), dwords 2t and 2t+1 (S == 8) or dword t / 2 (S == 2) of every group
-        const uint8_t *wrow = w_lds + stage * W_STAGE + lane * W_PITCH + (S == 2 ? (wave >> 1) * 4 : wave * S);
-        const uint32_t byte_pick = 0x0C0C0000u | (uint32_t)((2 + (wave & 1)) << 8) | (uint32_t)(wave & 1);
-        const float *mrow = m_lds + stage * M_STAGE + lane * M_PITCH;
+        const uint8_t *wrow = w_lds + stage * W_STAGE + lane_row * W_PITCH + (S == 2 ? (slice >> 1) * 4 : slice * S);
+        const uint32_t byte_pick = 0x0C0C0000u | (uint32_t)((2 + (slice & 1)) << 8) | (uint32_t)(slice & 1);
+        const float *mrow = m_lds + stage * M_STAGE + lane_row * M_PITCH;
 
         // LDS operands of group g of this step: the lane's nibbles and (scale', bias)
         auto fetch = [&](int g, uint32_t &w0, uint32_t &w1, float &scale, float &bias) {
@@ -493,11 +514,11 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
 #pragma unroll
     for (int t = 0; t < NB; ++t)
 #pragma unroll
-        for (int c = 0; c < S; ++c) fold[(t * TILE_ROWS + lane) * FOLD_PITCH + S * wave + c] = acc[t][c];
+        for (int c = 0; c < S; ++c) fold[(t * ROWS + lane_row) * FOLD_PITCH + S * slice + c] = acc[t][c];
     __syncthreads();
-    if (tid < NB * TILE_ROWS) {
-        const int t = tid >> 6;
-        const float *f = fold + (t * TILE_ROWS + lane) * FOLD_PITCH;
+    if (tid < NB * ROWS) {
+        const int t = tid / ROWS;
+        const float *f = fold + (t * ROWS + lane_row) * FOLD_PITCH;
         float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int a = 0; a < 8; ++a)
@@ -506,7 +527,7 @@ __global__ __launch_bounds__((32 / S) * 64) void q4_tile_kernel(const Q4Launch L
         const float even = part[0] + part[2];
         const float odd = part[1] + part[3];
         if (PRO != 2 || !L.moe.arrivals) {
-            if (lane < rows_here) y[(size_t)t * job.y_stride + row0 + lane] = even + odd;
+            if (lane_row < rows_here) y[(size_t)t * job.y_stride + row0 + lane_row] = even + odd;
         } else {                                        // uniform; NB == 1: these are the 64 lanes of wave 0
             // The layer output (reference gemma4_text.c:8301-8304: out = 0; out += o_i * w_i in ascending expert
             // order, product and sum rounded separately).  The topk workgroups that own these rows of the topk
@@ -594,9 +615,25 @@ __global__ __launch_bounds__(256) void q4_generic_kernel(const Q4Launch L) {
 // Launches of at most this many tiles (one per compute unit) use the wide-step variant and two chains per lane.
 constexpr int WIDE_TILE_LIMIT = 256;
 
+// Workgroups per tile of a single-token launch, as long as that gives more compute units work: sixteen-row workgroups up
+// to 96 tiles (beyond, the compute units that hold two of them take as long as with thirty-two rows), thirty-two-row ones
+// up to one per compute unit.  us before and after: 44 tiles of 2816 columns 10.8 / 6.8, of 8192 24.1 / 13.8, 96 of 2816
+// 10.9 / 7.5, 128 of 8192 25.7 / 17.3.
+int tile_split(int tiles, int cols) {
+    if (cols > SPLIT_MAX_COLS) return 1;
+    return tiles <= 96 ? 4 : 2 * tiles <= WIDE_TILE_LIMIT ? 2 : 1;
+}
+
 template <int S>
-int launch_tiles(const Q4Launch &L, hipStream_t stream) {
+int launch_tiles(const Q4Launch &L, bool may_split, hipStream_t stream) {
     const dim3 grid(L.total_tiles), block((32 / S) * 64);
+    const int split = S == 2 && L.tokens == 1 && may_split ? tile_split(L.total_tiles, L.cols) : 1;
+    if (split > 1) {
+        note_kernel("q4_tile_kernel<2,1,32,0,%d>", split);
+        if (split == 4) hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 0, 4>), dim3(4 * L.total_tiles), dim3(256), 0, stream, L);
+        else hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 0, 2>), dim3(2 * L.total_tiles), dim3(512), 0, stream, L);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
     // One token with few tiles: a workgroup has its compute unit to itself and stages twice as much per step.
     if (L.tokens == 1 && S <= 4 && L.total_tiles <= WIDE_TILE_LIMIT) {
         note_kernel("q4_tile_kernel<%d,1,32,0>", S);
@@ -648,7 +685,9 @@ int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream) {
     const dim3 grid(L.total_tiles + 1);                         // the extra workgroup publishes the router's outputs
     // measured at 176 tiles (eight experts of 704 rows): 1024-column steps 29.4 us per decode step, 512-column steps 29.1,
     // four chains per lane 30.4 and 33.4; the wide step is kept for launches that leave half the compute units idle
-    if (L.total_tiles <= WIDE_TILE_LIMIT / 2)
+    if (tile_split(L.total_tiles, L.cols) > 1)                  // two at most: the router needs a thread per expert
+        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 1, 2>), dim3(2 * L.total_tiles + 1), dim3(512), 0, stream, L);
+    else if (L.total_tiles <= WIDE_TILE_LIMIT / 2)
         hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 1>), grid, dim3(1024), 0, stream, L);
     else if (L.total_tiles <= WIDE_TILE_LIMIT)
         hipLaunchKernelGGL((q4_tile_kernel<2, 1, 16, 1>), grid, dim3(1024), 0, stream, L);
@@ -678,7 +717,12 @@ int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream) {
 int q4_activated_launch(const Q4Launch &L, hipStream_t stream) {
     if (L.total_tiles < 1 || L.tokens != 1 || L.cols < 64 || (L.cols & 63) || L.cols > MOE_FUSE_MAX_ROUTED) return -1;
     const dim3 grid(L.total_tiles);
-    if (L.total_tiles <= WIDE_TILE_LIMIT)
+    const int split = tile_split(L.total_tiles, L.cols);
+    if (split == 4)
+        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 3, 4>), dim3(4 * L.total_tiles), dim3(256), 0, stream, L);
+    else if (split == 2)
+        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 3, 2>), dim3(2 * L.total_tiles), dim3(512), 0, stream, L);
+    else if (L.total_tiles <= WIDE_TILE_LIMIT)
         hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 3>), grid, dim3(1024), 0, stream, L);
     else
         hipLaunchKernelGGL((q4_tile_kernel<4, 1, 16, 3>), grid, dim3(512), 0, stream, L);
@@ -695,9 +739,9 @@ int q4_launch(const Q4Launch &L, int chains_per_lane, hipStream_t stream) {
         S = L.total_tiles > WIDE_TILE_LIMIT ? 4 : 2;
     }
     switch (S) {
-        case 8: return launch_tiles<8>(L, stream);
-        case 4: return launch_tiles<4>(L, stream);
-        case 2: return launch_tiles<2>(L, stream);
+        case 8: return launch_tiles<8>(L, chains_per_lane == 0, stream);
+        case 4: return launch_tiles<4>(L, chains_per_lane == 0, stream);
+        case 2: return launch_tiles<2>(L, chains_per_lane == 0, stream);
         default: return -1;
     }
 }
