@@ -245,7 +245,7 @@ int salt_mi355_nvfp4_jobs_t_dev(const SaltMi355Fp4Job *jobs, int njobs, int C, i
 /* Prefill-sized NVFP4 matmul on the matrix cores (tolerance class): every
  * token is quantised and dequantised as salt_nvfp4_quantize_input_reference
  * does (nvfp4.c:82-130) and ys[token][row] approximates the reference matvec
- * (nvfp4.c:228-256) of that token: code * block scale is exact in bf16 for both
+ * (nvfp4.c:228-256) of that token: code * block scale is exact in fp16 for both
  * operands, products are exact, fp32 accumulation runs in the matrix cores'
  * order and the two per-tensor factors are applied once at the end.
  * xs: [B][C] fp32, ys: [B][R]; C a multiple of 64.  status_dev (optional device

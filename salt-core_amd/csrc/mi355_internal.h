@@ -144,7 +144,7 @@ int q4_dot_moe_down_launch(const MoeFuse &moe, hipStream_t stream);
 // ---------------------------------------------------------------- affine Q4 on MFMA (tolerance class)
 
 // One weight matrix against `tokens` activation rows that have been split
-// into three bf16 planes (x = hi + mid + lo) with per-64-column sums.
+// into two fp16 planes and notes on the row (see q4_mfma.hip).
 constexpr int MFMA_TM = 64;   // tokens per workgroup of the matrix-core kernel; its weight rows: mfma_tile_rows()
 
 struct MfmaJob {
@@ -175,7 +175,7 @@ struct MfmaLaunch {
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream);
 int mfma_tile_rows(int column_parts);
 int mfma_column_parts(long long wide_tiles, int ngrp);
-// rows of fp32 -> bf16 planes + group sums; output row r reads input row row_map[r] / map_divisor when a map is
+// rows of fp32 -> two fp16 planes + a plane of notes; output row r reads input row row_map[r] / map_divisor when a map is
 // given; with a gate the value split is gelu_tanh(gate) * x (gate has the layout of x)
 int x_split_launch(const float *x, const float *gate, const int *row_map, int map_divisor, int x_stride, int rows,
                    int cols, uint16_t *planes, size_t plane_stride, hipStream_t stream);
@@ -243,7 +243,7 @@ int fp4_qdq_flags_launch(const float *input, int cols, int tokens, float input_g
 // out_scale * sum_c (code * block scale)[row][c] * plane[token][c].
 struct Fp4MfmaLaunch {
     const uint8_t *packed, *scales;
-    const uint16_t *plane;    // [tokens][cols] bf16
+    const uint16_t *plane;    // [tokens][cols] fp16
     float *ys;                // [tokens][rows]
     float *partials;          // [ksplit][tokens][rows], used when ksplit > 1
     const int *status;        // nothing is published unless *status == 0 ...

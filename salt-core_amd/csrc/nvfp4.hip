@@ -97,8 +97,8 @@ __device__ __forceinline__ bool qdq_block(const float (&v)[16], float g, uint32_
         bytes[i >> 3] |= code << (4 * (i & 7));
         const float value = e2m1_decode(code);
         out[i] = value * from_code;
-        // code value * block scale: at most six significant bits, exact in bf16
-        const uint32_t h = __float_as_uint(value * scale) >> 16;
+        // code value * block scale: at most six significant bits between 2^-10 and 2688, exact in fp16
+        const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)(value * scale));
         if (i & 1) halves[i >> 1] |= h << 16; else halves[i >> 1] = h;
     }
     return true;

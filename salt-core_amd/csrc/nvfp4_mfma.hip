@@ -4,19 +4,29 @@
 // w_c = e2m1(code) * (e4m3(scale) * weight_global) and x_c the quantised and
 // dequantised activation e2m1(code) * (e4m3(scale) / input_global), in its
 // 32-chain order.  With hundreds of tokens the work is a dense contraction.
-// Both operands factor into a part that is exact in bf16,
-//     e2m1(code) * e4m3(block scale)        (two times four significant bits),
+// Both operands factor into a part that is exact in fp16,
+//     e2m1(code) * e4m3(block scale)        (two times four significant bits,
+//                                            between 2^-10 and 2688),
 // and a per-tensor fp32 factor, so the matrix cores see exact operands, the
 // products are exact in fp32 and only the order of the fp32 additions (and the
 // two per-tensor factors, applied once at the end) differs from the reference.
 //
-// Tiling: a workgroup of four waves computes 128 tokens x 128 weight rows, each
-// wave 64 x 64 as 2 x 2 blocks of v_mfma_f32_32x32x16_bf16.  Per 64-column chunk
-// the activation plane is copied and the weights are decoded (codes through
-// v_cvt_scalef32_pk_f32_fp4, scales through v_cvt_f32_fp8, one multiply, the
-// upper half kept) into one of two LDS stages with the next chunk's loads in
-// flight.  Long contractions with few tiles are split along the columns; the
-// partial sums are added in split order by a second kernel.
+// Tiling.  A wave computes 64 tokens x 64 weight rows as 2 x 2 blocks of
+// v_mfma_f32_32x32x16_f16.  The codes of its rows go through its own piece of
+// LDS, 128 bytes of a row at a time, to its registers and are decoded there:
+// one conversion and one packed multiply per pair, in the shadow of the matrix
+// instructions, and a quarter of the LDS reads that decoded weights would take
+// (with both operands read as 16-bit values the reads, 128 bytes per clock and
+// compute unit, took as long as the matrix work).  The token planes are staged
+// in LDS, 64 columns per stage, two stages.  Eight waves per workgroup, two per
+// SIMD: RW row blocks of 64 times 8 / RW parts of the columns, which meet in LDS
+// in part order; so a launch of 256 workgroups needs no partial sums in memory
+// and no second kernel.  Smaller ones are also split over workgroups, whose
+// partials a second kernel adds in split order.
+//
+// 8192 x 8192, 256 tokens: 64.2 -> 50.3 us with the activation pass, the kernel alone 51 + 9 (partial sums) -> 46.
+// Bound: lines from the cache to the compute unit (64 KB per stage of two rounds of matrix work, of which the planes
+// are half), then the matrix cores.
 #include "mi355_internal.h"
 
 #include <stddef.h>
@@ -24,21 +34,43 @@
 namespace mi355 {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef const u32x4 __attribute__((address_space(1))) *global_u128_ptr;
-typedef const uint16_t __attribute__((address_space(1))) *global_u16_ptr;
+typedef const uint8_t __attribute__((address_space(1))) *global_u8_ptr;
+typedef const void __attribute__((address_space(1))) *global_void_ptr;
+typedef float __attribute__((address_space(1))) *global_f32_out;
+typedef void __attribute__((address_space(3))) *lds_void_ptr;
+typedef const u32x4 __attribute__((address_space(3))) *lds_u128_ptr;
+typedef const uint32_t __attribute__((address_space(3))) *lds_u32_ptr;
 
-constexpr int TM = 128, TN = 128, KC = 64;
-constexpr int PITCH = 144;                     // bytes per staged row: 64 bf16 + 16 pad
-constexpr int A_BYTES = TM * PITCH, B_BYTES = TN * PITCH;
-constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
+constexpr int TM = 64, KC = 64, CH = 4;        // tokens per workgroup; columns per stage; stages per chunk of codes
+
+template <int WAVES, int RW> struct Shape {
+    static constexpr int KP = WAVES / RW;                            // parts of the columns
+    static constexpr int TN = 64 * RW;
+    static constexpr int X_BYTES = TM * 2 * KC;                      // one part's planes of one stage
+    static constexpr int STAGE_BYTES = KP * X_BYTES;
+    static constexpr int W_OFF = 2 * STAGE_BYTES, W_BYTES = 64 * 32 * CH;        // of one wave
+    static constexpr int S_OFF = W_OFF + WAVES * W_BYTES, S_BYTES = 64 * 4 * 2 * CH;
+    static constexpr int LDS_BYTES = S_OFF + WAVES * S_BYTES;
+    static constexpr int XT = TM / (8 * RW);                         // plane loads per wave and stage: eight tokens each
+    static constexpr int CODE_LOADS = 8;                             // per wave and chunk
+    static_assert((KP - 1) * RW * 64 * 64 * 4 <= S_OFF, "the parts' sums reuse the staging memory");
+};
 
 struct Geometry {
-    int m_tiles, n_tiles, chunks, chunks_per_split;
+    int m_tiles, n_tiles, chunks, chunks_per_split;                  // chunks of KC columns
 };
+
+// Piece p of a row lies at place p ^ place_mask(row): loads into LDS write 64 consecutive pieces, so rows cannot be
+// padded, and this spreads the sixteen rows of a read phase over all banks.
+__device__ __forceinline__ int place_mask(int row) { return (row >> 1) & 7; }
+
+template <int N> __device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 
 // Whether the activation pass rejected its input: the launch's status word, or the OR of the pass's per-workgroup
 // flags (every thread of the workgroup calls this; workgroup 0 then also publishes the outcome).
@@ -54,131 +86,255 @@ __device__ __forceinline__ bool rejected(const Fp4MfmaLaunch &L) {
     return any_bad != 0;
 }
 
-__device__ __forceinline__ uint32_t pack_upper_halves(float lo, float hi) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+// Eight E2M1 codes times their block's scale, in column order.
+__device__ __forceinline__ f16x8 weights_to_f16(uint32_t w, f16x2 s) {
+    u32x4 r;
+    r.x = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0)) * s));
+    r.y = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1)) * s));
+    r.z = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2)) * s));
+    r.w = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3)) * s));
+    return __builtin_bit_cast(f16x8, r);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void fp4_mfma_kernel(const Fp4MfmaLaunch L, const Geometry G) {
-    __shared__ __attribute__((aligned(16))) uint8_t stage[2 * STAGE_BYTES];
+template <int WAVES, int RW>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2))) void fp4_mfma_kernel(const Fp4MfmaLaunch L, const Geometry G) {
+    using S = Shape<WAVES, RW>;
+    __shared__ __attribute__((aligned(16))) uint8_t stage[S::LDS_BYTES];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int part = wave / RW, wn = wave % RW;
     const int l32 = lane & 31, half = lane >> 5;
 
-    // consecutive workgroups share a weight tile
-    const int mt = blockIdx.x % G.m_tiles;
-    const int nt = (blockIdx.x / G.m_tiles) % G.n_tiles;
-    const int split = blockIdx.x / (G.m_tiles * G.n_tiles);
-    const int tok0 = mt * TM, row0 = nt * TN;
+    // Workgroups go round the eight partitions of the device in turn; a partition takes one run of consecutive tiles,
+    // token tiles fastest, so that the tiles of the same weight rows meet in one partition's cache.
+    const int total = G.m_tiles * G.n_tiles * L.ksplit;
+    const int run = (total + 7) >> 3;
+    const int tile = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
+    const bool present = (int)(blockIdx.x >> 3) < run && tile < total;
+    if (!present) return;                           // uniform; workgroup 0 always has a tile
+    const int mt = tile % G.m_tiles, nt = (tile / G.m_tiles) % G.n_tiles, split = tile / (G.m_tiles * G.n_tiles);
+    const int tok0 = mt * TM, row0 = nt * S::TN + wn * 64;
     const int toks_here = L.tokens - tok0 < TM ? L.tokens - tok0 : TM;
-    const int rows_here = L.rows - row0 < TN ? L.rows - row0 : TN;
-    const int chunk0 = split * G.chunks_per_split;
-    const int chunk1 = chunk0 + G.chunks_per_split < G.chunks ? chunk0 + G.chunks_per_split : G.chunks;
+    const bool wide = toks_here > 32;               // both token blocks hold tokens
+    const bool live = row0 < L.rows;                // this wave has rows; the others only help to stage
     const int C = L.cols;
 
-    // activation plane: 128 tokens * 8 pieces of 16 bytes, four per thread
-    const global_u16_ptr plane = (global_u16_ptr)(uintptr_t)L.plane;
-    size_t a_src[4];
-    uint32_t a_dst[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int p = tid + i * 256;
-        const int tok = p >> 3, seg = p & 7;
-        const int tc = tok < toks_here ? tok : toks_here - 1;
-        a_src[i] = (size_t)(tok0 + tc) * C + seg * 8;
-        a_dst[i] = tok * PITCH + seg * 16;
-    }
-    // weights: 128 rows * 2 pieces of 32 codes (two scale blocks), one per thread
-    const int w_row = tid >> 1, w_half = tid & 1;
-    const int w_rc = w_row < rows_here ? w_row : rows_here - 1;
-    const global_u128_ptr w_src =
-        (global_u128_ptr)((uintptr_t)L.packed + (size_t)(row0 + w_rc) * (C >> 1) + w_half * 16);
-    const global_u16_ptr s_src = (global_u16_ptr)((uintptr_t)L.scales + (size_t)(row0 + w_rc) * (C >> 4) + w_half * 2);
+    // the split's columns, and the part's: `iterations` stages from first on, those from end on staged and unused
+    const int split0 = split * G.chunks_per_split;
+    const int split1 = split0 + G.chunks_per_split < G.chunks ? split0 + G.chunks_per_split : G.chunks;
+    const int even = (split1 - split0 + S::KP - 1) / S::KP;
+    const int iterations = even >= 4 * CH ? (even + CH - 1) / CH * CH : even;       // whole cache lines where it matters little
+    const int first = split0 + part * iterations;
+    const int end = first + iterations < split1 ? first + iterations : split1;
+    const int last_chunk = G.chunks - 1;
 
-    u32x4 areg[4], wreg;
-    uint32_t sreg = 0;
-    auto issue = [&](int chunk) {
+    // load i of a wave brings the eight token rows from (i * RW + wn) * 8 on; which piece of its row a lane fetches
+    // follows from the place that the load will put it in
+    const global_u8_ptr plane = (global_u8_ptr)(uintptr_t)L.plane + (size_t)tok0 * (size_t)(2 * C);
+    uint32_t x_src[S::XT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) areg[i] = *(global_u128_ptr)(plane + a_src[i] + (size_t)chunk * KC);
-        wreg = w_src[chunk * 2];
-        sreg = s_src[chunk * 2];
+    for (int i = 0; i < S::XT; ++i) {
+        const int r = (i * RW + wn) * 8 + (lane >> 3);
+        x_src[i] = (uint32_t)(r < toks_here ? r : toks_here - 1) * (uint32_t)(2 * C) + (uint32_t)((lane & 7) ^ place_mask(r)) * 16u;
+    }
+    const int rows_left = live ? L.rows - row0 : 1;
+    const int row_base = live ? row0 : 0;           // waves without rows fetch the first row and use nothing
+    const global_u8_ptr codes = (global_u8_ptr)(uintptr_t)L.packed + (size_t)row_base * (size_t)(C >> 1);
+    const global_u8_ptr scale_rows = (global_u8_ptr)(uintptr_t)L.scales + (size_t)row_base * (size_t)(C >> 4);
+
+    // Everything staged goes from memory into LDS without passing through registers, so that a wave's loads complete
+    // in the order they were sent in and a wait can leave the younger ones in flight.
+    auto issue_x = [&](int it) {
+        const int g = first + it < G.chunks ? first + it : last_chunk;
+        uint32_t at = (uint32_t)g * (2 * KC);
+        asm volatile("" : "+s"(at));
+        uint8_t *const x = stage + (it & 1) * S::STAGE_BYTES + part * S::X_BYTES + wn * 1024;
+#pragma unroll
+        for (int i = 0; i < S::XT; ++i) {
+            if (i * RW * 8 >= 32 && !wide) break;
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(plane + (x_src[i] + at)), (lds_void_ptr)(x + i * (RW * 1024)),
+                                             16, 0, 0);
+        }
     };
-    auto commit = [&](uint8_t *base) {
+    // A row's scales of a chunk are 16 bytes.  They come in one load where addresses allow it: 64 rows are 64 cache
+    // lines to look up however little of them is wanted, and eight loads of two bytes took longer than the matrix work.
+    const bool whole_scales = ((uintptr_t)L.scales & 3) == 0 && G.chunks >= CH;
+    auto issue_weights = [&](int it) {               // the chunk that starts with stage `it` of the part
+        const uint32_t at = (uint32_t)(first + it) * 32u, last = (uint32_t)G.chunks * 32u - 16u;
+        uint32_t lane_row = (uint32_t)lane >> 3;
+        uint32_t scale_at = (uint32_t)(lane < rows_left ? lane : rows_left - 1) * (uint32_t)(C >> 4);
+        asm volatile("" : "+v"(lane_row), "+v"(scale_at));   // addresses are made here, not kept in registers
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4 *>(base + a_dst[i]) = areg[i];
-        const uint32_t words[4] = {wreg.x, wreg.y, wreg.z, wreg.w};
-        uint32_t out[16];
+        for (int j = 0; j < 8; ++j) {
+            uint32_t r = j * 8 + lane_row;
+            uint32_t byte = at + (((uint32_t)lane & 7u) ^ (uint32_t)place_mask((int)r)) * 16u;
+            byte = byte < last ? byte : last;
+            r = r < (uint32_t)rows_left ? r : (uint32_t)rows_left - 1u;
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(codes + (__umul24(r, (uint32_t)(C >> 1)) + byte)),
+                                             (lds_void_ptr)(stage + S::W_OFF + wave * S::W_BYTES + j * 1024), 16, 0, 0);
+        }
+        if (whole_scales) {                          // a chunk's scales of a row at once, from the row's end backwards
+            const uint32_t s_at = (uint32_t)(first + it) * 4u, s_last = (uint32_t)G.chunks * 4u - 16u;
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(scale_rows + (scale_at + (s_at < s_last ? s_at : s_last))),
+                                             (lds_void_ptr)(stage + S::S_OFF + wave * S::S_BYTES), 16, 0, 0);
+            return;
+        }
 #pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
-            const float s = blk ? __builtin_amdgcn_cvt_f32_fp8((int)sreg, 1) : __builtin_amdgcn_cvt_f32_fp8((int)sreg, 0);
+        for (int k = 0; k < 2 * CH; ++k) {           // the two scales of each half of each stage
+            const int g = first + it + (k >> 1) < G.chunks ? first + it + (k >> 1) : last_chunk;
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(scale_rows + (scale_at + (uint32_t)(g * 4 + (k & 1) * 2))),
+                                             (lds_void_ptr)(stage + S::S_OFF + wave * S::S_BYTES + k * 256), 2, 0, 0);
+        }
+    };
+    struct Weights { u32x4 w[CH][2]; uint32_t s[CH][2]; };
+    auto take_weights = [&](int it, Weights &r) {    // and leave their place to the next chunk
+        const lds_u128_ptr w = (lds_u128_ptr)(stage + S::W_OFF + wave * S::W_BYTES);
+        const lds_u32_ptr sc = (lds_u32_ptr)(stage + S::S_OFF + wave * S::S_BYTES);
+        const int beyond = first + it - (G.chunks - CH), back = beyond > 0 ? beyond : 0;     // stages fetched from before the chunk
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const uint32_t w = words[blk * 2 + (b >> 2)];
-                f32x2 v;
-                switch (b & 3) {
-                    case 0: v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0); break;
-                    case 1: v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1); break;
-                    case 2: v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2); break;
-                    default: v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3); break;
-                }
-                out[blk * 8 + b] = pack_upper_halves(v.x * s, v.y * s);
+        for (int nb = 0; nb < 2; ++nb) {
+            const int at = (nb * 32 + l32) * 8, turn = place_mask(nb * 32 + l32);
+#pragma unroll
+            for (int gi = 0; gi < CH; ++gi) {
+                r.w[gi][nb] = w[at + ((gi * 2 + half) ^ turn)];
+                const int g = gi + back < CH ? gi + back : CH - 1;
+                if (whole_scales) r.s[gi][nb] = sc[(nb * 32 + l32) * 4 + g];
+                else r.s[gi][nb] = sc[(gi * 2 + half) * 64 + nb * 32 + l32];
             }
         }
-        u32x4 *dst = reinterpret_cast<u32x4 *>(base + A_BYTES + w_row * PITCH + w_half * 64);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (whole_scales) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) dst[q] = u32x4{out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]};
+            for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+                for (int gi = 0; gi < CH; ++gi) r.s[gi][nb] >>= half * 16;
+        }
     };
 
     const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     f32x16 acc[2][2] = {{zero, zero}, {zero, zero}};
 
-    issue(chunk0);
-    commit(stage);
+    issue_weights(0);
+    issue_x(0);
+    wait_loads<0>();
     __syncthreads();
-    for (int chunk = chunk0; chunk < chunk1; ++chunk) {
-        const uint8_t *cur = stage + ((chunk - chunk0) & 1) * STAGE_BYTES;
-        if (chunk + 1 < chunk1) issue(chunk + 1);
-        const uint8_t *arow = cur + (wm * 64 + l32) * PITCH + half * 16;
-        const uint8_t *brow = cur + A_BYTES + (wn * 64 + l32) * PITCH + half * 16;
+    if (iterations > 1) issue_x(1);
+
+    // The two lane halves of an instruction take columns 32 h + 8 k .. + 7 of a stage, so that a lane's codes of a
+    // stage are 16 consecutive bytes and its scales two.  While the matrix cores work on a step of 16 columns the
+    // operands of the next one are read and decoded; the workgroup meets before the last step of a stage, when its
+    // planes are in everybody's registers and their place can take the stage after the next one.
+    if (live) {
+        const int mix = place_mask(l32);             // rows 32 apart share it
+        Weights now;
+        f16x8 a[2][2], b[2][2];
+        auto read = [&](int it, int step, f16x8 (&to)[2]) {
+            const lds_u128_ptr x = (lds_u128_ptr)(stage + (it & 1) * S::STAGE_BYTES + part * S::X_BYTES + l32 * (2 * KC));
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            bf16x8 a[2], b[2];
+            for (int mb = 0; mb < 2; ++mb) to[mb] = __builtin_bit_cast(f16x8, x[mb * (32 * 8) + ((half * 4 + step) ^ mix)]);
+        };
+        auto decode = [&](const u32x4 (&w)[2], const uint32_t (&bits)[2], int step, bool inside, f16x8 (&to)[2]) {
 #pragma unroll
-            for (int blk = 0; blk < 2; ++blk) {
-                a[blk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(arow + blk * 32 * PITCH + ks * 32));
-                b[blk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(brow + blk * 32 * PITCH + ks * 32));
+            for (int nb = 0; nb < 2; ++nb) {
+                const uint32_t pair = inside ? bits[nb] : 0u;
+                const float scale = step < 2 ? __builtin_amdgcn_cvt_f32_fp8((int)pair, 0) : __builtin_amdgcn_cvt_f32_fp8((int)pair, 1);
+                const _Float16 h = (_Float16)scale;
+                to[nb] = weights_to_f16(w[nb][step], f16x2{h, h});
             }
+        };
+        auto multiply = [&](const f16x8 (&x)[2], const f16x8 (&w)[2]) {
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb)
-                    acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mb], b[nb], acc[mb][nb], 0, 0, 0);
-        }
-        if (chunk + 1 < chunk1) commit(stage + ((chunk + 1 - chunk0) & 1) * STAGE_BYTES);
-        __syncthreads();
-    }
-
-    const bool direct = L.ksplit == 1;
-    if (direct && rejected(L)) return;
-    float __attribute__((address_space(1))) *out =
-        (float __attribute__((address_space(1))) *)(uintptr_t)(direct ? L.ys
-                                                                      : L.partials + (size_t)split * L.tokens * L.rows);
-    const float factor = direct ? L.out_scale : 1.0f;
+                    acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[mb], w[nb], acc[mb][nb], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+            for (int k = 0; k < 4; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        take_weights(0, now);
+        if (CH < iterations) issue_weights(CH);
+        read(0, 0, a[0]);
+        decode(now.w[0], now.s[0], 0, first < end, b[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int it0 = 0; it0 < iterations; it0 += CH) {
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const int row = wn * 64 + nb * 32 + l32;
-            if (row >= rows_here) continue;
+            for (int gi = 0; gi < CH; ++gi) {
+                const int it = it0 + gi;
+                const bool inside = first + it < end;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int tok = wm * 64 + mb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                if (tok < toks_here) out[(size_t)(tok0 + tok) * L.rows + row0 + row] = acc[mb][nb][i] * factor;
+                for (int step = 0; step < 3; ++step) {
+                    read(it, step + 1, a[(step + 1) & 1]);
+                    decode(now.w[gi], now.s[gi], step + 1, inside, b[(step + 1) & 1]);
+                    multiply(a[step & 1], b[step & 1]);
+                }
+                // made here and not sunk to the use behind the workgroup's meeting, where nothing covers it
+                asm volatile("" : "+v"(b[1][0]), "+v"(b[1][1]));
+                // the next planes were sent for before the chunk that may still be on its way
+                if (gi == 0 && it0 + CH < iterations) {
+                    if (whole_scales) wait_loads<S::CODE_LOADS + 1>(); else wait_loads<S::CODE_LOADS + 2 * CH>();
+                } else {
+                    wait_loads<0>();
+                }
+                __syncthreads();
+                if (it + 2 < iterations) issue_x(it + 2);
+                if (gi == CH - 1) {
+                    take_weights(it + 1, now);
+                    if (it + 1 + CH < iterations) issue_weights(it + 1 + CH);
+                }
+                // after the last stage these are stale and unused
+                read(it + 1, 0, a[0]);
+                decode(now.w[gi == CH - 1 ? 0 : gi + 1], now.s[gi == CH - 1 ? 0 : gi + 1], 0, first + it + 1 < end, b[0]);
+                multiply(a[1], b[1]);
+                if (it + 1 >= iterations) break;
             }
         }
+    } else {
+        for (int it = 0; it < iterations; ++it) {    // a wave without rows helps to stage
+            wait_loads<0>();
+            __syncthreads();
+            if (it + 2 < iterations) issue_x(it + 2);
+        }
+    }
+
+    // ---- the parts meet in part order
+    float *sums = reinterpret_cast<float *>(stage);
+    if (S::KP > 1) __syncthreads();
+    if (part > 0) {
+        float *mine = sums + ((part - 1) * RW + wn) * 4096 + lane;
+#pragma unroll
+        for (int k = 0; k < 64; ++k) mine[k * 64] = acc[k >> 5][(k >> 4) & 1][k & 15];
+    }
+    if (S::KP > 1) __syncthreads();
+    const bool direct = L.ksplit == 1;
+    if (direct && rejected(L)) return;
+    if (part != 0 || !live) return;
+#pragma unroll
+    for (int p = 1; p < S::KP; ++p) {
+        const float *theirs = sums + ((p - 1) * RW + wn) * 4096 + lane;
+#pragma unroll
+        for (int k = 0; k < 64; ++k) acc[k >> 5][(k >> 4) & 1][k & 15] += theirs[k * 64];
+    }
+    const global_f32_out out = (global_f32_out)(uintptr_t)(direct ? L.ys : L.partials + (size_t)split * L.tokens * L.rows);
+    const float factor = direct ? L.out_scale : 1.0f;
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) {
+        global_f32_out line = out + (size_t)(tok0 + mb * 32 + half * 4) * L.rows + row0 + l32;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int tok = mb * 32 + half * 4 + (i >> 2) * 8 + (i & 3);
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+                if (tok < toks_here && row0 + nb * 32 + l32 < L.rows) line[nb * 32] = acc[mb][nb][i] * factor;
+            line += (size_t)L.rows * ((i & 3) == 3 ? 5 : 1);
+        }
+    }
 }
 
 // ys = out_scale * (partial 0 + partial 1 + ...), added in split order
@@ -209,12 +365,21 @@ __global__ __launch_bounds__(256) void fp4_split_sum_kernel(const Fp4MfmaLaunch 
 
 }  // namespace
 
+namespace {
+// Tiles of 64 x 256 by four waves, two workgroups on a compute unit, where there are enough of them; else tiles of
+// 64 x 128 by eight waves, four column parts.
+bool wide_tiles(int rows, int tokens) {
+    return (long long)((tokens + TM - 1) / TM) * ((rows + 255) / 256) >= 320;
+}
+}  // namespace
+
 int fp4_mfma_splits(int rows, int cols, int tokens) {
-    const int tiles = ((tokens + TM - 1) / TM) * ((rows + TN - 1) / TN);
+    const int tn = wide_tiles(rows, tokens) ? 256 : 128;
+    const int tiles = ((tokens + TM - 1) / TM) * ((rows + tn - 1) / tn);
     const int chunks = cols / KC;
-    int splits = (512 + tiles - 1) / tiles;            // aim at two workgroups per compute unit
+    int splits = 256 / tiles;                          // while every workgroup still has a compute unit of its own
     if (splits > 8) splits = 8;
-    if (splits > chunks / 4) splits = chunks / 4;      // at least four chunks per split
+    if (splits > chunks / 8) splits = chunks / 8;      // at least eight chunks per split, two per part
     // with chunks shared out in equal runs the last split must still own one (30 chunks in 7 splits of 5 would not)
     while (splits > 1 && (splits - 1) * ((chunks + splits - 1) / splits) >= chunks) --splits;
     return splits < 1 ? 1 : splits;
@@ -223,16 +388,20 @@ int fp4_mfma_splits(int rows, int cols, int tokens) {
 int fp4_mfma_launch(const Fp4MfmaLaunch &L, hipStream_t stream) {
     if (L.rows < 1 || L.tokens < 1 || L.cols < KC || (L.cols % KC) || L.ksplit < 1) return -1;
     if (L.flags ? (L.nflags < 1 || !L.outcome) : !L.status) return -1;
+    const bool wide = wide_tiles(L.rows, L.tokens);
+    const int tn = wide ? 256 : 128;
     Geometry G;
     G.m_tiles = (L.tokens + TM - 1) / TM;
-    G.n_tiles = (L.rows + TN - 1) / TN;
+    G.n_tiles = (L.rows + tn - 1) / tn;
     G.chunks = L.cols / KC;
     G.chunks_per_split = (G.chunks + L.ksplit - 1) / L.ksplit;
     if ((L.ksplit - 1) * G.chunks_per_split >= G.chunks) return -1;        // every split owns a chunk
     if (L.ksplit > 1 && !L.partials) return -1;
-    const long long grid = (long long)G.m_tiles * G.n_tiles * L.ksplit;
+    if (L.cols > (1 << 24)) return -1;                                     // 32-bit offsets inside a tile
+    const long long grid = ((long long)G.m_tiles * G.n_tiles * L.ksplit + 7) / 8 * 8;
     if (grid > 0x7FFFFFFFLL) return -1;
-    hipLaunchKernelGGL(fp4_mfma_kernel, dim3((unsigned)grid), dim3(256), 0, stream, L, G);
+    if (wide) hipLaunchKernelGGL((fp4_mfma_kernel<4, 4>), dim3((unsigned)grid), dim3(256), 0, stream, L, G);
+    else hipLaunchKernelGGL((fp4_mfma_kernel<8, 2>), dim3((unsigned)grid), dim3(512), 0, stream, L, G);
     if (L.ksplit > 1) {
         const size_t n = (size_t)L.tokens * L.rows;
         hipLaunchKernelGGL(fp4_split_sum_kernel, dim3((unsigned)((n / 4 + 256) / 256)), dim3(256), 0, stream, L, n);
