@@ -166,10 +166,11 @@ constexpr int x_batch_groups(int S, int NB) {
 // activations come from LDS as in the prologues above.
 // One token: 2816 x 2816 (44 tiles) 10.8 -> 6.8 us.
 template <int S, int NB, int CB, int PRO = 0, int SPLIT = 1>
-__global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const Q4Launch L) {
+__global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 1) void q4_tile_kernel(const Q4Launch L) {
     constexpr int CHUNK_BLOCKS = CB;
     constexpr int ROWS = TILE_ROWS / SPLIT;
     constexpr bool LDS_X = PRO >= 2 || SPLIT > 1;
+    constexpr bool STEP_X = SPLIT > 1 && S == 4;           // activations staged with each step's weights, not the whole row
     constexpr int CHUNK_GROUPS = CB / 2;                   // 64-column scale groups per step
     constexpr int W_PITCH = 16 * CB + 4;                   // bytes per staged row: odd dword pitch
     constexpr int M_PITCH = 2 * CHUNK_GROUPS + 2;          // floats per staged row of (scale, bias)
@@ -181,14 +182,14 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const 
     constexpr int ITEMS = (ROWS * CHUNK_GROUPS + THREADS - 1) / THREADS;
     constexpr int FOLD_BYTES = NB * ROWS * FOLD_PITCH * 4;
     constexpr int W_BYTES = 2 * W_STAGE > FOLD_BYTES ? 2 * W_STAGE : FOLD_BYTES;
-    constexpr int XG = LDS_X ? 2 : x_batch_groups(S, NB);        // LDS-fed activations sit in vector registers: short batches
+    constexpr int XG = STEP_X && NB >= 3 ? 1 : LDS_X ? 2 : x_batch_groups(S, NB);        // LDS-fed activations sit in vector registers: short batches
     constexpr int XN = XG * 2 * S;
     static_assert(THREADS >= NB * ROWS, "fold needs one thread per (token, row)");
-    static_assert(SPLIT == 1 || (NB == 1 && PRO != 2), "split tiles serve single tokens; the down launch counts whole tiles");
+    static_assert(SPLIT == 1 || (PRO != 2 && (NB == 1 || STEP_X)), "the down launch counts whole tiles; LDS holds one whole row");
 
     __shared__ __attribute__((aligned(16))) uint8_t w_lds[W_BYTES];
     __shared__ __attribute__((aligned(16))) float m_lds[2 * M_STAGE];
-    __shared__ __attribute__((aligned(16))) float x_lds[PRO >= 2 ? MOE_FUSE_MAX_ROUTED : SPLIT > 1 ? SPLIT_MAX_COLS : 4];
+    __shared__ __attribute__((aligned(16))) float x_lds[PRO >= 2 ? MOE_FUSE_MAX_ROUTED : STEP_X ? 2 * NB * CB * 32 : SPLIT > 1 ? SPLIT_MAX_COLS : 4];
     __shared__ int slow_flag;
     static_assert(PRO == 0 || NB == 1, "the MoE prologues serve the single-token kernel");
     static_assert(PRO != 1 || (sizeof(RouterShared) <= W_BYTES && THREADS >= MOE_FUSE_MAX_EXPERTS),
@@ -304,6 +305,14 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const 
     u32x4 wreg[ITEMS][2];
     uint32_t sreg[ITEMS], breg[ITEMS];               // raw bf16 bits; nothing may consume them before commit
 
+    // STEP_X: value k of a thread belongs to token k * THREADS / X_STEP
+    constexpr int X_STEP = CB * 32;
+    constexpr int X_ITEMS = STEP_X ? NB * X_STEP / THREADS : 1;
+    static_assert(!STEP_X || X_STEP % THREADS == 0, "a thread's values of one token lie THREADS apart");
+    const float __attribute__((address_space(1))) *const x_rows = (const float __attribute__((address_space(1))) *)(uintptr_t)job.x;
+    float xreg[X_ITEMS];
+    const float *x_step = x_lds;                           // STEP_X: column 0 of the row whose step lies in x_lds
+
     // Loads of step ck into registers.  In every step but a partial last one
     // the address is a wave-uniform base plus the fixed per-thread offset; in
     // the last one group indices past the end of the row are clamped (the data
@@ -315,6 +324,13 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const 
         return NB > 1 ? __builtin_nontemporal_load((global_u128_ptr)p) : *(global_u128_ptr)p;
     };
     auto issue = [&](int ck) {
+        if (STEP_X) {
+#pragma unroll
+            for (int k = 0; k < X_ITEMS; ++k) {
+                const int c = ck * X_STEP + (k * THREADS) % X_STEP + tid;
+                xreg[k] = c < L.cols ? x_rows[(size_t)((k * THREADS) / X_STEP) * job.x_stride + c] : 0.0f;
+            }
+        }
         if (!has_item) return;
         const bool tail = (ck + 1) * CHUNK_GROUPS > ngrp;
         if (!tail) {
@@ -344,6 +360,10 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const 
     };
 
     auto commit = [&](int stage) {
+        if (STEP_X) {
+#pragma unroll
+            for (int k = 0; k < X_ITEMS; ++k) x_lds[stage * (NB * X_STEP) + k * THREADS + tid] = xreg[k];
+        }
         if (!has_item) return;
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
@@ -375,10 +395,9 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const 
     if (PRO >= 2) {
         // after the first weights have been sent for: they are on their way while the activation is computed
         for (int i = tid; i < L.cols; i += THREADS) x_lds[i] = det_gelu_tanh(act_gate[i]) * act_up[i];
-    } else if (SPLIT > 1) {
-        const float __attribute__((address_space(1))) *src = (const float __attribute__((address_space(1))) *)(uintptr_t)job.x;
+    } else if (SPLIT > 1 && !STEP_X) {
 #pragma unroll 4
-        for (int i = tid; i < L.cols; i += THREADS) x_lds[i] = src[i];
+        for (int i = tid; i < L.cols; i += THREADS) x_lds[i] = x_rows[i];
     }
     __syncthreads();
 
@@ -387,10 +406,12 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const 
     // x of `groups` consecutive scale groups starting at group g0 of the row
     auto load_x = [&](int g0, float (&xq)[NB][XN], int groups) {
         if (LDS_X) {                      // every lane of a slice reads the same LDS words: the activations travel in vector registers
-            const float *xl = x_lds + g0 * 64 + S * slice;
+            const float *xl = x_step + g0 * 64 + S * slice;
 #pragma unroll
-            for (int k = 0; k < XN; ++k)
-                if (k < groups * 2 * S) xq[0][k] = xl[(k / S) * 32 + (k % S)];
+            for (int t = 0; t < NB; ++t)
+#pragma unroll
+                for (int k = 0; k < XN; ++k)
+                    if (k < groups * 2 * S) xq[t][k] = xl[t * X_STEP + (k / S) * 32 + (k % S)];
             return;
         }
         const uniform_f32_ptr xg = xbase + (size_t)g0 * 64;
@@ -410,10 +431,14 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64) void q4_tile_kernel(const 
         // The first batch of activations is requested before the barrier so
         // that its latency overlaps the staging writes and the wait.
         float xq[NB][XN];
-        if (full) load_x(ck * CHUNK_GROUPS, xq, XG);
+        if (full && !STEP_X) load_x(ck * CHUNK_GROUPS, xq, XG);
 
         commit(stage);
         __syncthreads();
+        if (STEP_X) {
+            x_step = x_lds + stage * (NB * X_STEP) - ck * X_STEP;
+            if (full) load_x(ck * CHUNK_GROUPS, xq, XG);
+        }
         if (ck + 1 < nchunk) issue(ck + 1);
 
         const int slow = __builtin_amdgcn_readfirstlane(slow_flag);
@@ -638,6 +663,22 @@ int launch_tiles(const Q4Launch &L, bool may_split, hipStream_t stream) {
     if (L.tokens == 1 && S <= 4 && L.total_tiles <= WIDE_TILE_LIMIT) {
         note_kernel("q4_tile_kernel<%d,1,32,0>", S);
         hipLaunchKernelGGL((q4_tile_kernel<S, 1, 32>), grid, block, 0, stream, L);
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
+    if (S == 4 && may_split && L.total_tiles > WIDE_TILE_LIMIT && L.total_tiles <= WIDE_TILE_LIMIT * 3 / 2) {
+        // Between one tile and one and a half per compute unit, some compute units have two and the rest wait for them:
+        // in halves they have three of them at most (264 tiles of 2816 columns, one to four tokens: 14.8 / 20.7 / 22.7 / 28.6
+        // us whole, 13.2 / 18.0 / 20.0 / 23.6 in halves).  Three waves a SIMD need 168 registers or fewer: without that
+        // bound three and four tokens took 26.9 and 32.2 us.
+        note_kernel("q4_tile_kernel<4,%d,16,0,2>", L.tokens);
+        const dim3 halves(2 * L.total_tiles);
+        switch (L.tokens) {
+            case 1: hipLaunchKernelGGL((q4_tile_kernel<4, 1, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
+            case 2: hipLaunchKernelGGL((q4_tile_kernel<4, 2, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
+            case 3: hipLaunchKernelGGL((q4_tile_kernel<4, 3, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
+            case 4: hipLaunchKernelGGL((q4_tile_kernel<4, 4, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
+            default: return -1;
+        }
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     note_kernel("q4_tile_kernel<%d,%d,16,0>", S, L.tokens);

@@ -29,6 +29,19 @@ def test_q4_parts_of_tiles(pkg, oracle, R, C):
     assert np.array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("R,C,B", [(16385, 576, 1), (16500, 512, 2), (20000, 64, 3), (24576, 1088, 4), (24577, 128, 3)])
+def test_q4_halves_between_one_and_one_and_a_half_tiles_per_compute_unit(pkg, oracle, R, C, B):
+    print(f"q4 halves R={R} C={C} B={B}", flush=True)
+    vals, scales, biases = synth.q4_tensor(R, C, R + C)
+    xs = synth.activations(C, B, 33)
+    got = pkg.lib.q4_matvec(vals, scales, biases, R, C, xs)
+    want = np.zeros((B, R), np.float32)
+    for t in range(B):
+        assert oracle.orc_q4_matvec_threads(ptr(vals), ptr(scales), ptr(biases), R, C, ptr(xs[t]), ptr(want[t]),
+                                            host_threads()) == 0
+    assert np.array_equal(bits(got), bits(want))
+
+
 @pytest.mark.parametrize("R,C", [(1, 64), (31, 544), (33, 4096), (100, 8192), (4096, 96), (4097, 96), (8192, 64), (8193, 64)])
 def test_nvfp4_parts_of_tiles(pkg, oracle, R, C):
     print(f"nvfp4 split R={R} C={C}", flush=True)
