@@ -170,7 +170,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
     constexpr int CHUNK_BLOCKS = CB;
     constexpr int ROWS = TILE_ROWS / SPLIT;
     constexpr bool LDS_X = PRO >= 2 || SPLIT > 1;
-    constexpr bool STEP_X = SPLIT > 1 && S == 4;           // activations staged with each step's weights, not the whole row
+    constexpr bool STEP_X = SPLIT > 1 && (S == 4 || NB > 1);   // activations staged with each step's weights, not the whole row
     constexpr int CHUNK_GROUPS = CB / 2;                   // 64-column scale groups per step
     constexpr int W_PITCH = 16 * CB + 4;                   // bytes per staged row: odd dword pitch
     constexpr int M_PITCH = 2 * CHUNK_GROUPS + 2;          // floats per staged row of (scale, bias)
@@ -640,10 +640,10 @@ __global__ __launch_bounds__(256) void q4_generic_kernel(const Q4Launch L) {
 // Launches of at most this many tiles (one per compute unit) use the wide-step variant and two chains per lane.
 constexpr int WIDE_TILE_LIMIT = 256;
 
-// Workgroups per tile of a single-token launch, as long as that gives more compute units work: sixteen-row workgroups up
+// Workgroups per tile of a launch, as long as that gives more compute units work: sixteen-row workgroups up
 // to 96 tiles (beyond, the compute units that hold two of them take as long as with thirty-two rows), thirty-two-row ones
 // up to one per compute unit.  us before and after: 44 tiles of 2816 columns 10.8 / 6.8, of 8192 24.1 / 13.8, 96 of 2816
-// 10.9 / 7.5, 128 of 8192 25.7 / 17.3.
+// 10.9 / 7.5, 128 of 8192 25.7 / 17.3; three tokens: 44 of 2816 16.4 / 10.7, 128 of 4096 22.1 / 14.3.
 int tile_split(int tiles, int cols) {
     if (cols > SPLIT_MAX_COLS) return 1;
     return tiles <= 96 ? 4 : 2 * tiles <= WIDE_TILE_LIMIT ? 2 : 1;
@@ -652,7 +652,21 @@ int tile_split(int tiles, int cols) {
 template <int S>
 int launch_tiles(const Q4Launch &L, bool may_split, hipStream_t stream) {
     const dim3 grid(L.total_tiles), block((32 / S) * 64);
-    const int split = S == 2 && L.tokens == 1 && may_split ? tile_split(L.total_tiles, L.cols) : 1;
+    const int split = S == 2 && may_split ? tile_split(L.total_tiles, L.tokens == 1 ? L.cols : 0) : 1;
+    if (split > 1 && L.tokens > 1) {
+        note_kernel("q4_tile_kernel<2,%d,16,0,%d>", L.tokens, split);
+        const dim3 parts(split * L.total_tiles), threads(1024 / split);
+        switch (L.tokens * 8 + split) {
+            case 2 * 8 + 2: hipLaunchKernelGGL((q4_tile_kernel<2, 2, 16, 0, 2>), parts, threads, 0, stream, L); break;
+            case 3 * 8 + 2: hipLaunchKernelGGL((q4_tile_kernel<2, 3, 16, 0, 2>), parts, threads, 0, stream, L); break;
+            case 4 * 8 + 2: hipLaunchKernelGGL((q4_tile_kernel<2, 4, 16, 0, 2>), parts, threads, 0, stream, L); break;
+            case 2 * 8 + 4: hipLaunchKernelGGL((q4_tile_kernel<2, 2, 16, 0, 4>), parts, threads, 0, stream, L); break;
+            case 3 * 8 + 4: hipLaunchKernelGGL((q4_tile_kernel<2, 3, 16, 0, 4>), parts, threads, 0, stream, L); break;
+            case 4 * 8 + 4: hipLaunchKernelGGL((q4_tile_kernel<2, 4, 16, 0, 4>), parts, threads, 0, stream, L); break;
+            default: return -1;
+        }
+        return hipGetLastError() == hipSuccess ? 0 : -1;
+    }
     if (split > 1) {
         note_kernel("q4_tile_kernel<2,1,32,0,%d>", split);
         if (split == 4) hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 0, 4>), dim3(4 * L.total_tiles), dim3(256), 0, stream, L);

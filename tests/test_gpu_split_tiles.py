@@ -1,6 +1,6 @@
-"""Single-token launches with few tiles run on parts of a tile (sixteen or thirty-two rows per workgroup, several chain
-slices per wave): the same bits as the CPU checker at the edges of the parts, of the tiles, of the rule's ranges and of the
-columns that the parts keep in LDS."""
+"""Launches with few tiles, or with up to one and a half per compute unit, run on parts of a tile (sixteen or thirty-two
+rows per workgroup, several chain slices per wave): the same bits as the CPU checker at the edges of the parts, of the
+tiles, of the rule's ranges and of the columns that the parts keep in LDS."""
 import numpy as np
 import pytest
 
@@ -29,9 +29,10 @@ def test_q4_parts_of_tiles(pkg, oracle, R, C):
     assert np.array_equal(bits(got), bits(want))
 
 
-@pytest.mark.parametrize("R,C,B", [(16385, 576, 1), (16500, 512, 2), (20000, 64, 3), (24576, 1088, 4), (24577, 128, 3)])
-def test_q4_halves_between_one_and_one_and_a_half_tiles_per_compute_unit(pkg, oracle, R, C, B):
-    print(f"q4 halves R={R} C={C} B={B}", flush=True)
+@pytest.mark.parametrize("R,C,B", [(1, 64, 2), (17, 8256, 3), (65, 576, 4), (6145, 192, 2), (8192, 128, 4), (8193, 128, 3),
+                                   (16385, 576, 1), (16500, 512, 2), (20000, 64, 3), (24576, 1088, 4), (24577, 128, 3)])
+def test_q4_parts_with_staged_activations(pkg, oracle, R, C, B):
+    print(f"q4 staged R={R} C={C} B={B}", flush=True)
     vals, scales, biases = synth.q4_tensor(R, C, R + C)
     xs = synth.activations(C, B, 33)
     got = pkg.lib.q4_matvec(vals, scales, biases, R, C, xs)
