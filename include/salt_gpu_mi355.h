@@ -167,6 +167,8 @@ int salt_mi355_q4_jobs_t_dev(const SaltMi355Q4Job *jobs, int njobs, int C, int t
  *   |error| <= 2^-20 * sum_c (|q_c s| + 16 |s| + |b|) |x_c| + 1e-6
  * (and <= 2^-18 * sum_c |w*x| + 1e-6 for activations without outliers).  Needs
  * C % 64 == 0 and device scratch of salt_mi355_q4_matmul_workspace_bytes().
+ * R and B choose how the columns are shared out and with it the order of the
+ * sums: the bits are the same for the same call, not for any other B.
  * The reference has no counterpart: its CPU and GPU paths keep the 32-chain
  * order at every batch size (kernels.c:1252-1261). */
 size_t salt_mi355_q4_matmul_workspace_bytes(int C, int B);
@@ -415,7 +417,8 @@ int salt_mi355_moe_decode_step_static_dev(const void *pool, size_t expert_stride
  * expert / token / rank order, :211-224 weighted sum over ranks in rank order
  * from +0; per-expert arithmetic gemma4_text.c:8749-9137).  The bucketing is
  * exact; the projections run on the matrix-core kernel of
- * salt_mi355_q4_matmul_dev and carry its tolerance.  selected / weights:
+ * salt_mi355_q4_matmul_dev and carry its tolerance; a token's bits do not
+ * depend on the tokens it comes with.  selected / weights:
  * [tokens][topk] (any order inside a token; experts distinct, weights
  * finite); inputs / outputs: [tokens][hidden].  Optional results: group_rows
  * [n_experts] rows per expert, row_pairs [tokens*topk] the pair index

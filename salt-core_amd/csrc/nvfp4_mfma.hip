@@ -397,7 +397,7 @@ int fp4_mfma_launch(const Fp4MfmaLaunch &L, hipStream_t stream) {
     G.chunks_per_split = (G.chunks + L.ksplit - 1) / L.ksplit;
     if ((L.ksplit - 1) * G.chunks_per_split >= G.chunks) return -1;        // every split owns a chunk
     if (L.ksplit > 1 && !L.partials) return -1;
-    if (L.cols > (1 << 24)) return -1;                                     // 32-bit offsets inside a tile
+    if (L.cols >= (1 << 25)) return -1;                                    // 32-bit offsets inside a tile
     const long long grid = ((long long)G.m_tiles * G.n_tiles * L.ksplit + 7) / 8 * 8;
     if (grid > 0x7FFFFFFFLL) return -1;
     if (wide) hipLaunchKernelGGL((fp4_mfma_kernel<4, 4>), dim3((unsigned)grid), dim3(256), 0, stream, L, G);
