@@ -167,8 +167,8 @@ int salt_mi355_q4_jobs_t_dev(const SaltMi355Q4Job *jobs, int njobs, int C, int t
  *   |error| <= 2^-20 * sum_c (|q_c s| + 16 |s| + |b|) |x_c| + 1e-6
  * (and <= 2^-18 * sum_c |w*x| + 1e-6 for activations without outliers).  Needs
  * C % 64 == 0 and device scratch of salt_mi355_q4_matmul_workspace_bytes().
- * R and B choose how the columns are shared out and with it the order of the
- * sums: the bits are the same for the same call, not for any other B.
+ * A token's bits depend on neither B nor the tokens it comes with, so a prompt
+ * may be cut into any pieces.
  * The reference has no counterpart: its CPU and GPU paths keep the 32-chain
  * order at every batch size (kernels.c:1252-1261). */
 size_t salt_mi355_q4_matmul_workspace_bytes(int C, int B);

@@ -145,7 +145,7 @@ int q4_dot_moe_down_launch(const MoeFuse &moe, hipStream_t stream);
 
 // One weight matrix against `tokens` activation rows that have been split
 // into two fp16 planes and notes on the row (see q4_mfma.hip).
-constexpr int MFMA_TM = 64;   // tokens per workgroup of the matrix-core kernel; its weight rows: mfma_tile_rows()
+constexpr int MFMA_TM = 64, MFMA_TN = 256;   // tokens and weight rows per workgroup of the matrix-core kernel
 
 struct MfmaJob {
     const uint8_t *vals, *scales, *biases;   // biases may be null
@@ -168,13 +168,10 @@ struct MfmaLaunch {
     const int *total_tiles_dev;   // workgroups past *total_tiles_dev exit at once
     const int *row_map;       // optional gather: token t of a job reads plane row row_map[row_base + t] / map_divisor
     int map_divisor;
-    int column_parts;         // the tile is tile_tokens (64 or 32) x 256 / column_parts rows (mfma_column_parts());
-    int tile_tokens;          // the launcher chooses both for a single job
+    int tile_tokens;          // tokens per tile: MFMA_TM or half of it; the launcher chooses for a single job
 };
 
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream);
-int mfma_tile_rows(int column_parts);
-int mfma_column_parts(long long wide_tiles, int ngrp);
 // rows of fp32 -> two fp16 planes + a plane of notes; output row r reads input row row_map[r] / map_divisor when a map is
 // given; with a gate the value split is gelu_tanh(gate) * x (gate has the layout of x)
 int x_split_launch(const float *x, const float *gate, const int *row_map, int map_divisor, int x_stride, int rows,

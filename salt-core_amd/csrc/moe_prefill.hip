@@ -104,7 +104,6 @@ struct ScanArgs {
     const uint8_t *pool;
     size_t expert_stride;
     int n_experts, hidden, routed;
-    int tn_up, tn_down;                  // weight rows per tile of the two matmul launches
     const int *counts;
     int *offsets;                        // [n_experts + 1] row offsets
     int *group_rows;                     // optional copy of the counts for the caller
@@ -130,7 +129,7 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
         a.offsets[e] = row0;
         if (a.group_rows) a.group_rows[e] = n;
     }
-    const int nt_up = (a.routed + a.tn_up - 1) / a.tn_up, nt_down = (a.hidden + a.tn_down - 1) / a.tn_down;
+    const int nt_up = (a.routed + MFMA_TN - 1) / MFMA_TN, nt_down = (a.hidden + MFMA_TN - 1) / MFMA_TN;
     const bool valid = a.plan->status == 0;          // written by the previous kernel on this stream
     if (e == 0) {
         a.offsets[a.n_experts] = rows_total;
@@ -278,11 +277,8 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
         return -1;
     const PrefillWorkspace w = carve(g, tokens, workspace);
     const int rows = tokens * g.topk;
-    // One column part whatever the number of tokens: a token's bits do not depend on the tokens it comes with.
     const int m_upper = rows / MFMA_TM + (g.n_experts < rows ? g.n_experts : rows);
-    const int parts_up = 1, parts_down = 1;
-    const int tn_up = mfma_tile_rows(parts_up), tn_down = mfma_tile_rows(parts_down);
-    const int nt_up = (g.routed + tn_up - 1) / tn_up, nt_down = (g.hidden + tn_down - 1) / tn_down;
+    const int nt_up = (g.routed + MFMA_TN - 1) / MFMA_TN, nt_down = (g.hidden + MFMA_TN - 1) / MFMA_TN;
     // plan and counts are adjacent 256-byte aligned pieces of the workspace: one clear covers both
     static_assert(sizeof(PrefillPlan) <= 256, "the plan fits the first aligned piece");
     if ((uint8_t *)w.counts != (uint8_t *)w.plan + 256) return -1;
@@ -292,7 +288,6 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
                        weights, tokens, g.topk, g.n_experts, w.counts, w.plan);
     ScanArgs a;
     a.pool = pool; a.expert_stride = expert_stride; a.n_experts = g.n_experts; a.hidden = g.hidden; a.routed = g.routed;
-    a.tn_up = tn_up; a.tn_down = tn_down;
     a.counts = w.counts; a.offsets = w.offsets; a.group_rows = group_rows; a.plan = w.plan; a.status_out = status_dev;
     a.gate_up_jobs = w.gate_up_jobs; a.down_jobs = w.down_jobs;
     a.planes_in = w.planes_in; a.planes_act = w.planes_act;
@@ -315,7 +310,7 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
     memset(&gu, 0, sizeof gu);
     gu.table = w.gate_up_jobs; gu.cols = g.hidden; gu.total_tiles = 2 * m_upper * nt_up;
     gu.plane_stride = (size_t)tokens * g.hidden;
-    gu.row_map = rp; gu.map_divisor = g.topk; gu.column_parts = parts_up; gu.tile_tokens = MFMA_TM;
+    gu.row_map = rp; gu.map_divisor = g.topk; gu.tile_tokens = MFMA_TM;
     gu.njobs_dev = &w.plan->gate_up_jobs; gu.total_tiles_dev = &w.plan->gate_up_tiles;
     if (q4_mfma_launch(gu, stream) != 0) return -1;
     // gelu(gate) * up, split for the down projection
@@ -326,7 +321,7 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
     memset(&dn, 0, sizeof dn);
     dn.table = w.down_jobs; dn.cols = g.routed; dn.total_tiles = m_upper * nt_down;
     dn.plane_stride = (size_t)rows * g.routed;
-    dn.column_parts = parts_down; dn.tile_tokens = MFMA_TM;
+    dn.tile_tokens = MFMA_TM;
     dn.njobs_dev = &w.plan->down_jobs; dn.total_tiles_dev = &w.plan->down_tiles;
     if (q4_mfma_launch(dn, stream) != 0) return -1;
     hipLaunchKernelGGL(prefill_reduce_kernel, dim3(tokens, (g.hidden + 1023) / 1024), dim3(256), 0, stream, w.down,

@@ -38,9 +38,21 @@
 // one barrier per stage.  Per 16 columns a wave reads 4 KB of LDS for eight
 // matrix instructions, 64 bytes per clock of the 128 a compute unit has, and
 // issues 24 other vector instructions in their shadow.  The four waves of a
-// workgroup are four row blocks (64 x 256 tile, 128 columns per stage) or, in
-// launches too small for that, also two or four parts of the columns, which
-// meet in LDS in part order.
+// workgroup are four row blocks: the tile is 64 tokens x 256 rows, or 32 tokens
+// where a launch is small.
+//
+// Order of the sums.  A wave walks all columns of its block from the first to
+// the last, so an output depends on its token and its row alone: not on the
+// number of tokens or rows in the call nor on the tile that holds it, and a
+// prompt cut into pieces gives the same bits.  Launches with fewer tiles than
+// compute units pay for that.  Two or four parts of the columns side by side in
+// a workgroup, added at the end, are faster there (33 tokens against 8192 x 2816
+// 25.6 us in four parts, 39.5 in one; against 8192 x 8192 51 and 97) and slower
+// in larger launches (333 tokens against 16384 x 2816: 175 us in four parts, 114
+// in two, 84 in one), so that the order would follow the number of tokens.
+// Fixed parts, one after the other in one workgroup where the launch is large,
+// cost that one 129 us (the sums meet in the output), and two fixed parts on
+// eight waves 102.
 //
 // Bound: the matrix cores, which execute twice the useful operations, at the
 // clock that their power leaves them: 44 % busy at 1.6 to 2.1 GHz in the grouped
@@ -97,34 +109,35 @@ __device__ __forceinline__ int eight_start(int c, int ngrp) {
     return 8 * c < last ? 8 * c : last;
 }
 
-// KP parts of the columns per workgroup: the tile is 64 tokens x 256 / KP rows.  LDS holds two stages of the token
-// planes, one scale group of each part, and for every wave one chunk, CH groups, of the codes and the scale bits of its
-// own 64 rows: 128 bytes of a row at a time, because a cache line that is fetched again for each of its quarters
-// costs as much as four lines.
-template <int KP> struct Shape {
-    static constexpr int ROW_WAVES = 4 / KP;
-    static constexpr int TN = 64 * ROW_WAVES;
-    static constexpr int CH = KP == 4 ? 2 : 4;
-    static constexpr int X_BYTES = X_PLANES * TM * 128;              // of one part
-    static constexpr int STAGE_BYTES = KP * X_BYTES;
-    static constexpr int W_OFF = 2 * STAGE_BYTES, W_BYTES = 64 * 32 * CH;        // of one wave
-    static constexpr int S_OFF = W_OFF + 4 * W_BYTES, S_BYTES = 64 * 4 * CH;
-    static constexpr int LDS_BYTES = S_OFF + 4 * S_BYTES;
-    static constexpr int XT = TM / (8 * ROW_WAVES);                  // loads per wave and plane: eight token rows each
-    static constexpr int PIECES = 2 * CH;                            // 16-byte pieces of a row's chunk
-    static constexpr int WT = PIECES;                                // loads per wave and chunk: 64 / PIECES rows each
-    static_assert((KP - 1) * ROW_WAVES * 64 * 64 * 4 <= 2 * STAGE_BYTES, "the parts' sums reuse the staging memory");
-};
+// LDS holds two stages of the token planes, one scale group each, and for every wave one chunk, CH groups, of the codes
+// and the scale bits of its own 64 rows: 128 bytes of a row at a time, because a cache line that is fetched again for
+// each of its quarters costs as much as four lines.
+constexpr int ROW_WAVES = 4;
+constexpr int CH = 4;
+constexpr int STAGE_BYTES = X_PLANES * TM * 128;
+constexpr int W_OFF = 2 * STAGE_BYTES, W_BYTES = 64 * 32 * CH;           // of one wave
+constexpr int S_OFF = W_OFF + ROW_WAVES * W_BYTES, S_BYTES = 64 * 4 * CH;
+constexpr int LDS_BYTES = S_OFF + ROW_WAVES * S_BYTES;
+constexpr int XT = TM / (8 * ROW_WAVES);         // loads per wave and plane: eight token rows each
+constexpr int PIECES = 2 * CH;                   // 16-byte pieces of a row's chunk
+constexpr int WT = PIECES;                       // loads per wave and chunk: 64 / PIECES rows each
+static_assert(MFMA_TN == 64 * ROW_WAVES, "a wave has 64 of the tile's rows");
 
 // Planes arrive in LDS by loads that write 64 consecutive 16-byte pieces, so rows cannot be padded: piece p of token
 // row r lies at place p ^ place_mask(r), which spreads the sixteen rows of an LDS read phase over all banks.  The
-// same for the codes; chunks of four pieces per row have four rows to a turn of the banks instead of two.
-template <int PIECES> __device__ __forceinline__ int place_mask(int row) {
-    return PIECES == 8 ? (row >> 1) & 7 : (row >> 2) & 3;
-}
+// same for the codes.
+static_assert(PIECES == 8, "place_mask covers rows of eight pieces");
+__device__ __forceinline__ int place_mask(int row) { return (row >> 1) & 7; }
 
 template <int N> __device__ __forceinline__ void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// The workgroup meets; a wave's LDS reads are done, its loads on their way stay there (__syncthreads waits for them).
+__device__ __forceinline__ void meet() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 }
 
 static_assert(sizeof(MfmaJob) == 56, "find_job reads a job record as seven 64-bit words");
@@ -199,13 +212,11 @@ __device__ __forceinline__ uint32_t pk_less_one(uint32_t a) {            // zero
 }
 
 // The codes and the scale bits of a lane's two rows for one chunk of scale groups.
-template <int CH> struct Weights { u32x4 w[CH][2]; uint32_t s[CH][2]; };
+struct Weights { u32x4 w[CH][2]; uint32_t s[CH][2]; };
 
-template <int KP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KP == 1 ? 2 : 1), amdgpu_num_vgpr(256)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2), amdgpu_num_vgpr(256)))
 void q4_mfma_kernel(const MfmaLaunch L) {
-    using S = Shape<KP>;
-    __shared__ __attribute__((aligned(16))) uint8_t stage[S::LDS_BYTES];
+    __shared__ __attribute__((aligned(16))) uint8_t stage[LDS_BYTES];
     __shared__ int s_down[TM];                     // per token: exponent of the power of two that undoes the split's scaling
     __shared__ int s_windows[4];
     __shared__ uint32_t s_row[TM];                 // per token: its row of the planes
@@ -213,7 +224,6 @@ void q4_mfma_kernel(const MfmaLaunch L) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int part = wave / S::ROW_WAVES, wn = wave % S::ROW_WAVES;
     const int l32 = lane & 31, half = lane >> 5;
 
     // Workgroups go round the eight partitions of the device in turn; a partition takes one run of consecutive tiles,
@@ -228,7 +238,7 @@ void q4_mfma_kernel(const MfmaLaunch L) {
     const int tm = L.tile_tokens;                   // TM, or half of it
     const int mtiles = (job.tokens + tm - 1) / tm;
     const int t = tile - job.tile0;
-    const int tok0 = (t % mtiles) * tm, row0 = (t / mtiles) * S::TN + wn * 64;
+    const int tok0 = (t % mtiles) * tm, row0 = (t / mtiles) * MFMA_TN + wave * 64;
     const int toks_here = job.tokens - tok0 < tm ? job.tokens - tok0 : tm;
     const bool wide = toks_here > 32;               // both token blocks hold tokens
     const bool live = row0 < job.rows;              // this wave has rows; the others only help to stage
@@ -243,21 +253,13 @@ void q4_mfma_kernel(const MfmaLaunch L) {
     const global_u8_ptr plane0 = (global_u8_ptr)(uintptr_t)job.planes;
     const global_u8_ptr plane1 = plane0 + 2 * L.plane_stride, notes = plane0 + 4 * L.plane_stride;
 
-    // The part's columns: `iterations` groups from g_first on, those from g_end on staged from inside the row and
-    // unused.  Whole chunks, for the sake of whole cache lines, where that leaves the parts about equal.
-    const int even = (ngrp + KP - 1) / KP;
-    const int per_part = even >= 4 * S::CH ? (even + S::CH - 1) / S::CH * S::CH : even;
-    const int iterations = per_part < ngrp ? per_part : ngrp;
-    const int g_first = part * per_part;
-    const int g_end = g_first + per_part < ngrp ? g_first + per_part : ngrp;
-
-    // Staging geometry of this lane: load i of a wave brings the eight token rows from (i * ROW_WAVES + wn) * 8 on;
+    // Staging geometry of this lane: load i of a wave brings the eight token rows from (i * ROW_WAVES + wave) * 8 on;
     // which piece of its row a lane fetches follows from the place that the load will put it in.
-    uint32_t x_src[S::XT];                          // byte offsets below 2^32
+    uint32_t x_src[XT];                          // byte offsets below 2^32
 #pragma unroll
-    for (int i = 0; i < S::XT; ++i) {
-        const int r = (i * S::ROW_WAVES + wn) * 8 + (lane >> 3);
-        const int piece = (lane & 7) ^ place_mask<8>(r);
+    for (int i = 0; i < XT; ++i) {
+        const int r = (i * ROW_WAVES + wave) * 8 + (lane >> 3);
+        const int piece = (lane & 7) ^ place_mask(r);
         x_src[i] = s_row[r] * (uint32_t)(2 * C) + (uint32_t)piece * 16u;
     }
 
@@ -277,54 +279,54 @@ void q4_mfma_kernel(const MfmaLaunch L) {
     const global_u8_ptr scale_rows = (global_u8_ptr)(uintptr_t)job.scales + (size_t)row_base * (size_t)(2 * ngrp);
 
     // Everything staged goes from memory into LDS without passing through registers, so that a wave's loads complete
-    // in the order they were sent in and a wait can leave the younger ones in flight.
+    // in the order they were sent in and a wait can leave the younger ones in flight (meet(), not __syncthreads, which
+    // waits for all of them: 33 tokens against 8192 x 2816 44.7 -> 39.5 us, grouped prefill of 2048 tokens 611 -> 602).
     auto issue_x = [&](int it) {
-        const int g = g_first + it < ngrp ? g_first + it : ngrp - 1;
-        uint8_t *const x = stage + (it & 1) * S::STAGE_BYTES + part * S::X_BYTES + wn * 1024;
-        uint32_t at = (uint32_t)g * 128u;
+        uint8_t *const x = stage + (it & 1) * STAGE_BYTES + wave * 1024;
+        uint32_t at = (uint32_t)it * 128u;
         asm volatile("" : "+s"(at));                 // addresses are made here, not kept in registers through the loops
 #pragma unroll
-        for (int i = 0; i < S::XT; ++i) {
-            if (i * S::ROW_WAVES * 8 >= 32 && !wide) break;
-            uint8_t *const to = x + i * (S::ROW_WAVES * 1024);
+        for (int i = 0; i < XT; ++i) {
+            if (i * ROW_WAVES * 8 >= 32 && !wide) break;
+            uint8_t *const to = x + i * (ROW_WAVES * 1024);
             __builtin_amdgcn_global_load_lds((global_void_ptr)(plane0 + (x_src[i] + at)), (lds_void_ptr)to, 16, 0, 0);
             __builtin_amdgcn_global_load_lds((global_void_ptr)(plane1 + (x_src[i] + at)), (lds_void_ptr)(to + TM * 128),
                                              16, 0, 0);
         }
     };
-    constexpr int CHUNK_LOADS = S::WT + S::CH;
-    auto issue_weights = [&](int it) {               // the chunk that starts with group `it` of the part
-        const uint32_t at = (uint32_t)(g_first + it) * 32u, last = (uint32_t)ngrp * 32u - 16u;
-        uint32_t lane_row = (uint32_t)lane / S::PIECES;
+    constexpr int CHUNK_LOADS = WT + CH;
+    auto issue_weights = [&](int it) {               // the chunk that starts with group `it`
+        const uint32_t at = (uint32_t)it * 32u, last = (uint32_t)ngrp * 32u - 16u;
+        uint32_t lane_row = (uint32_t)lane / PIECES;
         uint32_t scale_at = (uint32_t)(lane < rows_left ? lane : rows_left - 1) * (uint32_t)(2 * ngrp);
         asm volatile("" : "+v"(lane_row), "+v"(scale_at));
 #pragma unroll
-        for (int j = 0; j < S::WT; ++j) {
-            uint32_t r = j * (64 / S::PIECES) + lane_row;
-            const uint32_t piece = ((uint32_t)lane & (S::PIECES - 1)) ^ (uint32_t)place_mask<S::PIECES>((int)r);
+        for (int j = 0; j < WT; ++j) {
+            uint32_t r = j * (64 / PIECES) + lane_row;
+            const uint32_t piece = ((uint32_t)lane & (PIECES - 1)) ^ (uint32_t)place_mask((int)r);
             uint32_t byte = at + piece * 16u;
             byte = byte < last ? byte : last;
             r = r < (uint32_t)rows_left ? r : (uint32_t)rows_left - 1u;
             __builtin_amdgcn_global_load_lds((global_void_ptr)(codes + (__umul24(r, (uint32_t)(C >> 1)) + byte)),
-                                             (lds_void_ptr)(stage + S::W_OFF + wave * S::W_BYTES + j * 1024), 16, 0, 0);
+                                             (lds_void_ptr)(stage + W_OFF + wave * W_BYTES + j * 1024), 16, 0, 0);
         }
 #pragma unroll
-        for (int gi = 0; gi < S::CH; ++gi) {
-            const int g = g_first + it + gi;
+        for (int gi = 0; gi < CH; ++gi) {
+            const int g = it + gi;
             __builtin_amdgcn_global_load_lds((global_void_ptr)(scale_rows + (scale_at + 2u * (uint32_t)(g < ngrp ? g : ngrp - 1))),
-                                             (lds_void_ptr)(stage + S::S_OFF + wave * S::S_BYTES + gi * 256), 2, 0, 0);
+                                             (lds_void_ptr)(stage + S_OFF + wave * S_BYTES + gi * 256), 2, 0, 0);
         }
     };
     typedef const u32x4 __attribute__((address_space(3))) *lds_u128_ptr;
     typedef const uint32_t __attribute__((address_space(3))) *lds_u32_ptr;
-    auto take_weights = [&](Weights<S::CH> &r) {     // and leave their place to the next chunk
-        const lds_u128_ptr w = (lds_u128_ptr)(stage + S::W_OFF + wave * S::W_BYTES);
-        const lds_u32_ptr sc = (lds_u32_ptr)(stage + S::S_OFF + wave * S::S_BYTES);
+    auto take_weights = [&](Weights &r) {     // and leave their place to the next chunk
+        const lds_u128_ptr w = (lds_u128_ptr)(stage + W_OFF + wave * W_BYTES);
+        const lds_u32_ptr sc = (lds_u32_ptr)(stage + S_OFF + wave * S_BYTES);
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
-            const int at = (nb * 32 + l32) * S::PIECES, turn = place_mask<S::PIECES>(nb * 32 + l32);
+            const int at = (nb * 32 + l32) * PIECES, turn = place_mask(nb * 32 + l32);
 #pragma unroll
-            for (int gi = 0; gi < S::CH; ++gi) {
+            for (int gi = 0; gi < CH; ++gi) {
                 r.w[gi][nb] = w[at + ((gi * 2 + half) ^ turn)];
                 r.s[gi][nb] = sc[gi * 64 + nb * 32 + l32];
             }
@@ -381,20 +383,18 @@ void q4_mfma_kernel(const MfmaLaunch L) {
             for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) c.b[nb][j] &= keep;
-            if (KP == 1 || part == 0) {
 #pragma unroll
-                for (int plane = 0; plane < 3; ++plane)
+            for (int plane = 0; plane < 3; ++plane)
 #pragma unroll
-                    for (int mb = 0; mb < 2; ++mb)
+                for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-                        for (int nb = 0; nb < 2; ++nb) {
-                            const bf16x8 a = __builtin_bit_cast(bf16x8, x[plane][mb]);
-                            tb[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, c.b[nb]),
-                                                                                 tb[mb][nb], 0, 0, 0);
-                            ts[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, c.s[nb]),
-                                                                                 ts[mb][nb], 0, 0, 0);
-                        }
-            }
+                    for (int nb = 0; nb < 2; ++nb) {
+                        const bf16x8 a = __builtin_bit_cast(bf16x8, x[plane][mb]);
+                        tb[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, c.b[nb]),
+                                                                             tb[mb][nb], 0, 0, 0);
+                        ts[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, c.s[nb]),
+                                                                             ts[mb][nb], 0, 0, 0);
+                    }
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
@@ -452,24 +452,24 @@ void q4_mfma_kernel(const MfmaLaunch L) {
                 acc[mb][nb][i] = __builtin_amdgcn_ldexpf(acc[mb][nb][i], WEIGHT_TOP - top[nb] - down);
         }
 
-    const int mix = place_mask<8>(l32);             // rows 32 apart share it
+    const int mix = place_mask(l32);             // rows 32 apart share it
     uint32_t code_mask, sixteen;                    // opaque, so that (w & mask) | 16.0 stays one instruction
     asm("s_mov_b32 %0, 0x03C003C0" : "=s"(code_mask));
     asm("v_mov_b32 %0, 0x4C004C00" : "=v"(sixteen));
     int raise[2];                                   // row block nb: the power of two that its scales are brought up by
 
-    // The wave's walk over its part's columns for MB blocks of 32 tokens, in steps of 16 columns: while the matrix
+    // The wave's walk over the columns for MB blocks of 32 tokens, in steps of 16 columns: while the matrix
     // cores work on a step, the operands of the next one are read and converted (left to itself the compiler reads
     // a whole group ahead and spills).  The workgroup meets before the last step of a group: its planes are then in
     // everybody's registers, so their place takes the group after the next one.
     auto walk = [&](auto blocks) {
         constexpr int MB = decltype(blocks)::value;
-        constexpr int LAST = S::CH - 1;
-        Weights<S::CH> now;
+        constexpr int LAST = CH - 1;
+        Weights now;
         f16x8 a[2][MB][X_PLANES], b[2][2];
         f16x2 s[2], less[2], s_next[2], less_next[2];
         auto read = [&](int it, int step, f16x8 (&to)[MB][X_PLANES]) {
-            const lds_u128_ptr x = (lds_u128_ptr)(stage + (it & 1) * S::STAGE_BYTES + part * S::X_BYTES + l32 * 128);
+            const lds_u128_ptr x = (lds_u128_ptr)(stage + (it & 1) * STAGE_BYTES + l32 * 128);
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -477,12 +477,11 @@ void q4_mfma_kernel(const MfmaLaunch L) {
                     to[mb][plane] = __builtin_bit_cast(
                         f16x8, x[plane * (TM * 8) + mb * (32 * 8) + ((half * 4 + step) ^ mix)]);
         };
-        // Scales that the window does not bring into the WINDOW binades below 2^WEIGHT_TOP count as zero, and so do
-        // groups past the part's end.
-        auto scale = [&](const uint32_t (&bits)[2], bool inside, f16x2 (&s)[2], f16x2 (&less)[2]) {
+        // Scales that the window does not bring into the WINDOW binades below 2^WEIGHT_TOP count as zero.
+        auto scale = [&](const uint32_t (&bits)[2], f16x2 (&s)[2], f16x2 (&less)[2]) {
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-                const float value = bf16_to_f32(inside ? bits[nb] : 0u);
+                const float value = bf16_to_f32(bits[nb]);
                 const int place = __builtin_amdgcn_frexp_expf(value) + raise[nb];  // at most WEIGHT_TOP in this window
                 float raised = __builtin_amdgcn_ldexpf(value, raise[nb]);
                 const bool finite = __builtin_fabsf(value) < __builtin_inff();
@@ -519,82 +518,63 @@ void q4_mfma_kernel(const MfmaLaunch L) {
             for (int k = 0; k < 2; ++k) asm volatile("" : "+v"(values[k]));
         };
         take_weights(now);
-        if (S::CH < iterations) issue_weights(S::CH);
+        if (CH < ngrp) issue_weights(CH);
         read(0, 0, a[0]);
-        scale(now.s[0], g_first < g_end, s, less);
+        scale(now.s[0], s, less);
         convert(now.w[0], 0, b[0]);
         __builtin_amdgcn_sched_barrier(0);
-        for (int it0 = 0; it0 < iterations; it0 += S::CH) {
+        for (int it0 = 0; it0 < ngrp; it0 += CH) {
 #pragma unroll
-            for (int gi = 0; gi < S::CH; ++gi) {
+            for (int gi = 0; gi < CH; ++gi) {
                 const int it = it0 + gi;
 #pragma unroll
                 for (int step = 0; step < 3; ++step) {
                     read(it, step + 1, a[(step + 1) & 1]);
                     convert(now.w[gi], step + 1, b[(step + 1) & 1]);
                     if (step == 1 && gi < LAST) {
-                        scale(now.s[gi < LAST ? gi + 1 : 0], g_first + it + 1 < g_end, s_next, less_next);
+                        scale(now.s[gi < LAST ? gi + 1 : 0], s_next, less_next);
                         pin(s_next); pin(less_next);
                     }
                     multiply(a[step & 1], b[step & 1]);
                 }
                 pin(b[1]);
                 // the next planes were sent for before the chunk that may still be on its way
-                if (gi == 0 && it0 + S::CH < iterations) wait_loads<CHUNK_LOADS>(); else wait_loads<0>();
-                __syncthreads();
-                if (it + 2 < iterations) issue_x(it + 2);
-                if (gi == S::CH - 1) {
+                if (gi == 0 && it0 + CH < ngrp) wait_loads<CHUNK_LOADS>(); else wait_loads<0>();
+                meet();
+                if (it + 2 < ngrp) issue_x(it + 2);
+                if (gi == CH - 1) {
                     take_weights(now);
-                    if (it + 1 + S::CH < iterations) issue_weights(it + 1 + S::CH);
+                    if (it + 1 + CH < ngrp) issue_weights(it + 1 + CH);
                 }
                 // after the last group these are stale and unused
-                if (gi == LAST) scale(now.s[0], g_first + it + 1 < g_end, s_next, less_next);
+                if (gi == LAST) scale(now.s[0], s_next, less_next);
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) { s[nb] = s_next[nb]; less[nb] = less_next[nb]; }
                 read(it + 1, 0, a[0]);
                 convert(now.w[gi == LAST ? 0 : gi + 1], 0, b[0]);
                 multiply(a[1], b[1]);
-                if (it + 1 >= iterations) break;
+                if (it + 1 >= ngrp) break;
             }
         }
     };
     // A wave without rows helps to stage.
     auto stage_only = [&]() {
-        for (int it = 0; it < iterations; ++it) {
+        for (int it = 0; it < ngrp; ++it) {
             wait_loads<0>();
-            __syncthreads();
-            if (it + 2 < iterations) issue_x(it + 2);
+            meet();
+            if (it + 2 < ngrp) issue_x(it + 2);
         }
     };
     for (int window = 0;;) {
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) raise[nb] = WEIGHT_TOP - top[nb] + WINDOW * window;
-        // ---- main loop: acc += s (q - 8) x over the part's columns
-        if (iterations > 1) issue_x(1);
+        // ---- main loop: acc += s (q - 8) x
+        if (ngrp > 1) issue_x(1);
         if (!live) stage_only();
         else if (wide) walk(std::integral_constant<int, 2>{});
         else walk(std::integral_constant<int, 1>{});
 
-        // ---- the parts meet in part order
-        if (KP > 1) {
-            float *sums = reinterpret_cast<float *>(stage);
-            if (part > 0) {
-                float *mine = sums + ((part - 1) * S::ROW_WAVES + wn) * 4096 + lane;
-#pragma unroll
-                for (int k = 0; k < 64; ++k) mine[k * 64] = acc[k >> 5][(k >> 4) & 1][k & 15];
-            }
-            __syncthreads();
-            if (part == 0) {
-#pragma unroll
-                for (int p = 1; p < KP; ++p) {
-                    const float *theirs = sums + ((p - 1) * S::ROW_WAVES + wn) * 4096 + lane;
-#pragma unroll
-                    for (int k = 0; k < 64; ++k) acc[k >> 5][(k >> 4) & 1][k & 15] += theirs[k * 64];
-                }
-            }
-        }
-
-        if (live && part == 0) {
+        if (live) {
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb) {
                 if (mb == 1 && !wide) break;
@@ -618,7 +598,7 @@ void q4_mfma_kernel(const MfmaLaunch L) {
             }
         }
         if (++window >= windows) break;             // uniform over the workgroup
-        __syncthreads();                            // the parts' sums have been read
+        __syncthreads();                            // the last group has been read by every wave
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -740,45 +720,25 @@ __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ 
 
 }  // namespace
 
-int mfma_tile_rows(int column_parts) { return 256 / column_parts; }
-
 namespace {
-int mfma_tiles(int tokens, int tile_tokens, int rows, int column_parts) {
-    const int tn = mfma_tile_rows(column_parts);
-    return ((tokens + tile_tokens - 1) / tile_tokens) * ((rows + tn - 1) / tn);
+int mfma_tiles(int tokens, int tile_tokens, int rows) {
+    return ((tokens + tile_tokens - 1) / tile_tokens) * ((rows + MFMA_TN - 1) / MFMA_TN);
 }
 }  // namespace
-
-// Column parts for a launch of `wide_tiles` tiles of 64 x 256 over `ngrp` scale groups: as many as still leave every
-// workgroup a compute unit of its own.  A part shortens the walk of a workgroup that has its compute unit to itself;
-// beyond that it only adds rounds, and a workgroup of several parts fills a compute unit's LDS alone where two of one
-// part share it and hide each other's waits (16384 x 2816, 333 tokens, 384 tiles: 84 us in one part, 114 in two).
-int mfma_column_parts(long long wide_tiles, int ngrp) {
-    int parts = 1;
-    while (parts < 4 && wide_tiles * (2 * parts) <= 256 && ngrp >= 8 * parts) parts *= 2;
-    return parts;
-}
 
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream) {
     MfmaLaunch L = launch;
     if (L.cols < 64 || (L.cols & 63)) return -1;
     if (L.table == nullptr) {                   // one job: the tiling is chosen here
-        L.column_parts = mfma_column_parts(mfma_tiles(L.one.tokens, TM, L.one.rows, 1), L.cols >> 6);
         // Tiles of half the tokens where each still finds a compute unit of its own: half the matrix work per step of a
-        // walk that is bound by its waits (4096 x 4096, 64 tokens: 41 us in 64-token tiles, 32 in these).
-        const int halves = mfma_tiles(L.one.tokens, TM / 2, L.one.rows, L.column_parts);
-        L.tile_tokens = halves <= 256 ? TM / 2 : TM;
+        // walk that is bound by its waits (4096 x 4096, 64 tokens: 67 us in 64-token tiles, 54 in these).
+        L.tile_tokens = mfma_tiles(L.one.tokens, TM / 2, L.one.rows) <= 256 ? TM / 2 : TM;
         L.one.tile0 = 0;
-        L.total_tiles = mfma_tiles(L.one.tokens, L.tile_tokens, L.one.rows, L.column_parts);
+        L.total_tiles = mfma_tiles(L.one.tokens, L.tile_tokens, L.one.rows);
     }
     if (3 * (unsigned long long)L.plane_stride >= (1ull << 32)) return -1;      // 32-bit byte offsets inside a plane
     if (L.total_tiles < 1 || (L.tile_tokens != TM && L.tile_tokens != TM / 2) || (L.row_map && L.map_divisor < 1)) return -1;
-    switch (L.column_parts) {
-        case 1: hipLaunchKernelGGL(q4_mfma_kernel<1>, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L); break;
-        case 2: hipLaunchKernelGGL(q4_mfma_kernel<2>, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L); break;
-        case 4: hipLaunchKernelGGL(q4_mfma_kernel<4>, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L); break;
-        default: return -1;
-    }
+    hipLaunchKernelGGL(q4_mfma_kernel, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
