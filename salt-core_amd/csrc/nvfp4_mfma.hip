@@ -31,6 +31,8 @@
 
 #include <stddef.h>
 
+#include <type_traits>
+
 namespace mi355 {
 namespace {
 
@@ -46,6 +48,7 @@ typedef const u32x4 __attribute__((address_space(3))) *lds_u128_ptr;
 typedef const uint32_t __attribute__((address_space(3))) *lds_u32_ptr;
 
 constexpr int TM = 64, KC = 64, CH = 4;        // tokens per workgroup; columns per stage; stages per chunk of codes
+constexpr int FAR_COLS = 1 << 25;              // from here on the offsets inside a tile of 64 rows take 64 bits
 
 template <int WAVES, int RW> struct Shape {
     static constexpr int KP = WAVES / RW;                            // parts of the columns
@@ -96,9 +99,10 @@ __device__ __forceinline__ f16x8 weights_to_f16(uint32_t w, f16x2 s) {
     return __builtin_bit_cast(f16x8, r);
 }
 
-template <int WAVES, int RW>
+template <int WAVES, int RW, bool FAR>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2))) void fp4_mfma_kernel(const Fp4MfmaLaunch L, const Geometry G) {
     using S = Shape<WAVES, RW>;
+    using Offset = typename std::conditional<FAR, uint64_t, uint32_t>::type;
     __shared__ __attribute__((aligned(16))) uint8_t stage[S::LDS_BYTES];
 
     const int tid = threadIdx.x;
@@ -132,12 +136,12 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 
     // load i of a wave brings the eight token rows from (i * RW + wn) * 8 on; which piece of its row a lane fetches
     // follows from the place that the load will put it in
-    const global_u8_ptr plane = (global_u8_ptr)(uintptr_t)L.plane + (size_t)tok0 * (size_t)(2 * C);
-    uint32_t x_src[S::XT];
+    const global_u8_ptr plane = (global_u8_ptr)(uintptr_t)L.plane + (size_t)tok0 * (2 * (size_t)C);
+    Offset x_src[S::XT];
 #pragma unroll
     for (int i = 0; i < S::XT; ++i) {
         const int r = (i * RW + wn) * 8 + (lane >> 3);
-        x_src[i] = (uint32_t)(r < toks_here ? r : toks_here - 1) * (uint32_t)(2 * C) + (uint32_t)((lane & 7) ^ place_mask(r)) * 16u;
+        x_src[i] = (Offset)(r < toks_here ? r : toks_here - 1) * (2 * (Offset)C) + (uint32_t)((lane & 7) ^ place_mask(r)) * 16u;
     }
     const int rows_left = live ? L.rows - row0 : 1;
     const int row_base = live ? row0 : 0;           // waves without rows fetch the first row and use nothing
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
     // in the order they were sent in and a wait can leave the younger ones in flight.
     auto issue_x = [&](int it) {
         const int g = first + it < G.chunks ? first + it : last_chunk;
-        uint32_t at = (uint32_t)g * (2 * KC);
+        Offset at = (Offset)g * (2 * KC);
         asm volatile("" : "+s"(at));
         uint8_t *const x = stage + (it & 1) * S::STAGE_BYTES + part * S::X_BYTES + wn * 1024;
 #pragma unroll
@@ -164,7 +168,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
     auto issue_weights = [&](int it) {               // the chunk that starts with stage `it` of the part
         const uint32_t at = (uint32_t)(first + it) * 32u, last = (uint32_t)G.chunks * 32u - 16u;
         uint32_t lane_row = (uint32_t)lane >> 3;
-        uint32_t scale_at = (uint32_t)(lane < rows_left ? lane : rows_left - 1) * (uint32_t)(C >> 4);
+        Offset scale_at = (Offset)(lane < rows_left ? lane : rows_left - 1) * (uint32_t)(C >> 4);
         asm volatile("" : "+v"(lane_row), "+v"(scale_at));   // addresses are made here, not kept in registers
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -172,7 +176,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
             uint32_t byte = at + (((uint32_t)lane & 7u) ^ (uint32_t)place_mask((int)r)) * 16u;
             byte = byte < last ? byte : last;
             r = r < (uint32_t)rows_left ? r : (uint32_t)rows_left - 1u;
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(codes + (__umul24(r, (uint32_t)(C >> 1)) + byte)),
+            const Offset line = FAR ? (Offset)r * (uint32_t)(C >> 1) : (Offset)__umul24(r, (uint32_t)(C >> 1));
+            __builtin_amdgcn_global_load_lds((global_void_ptr)(codes + (line + byte)),
                                              (lds_void_ptr)(stage + S::W_OFF + wave * S::W_BYTES + j * 1024), 16, 0, 0);
         }
         if (whole_scales) {                          // a chunk's scales of a row at once, from the row's end backwards
@@ -367,14 +372,14 @@ __global__ __launch_bounds__(256) void fp4_split_sum_kernel(const Fp4MfmaLaunch 
 
 namespace {
 // Tiles of 64 x 256 by four waves, two workgroups on a compute unit, where there are enough of them; else tiles of
-// 64 x 128 by eight waves, four column parts.
-bool wide_tiles(int rows, int tokens) {
-    return (long long)((tokens + TM - 1) / TM) * ((rows + 255) / 256) >= 320;
+// 64 x 128 by eight waves, four column parts.  Rows of FAR_COLS columns and more have the one form.
+bool wide_tiles(int rows, int cols, int tokens) {
+    return cols < FAR_COLS && (long long)((tokens + TM - 1) / TM) * ((rows + 255) / 256) >= 320;
 }
 }  // namespace
 
 int fp4_mfma_splits(int rows, int cols, int tokens) {
-    const int tn = wide_tiles(rows, tokens) ? 256 : 128;
+    const int tn = wide_tiles(rows, cols, tokens) ? 256 : 128;
     const int tiles = ((tokens + TM - 1) / TM) * ((rows + tn - 1) / tn);
     const int chunks = cols / KC;
     int splits = 256 / tiles;                          // while every workgroup still has a compute unit of its own
@@ -388,7 +393,7 @@ int fp4_mfma_splits(int rows, int cols, int tokens) {
 int fp4_mfma_launch(const Fp4MfmaLaunch &L, hipStream_t stream) {
     if (L.rows < 1 || L.tokens < 1 || L.cols < KC || (L.cols % KC) || L.ksplit < 1) return -1;
     if (L.flags ? (L.nflags < 1 || !L.outcome) : !L.status) return -1;
-    const bool wide = wide_tiles(L.rows, L.tokens);
+    const bool wide = wide_tiles(L.rows, L.cols, L.tokens);
     const int tn = wide ? 256 : 128;
     Geometry G;
     G.m_tiles = (L.tokens + TM - 1) / TM;
@@ -397,11 +402,11 @@ int fp4_mfma_launch(const Fp4MfmaLaunch &L, hipStream_t stream) {
     G.chunks_per_split = (G.chunks + L.ksplit - 1) / L.ksplit;
     if ((L.ksplit - 1) * G.chunks_per_split >= G.chunks) return -1;        // every split owns a chunk
     if (L.ksplit > 1 && !L.partials) return -1;
-    if (L.cols >= (1 << 25)) return -1;                                    // 32-bit offsets inside a tile
     const long long grid = ((long long)G.m_tiles * G.n_tiles * L.ksplit + 7) / 8 * 8;
     if (grid > 0x7FFFFFFFLL) return -1;
-    if (wide) hipLaunchKernelGGL((fp4_mfma_kernel<4, 4>), dim3((unsigned)grid), dim3(256), 0, stream, L, G);
-    else hipLaunchKernelGGL((fp4_mfma_kernel<8, 2>), dim3((unsigned)grid), dim3(512), 0, stream, L, G);
+    if (wide) hipLaunchKernelGGL((fp4_mfma_kernel<4, 4, false>), dim3((unsigned)grid), dim3(256), 0, stream, L, G);
+    else if (L.cols < FAR_COLS) hipLaunchKernelGGL((fp4_mfma_kernel<8, 2, false>), dim3((unsigned)grid), dim3(512), 0, stream, L, G);
+    else hipLaunchKernelGGL((fp4_mfma_kernel<8, 2, true>), dim3((unsigned)grid), dim3(512), 0, stream, L, G);
     if (L.ksplit > 1) {
         const size_t n = (size_t)L.tokens * L.rows;
         hipLaunchKernelGGL(fp4_split_sum_kernel, dim3((unsigned)((n / 4 + 256) / 256)), dim3(256), 0, stream, L, n);

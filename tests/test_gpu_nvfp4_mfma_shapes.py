@@ -39,3 +39,29 @@ def test_tile_forms(pkg, oracle, R, C, B, offset):
     ratio = float((np.abs(got[:, rows].astype(np.float64) - want) / (2.0 ** -20 * mags + 1e-30)).max())
     print("max err / bound", ratio, flush=True)
     assert ratio <= 1.0
+
+
+def test_rows_beyond_32_bit_offsets(pkg, oracle):
+    """33 554 496 columns: the offset of the last of 64 token rows passes 2^32 bytes, that of a second weight row 2^24.
+    All tokens but the first and the last are zero."""
+    R, C, B = 2, (1 << 25) + 64, 64
+    print(f"nvfp4 mfma far rows C={C}", flush=True)
+    gpu = pkg.lib
+    lib = gpu.init()
+    packed, scales = synth.nvfp4_tensor(R, C, 3)
+    ends = synth.activations(C, 2, 5)
+    dp, ds, dx = gpu.DeviceBuffer.from_host(packed), gpu.DeviceBuffer.from_host(scales), gpu.DeviceBuffer(4 * B * C, fill=0)
+    dx.upload(ends[0])
+    dx.upload(ends[1], 4 * (B - 1) * C)
+    dy, status = gpu.DeviceBuffer(B * R * 4, fill=0xFF), gpu.DeviceBuffer(4, fill=0x7F)
+    ws = gpu.DeviceBuffer(lib.salt_mi355_nvfp4_matmul_workspace_bytes(R, C, B))
+    stream = lib.salt_mi355_stream()
+    gpu.check(lib.salt_mi355_nvfp4_matmul_dev(dp.ptr, ds.ptr, 2688.0, 64.0, R, C, B, dx.ptr, dy.ptr, status.ptr, ws.ptr, stream),
+              "nvfp4_matmul_dev")
+    gpu.check(lib.salt_mi355_stream_sync(stream), "sync")
+    got = dy.to_host(np.float32).reshape(B, R)
+    assert status.to_host(np.int32)[0] == 0 and (got[1:-1] == 0).all()
+    want, mags = reference(oracle, packed, scales, 2688.0, 64.0, R, C, ends)
+    ratio = float((np.abs(got[[0, -1]].astype(np.float64) - want) / (2.0 ** -20 * mags)).max())
+    print("max err / bound", ratio, flush=True)
+    assert ratio <= 1.0
