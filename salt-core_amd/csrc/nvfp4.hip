@@ -369,8 +369,9 @@ int launch_tiles(const Fp4Launch &L, hipStream_t stream) {
 
 // Four neighbouring lanes per 16-element block of one token, four elements each, so that a wave reads and writes whole
 // cache lines (a lane per block read 64 bytes apart: 256 tokens of 8192 columns 9.0 -> 7.2 us).  FLAGS: the workgroup
-// reports in flags[blockIdx.x] (0 or -1, always written) instead of setting *status.
+// reports in the flag of its own number (0 or -1, always written) instead of setting *status.
 constexpr int QDQ_THREADS = 1024, QDQ_BLOCKS = QDQ_THREADS / 4;
+constexpr unsigned QDQ_GRID_X = 1u << 20;      // a grid's dimension holds less than 2^32 threads: the rest goes into rows of this many
 
 template <bool FLAGS>
 __global__ __launch_bounds__(QDQ_THREADS) void fp4_qdq_kernel(const float *__restrict__ input, int cols, int tokens,
@@ -378,9 +379,11 @@ __global__ __launch_bounds__(QDQ_THREADS) void fp4_qdq_kernel(const float *__res
                                                       uint8_t *__restrict__ scales, float *__restrict__ dequant,
                                                       uint16_t *__restrict__ plane, int *__restrict__ status) {
     const int blocks_per_token = cols >> 4;
-    const long long item = (long long)blockIdx.x * QDQ_BLOCKS + (threadIdx.x >> 2);
+    const long long group = (long long)blockIdx.y * gridDim.x + blockIdx.x, items = (long long)blocks_per_token * tokens;
+    if (group * QDQ_BLOCKS >= items) return;                 // uniform: past the last workgroup of the last row
+    const long long item = group * QDQ_BLOCKS + (threadIdx.x >> 2);
     const int quarter = threadIdx.x & 3;
-    const bool present = item < (long long)blocks_per_token * tokens;
+    const bool present = item < items;
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (present) {
         const float4 f = reinterpret_cast<const float4 *>(input)[item * 4 + quarter];
@@ -401,7 +404,7 @@ __global__ __launch_bounds__(QDQ_THREADS) void fp4_qdq_kernel(const float *__res
     const bool good = top_bits < 0x7f800000u;                // the reference rejects the whole call
     if (FLAGS) {
         const int any_bad = __syncthreads_or(good ? 0 : 1);
-        if (threadIdx.x == 0) status[blockIdx.x] = any_bad ? -1 : 0;
+        if (threadIdx.x == 0) status[group] = any_bad ? -1 : 0;
         if (!present || !good) return;
     } else {
         if (present && !good) *status = -1;
@@ -442,12 +445,17 @@ int fp4_launch(const Fp4Launch &L, int chains_per_lane, hipStream_t stream) {
     }
 }
 
+namespace {
+dim3 qdq_grid(long long groups) {
+    return groups <= QDQ_GRID_X ? dim3((unsigned)groups) : dim3(QDQ_GRID_X, (unsigned)((groups + QDQ_GRID_X - 1) / QDQ_GRID_X));
+}
+}  // namespace
+
 int fp4_qdq_launch(const float *input, int cols, int tokens, float input_global_scale, uint8_t *packed,
                    uint8_t *scales, float *dequant, uint16_t *plane, int *status, hipStream_t stream) {
     const long long items = (long long)(cols >> 4) * tokens;
-    if (items < 1 || (cols & 15)) return -1;
-    const unsigned grid = (unsigned)((items + QDQ_BLOCKS - 1) / QDQ_BLOCKS);
-    hipLaunchKernelGGL(fp4_qdq_kernel<false>, dim3(grid), dim3(QDQ_THREADS), 0, stream, input, cols, tokens, input_global_scale,
+    if (items < 1 || items >= (1ll << 32) || (cols & 15)) return -1;
+    hipLaunchKernelGGL(fp4_qdq_kernel<false>, qdq_grid((items + QDQ_BLOCKS - 1) / QDQ_BLOCKS), dim3(QDQ_THREADS), 0, stream, input, cols, tokens, input_global_scale,
                        packed, scales, dequant, plane, status);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -461,7 +469,7 @@ int fp4_qdq_flags_launch(const float *input, int cols, int tokens, float input_g
                          int *flags, hipStream_t stream) {
     const int grid = fp4_qdq_flag_count(cols, tokens);
     if (grid < 1 || (cols & 15) || !flags) return -1;
-    hipLaunchKernelGGL(fp4_qdq_kernel<true>, dim3((unsigned)grid), dim3(QDQ_THREADS), 0, stream, input, cols, tokens,
+    hipLaunchKernelGGL(fp4_qdq_kernel<true>, qdq_grid(grid), dim3(QDQ_THREADS), 0, stream, input, cols, tokens,
                        input_global_scale, (uint8_t *)nullptr, (uint8_t *)nullptr, (float *)nullptr, plane, flags);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
