@@ -501,13 +501,14 @@ int salt_mi355_ffn_block_dev(const SaltMi355FfnLayer *layer, const float *residu
         hip_ok(hipStreamWaitEvent(side, g_state.fork, 0), "ffn block fork wait") != 0)
         return -1;
     // Whole tiles (a stated chain count): cut up, the dense branch would take compute units from the routed one, which
-    // is the longer of the two (92.2 us per block against 90.0 at 2816/2112/704).
-    const int down_chains = L.hidden <= 256 * 64 ? 2 : 0;
-    int rc = tileable ? q4_launch(gate_up, gate_up.total_tiles <= 256 ? 2 : 0, side) : q4_launch_generic(gate_up, side);
+    // is the longer of the two (92.2 us per block against 90.0 at 2816/2112/704).  From 257 tiles on there is nothing to
+    // choose between them (dense 8256, 9984, 12288: 106.0 / 112.1 / 118.5 us whole, 106.3 / 111.3 / 117.6 in halves).
+    const auto chains = [](int tiles) { return tiles <= 256 ? 2 : 4; };        // as q4_launch would choose
+    int rc = tileable ? q4_launch(gate_up, chains(gate_up.total_tiles), side) : q4_launch_generic(gate_up, side);
     if (rc == 0) rc = moe_activate_launch(ws.gate, ws.up, ws.act, (size_t)L.dense, side);
     if (rc == 0)
         rc = salt_mi355_q4_matvec_dev(L.dense_down[0], L.dense_down[1], L.dense_down[2], L.hidden, L.dense, 1, ws.act,
-                                      ws.dense_out, down_chains, side);
+                                      ws.dense_out, chains((L.hidden + 63) / 64), side);
     // the join is recorded even after a failure, so that the caller's stream never outruns the side stream
     const int recorded = hip_ok(hipEventRecord(g_state.join, side), "ffn block join");
     if (rc != 0 || recorded != 0) {

@@ -144,6 +144,23 @@ def test_ffn_block_matches_the_checker(gpu, oracle, H, D, F, E, K, seed):
     assert st == 0 and np.array_equal(bits(out3), bits(want))
 
 
+@pytest.mark.parametrize("H,D,kernel", [(16384, 64, "q4_tile_kernel<2,1,32,0>"), (16448, 64, "q4_tile_kernel<4,1,16,0>"),
+                                        (16448, 8256, "q4_tile_kernel<4,1,16,0>")])
+def test_ffn_block_dense_branch_runs_whole_tiles(gpu, oracle, H, D, kernel):
+    """256 and 257 tiles of the dense down projection, 2 and 258 of gate and up: neither side of the limit is cut into parts
+    (the down projection is the last launch that leaves its name)."""
+    F, E, K = 64, 4, 1
+    print("ffn block", H, D, F, E, K, flush=True)
+    w = synth.ffn_layer(H, D, F, E, K, 11)
+    block = gpu.FfnBlock(w)
+    residual = (synth.activations(H, 1, 12)[0] * 3).astype(f32)
+    st, sel, wt, out = block.step(residual)
+    assert gpu.load().salt_mi355_last_kernel().decode() == kernel
+    want = np.zeros(H, f32); osel = np.zeros(K, np.int32); owt = np.zeros(K, f32)
+    assert oracle.orc_ffn_block(C.byref(ffn_layer_struct(w)), ptr(residual), ptr(want), ptr(osel), ptr(owt), host_threads()) == 0
+    assert st == 0 and np.array_equal(sel, osel) and np.array_equal(bits(wt), bits(owt)) and np.array_equal(bits(out), bits(want))
+
+
 def test_ffn_block_argument_errors(gpu):
     w = synth.ffn_layer(256, 192, 128, 4, 2, 9)
     block = gpu.FfnBlock(w)
