@@ -7,7 +7,7 @@
 
 namespace mi355 {
 
-// Name and template arguments of the matvec kernel launched last (diagnostics: salt_mi355_last_kernel).
+// Name and template arguments of the matvec or matmul kernel launched last (diagnostics: salt_mi355_last_kernel).
 void note_kernel(const char *format, ...) __attribute__((format(printf, 1, 2)));
 
 // ---------------------------------------------------------------- affine Q4

@@ -404,6 +404,7 @@ int fp4_mfma_launch(const Fp4MfmaLaunch &L, hipStream_t stream) {
     if (L.ksplit > 1 && !L.partials) return -1;
     const long long grid = ((long long)G.m_tiles * G.n_tiles * L.ksplit + 7) / 8 * 8;
     if (grid > 0x7FFFFFFFLL) return -1;
+    note_kernel("fp4_mfma_kernel<%s> ksplit %d", wide ? "4,4,0" : L.cols < FAR_COLS ? "8,2,0" : "8,2,1", L.ksplit);
     if (wide) hipLaunchKernelGGL((fp4_mfma_kernel<4, 4, false>), dim3((unsigned)grid), dim3(256), 0, stream, L, G);
     else if (L.cols < FAR_COLS) hipLaunchKernelGGL((fp4_mfma_kernel<8, 2, false>), dim3((unsigned)grid), dim3(512), 0, stream, L, G);
     else hipLaunchKernelGGL((fp4_mfma_kernel<8, 2, true>), dim3((unsigned)grid), dim3(512), 0, stream, L, G);

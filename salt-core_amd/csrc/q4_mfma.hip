@@ -738,6 +738,7 @@ int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream) {
     }
     if (3 * (unsigned long long)L.plane_stride >= (1ull << 32)) return -1;      // 32-bit byte offsets inside a plane
     if (L.total_tiles < 1 || (L.tile_tokens != TM && L.tile_tokens != TM / 2) || (L.row_map && L.map_divisor < 1)) return -1;
+    note_kernel("q4_mfma_kernel, tiles of %d tokens", L.tile_tokens);
     hipLaunchKernelGGL(q4_mfma_kernel, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

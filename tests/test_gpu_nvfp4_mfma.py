@@ -1,6 +1,6 @@
 """Prefill-sized NVFP4 matmul on the matrix cores: tolerance class.
 
-Both operands reach the matrix cores as exact bf16 values (code * block scale),
+Both operands reach the matrix cores as exact fp16 values (code * block scale),
 so the result differs from the reference matvec (src/nvfp4.c:228-256) only by
 the order of the fp32 additions and by where the two per-tensor factors are
 rounded.  Stated tolerance per output, checked against the bit-exact CPU
@@ -54,7 +54,7 @@ def test_matmul_within_stated_tolerance(pkg, oracle, R, Cc, B, g):
 
 
 def test_cfg4_8192x8192_batch256_sampled_rows(pkg, oracle):
-    """BASELINE configs[4] at batch 256 and full size (128 tiles x 4 K-splits plus the split sum): 32 rows x 256
+    """8192 x 8192 at batch 256 (256 workgroups of eight waves, four column parts each, no split sum): 32 rows x 256
     tokens against the checker."""
     R = Cc = 8192
     B = 256

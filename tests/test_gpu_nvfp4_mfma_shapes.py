@@ -17,6 +17,10 @@ synth = cases.synth
     (27400, 64, 130, 0), (27400, 320, 130, 0), (27400, 320, 130, 2),                # 64 x 256 tiles
 ])
 def test_tile_forms(pkg, oracle, R, C, B, offset):
+    """The expected form: 64 x 256 tiles from 320 of them on; else 64 x 128 and the columns split over workgroups while each
+    still has a compute unit, eight chunks of 64 columns at least per split."""
+    wide = -(-B // 64) * -(-R // 256) >= 320
+    split = 1 if wide else max(1, min(256 // (-(-B // 64) * -(-R // 128)), 8, C // 64 // 8))
     print(f"nvfp4 mfma forms R={R} C={C} B={B} offset={offset}", flush=True)
     gpu = pkg.lib
     lib = gpu.init()
@@ -31,6 +35,9 @@ def test_tile_forms(pkg, oracle, R, C, B, offset):
                                               stream), "nvfp4_matmul_dev")
     gpu.check(lib.salt_mi355_stream_sync(stream), "sync")
     got = dy.to_host(np.float32).reshape(B, R)
+    form, _, splits = lib.salt_mi355_last_kernel().decode().rpartition(" ksplit ")
+    assert form == ("fp4_mfma_kernel<4,4,0>" if wide else "fp4_mfma_kernel<8,2,0>")
+    assert int(splits) == split
     assert status.to_host(np.int32)[0] == 0 and np.isfinite(got).all()
     rows = np.unique(np.r_[np.arange(0, R, max(1, R // 60)), R - 1])
     sub_packed = np.ascontiguousarray(packed.reshape(R, C // 2)[rows]).reshape(-1)
@@ -60,6 +67,7 @@ def test_rows_beyond_32_bit_offsets(pkg, oracle):
               "nvfp4_matmul_dev")
     gpu.check(lib.salt_mi355_stream_sync(stream), "sync")
     got = dy.to_host(np.float32).reshape(B, R)
+    assert lib.salt_mi355_last_kernel().decode() == "fp4_mfma_kernel<8,2,1> ksplit 8"
     assert status.to_host(np.int32)[0] == 0 and (got[1:-1] == 0).all()
     want, mags = reference(oracle, packed, scales, 2688.0, 64.0, R, C, ends)
     ratio = float((np.abs(got[[0, -1]].astype(np.float64) - want) / (2.0 ** -20 * mags)).max())

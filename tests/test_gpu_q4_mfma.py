@@ -1,8 +1,8 @@
 """Prefill-sized affine-Q4 matmul on the matrix cores: tolerance class.
 
-The kernel evaluates the affine form per scale group, s * sum(q x) + b * sum(x),
-so its rounding error scales with the magnitudes of the two terms, not with
-their (possibly cancelling) sum.  Stated tolerance per output, checked against
+The kernel evaluates the affine form as sum s (q - 8) x plus, per scale group,
+(b + 8 s) sum(x), so its rounding error scales with the magnitudes of the two
+terms, not with their (possibly cancelling) sum.  Stated tolerance per output, checked against
 the bit-exact CPU checker:
 
     |error| <= 2^-20 * sum_c (|q_c s| + 16 |s| + |b|) * |x_c| + 1e-6

@@ -13,8 +13,20 @@ pytestmark = pytest.mark.gpu
 synth = cases.synth
 
 
-def check(pkg, oracle, vals, scales, biases, R, C, xs):
+def tile_tokens(R, B):
+    """32 where that many tiles of 32 tokens x 256 rows still have a compute unit each."""
+    return 32 if -(-B // 32) * -(-R // 256) <= 256 else 64
+
+
+def matmul(pkg, vals, scales, biases, R, C, xs):
     got = pkg.lib.q4_matmul(vals, scales, biases, R, C, xs)
+    form = f"q4_mfma_kernel, tiles of {tile_tokens(R, xs.shape[0])} tokens"
+    assert pkg.lib.load().salt_mi355_last_kernel().decode() == form
+    return got
+
+
+def check(pkg, oracle, vals, scales, biases, R, C, xs):
+    got = matmul(pkg, vals, scales, biases, R, C, xs)
     want = reference(oracle, vals, scales, biases, R, C, xs)
     assert np.isfinite(got).all()
     bound = 2.0 ** -20 * magnitude_sums(vals, scales, biases, R, C, xs)[1] + 1e-6
@@ -35,8 +47,22 @@ def test_tile_forms(pkg, oracle, R, C, B):
     check(pkg, oracle, vals, scales, biases, R, C, synth.activations(C, B, 23))
 
 
-@pytest.mark.parametrize("R,C,B", [(100, 640, 40), (300, 2112, 70)])
-def test_scales_far_apart(pkg, oracle, R, C, B):
+@pytest.mark.parametrize("R,C,B", [(130, 576, 33), (300, 448, 65), (16640, 192, 130), (16448, 704, 129)])
+def test_without_biases(pkg, oracle, R, C, B):
+    print(f"mfma no biases R={R} C={C} B={B}", flush=True)
+    vals, scales, _ = synth.q4_tensor(R, C, R + C + B)
+    check(pkg, oracle, vals, scales, None, R, C, synth.activations(C, B, 24))
+
+
+def test_both_tile_forms_are_reached():
+    """The sizes in this file on both sides of the rule, with and without missing tokens in the second half of a tile."""
+    small, large = [(65, 33), (300, 65), (200, 100), (130, 33)], [(16640, 130), (16448, 129), (16640, 120)]
+    assert all(tile_tokens(*s) == 32 for s in small) and all(tile_tokens(*s) == 64 for s in large)
+
+
+@pytest.mark.parametrize("R,C,B", [(100, 640, 40), (300, 2112, 70), (16640, 192, 130), (16500, 640, 120)])
+@pytest.mark.parametrize("with_biases", [True, False])
+def test_scales_far_apart(pkg, oracle, R, C, B, with_biases):
     """Groups of a row up to 2^70 apart.  All but the first token see zeros where the scales are large, so that only the
     small ones decide their outputs."""
     print(f"mfma windows R={R} C={C} B={B}", flush=True)
@@ -50,7 +76,40 @@ def test_scales_far_apart(pkg, oracle, R, C, B):
     biases = ((-7.5 * synth.bf16_bits_to_f32(scales)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
     xs = synth.activations(C, B, 29)
     xs[1:, np.repeat(far, 64)] = 0.0
-    check(pkg, oracle, vals, scales, biases, R, C, xs)
+    check(pkg, oracle, vals, scales, biases if with_biases else None, R, C, xs)
+
+
+@pytest.mark.parametrize("R,C,B", [(300, 640, 40), (16640, 256, 130)])
+@pytest.mark.parametrize("kind", ["scale inf", "scale nan", "bias inf", "x inf", "x nan", "x 1e37", "scale 2^100", "scale subnormal"])
+def test_extreme_values_stay_in_their_row_or_token(pkg, oracle, R, C, B, kind):
+    """What is not finite makes the outputs of its row or token not finite and leaves the bits of all others alone; what is
+    finite and extreme keeps the bound."""
+    print(f"mfma {kind} R={R} C={C} B={B}", flush=True)
+    vals, scales, biases = synth.q4_tensor(R, C, 5)
+    xs = synth.activations(C, B, 6)
+    plain = matmul(pkg, vals, scales, biases, R, C, xs)
+    s, b, x, row, token = scales.reshape(R, -1).copy(), biases.reshape(R, -1).copy(), xs.copy(), 3, 5
+    if kind == "scale inf": s[row, 1] = 0x7F80
+    if kind == "scale nan": s[row, 1] = 0x7FC0
+    if kind == "bias inf": b[row, 2] = 0xFF80
+    if kind == "x inf": x[token, 70] = np.inf
+    if kind == "x nan": x[token, 70] = np.nan
+    if kind == "x 1e37": x[token] *= np.float32(1e36)
+    if kind == "scale 2^100": s[row] = 0x7180; b[row] = 0xF300       # 2^100 and -8 times that
+    if kind == "scale subnormal": s[row] = 1; b[row] = 0
+    got = matmul(pkg, vals, s.reshape(-1), b.reshape(-1), R, C, x)
+    hit = np.zeros((B, R), bool)
+    if kind.startswith("x"): hit[token] = True
+    else: hit[:, row] = True
+    assert np.array_equal(got.view(np.uint32)[~hit], plain.view(np.uint32)[~hit])
+    if "inf" in kind or "nan" in kind:
+        assert not np.isfinite(got[hit]).any()
+        return
+    tokens, rows = ([token], np.arange(R)) if kind.startswith("x") else (np.arange(B), [row])
+    pick = np.ascontiguousarray(vals.reshape(R, -1)[rows]).reshape(-1), s[rows].reshape(-1), b[rows].reshape(-1)
+    want = reference(oracle, *pick, len(rows), C, x[tokens])
+    bound = 2.0 ** -20 * magnitude_sums(*pick, len(rows), C, x[tokens])[1] + 1e-6
+    assert (np.abs(got[np.ix_(tokens, rows)].astype(np.float64) - want) <= bound).all()
 
 
 def test_token_bits_do_not_depend_on_the_call(pkg):

@@ -43,6 +43,43 @@ def test_q4_parts_with_staged_activations(pkg, oracle, R, C, B):
     assert np.array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("kernel,rows,C", [
+    ("q4_tile_kernel<2,{},16,0,4>", (70, 1, 1040, 333), 576),                     # 24 tiles: quarters
+    ("q4_tile_kernel<2,{},16,0,2>", (2112, 2100, 2112, 6), 192),                  # 100 tiles: halves
+    ("q4_tile_kernel<4,{},16,0,2>", (2112, 2112, 2100, 2112, 2112, 2111, 2112, 2049), 576),    # 264 tiles: halves, four chains
+    ("q4_tile_kernel<4,{},16,0,2>", (8192, 8190, 8130), 128),                     # 384 tiles, the last one of two rows
+])
+@pytest.mark.parametrize("tokens", [1, 2, 3, 4])
+def test_q4_job_tables_in_parts(pkg, oracle, kernel, rows, C, tokens):
+    """Several jobs with ragged last tiles, and in the second job a scale that takes the path for scales the converter's power
+    of two overflows."""
+    if tokens == 1:
+        kernel = kernel.replace("<2,{},16", "<2,1,32")
+    print(f"q4 jobs in parts {kernel} tokens={tokens}", flush=True)
+    lib = pkg.lib.init()
+    stream = lib.salt_mi355_stream()
+    hold, jobs, want = [], (pkg.lib.Q4Job * len(rows))(), []
+    for j, R in enumerate(rows):
+        vals, scales, biases = synth.q4_tensor(R, C, 50 + j)
+        if j == 1:
+            scales = scales.copy()
+            scales[-1] = 0x7B80                  # 2^120, in the job's last row
+            scales[0] = 0xFB80
+        xs = synth.activations(C, tokens, 60 + j)
+        y = np.zeros((tokens, R), np.float32)
+        for t in range(tokens):
+            assert oracle.orc_q4_matvec_threads(ptr(vals), ptr(scales), ptr(biases), R, C, ptr(xs[t]), ptr(y[t]), host_threads()) == 0
+        bufs = [pkg.lib.DeviceBuffer.from_host(a) for a in (vals, scales, biases, xs)] + [pkg.lib.DeviceBuffer(y.nbytes, fill=0xFF)]
+        jobs[j] = pkg.lib.Q4Job(*[b.ptr for b in bufs], R)
+        hold.append(bufs)
+        want.append(y)
+    pkg.lib.check(lib.salt_mi355_q4_jobs_dev(jobs, len(rows), C, tokens, 0, stream), "q4_jobs_dev")
+    pkg.lib.check(lib.salt_mi355_stream_sync(stream), "sync")
+    assert lib.salt_mi355_last_kernel().decode() == kernel.format(tokens)
+    for bufs, y in zip(hold, want):
+        assert np.array_equal(bits(bufs[4].to_host(np.float32).reshape(y.shape)), bits(y))
+
+
 @pytest.mark.parametrize("R,C", [(1, 64), (31, 544), (33, 4096), (100, 8192), (4096, 96), (4097, 96), (8192, 64), (8193, 64)])
 def test_nvfp4_parts_of_tiles(pkg, oracle, R, C):
     print(f"nvfp4 split R={R} C={C}", flush=True)
