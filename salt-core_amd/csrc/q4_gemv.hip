@@ -289,7 +289,9 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
     // group holds bytes 2t, 2t+1 of the first block and of the second, which is
     // exactly the pair of two-byte slices a four-chain wave consumes.
     constexpr int ROW_STEP = THREADS / CHUNK_GROUPS;
-    const bool has_item = tid < ROWS * CHUNK_GROUPS;    // only narrower than the block when THREADS == 1024
+    // Fewer items than threads with 1024 threads, and in parts of a tile whose steps are sixteen blocks: threads without
+    // one still bring activations (STEP_X), which issue() and commit() therefore do first.
+    const bool has_item = tid < ROWS * CHUNK_GROUPS;
     const uint32_t it_grp = tid % CHUNK_GROUPS;
     const uint32_t w_dst0 = ((tid / CHUNK_GROUPS) & (ROWS - 1)) * W_PITCH + it_grp * 32;
     const uint32_t m_dst0 = ((tid / CHUNK_GROUPS) & (ROWS - 1)) * M_PITCH + 2 * it_grp;
@@ -640,10 +642,13 @@ __global__ __launch_bounds__(256) void q4_generic_kernel(const Q4Launch L) {
 // Launches of at most this many tiles (one per compute unit) use the wide-step variant and two chains per lane.
 constexpr int WIDE_TILE_LIMIT = 256;
 
-// Workgroups per tile of a launch, as long as that gives more compute units work: sixteen-row workgroups up
-// to 96 tiles (beyond, the compute units that hold two of them take as long as with thirty-two rows), thirty-two-row ones
-// up to one per compute unit.  us before and after: 44 tiles of 2816 columns 10.8 / 6.8, of 8192 24.1 / 13.8, 96 of 2816
-// 10.9 / 7.5, 128 of 8192 25.7 / 17.3; three tokens: 44 of 2816 16.4 / 10.7, 128 of 4096 22.1 / 14.3.
+// Workgroups per tile of a launch of at most one tile per compute unit: sixteen-row workgroups up to 96 tiles,
+// thirty-two-row ones up to 128.  us whole / in halves / in quarters, one token, 2816 columns: 16 to 64 tiles 10.8 / 7.2 /
+// 6.8, 72 to 96 10.9 / 7.3 / 7.6, 112 and 128 11.0 / 7.4 / 7.7; three tokens 16.3 / 10.3 / 10.5, 16.6 / 10.5 / 11.5,
+// 16.6 / 10.7 / 11.7; 8192 columns, one token: 64 tiles 24.6 / 16.3 / 15.4, 96 24.7 / 16.6 / 17.2, 128 26.0 / 17.1 / 17.7.
+// So quarters pay for one token up to 64 tiles; the line at 96 costs up to 4 % there and, with three tokens, 10 %.
+// Beyond 128 tiles launches are left whole although parts are faster there too: 160 and 192 tiles 11.0 / 10.0 / 9.1
+// (three tokens 16.6 / 15.4 / 13.9), 256 11.4 / 10.3 / 13.2 (16.7 / 15.5 / 16.5).
 int tile_split(int tiles, int cols) {
     if (cols > SPLIT_MAX_COLS) return 1;
     return tiles <= 96 ? 4 : 2 * tiles <= WIDE_TILE_LIMIT ? 2 : 1;
@@ -682,7 +687,8 @@ int launch_tiles(const Q4Launch &L, bool may_split, hipStream_t stream) {
     if (S == 4 && may_split && L.total_tiles > WIDE_TILE_LIMIT && L.total_tiles <= WIDE_TILE_LIMIT * 3 / 2) {
         // Between one tile and one and a half per compute unit, some compute units have two and the rest wait for them:
         // in halves they have three of them at most (264 tiles of 2816 columns, one to four tokens: 14.8 / 20.7 / 22.7 / 28.6
-        // us whole, 13.2 / 18.0 / 20.0 / 23.6 in halves).  Three waves a SIMD need 168 registers or fewer: without that
+        // us whole, 13.2 / 18.0 / 20.0 / 23.6 in halves; 400 tiles 15.0 whole and 15.6 in halves, three tokens 22.9 and
+        // 26.8).  Quarters with two chains per lane do not pay up to 320 tiles (one token 15.3 us, three 19.5).  Three waves a SIMD need 168 registers or fewer: without that
         // bound three and four tokens took 26.9 and 32.2 us.
         note_kernel("q4_tile_kernel<4,%d,16,0,2>", L.tokens);
         const dim3 halves(2 * L.total_tiles);
