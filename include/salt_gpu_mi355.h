@@ -52,7 +52,8 @@ const char *salt_mi355_last_kernel(void);
  * returns for the low and high nibble of byte b.  Host arrays of 256 / 512. */
 int salt_mi355_converter_tables(float *fp8, float *fp4);
 
-/* ---- device memory and timing helpers for host harnesses --------------- */
+/* ---- device memory and timing helpers for host harnesses ---------------
+ * Uploads, downloads and fills are done when they return. */
 
 void *salt_mi355_dev_alloc(size_t nbytes);
 int salt_mi355_dev_free(void *device_ptr);

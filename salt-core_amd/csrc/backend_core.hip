@@ -230,7 +230,9 @@ int salt_mi355_dev_download(void *dst, const void *src, size_t nbytes) {
     return hip_ok(hipMemcpy(dst, src, nbytes, hipMemcpyDeviceToHost), "hipMemcpy D2H");
 }
 int salt_mi355_dev_fill(void *dst, int value, size_t nbytes) {
-    return hip_ok(hipMemset(dst, value, nbytes), "hipMemset");
+    // hipMemset returns before the memory is set, and the library's streams do not wait for the null stream it runs on
+    const int rc = hip_ok(hipMemset(dst, value, nbytes), "hipMemset");
+    return rc != 0 ? rc : hip_ok(hipStreamSynchronize(nullptr), "hipMemset sync");
 }
 void *salt_mi355_stream(void) { return g_state.stream; }
 int salt_mi355_stream_sync(void *stream) {
