@@ -3,8 +3,8 @@
 // exact cells, include/salt/gpu.h:211-234, src/gpu_hip.cpp:2034-2063, 2389-2458, 2688-2745).
 //
 // Every norm needs ss = x0*x0 + x1*x1 + ... added left to right in fp32.  The squares are computed by the whole
-// workgroup into LDS; one lane then walks them with dependent additions (several vectors at once ride in
-// neighbouring lanes of that wave).  inv = pow(ss / n + eps, -0.5) is six double-precision Newton steps from the
+// workgroup into LDS; one wave per vector then adds them (ordered_sum: the bits of the left-to-right chain, most of it
+// not walked).  inv = pow(ss / n + eps, -0.5) is six double-precision Newton steps from the
 // 0x5f3759df seed (src/bitmath.c:114-142).  A cell that meets a non-finite input or result publishes nothing and
 // sets the sticky status word to -1; a cell that finds the status word set does nothing.
 #include "device_math.h"
@@ -111,55 +111,287 @@ __device__ __forceinline__ float add_staged(const float *mine, int count, float 
     return acc;
 }
 
-// The same sums for at most SQ_CHUNK elements that the threads already hold: val[v][k] is element tid + k * THREADS of
-// vector v.
-template <int V>
-__device__ __forceinline__ void chains_from_registers(const float (&val)[V][SLOTS], int n, float *sq, float *shared,
-                                                      float (&ss)[V]) {
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int v = 0; v < V; ++v)
-#pragma unroll
-        for (int k = 0; k < SLOTS; ++k) {
-            const int i = tid + k * THREADS;
-            if (i < n) sq[v * SQ_CHUNK + i] = val[v][k] * val[v][k];
-        }
-    __syncthreads();
-    if (tid < V) shared[tid] = add_staged(sq + tid * SQ_CHUNK, n, 0.0f);
-    __syncthreads();
-#pragma unroll
-    for (int v = 0; v < V; ++v) ss[v] = shared[v];
-    __syncthreads();
+// ---- the same chain, not walked
+//
+// Between two powers of two every value of the accumulator is a multiple of one unit u, and adding x >= 0 moves it by
+// rint(x / u) units; only when x / u ends in exactly one half does the step depend on the accumulator, and then on its
+// last bit alone.  So while it stays in one binade the accumulator's bit pattern moves by an integer that is a function
+// of its last bit, and such functions compose: {d0, d1} is the number of units that a run of addends adds to an even
+// and to an odd accumulator.  A wave cuts the addends into 256 parts (lane l has parts 4 l .. 4 l + 3), guesses where
+// the chain stands at each part from plain sums, finds each part's {d0, d1} by adding its values to an even and an odd
+// number of that binade, and composes them over the wave.  Parts in which a guess leaves its binade are walked; where
+// the chain turns out to be in another binade than the guess, everything is: the guesses decide what is walked, never
+// the result.
+// (Subnormals and the lowest normal binade share their unit; a zero accumulator is even; infinities and NaN are walked.)
+//
+// 2816 squares of a normal vector: 9 of 235 parts are walked, 3.0 us instead of 10.1 for the chain (a lone wave issues a
+// vector instruction every eight clocks, 3.6 ns, which is what counts here).  The feed-forward block of 2816/2112/704
+// with 128 experts, three such sums deep: 90.1 -> 63.8 us; its first cell 13.5 -> 6.2 us, its last 30.6 -> 11.2.
+constexpr int ORDERED_MIN = 512;      // below, the chain is as quick
+constexpr int PARTS = 4;              // of a lane
+constexpr int ORDERED_FLOATS = 64 * (SQ_CHUNK / 64 + 4);     // LDS of SQ_CHUNK addends; a lane's block is 4 floats apart
+                                                             // from the next, so that 16-byte reads hit all banks
+struct OrderedScratch { int4 run[64 * PARTS + 1]; int walked[64 * PARTS + 1]; };
+
+// 16-byte words of a part: 1 to 4, so that 256 parts hold count <= SQ_CHUNK addends
+__device__ __forceinline__ int part_words(int count) { return (count + 1023) >> 10; }
+// place of addend i in LDS
+__device__ __forceinline__ int ordered_place(int i, int words) {
+    const int third = words == 3 ? 171 : 512 >> (words >> 1);     // (i / 16) / words, exact below 256
+    const int lane = ((i >> 4) * third) >> 9;
+    return i + 4 * lane;
 }
 
-// Serial sums of squares of `vectors` (1 or 2) vectors of n floats: lane v of wave 0 adds vector v's squares left to
-// right.  Returns the sums in ss_out[] on every thread; `bad` collects non-finite elements.  sq is LDS scratch of
-// vectors * SQ_CHUNK + SQ_TAIL floats, shared of at least `vectors` floats.
-__device__ void serial_square_sums(const float *const *x, int vectors, int n, float *sq, float *ss_out, float *shared,
+struct Units { int d0, d1; bool cut; };             // cut: a walked part lies inside, what came before it is forgotten
+__device__ __forceinline__ Units then(const Units &a, const Units &b) {
+    const int a0 = a.d0, a1 = a.d1, b0 = b.d0, b1 = b.d1;         // values: a choice between members is one of addresses
+    const int r0 = a0 + ((a0 & 1) ? b1 : b0), r1 = a1 + ((a1 & 1) ? b0 : b1);
+    return {b.cut ? b0 : r0, b.cut ? b1 : r1, a.cut || b.cut};
+}
+
+// The value of another lane as the data-parallel control says; lanes and rows it gives nothing to get `none`.
+template <int CTRL, int ROWS> __device__ __forceinline__ int from_lane(int none, int v) {
+    return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ void scan_step(float &v) {
+    v = __int_as_float(from_lane<CTRL, ROWS>(0, __float_as_int(v))) + v;
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ void scan_step(Units &v) {
+    const Units before = {from_lane<CTRL, ROWS>(0, v.d0), from_lane<CTRL, ROWS>(0, v.d1),
+                          from_lane<CTRL, ROWS>(0, (int)v.cut) != 0};
+    v = then(before, v);
+}
+// inclusive scan over the wave: within rows of 16 lanes (row_shr 1, 2, 4, 8), then across them (row_bcast 15, 31)
+template <typename T> __device__ __forceinline__ void wave_scan(T &v) {
+    scan_step<0x111, 0xf>(v); scan_step<0x112, 0xf>(v); scan_step<0x114, 0xf>(v); scan_step<0x118, 0xf>(v);
+    scan_step<0x142, 0xa>(v); scan_step<0x143, 0xc>(v);
+}
+constexpr int WAVE_SHR1 = 0x138;
+
+// acc + addend 0 + addend 1 + ..., left to right, by one whole wave; up to 1024 * WORDS addends at their ordered_place,
+// zeros behind the last; finite or not, never negative.
+template <int WORDS>
+__device__ __forceinline__ float ordered_sum(const float *addends, float acc, OrderedScratch &scratch) {
+    constexpr int PITCH = 16 * WORDS + 4;
+    typedef const float4 *words_ptr;
+    const int lane = threadIdx.x & 63;
+    const words_ptr mine = (words_ptr)(addends + lane * PITCH);
+    float total = 0.0f, sum[PARTS];
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+        sum[p] = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w) {
+            const float4 v = mine[p * WORDS + w];
+            sum[p] += (v.x + v.y) + (v.z + v.w);
+        }
+        total += sum[p];
+    }
+    wave_scan(total);
+    float guess = acc + __int_as_float(from_lane<WAVE_SHR1, 0xf>(0, __float_as_int(total)));
+    Units run[PARTS];
+    int binade[PARTS];                              // of a part that stays in one, else -1
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+        const int start = __float_as_int(guess) & ~1;
+        float even = __int_as_float(start), odd = __int_as_float(start | 1);
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w) {
+            const float4 v = mine[p * WORDS + w];
+            even = even + v.x; odd = odd + v.x;
+            even = even + v.y; odd = odd + v.y;
+            even = even + v.z; odd = odd + v.z;
+            even = even + v.w; odd = odd + v.w;
+        }
+        const int b = start >> 23;
+        const bool stays = (__float_as_int(even) >> 23) == b && (__float_as_int(odd) >> 23) == b && b != 255;
+        binade[p] = stays ? b : -1;
+        run[p] = {stays ? __float_as_int(even) - start : 0, stays ? __float_as_int(odd) - (start | 1) : 0, !stays};
+        guess += sum[p];
+    }
+    int before = from_lane<WAVE_SHR1, 0xf>(-1, binade[PARTS - 1]);
+    int position = 0, walks = 0;                    // among the walked parts: of this lane's first, and their number
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+        if (before >= 0 && binade[p] >= 0 && before != binade[p]) run[p] = {0, 0, true};      // the next binade starts here
+        before = binade[p];
+        const uint64_t walked = __ballot(run[p].cut);
+        position += __builtin_amdgcn_mbcnt_hi((uint32_t)(walked >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)walked, 0));
+        walks += __popcll(walked);
+    }
+    // Record r of `run` stands before part r: what the parts since the last walked one add, the bits that their binade
+    // has above the significand, and which of those bits to hold against it (none where the part before is walked itself).
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p)
+        if (run[p].cut) scratch.walked[position++] = lane * PARTS + p;
+    if (lane == 0) {
+        scratch.walked[walks] = 64 * PARTS;
+        scratch.run[0] = make_int4(0, 0, 0, 0);
+    }
+    bool cut[PARTS];
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) cut[p] = run[p].cut;
+#pragma unroll
+    for (int p = 1; p < PARTS; ++p) run[p] = then(run[p - 1], run[p]);
+    Units lanes = run[PARTS - 1];
+    wave_scan(lanes);
+    lanes = {from_lane<WAVE_SHR1, 0xf>(0, lanes.d0), from_lane<WAVE_SHR1, 0xf>(0, lanes.d1),
+             from_lane<WAVE_SHR1, 0xf>(0, (int)lanes.cut) != 0};
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+        const Units all = then(lanes, run[p]);
+        scratch.run[lane * PARTS + p + 1] = make_int4(all.d0, all.d1, binade[p] << 23, cut[p] ? 0 : (int)0xff800000u);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+    // From here on every lane does the same: the parts between two walked ones in one addition to the bit pattern, the
+    // walked ones addend by addend.  Lane l holds where the l-th walked part of a round of 64 lies; its record and its
+    // addends are read one walked part ahead.  Few instructions matter here: a lone wave issues one every eight clocks.
+    auto words_of = [&](int part) { return (words_ptr)(addends + (part >> 2) * PITCH + (part & 3) * 4 * WORDS); };
+    auto add = [&](const float4 &v) {
+        acc = acc + v.x;
+        acc = acc + v.y;
+        acc = acc + v.z;
+        acc = acc + v.w;
+    };
+    const float before_all = acc;
+    int wrong = 0;                                  // bits of a binade that was not the chain's
+    for (int k0 = 0; k0 <= walks; k0 += 64) {
+        const int part = scratch.walked[k0 + lane <= walks ? k0 + lane : walks];
+        const int here = walks + 1 - k0 < 64 ? walks + 1 - k0 : 64;
+        struct Ahead { int4 leap; float4 v[WORDS]; } even, odd;
+        auto read = [&](Ahead &to, int l) {
+            const int next = __builtin_amdgcn_readlane(part, l);
+            to.leap = scratch.run[next];
+            const words_ptr from = words_of(next < 64 * PARTS ? next : 0);
+#pragma unroll
+            for (int w = 0; w < WORDS; ++w) to.v[w] = from[w];
+        };
+        auto leap = [&](const Ahead &of) {
+            const int bits = __float_as_int(acc), d0 = of.leap.x, d1 = of.leap.y;
+            const int moved = bits + ((bits & 1) ? d1 : d0);
+            wrong |= ((bits ^ of.leap.z) | (moved ^ of.leap.z)) & of.leap.w;
+            acc = __int_as_float(moved);
+        };
+        auto walk = [&](const Ahead &of) {
+#pragma unroll
+            for (int w = 0; w < WORDS; ++w) add(of.v[w]);
+        };
+        const bool last_round = k0 + 64 > walks;    // its last entry is the end: a leap, nothing to walk
+        read(even, 0);
+        for (int l = 0;;) {
+            read(odd, l + 1 < 64 ? l + 1 : 63);
+            leap(even);
+            if (++l == here && last_round) break;
+            walk(even);
+            if (l == here) break;
+            read(even, l + 1 < 64 ? l + 1 : 63);
+            leap(odd);
+            if (++l == here && last_round) break;
+            walk(odd);
+            if (l == here) break;
+        }
+    }
+    if (__builtin_amdgcn_readfirstlane(wrong)) {    // a guess on the other side of a power of two: rare, so in full
+        acc = before_all;
+        for (int part = 0; part < 64 * PARTS; ++part)
+#pragma unroll
+            for (int w = 0; w < WORDS; ++w) add(words_of(part)[w]);
+    }
+    return acc;
+}
+
+// LDS of the sums of V vectors
+template <int V> struct SumScratch {
+    __attribute__((aligned(16))) float sq[V * ORDERED_FLOATS + SQ_TAIL];
+    OrderedScratch ordered[V];
+    float ss[V];
+};
+static_assert(ORDERED_FLOATS >= SQ_CHUNK && ORDERED_MIN <= SQ_CHUNK, "both layouts fit");
+
+// Sums of at most SQ_CHUNK staged squares: place(i) is where the square of element i of a vector of ORDERED_FLOATS goes;
+// add(v, acc) is called by the whole wave v.
+struct Staged {
+    int count, words;
+    bool chain;
+    __device__ explicit Staged(int n) : count(n), words(part_words(n)), chain(n < ORDERED_MIN) {}
+    __device__ int end() const { return chain ? count : 1024 * words; }
+    __device__ int place(int i) const { return chain ? i : ordered_place(i, words); }
+    __device__ __forceinline__ float add(const float *sq, float acc, OrderedScratch &scratch) const {
+        if (chain) return add_staged(sq, count, acc);
+        switch (words) {
+        case 1: return ordered_sum<1>(sq, acc, scratch);
+        case 2: return ordered_sum<2>(sq, acc, scratch);
+        case 3: return ordered_sum<3>(sq, acc, scratch);
+        default: return ordered_sum<4>(sq, acc, scratch);
+        }
+    }
+};
+
+// The sums of squares of `vectors` (at most V) vectors of at most SQ_CHUNK elements, a multiple of SLOTS, that the
+// threads already hold: val[v][k] is element SLOTS * tid + k of vector v (any value past the end).
+template <int V>
+__device__ __forceinline__ void chains_from_registers(const float (&val)[V][SLOTS], int vectors, int n,
+                                                      SumScratch<V> &scratch, float (&ss)[V]) {
+    static_assert(SLOTS == 4, "a thread's elements are 16 bytes");
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = SLOTS * tid;
+    const Staged staged(n);
+    if (i < staged.end())
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const float4 square = make_float4(val[v][0] * val[v][0], val[v][1] * val[v][1], val[v][2] * val[v][2],
+                                              val[v][3] * val[v][3]);
+            *(float4 *)&scratch.sq[v * ORDERED_FLOATS + staged.place(i)] = i < n ? square : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+    __syncthreads();
+    if (wave < vectors) {
+        const float sum = staged.add(scratch.sq + wave * ORDERED_FLOATS, 0.0f, scratch.ordered[wave]);
+        if ((tid & 63) == 0) scratch.ss[wave] = sum;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < V; ++v) ss[v] = scratch.ss[v];
+}
+
+// SLOTS consecutive floats on any four-byte boundary
+typedef float any_float4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_slots(const float *from, float (&to)[SLOTS]) {
+    const any_float4 v = *(const any_float4 *)from;
+    to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
+}
+__device__ __forceinline__ void store_slots(float *to, const float (&from)[SLOTS]) {
+    *(any_float4 *)to = any_float4{from[0], from[1], from[2], from[3]};
+}
+
+// Serial sums of squares of V vectors of n floats: wave v adds vector v's squares left to right.  Returns the sums in
+// ss_out[] on every thread; `bad` collects non-finite elements.
+template <int V>
+__device__ __forceinline__ void serial_square_sums(const float *const (&x)[V], int n, SumScratch<V> &scratch, float (&ss_out)[V],
                                    unsigned &bad) {
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     float acc = 0.0f;
     for (int base = 0; base < n; base += SQ_CHUNK) {
-        const int count = n - base < SQ_CHUNK ? n - base : SQ_CHUNK;
-        for (int v = 0; v < vectors; ++v) {
+        const Staged staged(n - base < SQ_CHUNK ? n - base : SQ_CHUNK);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
             const float *src = x[v] + base;
 #pragma unroll
             for (int k = 0; k < SLOTS; ++k) {
                 const int i = tid + k * THREADS;
-                if (i < count) {
-                    const float value = src[i];
-                    bad |= nonfinite(value);
-                    sq[v * SQ_CHUNK + i] = value * value;
-                }
+                const float value = i < staged.count ? src[i] : 0.0f;
+                bad |= nonfinite(value);
+                if (i < staged.end()) scratch.sq[v * ORDERED_FLOATS + staged.place(i)] = value * value;
             }
         }
         __syncthreads();
-        if (tid < vectors) acc = add_staged(sq + tid * SQ_CHUNK, count, acc);
+        if (wave < V) acc = staged.add(scratch.sq + wave * ORDERED_FLOATS, acc, scratch.ordered[wave]);
         __syncthreads();
     }
-    if (tid < vectors) shared[tid] = acc;
+    if (wave < V && (tid & 63) == 0) scratch.ss[wave] = acc;
     __syncthreads();
-    for (int v = 0; v < vectors; ++v) ss_out[v] = shared[v];
+#pragma unroll
+    for (int v = 0; v < V; ++v) ss_out[v] = scratch.ss[v];
     __syncthreads();
 }
 
@@ -180,14 +412,13 @@ struct NormArgs {
 };
 
 __global__ __launch_bounds__(THREADS) void norm_cell_kernel(NormArgs a) {
-    __shared__ __attribute__((aligned(16))) float sq[SQ_CHUNK + SQ_TAIL];
-    __shared__ float shared[4];
+    __shared__ SumScratch<1> scratch;
     if (*a.status != 0) return;
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps);
-    const float *vec[1] = {a.x};
-    float ss;
-    serial_square_sums(vec, 1, a.n, sq, &ss, shared, bad);
-    const float inv = inverse_from_sum(ss, a.n, a.eps);
+    const float *const vec[1] = {a.x};
+    float ss[1];
+    serial_square_sums<1>(vec, a.n, scratch, ss, bad);
+    const float inv = inverse_from_sum(ss[0], a.n, a.eps);
     bad |= nonfinite(inv);
     float root = a.root;
     if (a.kind == 1 && !(root > 0.0f)) root = 1.0f / det_sqrtf((float)a.n);
@@ -222,24 +453,21 @@ struct PreArgs {
     int *status;               // written, not only set: this kernel opens the block
 };
 
-// n <= SQ_CHUNK: every input is requested once, up front, and lives in registers from then on
+// n <= SQ_CHUNK, a multiple of SLOTS: every input is requested once, up front, and lives in registers from then on; a
+// thread has SLOTS consecutive elements
 __global__ __launch_bounds__(THREADS) void ffn_pre_small_kernel(PreArgs a) {
-    __shared__ __attribute__((aligned(16))) float sq[SQ_CHUNK + SQ_TAIL];
-    __shared__ float shared[4];
+    __shared__ SumScratch<1> scratch;
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps);
+    const int i = SLOTS * (int)threadIdx.x, at = i < a.n ? i : a.n - SLOTS;       // past the end the last elements again
     float r[1][SLOTS], w1[SLOTS], w2[SLOTS], rs[SLOTS];
+    load_slots(a.residual + at, r[0]);
+    load_slots(a.w1 + at, w1);
+    load_slots(a.w2 + at, w2);
+    load_slots(a.router_scale + at, rs);
 #pragma unroll
-    for (int k = 0; k < SLOTS; ++k) {
-        const int i = (int)threadIdx.x + k * THREADS;
-        const bool live = i < a.n;
-        r[0][k] = live ? a.residual[i] : 0.0f;
-        w1[k] = live ? a.w1[i] : 0.0f;
-        w2[k] = live ? a.w2[i] : 0.0f;
-        rs[k] = live ? a.router_scale[i] : 0.0f;
-        bad |= nonfinite(r[0][k]) | nonfinite(w1[k]) | nonfinite(w2[k]) | nonfinite(rs[k]);
-    }
+    for (int k = 0; k < SLOTS; ++k) bad |= nonfinite(r[0][k]) | nonfinite(w1[k]) | nonfinite(w2[k]) | nonfinite(rs[k]);
     float ss[1];
-    chains_from_registers<1>(r, a.n, sq, shared, ss);
+    chains_from_registers<1>(r, 1, a.n, scratch, ss);
     const float inv = inverse_from_sum(ss[0], a.n, a.eps);
     bad |= nonfinite(inv);
     const float root = 1.0f / det_sqrtf((float)a.n);
@@ -254,22 +482,19 @@ __global__ __launch_bounds__(THREADS) void ffn_pre_small_kernel(PreArgs a) {
     }
     const bool failed = __syncthreads_or((int)bad);
     if (threadIdx.x == 0) *a.status = failed ? -1 : 0;
-    if (failed) return;
-#pragma unroll
-    for (int k = 0; k < SLOTS; ++k) {
-        const int i = (int)threadIdx.x + k * THREADS;
-        if (i < a.n) { a.norm_a[i] = na[k]; a.norm_b[i] = nb[k]; a.router_in[i] = ri[k]; }
-    }
+    if (failed || i >= a.n) return;
+    store_slots(a.norm_a + i, na);
+    store_slots(a.norm_b + i, nb);
+    store_slots(a.router_in + i, ri);
 }
 
 __global__ __launch_bounds__(THREADS) void ffn_pre_kernel(PreArgs a) {
-    __shared__ __attribute__((aligned(16))) float sq[SQ_CHUNK + SQ_TAIL];
-    __shared__ float shared[4];
+    __shared__ SumScratch<1> scratch;
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps);
-    const float *vec[1] = {a.residual};
-    float ss;
-    serial_square_sums(vec, 1, a.n, sq, &ss, shared, bad);
-    const float inv = inverse_from_sum(ss, a.n, a.eps);
+    const float *const vec[1] = {a.residual};
+    float ss[1];
+    serial_square_sums<1>(vec, a.n, scratch, ss, bad);
+    const float inv = inverse_from_sum(ss[0], a.n, a.eps);
     bad |= nonfinite(inv);
     const float root = 1.0f / det_sqrtf((float)a.n);
     each_element(a.n, [&](int i) {
@@ -302,64 +527,80 @@ struct CombineArgs {
     int topk;
 };
 
-// n <= SQ_CHUNK: one load phase, everything else in registers and LDS
+// n <= SQ_CHUNK, a multiple of SLOTS: one load phase, everything else in registers and LDS; a thread has SLOTS consecutive
+// elements.  Bound by what one compute unit can fetch (six vectors and topk expert outputs, 158 KB at 2816 and eight, in
+// 2 us; a wait for each expert and four bytes per load took 7), then by the two rounds of sums, 3 us each.
 __global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
-    __shared__ __attribute__((aligned(16))) float sq[2 * SQ_CHUNK + SQ_TAIL];
-    __shared__ float shared[4];
-    if (*a.status != 0) return;
-    if (a.other && *a.other != 0) {
-        if (threadIdx.x == 0) *a.status = -1;
-        return;
-    }
+    __shared__ SumScratch<2> scratch;
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps) || nonfinite(a.scalar);
+    // Every input is asked for before anything is waited for, the status words among them; the experts' outputs eight
+    // at a time.
+    const int status = *a.status, other = a.other ? *a.other : 0;
+    const int i = SLOTS * (int)threadIdx.x, at = i < a.n ? i : a.n - SLOTS;       // past the end the last elements again
     float dr[2][SLOTS], res[SLOTS], wd[SLOTS], wr[SLOTS], wf[SLOTS];
+    load_slots(a.dense + at, dr[0]);
+    if (!a.expert_out) load_slots(a.routed + at, dr[1]);
+    else {
 #pragma unroll
-    for (int k = 0; k < SLOTS; ++k) {
-        const int i = (int)threadIdx.x + k * THREADS;
-        const bool live = i < a.n;
-        res[k] = live ? a.residual[i] : 0.0f;
-        wd[k] = live ? a.wd[i] : 0.0f;
-        wr[k] = live ? a.wr[i] : 0.0f;
-        wf[k] = live ? a.wf[i] : 0.0f;
-        dr[0][k] = live ? a.dense[i] : 0.0f;
-        dr[1][k] = live && !a.expert_out ? a.routed[i] : 0.0f;
-    }
-    if (a.expert_out)
-        for (int e = 0; e < a.topk; ++e) {
-            const float w = a.weights[e];
+        for (int k = 0; k < SLOTS; ++k) dr[1][k] = 0.0f;
+        for (int e0 = 0; e0 < a.topk; e0 += 8) {
+            float term[8][SLOTS], w[8];
 #pragma unroll
-            for (int k = 0; k < SLOTS; ++k) {
-                const int i = (int)threadIdx.x + k * THREADS;
-                if (i < a.n) {
-                    const float term = a.expert_out[(size_t)e * a.n + i] * w;
-                    dr[1][k] = dr[1][k] + term;
+            for (int e = 0; e < 8; ++e) {
+                if (e0 + e >= a.topk) break;
+                w[e] = a.weights[e0 + e];
+                load_slots(a.expert_out + (size_t)(e0 + e) * a.n + at, term[e]);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (e0 + e >= a.topk) break;
+#pragma unroll
+                for (int k = 0; k < SLOTS; ++k) {
+                    const float product = term[e][k] * w[e];
+                    dr[1][k] = dr[1][k] + product;
                 }
             }
         }
+    }
+    load_slots(a.residual + at, res);
+    load_slots(a.wd + at, wd);
+    load_slots(a.wr + at, wr);
+    load_slots(a.wf + at, wf);
+    if (status != 0) return;
+    if (other != 0) {
+        if (threadIdx.x == 0) *a.status = -1;
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < SLOTS; ++k)
         bad |= nonfinite(res[k]) | nonfinite(wd[k]) | nonfinite(wr[k]) | nonfinite(wf[k]) | nonfinite(dr[0][k]) |
                nonfinite(dr[1][k]);
-    float ss[2];
-    chains_from_registers<2>(dr, a.n, sq, shared, ss);
-    const float inv_d = inverse_from_sum(ss[0], a.n, a.eps), inv_r = inverse_from_sum(ss[1], a.n, a.eps);
-    bad |= nonfinite(inv_d) | nonfinite(inv_r);
-    float sum[1][SLOTS];
+    // Two rounds of sums through the same instructions (twice the code is twice the time to fetch it): the two branches,
+    // then their sum in dr[0].
+    float inv = 0.0f;
+#pragma unroll 1
+    for (int vectors = 2; vectors >= 1; --vectors) {
+        float ss[2];
+        chains_from_registers<2>(dr, vectors, a.n, scratch, ss);
+        // odd lanes see to the routed branch
+        const bool odd = (threadIdx.x & 1) != 0 && vectors == 2;
+        inv = inverse_from_sum(odd ? ss[1] : ss[0], a.n, a.eps);
+        bad |= nonfinite(inv);
+        if (vectors == 1) break;
+        const float inv_d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), 0));
+        const float inv_r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), 1));
 #pragma unroll
-    for (int k = 0; k < SLOTS; ++k) {
-        const float d0 = dr[0][k] * inv_d, r0 = dr[1][k] * inv_r;
-        const float d = d0 * wd[k], r = r0 * wr[k];
-        sum[0][k] = d + r;
-        bad |= nonfinite(d0) | nonfinite(r0) | nonfinite(d) | nonfinite(r) | nonfinite(sum[0][k]);
+        for (int k = 0; k < SLOTS; ++k) {
+            const float d0 = dr[0][k] * inv_d, r0 = dr[1][k] * inv_r;
+            const float d = d0 * wd[k], r = r0 * wr[k];
+            dr[0][k] = d + r;
+            bad |= nonfinite(d0) | nonfinite(r0) | nonfinite(d) | nonfinite(r) | nonfinite(dr[0][k]);
+        }
     }
-    float ss_sum[1];
-    chains_from_registers<1>(sum, a.n, sq, shared, ss_sum);
-    const float inv_f = inverse_from_sum(ss_sum[0], a.n, a.eps);
-    bad |= nonfinite(inv_f);
     float y[SLOTS];
 #pragma unroll
     for (int k = 0; k < SLOTS; ++k) {
-        const float f0 = sum[0][k] * inv_f;
+        const float f0 = dr[0][k] * inv;
         const float f = f0 * wf[k];
         y[k] = (res[k] + f) * a.scalar;
         bad |= nonfinite(f0) | nonfinite(f) | nonfinite(y[k]);
@@ -368,16 +609,12 @@ __global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
         if (threadIdx.x == 0) *a.status = -1;
         return;
     }
-#pragma unroll
-    for (int k = 0; k < SLOTS; ++k) {
-        const int i = (int)threadIdx.x + k * THREADS;
-        if (i < a.n) a.out[i] = y[k];
-    }
+    if (i < a.n) store_slots(a.out + i, y);
 }
 
 __global__ __launch_bounds__(THREADS) void combine_cell_kernel(CombineArgs a) {
-    __shared__ __attribute__((aligned(16))) float sq[2 * SQ_CHUNK + SQ_TAIL];
-    __shared__ float shared[4];
+    __shared__ SumScratch<2> scratch;
+    __shared__ SumScratch<1> scratch_sum;
     if (*a.status != 0) return;
     if (a.other && *a.other != 0) {
         if (threadIdx.x == 0) *a.status = -1;
@@ -408,9 +645,9 @@ __global__ __launch_bounds__(THREADS) void combine_cell_kernel(CombineArgs a) {
             }
         }
     }
-    const float *vec[2] = {a.dense, a.routed};
+    const float *const vec[2] = {a.dense, a.routed};
     float ss[2];
-    serial_square_sums(vec, 2, a.n, sq, ss, shared, bad);
+    serial_square_sums<2>(vec, a.n, scratch, ss, bad);
     const float inv_d = inverse_from_sum(ss[0], a.n, a.eps), inv_r = inverse_from_sum(ss[1], a.n, a.eps);
     bad |= nonfinite(inv_d) | nonfinite(inv_r);
     each_element(a.n, [&](int i) {
@@ -422,10 +659,10 @@ __global__ __launch_bounds__(THREADS) void combine_cell_kernel(CombineArgs a) {
                nonfinite(s);
         a.sum[i] = s;
     });
-    const float *vec2[1] = {a.sum};                     // a thread reads back the elements it wrote itself
-    float ss_sum;
-    serial_square_sums(vec2, 1, a.n, sq, &ss_sum, shared, bad);
-    const float inv_f = inverse_from_sum(ss_sum, a.n, a.eps);
+    const float *const vec2[1] = {a.sum};               // a thread reads back the elements it wrote itself
+    float ss_sum[1];
+    serial_square_sums<1>(vec2, a.n, scratch_sum, ss_sum, bad);
+    const float inv_f = inverse_from_sum(ss_sum[0], a.n, a.eps);
     bad |= nonfinite(inv_f);
     each_element(a.n, [&](int i) {
         const float f0 = a.sum[i] * inv_f;
@@ -478,7 +715,7 @@ int ffn_pre_launch(const float *residual, const float *w1, const float *w2, cons
                    float *norm_b, float *router_in, int n, float eps, int *status, hipStream_t stream) {
     if (!residual || !w1 || !w2 || !router_scale || !norm_a || !norm_b || !router_in || !status || n < 1) return -1;
     PreArgs a = {residual, w1, w2, router_scale, norm_a, norm_b, router_in, n, eps, status};
-    if (n <= SQ_CHUNK) ffn_pre_small_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
+    if (n <= SQ_CHUNK && n % SLOTS == 0) ffn_pre_small_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
     else ffn_pre_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
     return launched() ? 0 : -1;
 }
@@ -492,7 +729,7 @@ int combine_cell_launch(const float *residual, const float *dense, const float *
         return -1;
     CombineArgs a = {residual, dense, routed, wd, wr, wf, sum_scratch, out, n, eps, scalar, status, other_status,
                      expert_out, weights, topk};
-    if (n <= SQ_CHUNK) combine_small_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
+    if (n <= SQ_CHUNK && n % SLOTS == 0) combine_small_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
     else combine_cell_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
     return launched() ? 0 : -1;
 }
