@@ -43,10 +43,12 @@ struct MoeFuse {
     int *status;                  // 0, or -1 when the router rejected its input (then nothing else is written)
     int n_experts, topk, hidden, routed;
     // q4_moe_gate_up_launch / q4_moe_down_launch only, both null or both set: the down launch also writes the layer
-    // output.  arrivals holds one counter per 64-row tile of the output; the gate/up launch zeroes them, and the last
-    // of the topk workgroups of the down launch to finish a tile adds that tile's expert outputs in expert order.
+    // output.  arrivals holds one counter per arrival_rows rows of the output (q4_moe_arrival_rows: 64, or the rows of
+    // the down launch's parts of a tile); the gate/up launch zeroes them, and the last of the topk workgroups of the
+    // down launch to finish those rows adds their expert outputs in expert order.
     float *out;                   // [hidden]
-    int *arrivals;                // [ceil(hidden / 64)]
+    int *arrivals;                // [ceil(hidden / arrival_rows)]
+    int arrival_rows;
 };
 constexpr int MOE_FUSE_MAX_ROUTED = 4096;      // activations of one expert held in LDS by the down launch
 constexpr int MOE_FUSE_MAX_EXPERTS = 512;      // one thread per expert in the gate/up prologue
@@ -70,6 +72,7 @@ struct Q4Launch {
 };
 int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream);   // fills tiles and jobs from launch.moe
 int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream);
+int q4_moe_arrival_rows(int hidden, int routed, int topk);     // as the down launch prefers; 64 is always possible
 
 // chains_per_lane: 8, 4 or 2; 0 lets the launcher choose from the tile count.
 int q4_launch(const Q4Launch &launch, int chains_per_lane, hipStream_t stream);

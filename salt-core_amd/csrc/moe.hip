@@ -168,7 +168,16 @@ int moe_decode_step_launch(const MoeGeometry &g, const uint8_t *pool, size_t exp
         m.logits = logits; m.per_expert_scale = per_expert_scale; m.pool = pool; m.expert_stride = expert_stride;
         m.x = x; m.gate = ws.gate; m.up = ws.up; m.expert_out = eo; m.selected = selected; m.weights = weights;
         m.status = ws.status; m.n_experts = g.n_experts; m.topk = g.topk; m.hidden = g.hidden; m.routed = g.routed;
-        m.out = out; m.arrivals = out ? ws.arrivals : nullptr;
+        m.out = out;
+        if (out) {
+            // counters of parts of a tile lie where this plan keeps nothing else, or the down launch runs whole tiles
+            m.arrival_rows = q4_moe_arrival_rows(g.hidden, g.routed, g.topk);
+            m.arrivals = (int *)ws.act;
+            if (m.arrival_rows == 64 || (long long)(g.hidden + m.arrival_rows - 1) / m.arrival_rows > (long long)g.topk * g.routed) {
+                m.arrival_rows = 64;
+                m.arrivals = ws.arrivals;
+            }
+        }
         if (q4_moe_gate_up_launch(fused, stream) != 0) return -1;
         return q4_moe_down_launch(fused, stream);
     }

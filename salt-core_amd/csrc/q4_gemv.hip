@@ -119,7 +119,12 @@ template <int S, int NB, int XN, int NNIB, bool SLOW>
 __device__ __forceinline__ void consume_word(uint32_t w, int first_block, int xbase, float scale, float bias,
                                              const float (&x)[NB][XN], float code_scale, float (&acc)[NB][S]) {
     float q[8];
-    nibbles_to_f32(w, q);
+    if (S == 1) {                    // one nibble in each of the two low bytes: the first block's and the second's
+        const f32x2 pair = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
+        q[0] = pair.x; q[1] = pair.y;
+    } else {
+        nibbles_to_f32(w, q);
+    }
 #pragma unroll
     for (int n = 0; n < NNIB; ++n) {
         const int blk = first_block + ((S == 8) ? 0 : n / S);
@@ -163,14 +168,16 @@ constexpr int x_batch_groups(int S, int NB) {
 // a wave then holds SPLIT chain slices of ROWS rows, lane l row l % ROWS of slice SPLIT * wave + l / ROWS, so a
 // workgroup has 1 / SPLIT of the waves and a wave the same work.  The chain order leaves rows as the only axis to cut
 // along, and a wave's instruction count does not shrink with idle lanes.  The slice differs inside a wave, so the
-// activations come from LDS as in the prologues above.
-// One token: 2816 x 2816 (44 tiles) 10.8 -> 6.8 us.
+// activations come from LDS as in the prologues above.  One chain per lane (S = 1) leaves a wave with fewer than half of
+// the instructions of two and doubles the waves: a lone wave issues one every eight clocks, two on a SIMD fill it.
+// One token, 2816 x 2816 (44 tiles): 10.8 us whole, 6.9 in quarters with two chains per lane, 5.9 with one.
 template <int S, int NB, int CB, int PRO = 0, int SPLIT = 1>
 __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 1) void q4_tile_kernel(const Q4Launch L) {
     constexpr int CHUNK_BLOCKS = CB;
     constexpr int ROWS = TILE_ROWS / SPLIT;
     constexpr bool LDS_X = PRO >= 2 || SPLIT > 1;
-    constexpr bool STEP_X = SPLIT > 1 && (S == 4 || NB > 1);   // activations staged with each step's weights, not the whole row
+    // activations staged with each step's weights, not the whole row (a prologue that computes them computes the whole row)
+    constexpr bool STEP_X = PRO < 2 && SPLIT > 1 && (S == 4 || NB > 1);
     constexpr int CHUNK_GROUPS = CB / 2;                   // 64-column scale groups per step
     constexpr int W_PITCH = 16 * CB + 4;                   // bytes per staged row: odd dword pitch
     constexpr int M_PITCH = 2 * CHUNK_GROUPS + 2;          // floats per staged row of (scale, bias)
@@ -185,15 +192,15 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
     constexpr int XG = STEP_X && NB >= 3 ? 1 : LDS_X ? 2 : x_batch_groups(S, NB);        // LDS-fed activations sit in vector registers: short batches
     constexpr int XN = XG * 2 * S;
     static_assert(THREADS >= NB * ROWS, "fold needs one thread per (token, row)");
-    static_assert(SPLIT == 1 || (PRO != 2 && (NB == 1 || STEP_X)), "the down launch counts whole tiles; LDS holds one whole row");
+    static_assert(SPLIT == 1 || NB == 1 || STEP_X, "LDS holds one whole row");
 
     __shared__ __attribute__((aligned(16))) uint8_t w_lds[W_BYTES];
     __shared__ __attribute__((aligned(16))) float m_lds[2 * M_STAGE];
     __shared__ __attribute__((aligned(16))) float x_lds[PRO >= 2 ? MOE_FUSE_MAX_ROUTED : STEP_X ? 2 * NB * CB * 32 : SPLIT > 1 ? SPLIT_MAX_COLS : 4];
     __shared__ int slow_flag;
     static_assert(PRO == 0 || NB == 1, "the MoE prologues serve the single-token kernel");
-    static_assert(PRO != 1 || (sizeof(RouterShared) <= W_BYTES && THREADS >= MOE_FUSE_MAX_EXPERTS),
-                  "the router prologue borrows the weight staging memory and one thread per expert");
+    // the router prologue borrows memory that is used later, and one thread per expert (q4_moe_gate_up_launch sees to that)
+    static_assert(PRO != 1 || sizeof(RouterShared) <= (SPLIT > 1 && !STEP_X ? sizeof x_lds : W_BYTES), "the router fits");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -202,7 +209,8 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
     // lane's row of the tile and its slice of the chains
     const int lane_row = lane & (ROWS - 1);
     const int slice = SPLIT == 1 ? wave : wave * SPLIT + lane / ROWS;
-    const int tile = SPLIT == 1 ? (int)blockIdx.x : (int)blockIdx.x / SPLIT;
+    const int part = (int)blockIdx.x - (PRO == 1 ? 1 : 0);      // workgroup 0 of the MoE gate/up launch is the router's publisher
+    const int tile = SPLIT == 1 ? part : part / SPLIT;
 
     Q4Job job;
     const float *act_gate = nullptr, *act_up = nullptr;     // PRO >= 2: the activation row is gelu_tanh(gate) * up
@@ -217,10 +225,10 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
         const size_t n = (size_t)m.hidden * (size_t)m.routed;
         const size_t vals_bytes = n / 2, meta_bytes = (n / 64) * 2, proj_bytes = vals_bytes + 2 * meta_bytes;
         if (PRO == 1) {
-            RouterShared &sh = *reinterpret_cast<RouterShared *>(w_lds);
-            const bool publisher = tile == L.total_tiles;                  // one workgroup past the tiles
+            RouterShared &sh = *reinterpret_cast<RouterShared *>(SPLIT > 1 && !STEP_X ? (uint8_t *)x_lds : w_lds);
+            const bool publisher = blockIdx.x == 0;
             const int up_tiles = (m.routed + TILE_ROWS - 1) / TILE_ROWS;
-            const int slot_index = tile / up_tiles;                        // 2 * place + (0 gate | 1 up)
+            const int slot_index = tile / up_tiles;                        // 2 * place + (0 gate | 1 up); of tiles
             const int place = slot_index >> 1, proj = slot_index & 1;
             int expert;
             if (!publisher && m.n_experts <= ROUTER_WAVE_MAX_EXPERTS) {
@@ -234,8 +242,8 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
                 if (publisher) {
                     if (tid == 0) *m.status = bad ? -1 : 0;
                     if (tid < m.topk && !bad) { m.selected[tid] = sh.out_sel[tid]; m.weights[tid] = sh.out_w[tid]; }
-                    if (m.arrivals)                 // the down launch counts its workgroups per tile of the output
-                        for (int i = tid; i < (m.hidden + TILE_ROWS - 1) / TILE_ROWS; i += THREADS) m.arrivals[i] = 0;
+                    if (m.arrivals)                 // the down launch counts its workgroups per tile, or part, of the output
+                        for (int i = tid; i < (m.hidden + m.arrival_rows - 1) / m.arrival_rows; i += THREADS) m.arrivals[i] = 0;
                     return;
                 }
                 if (bad) return;                                           // uniform
@@ -252,7 +260,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
         } else {
             if (*(const int __attribute__((address_space(4))) *)(uintptr_t)m.status != 0) return;
             const int down_tiles = (m.hidden + TILE_ROWS - 1) / TILE_ROWS;
-            const int place = (int)blockIdx.x / down_tiles;
+            const int place = tile / down_tiles;
             const int expert = ((const int __attribute__((address_space(4))) *)(uintptr_t)m.selected)[place];
             act_gate = m.gate + (size_t)place * m.routed; act_up = m.up + (size_t)place * m.routed;
             job.vals = m.pool + (size_t)expert * m.expert_stride + 2 * proj_bytes;
@@ -266,7 +274,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
         job.scales = job.vals + vals_bytes;
         job.biases = job.scales + meta_bytes;
     }
-    const int row0 = (tile - job.tile0) * TILE_ROWS + (SPLIT == 1 ? 0 : ((int)blockIdx.x % SPLIT) * ROWS);
+    const int row0 = (tile - job.tile0) * TILE_ROWS + (SPLIT == 1 ? 0 : (part % SPLIT) * ROWS);
     const int R = job.rows;
     if (SPLIT > 1 && row0 >= R) return;             // uniform: the rest of a job's last tile
     const int rows_here = R - row0 < ROWS ? R - row0 : ROWS;
@@ -445,8 +453,9 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
 
         const int slow = __builtin_amdgcn_readfirstlane(slow_flag);
         // wave t reads dword t (S == 4), dwords 2t and 2t+1 (S == 8) or dword t / 2 (S == 2) of every group
-        const uint8_t *wrow = w_lds + stage * W_STAGE + lane_row * W_PITCH + (S == 2 ? (slice >> 1) * 4 : slice * S);
-        const uint32_t byte_pick = 0x0C0C0000u | (uint32_t)((2 + (slice & 1)) << 8) | (uint32_t)(slice & 1);
+        const uint8_t *wrow = w_lds + stage * W_STAGE + lane_row * W_PITCH + (S == 1 ? (slice >> 2) * 4 : S == 2 ? (slice >> 1) * 4 : slice * S);
+        const int byte_of = S == 1 ? (slice >> 1) & 1 : slice & 1;
+        const uint32_t byte_pick = 0x0C0C0000u | (uint32_t)((2 + byte_of) << 8) | (uint32_t)byte_of;
         const float *mrow = m_lds + stage * M_STAGE + lane_row * M_PITCH;
 
         // LDS operands of group g of this step: the lane's nibbles and (scale', bias)
@@ -464,6 +473,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
             } else {                 // S == 2: byte (t & 1) of each half of dword t / 2
                 const uint32_t d = *reinterpret_cast<const uint32_t *>(wrow + g * 32);
                 w0 = __builtin_amdgcn_perm(0u, d, byte_pick);
+                if (S == 1) w0 = (w0 >> (4 * (slice & 1))) & 0x0F0Fu;      // and one nibble of each
             }
         };
 
@@ -481,7 +491,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
                         consume_word<S, NB, XN, 8, false>(w0, 0, gl * 2 * S, scale, bias, xq, L.code_scale, acc);
                         consume_word<S, NB, XN, 8, false>(w1, 1, gl * 2 * S, scale, bias, xq, L.code_scale, acc);
                     } else {
-                        consume_word<S, NB, XN, (S == 4 ? 8 : 4), false>(w0, 0, gl * 2 * S, scale, bias, xq,
+                        consume_word<S, NB, XN, 2 * S, false>(w0, 0, gl * 2 * S, scale, bias, xq,
                                                                                  L.code_scale, acc);
                     }
                 }
@@ -502,7 +512,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
                             consume_word<S, NB, XN, 8, false>(w0, 0, gl * 2 * S, scale, bias, xq, L.code_scale, acc);
                             consume_word<S, NB, XN, 8, false>(w1, 1, gl * 2 * S, scale, bias, xq, L.code_scale, acc);
                         } else {
-                            consume_word<S, NB, XN, (S == 4 ? 8 : 4), false>(w0, 0, gl * 2 * S, scale, bias, xq,
+                            consume_word<S, NB, XN, 2 * S, false>(w0, 0, gl * 2 * S, scale, bias, xq,
                                                                                      L.code_scale, acc);
                         }
                     }
@@ -519,7 +529,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
                         consume_word<S, NB, XN, 8, true>(w0, 0, 0, scale, bias, xq, L.code_scale, acc);
                         consume_word<S, NB, XN, 8, true>(w1, 1, 0, scale, bias, xq, L.code_scale, acc);
                     } else {
-                        consume_word<S, NB, XN, (S == 4 ? 8 : 4), true>(w0, 0, 0, scale, bias, xq,
+                        consume_word<S, NB, XN, 2 * S, true>(w0, 0, 0, scale, bias, xq,
                                                                                 L.code_scale, acc);
                     }
                 } else {
@@ -527,7 +537,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
                         consume_word<S, NB, XN, 8, false>(w0, 0, 0, scale, bias, xq, L.code_scale, acc);
                         consume_word<S, NB, XN, 8, false>(w1, 1, 0, scale, bias, xq, L.code_scale, acc);
                     } else {
-                        consume_word<S, NB, XN, (S == 4 ? 8 : 4), false>(w0, 0, 0, scale, bias, xq,
+                        consume_word<S, NB, XN, 2 * S, false>(w0, 0, 0, scale, bias, xq,
                                                                                  L.code_scale, acc);
                     }
                 }
@@ -555,7 +565,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
         const float odd = part[1] + part[3];
         if (PRO != 2 || !L.moe.arrivals) {
             if (lane_row < rows_here) y[(size_t)t * job.y_stride + row0 + lane_row] = even + odd;
-        } else {                                        // uniform; NB == 1: these are the 64 lanes of wave 0
+        } else {                                        // uniform; NB == 1: these are the first ROWS lanes of wave 0
             // The layer output (reference gemma4_text.c:8301-8304: out = 0; out += o_i * w_i in ascending expert
             // order, product and sum rounded separately).  The topk workgroups that own these rows of the topk
             // experts count themselves in; the one that arrives last finds every expert's rows written and adds
@@ -569,7 +579,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
             if (lane < rows_here) __hip_atomic_store(mine + lane, even + odd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             int before = 0;
-            if (tid == 0) before = __hip_atomic_fetch_add(m.arrivals + (row0 / TILE_ROWS), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (tid == 0) before = __hip_atomic_fetch_add(m.arrivals + (row0 / ROWS), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             before = __builtin_amdgcn_readfirstlane(before);    // waits for the count's return
             if (before == m.topk - 1 && lane < rows_here) {
                 float total = 0.0f;
@@ -639,77 +649,99 @@ __global__ __launch_bounds__(256) void q4_generic_kernel(const Q4Launch L) {
     }
 }
 
-// Launches of at most this many tiles (one per compute unit) use the wide-step variant and two chains per lane.
-constexpr int WIDE_TILE_LIMIT = 256;
+// How a launch is cut: chains per lane, blocks staged per step, workgroups per tile.
+struct TileShape {
+    int chains, blocks, split;
+    int threads() const { return 64 * 32 / (chains * split); }
+};
 
-// Workgroups per tile of a launch of at most one tile per compute unit: sixteen-row workgroups up to 96 tiles,
-// thirty-two-row ones up to 128.  us whole / in halves / in quarters, one token, 2816 columns: 16 to 64 tiles 10.8 / 7.2 /
-// 6.8, 72 to 96 10.9 / 7.3 / 7.6, 112 and 128 11.0 / 7.4 / 7.7; three tokens 16.3 / 10.3 / 10.5, 16.6 / 10.5 / 11.5,
-// 16.6 / 10.7 / 11.7; 8192 columns, one token: 64 tiles 24.6 / 16.3 / 15.4, 96 24.7 / 16.6 / 17.2, 128 26.0 / 17.1 / 17.7.
-// So quarters pay for one token up to 64 tiles; the line at 96 costs up to 4 % there and, with three tokens, 10 %.
-// Beyond 128 tiles launches are left whole although parts are faster there too: 160 and 192 tiles 11.0 / 10.0 / 9.1
-// (three tokens 16.6 / 15.4 / 13.9), 256 11.4 / 10.3 / 13.2 (16.7 / 15.5 / 16.5).
-int tile_split(int tiles, int cols) {
-    if (cols > SPLIT_MAX_COLS) return 1;
-    return tiles <= 96 ? 4 : 2 * tiles <= WIDE_TILE_LIMIT ? 2 : 1;
+constexpr int COMPUTE_UNITS = 256;
+
+// Whole tiles: up to one per compute unit, sixteen waves per tile (two chains per lane) hide more of the LDS and
+// scalar-load latency, and a single token's workgroup, alone on its compute unit, stages twice as much per step; beyond
+// that four chains per lane win (one token, 2816 columns: 10.4 against 10.8 us at 256 tiles, 14.2 against 20.3 at 264;
+// eight chains per lane never do).
+TileShape whole_shape(int chains, int tiles, int tokens) {
+    return {chains, tokens == 1 && chains <= 4 && tiles <= COMPUTE_UNITS ? 32 : 16, 1};
 }
 
-template <int S>
-int launch_tiles(const Q4Launch &L, bool may_split, hipStream_t stream) {
-    const dim3 grid(L.total_tiles), block((32 / S) * 64);
-    const int split = S == 2 && may_split ? tile_split(L.total_tiles, L.tokens == 1 ? L.cols : 0) : 1;
-    if (split > 1 && L.tokens > 1) {
-        note_kernel("q4_tile_kernel<2,%d,16,0,%d>", L.tokens, split);
-        const dim3 parts(split * L.total_tiles), threads(1024 / split);
-        switch (L.tokens * 8 + split) {
-            case 2 * 8 + 2: hipLaunchKernelGGL((q4_tile_kernel<2, 2, 16, 0, 2>), parts, threads, 0, stream, L); break;
-            case 3 * 8 + 2: hipLaunchKernelGGL((q4_tile_kernel<2, 3, 16, 0, 2>), parts, threads, 0, stream, L); break;
-            case 4 * 8 + 2: hipLaunchKernelGGL((q4_tile_kernel<2, 4, 16, 0, 2>), parts, threads, 0, stream, L); break;
-            case 2 * 8 + 4: hipLaunchKernelGGL((q4_tile_kernel<2, 2, 16, 0, 4>), parts, threads, 0, stream, L); break;
-            case 3 * 8 + 4: hipLaunchKernelGGL((q4_tile_kernel<2, 3, 16, 0, 4>), parts, threads, 0, stream, L); break;
-            case 4 * 8 + 4: hipLaunchKernelGGL((q4_tile_kernel<2, 4, 16, 0, 4>), parts, threads, 0, stream, L); break;
-            default: return -1;
-        }
-        return hipGetLastError() == hipSuccess ? 0 : -1;
+// The shape of a launch whose caller leaves it open.  A compute unit's time follows the rows of the fullest one, so parts
+// pay where whole tiles leave some idle or some with one tile more than the rest.  us, 2816 columns:
+//   tiles      one token                                      three tokens
+//   16 - 64    quarters <1> 5.9, <2> 7.0, halves 7.4, whole 10.8   8.7 / 10.9 / 10.6 / 16.4
+//   65 - 96    eighths <1> 6.9, quarters <1> 7.5, halves 7.4      quarters <1> 10.9, halves 10.5, quarters <2> 11.7
+//   97 - 128   halves 7.4, quarters <1> 7.6                       halves 10.6, quarters <1> 11.2
+//   129 - 192  quarters <2> 8.9, halves 9.7, whole 10.2            14.3 / 15.7 / 16.4
+//   193 - 256  halves 10.0, quarters <2> 13.7, whole 10.3           15.7 / 16.6 / 16.4
+//   257 - 384  halves <4> 12.3, quarters <2> 14.7, whole <4> 14.2  20.3 / 19.7 / 22.8
+//   385 - 512  whole <4> 14.9, halves <4> 15.7                    22.8 / 27.6
+//   513 - 640  whole <4> 19.1, halves <4> 19.2                    35.0 / 31.3
+// (<n>: chains per lane.  257 - 384 with three or four tokens: three waves a SIMD need 168 registers or fewer; without
+// that bound halves took 26.9 and 32.2 us.)  Two and four tokens as three.  Below 1024 columns one chain per lane gives
+// nothing (a launch of any shape takes 4.2 to 4.6 us), and at 513 - 640 tiles 5 to 7 % as everywhere.
+// A single token's parts keep its whole row in LDS, except <4>, which stages activations with each step's weights.
+TileShape open_shape(int tiles, int cols, int tokens) {
+    const int wide = tokens == 1 ? 32 : 16;
+    if (tiles > COMPUTE_UNITS) {
+        const bool uneven = tiles <= COMPUTE_UNITS * 3 / 2 || (tokens > 1 && tiles > 2 * COMPUTE_UNITS && tiles <= COMPUTE_UNITS * 5 / 2);
+        return uneven ? TileShape{4, 16, 2} : whole_shape(4, tiles, tokens);
     }
-    if (split > 1) {
-        note_kernel("q4_tile_kernel<2,1,32,0,%d>", split);
-        if (split == 4) hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 0, 4>), dim3(4 * L.total_tiles), dim3(256), 0, stream, L);
-        else hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 0, 2>), dim3(2 * L.total_tiles), dim3(512), 0, stream, L);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
+    if (tokens == 1 && cols > SPLIT_MAX_COLS) return whole_shape(2, tiles, tokens);
+    const bool narrow = cols < 1024;
+    if (tiles <= COMPUTE_UNITS / 4) return {narrow ? 2 : 1, wide, 4};
+    if (tokens == 1 && tiles <= COMPUTE_UNITS * 3 / 8) return narrow ? TileShape{2, wide, 4} : TileShape{1, wide, 8};
+    if (tiles <= COMPUTE_UNITS / 2) return {2, wide, 2};
+    if (tiles <= COMPUTE_UNITS * 3 / 4) return {2, 16, 4};
+    return {2, 16, 2};
+}
+
+constexpr int shape_key(int chains, int blocks, int split) { return (chains * 64 + blocks) * 16 + split; }
+
+template <int S, int NB, int CB, int PRO, int SPLIT>
+int launch_as(const Q4Launch &L, int extra, hipStream_t stream) {
+    if (PRO == 0) {
+        if (SPLIT == 1) note_kernel("q4_tile_kernel<%d,%d,%d,0>", S, NB, CB);
+        else note_kernel("q4_tile_kernel<%d,%d,%d,0,%d>", S, NB, CB, SPLIT);
     }
-    // One token with few tiles: a workgroup has its compute unit to itself and stages twice as much per step.
-    if (L.tokens == 1 && S <= 4 && L.total_tiles <= WIDE_TILE_LIMIT) {
-        note_kernel("q4_tile_kernel<%d,1,32,0>", S);
-        hipLaunchKernelGGL((q4_tile_kernel<S, 1, 32>), grid, block, 0, stream, L);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    if (S == 4 && may_split && L.total_tiles > WIDE_TILE_LIMIT && L.total_tiles <= WIDE_TILE_LIMIT * 3 / 2) {
-        // Between one tile and one and a half per compute unit, some compute units have two and the rest wait for them:
-        // in halves they have three of them at most (264 tiles of 2816 columns, one to four tokens: 14.8 / 20.7 / 22.7 / 28.6
-        // us whole, 13.2 / 18.0 / 20.0 / 23.6 in halves; 400 tiles 15.0 whole and 15.6 in halves, three tokens 22.9 and
-        // 26.8).  Quarters with two chains per lane do not pay up to 320 tiles (one token 15.3 us, three 19.5).  Three waves a SIMD need 168 registers or fewer: without that
-        // bound three and four tokens took 26.9 and 32.2 us.
-        note_kernel("q4_tile_kernel<4,%d,16,0,2>", L.tokens);
-        const dim3 halves(2 * L.total_tiles);
-        switch (L.tokens) {
-            case 1: hipLaunchKernelGGL((q4_tile_kernel<4, 1, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
-            case 2: hipLaunchKernelGGL((q4_tile_kernel<4, 2, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
-            case 3: hipLaunchKernelGGL((q4_tile_kernel<4, 3, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
-            case 4: hipLaunchKernelGGL((q4_tile_kernel<4, 4, 16, 0, 2>), halves, dim3(256), 0, stream, L); break;
-            default: return -1;
-        }
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
-    note_kernel("q4_tile_kernel<%d,%d,16,0>", S, L.tokens);
-    switch (L.tokens) {
-        case 1: hipLaunchKernelGGL((q4_tile_kernel<S, 1, 16>), grid, block, 0, stream, L); break;
-        case 2: hipLaunchKernelGGL((q4_tile_kernel<S, 2, 16>), grid, block, 0, stream, L); break;
-        case 3: hipLaunchKernelGGL((q4_tile_kernel<S, 3, 16>), grid, block, 0, stream, L); break;
-        case 4: hipLaunchKernelGGL((q4_tile_kernel<S, 4, 16>), grid, block, 0, stream, L); break;
-        default: return -1;
-    }
+    hipLaunchKernelGGL((q4_tile_kernel<S, NB, CB, PRO, SPLIT>), dim3(SPLIT * L.total_tiles + extra), dim3(64 * 32 / (S * SPLIT)),
+                       0, stream, L);
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// One token.  `extra` workgroups follow those of the tiles.
+template <int PRO>
+int launch_one(const Q4Launch &L, const TileShape &shape, int extra, hipStream_t stream) {
+    switch (shape_key(shape.chains, shape.blocks, shape.split)) {
+        case shape_key(1, 32, 4): return launch_as<1, 1, 32, PRO, 4>(L, extra, stream);
+        case shape_key(1, 32, 8): return launch_as<1, 1, 32, PRO, 8>(L, extra, stream);
+        case shape_key(2, 32, 1): return launch_as<2, 1, 32, PRO, 1>(L, extra, stream);
+        case shape_key(2, 32, 2): return launch_as<2, 1, 32, PRO, 2>(L, extra, stream);
+        case shape_key(2, 32, 4): return launch_as<2, 1, 32, PRO, 4>(L, extra, stream);
+        case shape_key(2, 16, 2): return launch_as<2, 1, 16, PRO, 2>(L, extra, stream);
+        case shape_key(2, 16, 4): return launch_as<2, 1, 16, PRO, 4>(L, extra, stream);
+        case shape_key(4, 16, 1): return launch_as<4, 1, 16, PRO, 1>(L, extra, stream);
+        case shape_key(4, 16, 2): return launch_as<4, 1, 16, PRO, 2>(L, extra, stream);
+    }
+    if (PRO == 0) switch (shape_key(shape.chains, shape.blocks, shape.split)) {         // as the caller asked
+        case shape_key(2, 16, 1): return launch_as<2, 1, 16, 0, 1>(L, extra, stream);
+        case shape_key(4, 32, 1): return launch_as<4, 1, 32, 0, 1>(L, extra, stream);
+        case shape_key(8, 16, 1): return launch_as<8, 1, 16, 0, 1>(L, extra, stream);
+    }
+    return -1;
+}
+
+template <int NB>
+int launch_several(const Q4Launch &L, const TileShape &shape, hipStream_t stream) {
+    switch (shape_key(shape.chains, shape.blocks, shape.split)) {
+        case shape_key(1, 16, 4): return launch_as<1, NB, 16, 0, 4>(L, 0, stream);
+        case shape_key(2, 16, 1): return launch_as<2, NB, 16, 0, 1>(L, 0, stream);
+        case shape_key(2, 16, 2): return launch_as<2, NB, 16, 0, 2>(L, 0, stream);
+        case shape_key(2, 16, 4): return launch_as<2, NB, 16, 0, 4>(L, 0, stream);
+        case shape_key(4, 16, 1): return launch_as<4, NB, 16, 0, 1>(L, 0, stream);
+        case shape_key(4, 16, 2): return launch_as<4, NB, 16, 0, 2>(L, 0, stream);
+        case shape_key(8, 16, 1): return launch_as<8, NB, 16, 0, 1>(L, 0, stream);
+    }
+    return -1;
 }
 
 }  // namespace
@@ -735,6 +767,30 @@ int q4_uniform_tiles(const Q4Job *table, int njobs) {
     return first;
 }
 
+namespace {
+// Every wave of the MoE step's gate/up launch first finds its expert, so that more and shorter workgroups cost more than in
+// a plain launch.  us per decode step, whole / halves <2> / quarters <2> or halves <4>: 40 tiles of 2048 columns 17.2 / 14.1
+// (quarters <1> 14.0), 64 of 2048 16.9 / 14.1 (14.7), 64 of 2816 20.3 / 16.1 (15.1), 120 of 2816 21.2 / 17.2; 144 of 1600
+// 18.5 / 18.2 / quarters 18.9; 176 of 1024 17.0 / 16.7 / quarters 18.8, of 1536 17.5 / 17.2 / 16.5, of 2816 24.3 / 22.7 /
+// 21.4; 192 of 2816 (four quarters a compute unit, with the publisher) 23.5 / 21.9 / 23.4; 256 of 1024 21.1 / 18.8 / halves
+// <4> 16.3, of 2048 24.9 / 23.0 / 19.9, 208 of 2816 24.0 / 22.5 / 22.7.
+TileShape gate_up_shape(const MoeFuse &m, int tiles) {
+    TileShape shape = open_shape(tiles, m.hidden, 1);
+    if (shape.split > 1 && tiles <= COMPUTE_UNITS) {
+        if (tiles <= COMPUTE_UNITS / 2) {
+            if (shape.chains == 2 || shape.split == 8 || m.hidden <= 2048) shape = {2, 32, 2};
+        } else if (tiles <= COMPUTE_UNITS * 3 / 4) {
+            if (tiles <= COMPUTE_UNITS * 3 / 5 || 4 * tiles + 1 > 3 * COMPUTE_UNITS || m.hidden < 1280) shape = {2, 16, 2};
+        } else {
+            shape = {4, 16, 2};
+        }
+    }
+    if (shape.threads() >= m.n_experts) return shape;            // the router wants a thread per expert
+    if (tiles > COMPUTE_UNITS) return whole_shape(4, tiles, 1);
+    return {2, tiles <= COMPUTE_UNITS / 2 ? 32 : 16, 2};         // open_shape gave parts: the row fits in LDS
+}
+}  // namespace
+
 int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream) {
     Q4Launch L = launch;
     const MoeFuse &m = L.moe;
@@ -743,18 +799,31 @@ int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream) {
         return -1;
     L.table = nullptr; L.njobs = 1; L.cols = m.hidden; L.tokens = 1;
     L.total_tiles = 2 * m.topk * ((m.routed + TILE_ROWS - 1) / TILE_ROWS);
-    const dim3 grid(L.total_tiles + 1);                         // the extra workgroup publishes the router's outputs
-    // measured at 176 tiles (eight experts of 704 rows): 1024-column steps 29.4 us per decode step, 512-column steps 29.1,
-    // four chains per lane 30.4 and 33.4; the wide step is kept for launches that leave half the compute units idle
-    if (tile_split(L.total_tiles, L.cols) > 1)                  // two at most: the router needs a thread per expert
-        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 1, 2>), dim3(2 * L.total_tiles + 1), dim3(512), 0, stream, L);
-    else if (L.total_tiles <= WIDE_TILE_LIMIT / 2)
-        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 1>), grid, dim3(1024), 0, stream, L);
-    else if (L.total_tiles <= WIDE_TILE_LIMIT)
-        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 16, 1>), grid, dim3(1024), 0, stream, L);
-    else
-        hipLaunchKernelGGL((q4_tile_kernel<4, 1, 16, 1>), grid, dim3(512), 0, stream, L);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    // one more workgroup, the first, publishes the router's outputs
+    return launch_one<1>(L, gate_up_shape(m, L.total_tiles), 1, stream);
+}
+
+namespace {
+// Launches whose workgroups compute the activation row in a prologue repeat that work in every part.  us per MoE decode
+// step, down launch whole / in parts: 44 tiles of 704 columns 20.0 / quarters <1> 19.6, 64 of 1024 15.3 / 14.8 (halves 14.9);
+// 100 of 896 18.5 / halves 18.1, 128 of 1024 21.0 / 20.3; 150 of 896 18.6 / 18.8, 192 of 640 18.4 / 18.9; 352 of 704
+// 24.0 / halves <4> 25.0.
+TileShape activated_shape(int tiles) {
+    if (tiles > COMPUTE_UNITS / 2) return whole_shape(tiles <= COMPUTE_UNITS ? 2 : 4, tiles, 1);
+    return tiles <= COMPUTE_UNITS / 4 ? TileShape{1, 32, 4} : TileShape{2, 32, 2};
+}
+TileShape down_shape(const MoeFuse &m) {
+    const int tiles = m.topk * ((m.hidden + TILE_ROWS - 1) / TILE_ROWS);
+    const TileShape shape = activated_shape(tiles);
+    const bool counts_otherwise = m.arrivals && m.arrival_rows != TILE_ROWS / shape.split;
+    return counts_otherwise ? whole_shape(tiles <= COMPUTE_UNITS ? 2 : 4, tiles, 1) : shape;
+}
+}  // namespace
+
+int q4_moe_arrival_rows(int hidden, int routed, int topk) {
+    MoeFuse m = {};
+    m.hidden = hidden; m.routed = routed; m.topk = topk;
+    return TILE_ROWS / down_shape(m).split;
 }
 
 int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream) {
@@ -765,45 +834,24 @@ int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream) {
         return -1;
     L.table = nullptr; L.njobs = 1; L.cols = m.routed; L.tokens = 1;
     L.total_tiles = m.topk * ((m.hidden + TILE_ROWS - 1) / TILE_ROWS);
-    const dim3 grid(L.total_tiles);
-    // measured at 352 tiles (eight experts of 2816 rows): two chains per lane 31.4 us per decode step, four 29.4,
-    // eight 31.4, wide steps 32.7 and 34.5
-    if (L.total_tiles <= WIDE_TILE_LIMIT)
-        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 2>), grid, dim3(1024), 0, stream, L);
-    else
-        hipLaunchKernelGGL((q4_tile_kernel<4, 1, 16, 2>), grid, dim3(512), 0, stream, L);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return launch_one<2>(L, down_shape(m), 0, stream);
 }
 
 int q4_activated_launch(const Q4Launch &L, hipStream_t stream) {
     if (L.total_tiles < 1 || L.tokens != 1 || L.cols < 64 || (L.cols & 63) || L.cols > MOE_FUSE_MAX_ROUTED) return -1;
-    const dim3 grid(L.total_tiles);
-    const int split = tile_split(L.total_tiles, L.cols);
-    if (split == 4)
-        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 3, 4>), dim3(4 * L.total_tiles), dim3(256), 0, stream, L);
-    else if (split == 2)
-        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 3, 2>), dim3(2 * L.total_tiles), dim3(512), 0, stream, L);
-    else if (L.total_tiles <= WIDE_TILE_LIMIT)
-        hipLaunchKernelGGL((q4_tile_kernel<2, 1, 32, 3>), grid, dim3(1024), 0, stream, L);
-    else
-        hipLaunchKernelGGL((q4_tile_kernel<4, 1, 16, 3>), grid, dim3(512), 0, stream, L);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return launch_one<3>(L, activated_shape(L.total_tiles), 0, stream);
 }
 
 int q4_launch(const Q4Launch &L, int chains_per_lane, hipStream_t stream) {
     if (L.total_tiles < 1 || L.tokens < 1 || L.tokens > 4 || L.cols < 64 || (L.cols & 63)) return -1;
-    int S = chains_per_lane;
-    if (S == 0) {
-        // Up to one tile per compute unit, sixteen waves per tile (two chains per lane) hide more of the LDS and
-        // scalar-load latency; beyond that four chains per lane win (one token, 2816 columns: 12.4 against 15.5 us at
-        // 256 tiles, 20.7 against 15.2 at 320, 23.3 against 17.6 at 512; eight chains per lane never do).
-        S = L.total_tiles > WIDE_TILE_LIMIT ? 4 : 2;
-    }
-    switch (S) {
-        case 8: return launch_tiles<8>(L, chains_per_lane == 0, stream);
-        case 4: return launch_tiles<4>(L, chains_per_lane == 0, stream);
-        case 2: return launch_tiles<2>(L, chains_per_lane == 0, stream);
-        default: return -1;
+    if (chains_per_lane != 0 && chains_per_lane != 2 && chains_per_lane != 4 && chains_per_lane != 8) return -1;
+    const TileShape shape = chains_per_lane ? whole_shape(chains_per_lane, L.total_tiles, L.tokens)
+                                            : open_shape(L.total_tiles, L.cols, L.tokens);
+    switch (L.tokens) {
+        case 1: return launch_one<0>(L, shape, 0, stream);
+        case 2: return launch_several<2>(L, shape, stream);
+        case 3: return launch_several<3>(L, shape, stream);
+        default: return launch_several<4>(L, shape, stream);
     }
 }
 
