@@ -450,6 +450,17 @@ bool ffn_layer_ok(const SaltMi355FfnLayer *L) {
     return ((uintptr_t)L->pool & 3) == 0 && (L->expert_stride & 15) == 0 && L->expert_stride >= 3 * (n / 2 + 4 * (n / 64));
 }
 
+int ffn_combine(const SaltMi355FfnLayer &L, const float *residual, const FfnWorkspace &ws, const MoeWorkspace &moe,
+                const float *weights, int *status_dev, float *out, hipStream_t stream) {
+    if (combine_cell_launch(residual, ws.dense_out, ws.routed_out, L.post_norm_1, L.post_norm_2, L.post_norm, ws.sum, out,
+                            L.hidden, L.eps, L.layer_scalar, status_dev, moe.status, ws.expert_out, weights, L.topk,
+                            stream) != 0) {
+        set_error("ffn block: combine launch failed");
+        return -1;
+    }
+    return 0;
+}
+
 }  // namespace
 
 size_t salt_mi355_ffn_block_workspace_bytes(const SaltMi355FfnLayer *layer) {
@@ -495,7 +506,35 @@ int salt_mi355_ffn_block_dev(const SaltMi355FfnLayer *layer, const float *residu
         set_error("ffn block: pre-norm launch failed");
         return -1;
     }
-    // The dense branch runs beside the routed one on the library's second stream.
+    Q8Launch gate;
+    gate.vals = (const uint8_t *)L.router[0]; gate.scales = (const uint8_t *)L.router[1]; gate.biases = (const uint8_t *)L.router[2];
+    gate.x = ws.router_in; gate.y = ws.logits;
+    gate.rows = L.n_experts; gate.cols = L.hidden; gate.tokens = 1;
+    gate.x_stride = L.hidden; gate.y_stride = L.n_experts;
+    Q4Launch down;
+    memset(&down, 0, sizeof down);
+    down.one.vals = (const uint8_t *)L.dense_down[0]; down.one.scales = (const uint8_t *)L.dense_down[1];
+    down.one.biases = (const uint8_t *)L.dense_down[2];
+    down.one.x = ws.gate; down.one.y = ws.dense_out;
+    down.one.rows = L.hidden; down.one.x_stride = L.dense; down.one.y_stride = L.hidden;
+    down.act_delta = ws.up - ws.gate;
+    down.njobs = 1; down.cols = L.dense; down.tokens = 1; down.code_scale = g_state.code_scale;
+    down.total_tiles = (L.hidden + 63) / 64;
+    if (tileable && q4_job_is_tileable(down.one, L.dense) &&
+        q4_ffn_serves({L.hidden, L.dense, L.routed, L.n_experts, L.topk}, gate)) {
+        // Both branches in the same launches, on the caller's stream alone.  A rejected residual leaves their inputs
+        // unwritten: the router then works on whatever they held, which it either rejects or routes harmlessly, and the
+        // combine publishes nothing in both cases.
+        if (q4_ffn_gate_launch(gate_up, gate, stream) != 0 ||
+            moe_decode_experts_launch(g, (const uint8_t *)L.pool, L.expert_stride, ws.logits, L.per_expert_scale, ws.norm_b,
+                                      selected, weights, ws.expert_out, moe, g_state.code_scale, &down, stream) != 0) {
+            set_error("ffn block: branches failed to launch");
+            return -1;
+        }
+        return ffn_combine(L, residual, ws, moe, weights, status_dev, out, stream);
+    }
+
+    // Else the dense branch runs beside the routed one on the library's second stream.
     hipStream_t side = g_state.side;
     if (hip_ok(hipEventRecord(g_state.fork, stream), "ffn block fork") != 0 ||
         hip_ok(hipStreamWaitEvent(side, g_state.fork, 0), "ffn block fork wait") != 0)
@@ -528,13 +567,7 @@ int salt_mi355_ffn_block_dev(const SaltMi355FfnLayer *layer, const float *residu
         return -1;
     }
     if (hip_ok(hipStreamWaitEvent(stream, g_state.join, 0), "ffn block join wait") != 0) return -1;
-    if (combine_cell_launch(residual, ws.dense_out, ws.routed_out, L.post_norm_1, L.post_norm_2, L.post_norm, ws.sum, out,
-                            L.hidden, L.eps, L.layer_scalar, status_dev, moe.status, ws.expert_out, weights, L.topk,
-                            stream) != 0) {
-        set_error("ffn block: combine launch failed");
-        return -1;
-    }
-    return 0;
+    return ffn_combine(L, residual, ws, moe, weights, status_dev, out, stream);
 }
 
 int salt_mi355_router_topk_dev(const float *logits, const float *per_expert_scale, int n_experts, int topk,

@@ -286,6 +286,14 @@ struct Q8Launch {
 };
 int q8_launch(const Q8Launch &launch, hipStream_t stream);
 
+// The two launches of a feed-forward block that carry the routed branch and the dense one side by side: the router's gate
+// beside the dense gate and up (two jobs in dense.inline_jobs), the routed down projections (as q4_moe_down_launch) beside
+// the dense one (one job, as for q4_activated_launch).  q4_ffn_serves: both take these shapes.
+struct FfnShape { int hidden, dense, routed, n_experts, topk; };
+bool q4_ffn_serves(const FfnShape &shape, const Q8Launch &gate);
+int q4_ffn_gate_launch(const Q4Launch &dense, const Q8Launch &gate, hipStream_t stream);
+int q4_ffn_down_launch(const Q4Launch &moe, const Q4Launch &dense, hipStream_t stream);
+
 // ---------------------------------------------------------------- fp32 cells of a decoder block
 
 // Each launcher enqueues kernels that do nothing when *status != 0 and set it to -1 (publishing nothing) when an
@@ -336,6 +344,12 @@ int moe_decode_step_launch(const MoeGeometry &g, const uint8_t *pool, size_t exp
                            const float *logits, const float *per_expert_scale, const float *x,
                            int *selected, float *weights, float *expert_out, float *out,
                            const MoeWorkspace &ws, float code_scale, hipStream_t stream);
+// The same without the reduction, with another branch's down projection beside the experts' (q4_ffn_down_launch), for
+// geometries that q4_ffn_serves takes.
+int moe_decode_experts_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_stride, const float *logits,
+                              const float *per_expert_scale, const float *x, int *selected, float *weights,
+                              float *expert_out, const MoeWorkspace &ws, float code_scale, const Q4Launch *beside,
+                              hipStream_t stream);
 
 // tolerance class (q4_dot.hip); -1 when the geometry is not served (more than 256 experts, widths the streaming
 // kernel does not take)

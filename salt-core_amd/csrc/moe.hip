@@ -150,6 +150,30 @@ int moe_reduce_launch(const float *expert_out, const float *weights, int topk, i
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+namespace {
+Q4Launch moe_fused(const MoeGeometry &g, const uint8_t *pool, size_t expert_stride, const float *logits,
+                   const float *per_expert_scale, const float *x, int *selected, float *weights, float *expert_out,
+                   const MoeWorkspace &ws, float code_scale) {
+    Q4Launch fused;
+    memset(&fused, 0, sizeof fused);
+    fused.code_scale = code_scale;
+    MoeFuse &m = fused.moe;
+    m.logits = logits; m.per_expert_scale = per_expert_scale; m.pool = pool; m.expert_stride = expert_stride;
+    m.x = x; m.gate = ws.gate; m.up = ws.up; m.expert_out = expert_out; m.selected = selected; m.weights = weights;
+    m.status = ws.status; m.n_experts = g.n_experts; m.topk = g.topk; m.hidden = g.hidden; m.routed = g.routed;
+    return fused;
+}
+}  // namespace
+
+int moe_decode_experts_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_stride, const float *logits,
+                              const float *per_expert_scale, const float *x, int *selected, float *weights,
+                              float *expert_out, const MoeWorkspace &ws, float code_scale, const Q4Launch *beside,
+                              hipStream_t stream) {
+    const Q4Launch fused = moe_fused(g, pool, expert_stride, logits, per_expert_scale, x, selected, weights, expert_out, ws, code_scale);
+    if (q4_moe_gate_up_launch(fused, stream) != 0) return -1;
+    return q4_ffn_down_launch(fused, *beside, stream);
+}
+
 int moe_decode_step_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_stride, const float *logits,
                            const float *per_expert_scale, const float *x, int *selected, float *weights,
                            float *expert_out, float *out, const MoeWorkspace &ws, float code_scale,
@@ -161,13 +185,8 @@ int moe_decode_step_launch(const MoeGeometry &g, const uint8_t *pool, size_t exp
     if (g.n_experts <= MOE_FUSE_MAX_EXPERTS && g.routed <= MOE_FUSE_MAX_ROUTED) {
         // Two launches: router + gate/up, then activation + down + the ordered reduction (by the last workgroup
         // to finish each tile of the output).
-        Q4Launch fused;
-        memset(&fused, 0, sizeof fused);
-        fused.code_scale = code_scale;
+        Q4Launch fused = moe_fused(g, pool, expert_stride, logits, per_expert_scale, x, selected, weights, eo, ws, code_scale);
         MoeFuse &m = fused.moe;
-        m.logits = logits; m.per_expert_scale = per_expert_scale; m.pool = pool; m.expert_stride = expert_stride;
-        m.x = x; m.gate = ws.gate; m.up = ws.up; m.expert_out = eo; m.selected = selected; m.weights = weights;
-        m.status = ws.status; m.n_experts = g.n_experts; m.topk = g.topk; m.hidden = g.hidden; m.routed = g.routed;
         m.out = out;
         if (out) {
             // counters of parts of a tile lie where this plan keeps nothing else, or the down launch runs whole tiles

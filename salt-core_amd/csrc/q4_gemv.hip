@@ -26,6 +26,7 @@
 //  * The per-row fold runs in the documented order from LDS.
 #include "device_math.h"
 #include "mi355_internal.h"
+#include "q8_chain.h"
 #include "router_device.h"
 
 #include <stddef.h>
@@ -171,37 +172,58 @@ constexpr int x_batch_groups(int S, int NB) {
 // activations come from LDS as in the prologues above.  One chain per lane (S = 1) leaves a wave with fewer than half of
 // the instructions of two and doubles the waves: a lone wave issues one every eight clocks, two on a SIMD fill it.
 // One token, 2816 x 2816 (44 tiles): 10.8 us whole, 6.9 in quarters with two chains per lane, 5.9 with one.
-template <int S, int NB, int CB, int PRO = 0, int SPLIT = 1>
-__global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 1) void q4_tile_kernel(const Q4Launch L) {
-    constexpr int CHUNK_BLOCKS = CB;
-    constexpr int ROWS = TILE_ROWS / SPLIT;
-    constexpr bool LDS_X = PRO >= 2 || SPLIT > 1;
+template <int S, int NB, int CB, int PRO, int SPLIT>
+struct TileKernel {
+    static constexpr int CHUNK_BLOCKS = CB;
+    static constexpr int ROWS = TILE_ROWS / SPLIT;
+    static constexpr bool LDS_X = PRO >= 2 || SPLIT > 1;
     // activations staged with each step's weights, not the whole row (a prologue that computes them computes the whole row)
-    constexpr bool STEP_X = PRO < 2 && SPLIT > 1 && (S == 4 || NB > 1);
-    constexpr int CHUNK_GROUPS = CB / 2;                   // 64-column scale groups per step
-    constexpr int W_PITCH = 16 * CB + 4;                   // bytes per staged row: odd dword pitch
-    constexpr int M_PITCH = 2 * CHUNK_GROUPS + 2;          // floats per staged row of (scale, bias)
-    constexpr int W_STAGE = ROWS * W_PITCH;
-    constexpr int M_STAGE = ROWS * M_PITCH;
-    constexpr int WAVES = 32 / (S * SPLIT);
-    constexpr int THREADS = WAVES * 64;
+    static constexpr bool STEP_X = PRO < 2 && SPLIT > 1 && (S == 4 || NB > 1);
+    static constexpr int CHUNK_GROUPS = CB / 2;                   // 64-column scale groups per step
+    static constexpr int W_PITCH = 16 * CB + 4;                   // bytes per staged row: odd dword pitch
+    static constexpr int M_PITCH = 2 * CHUNK_GROUPS + 2;          // floats per staged row of (scale, bias)
+    static constexpr int W_STAGE = ROWS * W_PITCH;
+    static constexpr int M_STAGE = ROWS * M_PITCH;
+    static constexpr int WAVES = 32 / (S * SPLIT);
+    static constexpr int THREADS = WAVES * 64;
     // A staging item is one scale group of one row: 32 bytes of codes (two blocks) and its (scale, bias).
-    constexpr int ITEMS = (ROWS * CHUNK_GROUPS + THREADS - 1) / THREADS;
-    constexpr int FOLD_BYTES = NB * ROWS * FOLD_PITCH * 4;
-    constexpr int W_BYTES = 2 * W_STAGE > FOLD_BYTES ? 2 * W_STAGE : FOLD_BYTES;
-    constexpr int XG = STEP_X && NB >= 3 ? 1 : LDS_X ? 2 : x_batch_groups(S, NB);        // LDS-fed activations sit in vector registers: short batches
-    constexpr int XN = XG * 2 * S;
+    static constexpr int ITEMS = (ROWS * CHUNK_GROUPS + THREADS - 1) / THREADS;
+    static constexpr int FOLD_BYTES = NB * ROWS * FOLD_PITCH * 4;
+    static constexpr int W_BYTES = 2 * W_STAGE > FOLD_BYTES ? 2 * W_STAGE : FOLD_BYTES;
+    static constexpr int XG = STEP_X && NB >= 3 ? 1 : LDS_X ? 2 : x_batch_groups(S, NB); // LDS-fed activations sit in vector registers: short batches
+    static constexpr int XN = XG * 2 * S;
+    static constexpr int X_FLOATS = PRO >= 2 ? MOE_FUSE_MAX_ROUTED : STEP_X ? 2 * NB * CB * 32 : SPLIT > 1 ? SPLIT_MAX_COLS : 4;
+    static constexpr int MIN_WAVES = SPLIT > 1 && S == 4 ? 3 : 1;
     static_assert(THREADS >= NB * ROWS, "fold needs one thread per (token, row)");
     static_assert(SPLIT == 1 || NB == 1 || STEP_X, "LDS holds one whole row");
-
-    __shared__ __attribute__((aligned(16))) uint8_t w_lds[W_BYTES];
-    __shared__ __attribute__((aligned(16))) float m_lds[2 * M_STAGE];
-    __shared__ __attribute__((aligned(16))) float x_lds[PRO >= 2 ? MOE_FUSE_MAX_ROUTED : STEP_X ? 2 * NB * CB * 32 : SPLIT > 1 ? SPLIT_MAX_COLS : 4];
-    __shared__ int slow_flag;
     static_assert(PRO == 0 || NB == 1, "the MoE prologues serve the single-token kernel");
-    // the router prologue borrows memory that is used later, and one thread per expert (q4_moe_gate_up_launch sees to that)
-    static_assert(PRO != 1 || sizeof(RouterShared) <= (SPLIT > 1 && !STEP_X ? sizeof x_lds : W_BYTES), "the router fits");
 
+    struct Lds {
+        __attribute__((aligned(16))) uint8_t w[W_BYTES];
+        __attribute__((aligned(16))) float m[2 * M_STAGE];
+        __attribute__((aligned(16))) float x[X_FLOATS];
+        int slow;
+    };
+    // the router prologue borrows memory that is used later, and one thread per expert (q4_moe_gate_up_launch sees to that)
+    static_assert(PRO != 1 || sizeof(RouterShared) <= (SPLIT > 1 && !STEP_X ? sizeof(Lds::x) : sizeof(Lds::w)), "the router fits");
+
+    // `block` numbers the launch's workgroups from 0
+    static __device__ __forceinline__ void run(const Q4Launch &L, int block, Lds &lds);
+};
+
+template <int S, int NB, int CB, int PRO = 0, int SPLIT = 1>
+__global__ __launch_bounds__((TileKernel<S, NB, CB, PRO, SPLIT>::THREADS), (TileKernel<S, NB, CB, PRO, SPLIT>::MIN_WAVES))
+void q4_tile_kernel(const Q4Launch L) {
+    __shared__ typename TileKernel<S, NB, CB, PRO, SPLIT>::Lds lds;
+    TileKernel<S, NB, CB, PRO, SPLIT>::run(L, (int)blockIdx.x, lds);
+}
+
+template <int S, int NB, int CB, int PRO, int SPLIT>
+__device__ __forceinline__ void TileKernel<S, NB, CB, PRO, SPLIT>::run(const Q4Launch &L, const int block, Lds &lds) {
+    auto &w_lds = lds.w;
+    auto &m_lds = lds.m;
+    auto &x_lds = lds.x;
+    int &slow_flag = lds.slow;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -209,7 +231,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
     // lane's row of the tile and its slice of the chains
     const int lane_row = lane & (ROWS - 1);
     const int slice = SPLIT == 1 ? wave : wave * SPLIT + lane / ROWS;
-    const int part = (int)blockIdx.x - (PRO == 1 ? 1 : 0);      // workgroup 0 of the MoE gate/up launch is the router's publisher
+    const int part = block - (PRO == 1 ? 1 : 0);      // workgroup 0 of the MoE gate/up launch is the router's publisher
     const int tile = SPLIT == 1 ? part : part / SPLIT;
 
     Q4Job job;
@@ -226,7 +248,7 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
         const size_t vals_bytes = n / 2, meta_bytes = (n / 64) * 2, proj_bytes = vals_bytes + 2 * meta_bytes;
         if (PRO == 1) {
             RouterShared &sh = *reinterpret_cast<RouterShared *>(SPLIT > 1 && !STEP_X ? (uint8_t *)x_lds : w_lds);
-            const bool publisher = blockIdx.x == 0;
+            const bool publisher = block == 0;
             const int up_tiles = (m.routed + TILE_ROWS - 1) / TILE_ROWS;
             const int slot_index = tile / up_tiles;                        // 2 * place + (0 gate | 1 up); of tiles
             const int place = slot_index >> 1, proj = slot_index & 1;
@@ -416,12 +438,17 @@ __global__ __launch_bounds__((32 / (S * SPLIT)) * 64, SPLIT > 1 && S == 4 ? 3 : 
     // x of `groups` consecutive scale groups starting at group g0 of the row
     auto load_x = [&](int g0, float (&xq)[NB][XN], int groups) {
         if (LDS_X) {                      // every lane of a slice reads the same LDS words: the activations travel in vector registers
+            typedef float f32xS __attribute__((ext_vector_type(S)));        // a slice's activations of one block, one LDS read
             const float *xl = x_step + g0 * 64 + S * slice;
 #pragma unroll
             for (int t = 0; t < NB; ++t)
 #pragma unroll
-                for (int k = 0; k < XN; ++k)
-                    if (k < groups * 2 * S) xq[t][k] = xl[t * X_STEP + (k / S) * 32 + (k % S)];
+                for (int b = 0; b < XN / S; ++b)
+                    if (b < groups * 2) {
+                        const f32xS v = *reinterpret_cast<const f32xS *>(xl + t * X_STEP + b * 32);
+#pragma unroll
+                        for (int k = 0; k < S; ++k) xq[t][b * S + k] = v[k];
+                    }
             return;
         }
         const uniform_f32_ptr xg = xbase + (size_t)g0 * 64;
@@ -791,16 +818,23 @@ TileShape gate_up_shape(const MoeFuse &m, int tiles) {
 }
 }  // namespace
 
-int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream) {
-    Q4Launch L = launch;
+namespace {
+bool prepare_gate_up(Q4Launch &L) {
     const MoeFuse &m = L.moe;
     if (m.n_experts < 1 || m.n_experts > MOE_FUSE_MAX_EXPERTS || m.topk < 1 || m.topk > m.n_experts ||
         m.topk > ROUTER_MAX_TOPK || m.hidden < 64 || (m.hidden & 63) || m.routed < 64 || (m.routed & 63))
-        return -1;
+        return false;
     L.table = nullptr; L.njobs = 1; L.cols = m.hidden; L.tokens = 1;
     L.total_tiles = 2 * m.topk * ((m.routed + TILE_ROWS - 1) / TILE_ROWS);
+    return true;
+}
+}  // namespace
+
+int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream) {
+    Q4Launch L = launch;
+    if (!prepare_gate_up(L)) return -1;
     // one more workgroup, the first, publishes the router's outputs
-    return launch_one<1>(L, gate_up_shape(m, L.total_tiles), 1, stream);
+    return launch_one<1>(L, gate_up_shape(L.moe, L.total_tiles), 1, stream);
 }
 
 namespace {
@@ -826,20 +860,104 @@ int q4_moe_arrival_rows(int hidden, int routed, int topk) {
     return TILE_ROWS / down_shape(m).split;
 }
 
-int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream) {
-    Q4Launch L = launch;
+namespace {
+bool prepare_down(Q4Launch &L) {
     const MoeFuse &m = L.moe;
     if (m.topk < 1 || m.hidden < 64 || (m.hidden & 63) || m.routed < 64 || (m.routed & 63) ||
         m.routed > MOE_FUSE_MAX_ROUTED || (m.out == nullptr) != (m.arrivals == nullptr))
-        return -1;
+        return false;
     L.table = nullptr; L.njobs = 1; L.cols = m.routed; L.tokens = 1;
     L.total_tiles = m.topk * ((m.hidden + TILE_ROWS - 1) / TILE_ROWS);
-    return launch_one<2>(L, down_shape(m), 0, stream);
+    return true;
+}
+}  // namespace
+
+int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream) {
+    Q4Launch L = launch;
+    if (!prepare_down(L)) return -1;
+    return launch_one<2>(L, down_shape(L.moe), 0, stream);
 }
 
 int q4_activated_launch(const Q4Launch &L, hipStream_t stream) {
     if (L.total_tiles < 1 || L.tokens != 1 || L.cols < 64 || (L.cols & 63) || L.cols > MOE_FUSE_MAX_ROUTED) return -1;
     return launch_one<3>(L, activated_shape(L.total_tiles), 0, stream);
+}
+
+// ---------------------------------------------------------------- a feed-forward block's branches side by side
+// The dense branch beside the routed one in the same launches, where it used to run on a second stream: that took three
+// launches and four event calls more, and enqueuing them was what bounded a block (57 us at 16 experts, top-1, 1024/512 with
+// a dense branch of 1024, now 34).  The down projections go together because the routed gate/up launch fills the chip by
+// itself (2816/2112/704, 128 experts, top-8: dense down beside gate/up 61.4 us a block, beside the routed down 57.5, on a
+// second stream 65.5).
+namespace {
+
+using DenseGateUp = TileKernel<4, 1, 16, 0, 2>;     // the gate's chain takes twice as long: any shape of 256 threads serves
+
+union FfnGateLds {
+    Q8ChainLds gate;
+    DenseGateUp::Lds dense;
+};
+// the launch record comes first: a job's record is read from the kernel arguments (find_job)
+__global__ __launch_bounds__(256) void ffn_gate_kernel(const Q4Launch dense, const Q8Launch gate, const int gate_blocks) {
+    __shared__ FfnGateLds lds;
+    if ((int)blockIdx.x < gate_blocks) q8_chain(gate, (int)blockIdx.x, 0, lds.gate);
+    else DenseGateUp::run(dense, (int)blockIdx.x - gate_blocks, lds.dense);
+}
+
+// Dense down projection in workgroups of THREADS threads, numbered before the routed ones, whose rows are shorter.
+template <int THREADS> struct DenseDown;
+template <> struct DenseDown<512> { using Kernel = TileKernel<2, 1, 32, 3, 2>; static constexpr int SPLIT = 2; };
+template <> struct DenseDown<1024> { using Kernel = TileKernel<2, 1, 32, 3, 1>; static constexpr int SPLIT = 1; };
+
+template <int S, int CB, int SPLIT>
+__global__ __launch_bounds__((TileKernel<S, 1, CB, 2, SPLIT>::THREADS))
+void ffn_down_kernel(const Q4Launch moe, const Q4Launch dense, const int dense_blocks) {
+    using Routed = TileKernel<S, 1, CB, 2, SPLIT>;
+    using Dense = typename DenseDown<Routed::THREADS>::Kernel;
+    __shared__ union Lds { typename Routed::Lds routed; typename Dense::Lds dense; } lds;
+    if ((int)blockIdx.x < dense_blocks) Dense::run(dense, (int)blockIdx.x, lds.dense);
+    else Routed::run(moe, (int)blockIdx.x - dense_blocks, lds.routed);
+}
+
+template <int S, int CB, int SPLIT>
+int launch_downs(const Q4Launch &moe, const Q4Launch &dense, hipStream_t stream) {
+    constexpr int THREADS = TileKernel<S, 1, CB, 2, SPLIT>::THREADS;
+    const int dense_blocks = DenseDown<THREADS>::SPLIT * dense.total_tiles;
+    hipLaunchKernelGGL((ffn_down_kernel<S, CB, SPLIT>), dim3(dense_blocks + SPLIT * moe.total_tiles), dim3(THREADS), 0, stream, moe,
+                       dense, dense_blocks);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+}  // namespace
+
+bool q4_ffn_serves(const FfnShape &f, const Q8Launch &gate) {
+    // (a chain's width, 4096, also lets every shape of gate_up_shape but the whole tiles of wider rows through)
+    return q8_chain_takes(gate) && f.dense <= MOE_FUSE_MAX_ROUTED && f.routed <= MOE_FUSE_MAX_ROUTED &&
+           f.n_experts <= MOE_FUSE_MAX_EXPERTS && f.topk <= ROUTER_MAX_TOPK;
+}
+
+int q4_ffn_gate_launch(const Q4Launch &dense, const Q8Launch &gate, hipStream_t stream) {
+    if (dense.total_tiles < 1 || dense.tokens != 1 || dense.table || dense.cols < 64 || (dense.cols & 63) || gate.rows < 1 ||
+        gate.tokens != 1 || !q8_chain_takes(gate))
+        return -1;
+    const int gate_blocks = (gate.rows + CH_ROWS - 1) / CH_ROWS;
+    hipLaunchKernelGGL(ffn_gate_kernel, dim3(gate_blocks + 2 * dense.total_tiles), dim3(256), 0, stream, dense, gate, gate_blocks);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int q4_ffn_down_launch(const Q4Launch &launch, const Q4Launch &dense, hipStream_t stream) {
+    Q4Launch moe = launch;
+    if (!prepare_down(moe) || dense.total_tiles < 1 || dense.tokens != 1 || dense.cols < 64 || (dense.cols & 63) ||
+        dense.cols > MOE_FUSE_MAX_ROUTED)
+        return -1;
+    const TileShape shape = down_shape(moe.moe);
+    switch (shape_key(shape.chains, shape.blocks, shape.split)) {
+        case shape_key(1, 32, 4): return launch_downs<1, 32, 4>(moe, dense, stream);
+        case shape_key(2, 32, 2): return launch_downs<2, 32, 2>(moe, dense, stream);
+        case shape_key(2, 32, 1): return launch_downs<2, 32, 1>(moe, dense, stream);
+        case shape_key(4, 16, 1): return launch_downs<4, 16, 1>(moe, dense, stream);
+    }
+    return -1;
 }
 
 int q4_launch(const Q4Launch &L, int chains_per_lane, hipStream_t stream) {
