@@ -56,17 +56,22 @@
 //
 // Bound: the matrix cores, which execute twice the useful operations, at the
 // clock that their power leaves them: 44 % busy at 1.6 to 2.1 GHz in the grouped
-// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 602 us a layer);
-// one 16384 x 2816 matrix, 333 tokens: 101 -> 82 us, 384 tiles on 256 compute
+// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 590 us a layer);
+// one 16384 x 2816 matrix, 333 tokens: 101 -> 78 us, 384 tiles on 256 compute
 // units.  Before, every scale group cost 16 multiply-adds per block and a
 // conversion in each of two waves, and each 32 bytes of codes and each scale
-// fetched a cache line of its own.
+// fetched a cache line of its own.  Calls of few tiles are bound by one wave per
+// SIMD that issues an instruction every eight clocks: 33 tokens, 8192 x 2816
+// 39.5 -> 34.1 us and 8192 x 8192 98.7 -> 84.9, 64 tokens, 4096 x 4096 54.3 ->
+// 46.2 once nothing in the walk waits but what has to (lds_load.h).  Four
+// stages of planes instead of two gained nothing there.
 //
 // Inside every aligned run of eight columns the planes are stored in the order
 // 0,4,1,5,2,6,3,7, which is the order the pair extraction yields the codes in;
 // the two lane halves of an instruction take columns 32 h + 8 k .. + 7 of a
 // scale group, so that a lane's codes of a group are 16 consecutive bytes.
 #include "device_math.h"
+#include "lds_load.h"
 #include "mi355_internal.h"
 
 #include <stddef.h>
@@ -87,8 +92,6 @@ typedef const u32x4 __attribute__((address_space(1))) *global_u128_ptr;
 typedef const u32x4_any __attribute__((address_space(1))) *global_u128_any_ptr;
 typedef const uint16_t __attribute__((address_space(1))) *global_u16_ptr;
 typedef const uint8_t __attribute__((address_space(1))) *global_u8_ptr;
-typedef const void __attribute__((address_space(1))) *global_void_ptr;
-typedef void __attribute__((address_space(3))) *lds_void_ptr;
 typedef const int __attribute__((address_space(1))) *global_i32_ptr;
 typedef float __attribute__((address_space(1))) *global_f32_out;
 
@@ -99,11 +102,13 @@ constexpr int MAX_WINDOWS = 10;             // all of a bf16's binades
 constexpr int WEIGHT_TOP = 11;              // scales are brought below 2^WEIGHT_TOP: 24 * 2^11 is inside fp16
 
 // A row of the third plane holds what the split has to say about its row of x: at byte 0 the exponent k of the power
-// of two 2^-k that undoes its scaling, from byte 16 on the group sums as three bf16 planes of padded_groups() entries.
+// of two 2^-k that undoes its scaling, from byte 16 on the group sums in blocks of sixteen groups, a block as three bf16
+// planes of sixteen entries (96 bytes).
 // The bias pass reads scales, biases and sums eight groups at a time, the last eight of a row from its end backwards,
 // so that it never reads past the row: entry j of eight c stands for group eight_start(c) + j, and is zero where an
 // earlier eight already holds that group.  16 + 6 * padded_groups(C / 64) bytes fit the 2 * C of the row for every C.
 __host__ __device__ constexpr int padded_groups(int ngrp) { return (ngrp + 15) & ~15; }
+__device__ __forceinline__ int sum_entry(int at, int plane) { return 8 + (at >> 4) * 48 + plane * 16 + (at & 15); }   // in halves
 __device__ __forceinline__ int eight_start(int c, int ngrp) {
     const int last = ngrp > 8 ? ngrp - 8 : 0;
     return 8 * c < last ? 8 * c : last;
@@ -117,7 +122,12 @@ constexpr int CH = 4;
 constexpr int STAGE_BYTES = X_PLANES * TM * 128;
 constexpr int W_OFF = 2 * STAGE_BYTES, W_BYTES = 64 * 32 * CH;           // of one wave
 constexpr int S_OFF = W_OFF + ROW_WAVES * W_BYTES, S_BYTES = 64 * 4 * CH;
-constexpr int LDS_BYTES = S_OFF + ROW_WAVES * S_BYTES;
+// Blocks of group sums of all tokens for the bias pass: three at a time, two of them where the second stage of planes comes
+// later and one of its own.
+constexpr int SUM_BYTES = TM * 96, SUM_OFF = S_OFF + ROW_WAVES * S_BYTES, SUM_BLOCKS = 3;
+constexpr int LDS_BYTES = SUM_OFF + SUM_BYTES;
+static_assert(2 * SUM_BYTES <= STAGE_BYTES && 2 * (LDS_BYTES + 2048) <= 160 * 1024, "two workgroups per compute unit");
+__device__ __forceinline__ int sum_place(int block) { return block < 2 ? STAGE_BYTES + block * SUM_BYTES : SUM_OFF; }
 constexpr int XT = TM / (8 * ROW_WAVES);         // loads per wave and plane: eight token rows each
 constexpr int PIECES = 2 * CH;                   // 16-byte pieces of a row's chunk
 constexpr int WT = PIECES;                       // loads per wave and chunk: 64 / PIECES rows each
@@ -250,7 +260,7 @@ void q4_mfma_kernel(const MfmaLaunch L) {
         s_row[tid] = L.row_map ? (uint32_t)(L.row_map[job.row_base + tok0 + tc] / L.map_divisor) : (uint32_t)(tok0 + tc);
     }
     __syncthreads();
-    const global_u8_ptr plane0 = (global_u8_ptr)(uintptr_t)job.planes;
+    const global_u8_ptr plane0 = uniform_address((global_u8_ptr)(uintptr_t)job.planes);
     const global_u8_ptr plane1 = plane0 + 2 * L.plane_stride, notes = plane0 + 4 * L.plane_stride;
 
     // Staging geometry of this lane: load i of a wave brings the eight token rows from (i * ROW_WAVES + wave) * 8 on;
@@ -275,8 +285,8 @@ void q4_mfma_kernel(const MfmaLaunch L) {
     // codes of the wave's rows: load j of a chunk brings rows j * 64 / PIECES .., clamped to the matrix
     const int rows_left = live ? job.rows - row0 : 1;
     const int row_base = live ? row0 : 0;           // waves without rows fetch the first row and use nothing
-    const global_u8_ptr codes = (global_u8_ptr)(uintptr_t)job.vals + (size_t)row_base * (size_t)(C >> 1);
-    const global_u8_ptr scale_rows = (global_u8_ptr)(uintptr_t)job.scales + (size_t)row_base * (size_t)(2 * ngrp);
+    const global_u8_ptr codes = uniform_address((global_u8_ptr)(uintptr_t)job.vals + (size_t)row_base * (size_t)(C >> 1));
+    const global_u8_ptr scale_rows = uniform_address((global_u8_ptr)(uintptr_t)job.scales + (size_t)row_base * (size_t)(2 * ngrp));
 
     // Everything staged goes from memory into LDS without passing through registers, so that a wave's loads complete
     // in the order they were sent in and a wait can leave the younger ones in flight (meet(), not __syncthreads, which
@@ -289,9 +299,8 @@ void q4_mfma_kernel(const MfmaLaunch L) {
         for (int i = 0; i < XT; ++i) {
             if (i * ROW_WAVES * 8 >= 32 && !wide) break;
             uint8_t *const to = x + i * (ROW_WAVES * 1024);
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(plane0 + (x_src[i] + at)), (lds_void_ptr)to, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(plane1 + (x_src[i] + at)), (lds_void_ptr)(to + TM * 128),
-                                             16, 0, 0);
+            load_to_lds<16>(plane0, x_src[i] + at, to);
+            load_to_lds<16>(plane1, x_src[i] + at, to + TM * 128);
         }
     };
     constexpr int CHUNK_LOADS = WT + CH;
@@ -307,14 +316,12 @@ void q4_mfma_kernel(const MfmaLaunch L) {
             uint32_t byte = at + piece * 16u;
             byte = byte < last ? byte : last;
             r = r < (uint32_t)rows_left ? r : (uint32_t)rows_left - 1u;
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(codes + (__umul24(r, (uint32_t)(C >> 1)) + byte)),
-                                             (lds_void_ptr)(stage + W_OFF + wave * W_BYTES + j * 1024), 16, 0, 0);
+            load_to_lds<16>(codes, __umul24(r, (uint32_t)(C >> 1)) + byte, stage + W_OFF + wave * W_BYTES + j * 1024);
         }
 #pragma unroll
         for (int gi = 0; gi < CH; ++gi) {
             const int g = it + gi;
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(scale_rows + (scale_at + 2u * (uint32_t)(g < ngrp ? g : ngrp - 1))),
-                                             (lds_void_ptr)(stage + S_OFF + wave * S_BYTES + gi * 256), 2, 0, 0);
+            load_to_lds<2>(scale_rows, scale_at + 2u * (uint32_t)(g < ngrp ? g : ngrp - 1), stage + S_OFF + wave * S_BYTES + gi * 256);
         }
     };
     typedef const u32x4 __attribute__((address_space(3))) *lds_u128_ptr;
@@ -334,51 +341,85 @@ void q4_mfma_kernel(const MfmaLaunch L) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
 
+    // What the bias pass needs is sent for before the first planes and codes, whose arrival nobody has to wait for there.
+    // The group sums go to LDS once for all waves, in 16-byte pieces of a token's contiguous 96: read by every wave for
+    // itself, 32 tokens a load, they were more than half of the cache lines that a tile's start asks for.
+    const int blocks = padded_groups(ngrp) >> 4;
+    auto issue_sums = [&](int first) {              // blocks first .. first + SUM_BLOCKS - 1
+        for (int i = wave; i < 6 * SUM_BLOCKS; i += ROW_WAVES) {
+            const int block = i / 6;
+            if (first + block >= blocks) break;     // uniform over the wave
+            const int piece = (i - 6 * block) * 64 + lane, token = piece / 6;
+            load_to_lds<16>(notes, s_row[token] * (uint32_t)(2 * C) + (uint32_t)(16 + (first + block) * 96 + (piece - 6 * token) * 16),
+                            stage + sum_place(block) + (i - 6 * block) * 1024);
+        }
+    };
+    global_u16_ptr biases[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        biases[k] = (global_u16_ptr)(uintptr_t)(job.biases ? job.biases : job.scales) + (size_t)row[k] * (size_t)ngrp;
+    struct Eights { u32x4 s[2], b[2]; };            // sixteen groups, eight per lane half
+    auto fetch = [&](int block, Eights &e) {
+        const int first = eight_start(2 * block + half, ngrp);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            e.s[k] = *(global_u128_any_ptr)(scales[k] + first);
+            e.b[k] = *(global_u128_any_ptr)(biases[k] + first);
+        }
+    };
+    constexpr int AHEAD = SUM_BLOCKS;
+    issue_sums(0);
+    int my_down = 0;
+    if (tid < TM) my_down = *(global_i32_ptr)(notes + (size_t)s_row[tid] * (size_t)(2 * C));
+    Eights e[AHEAD];
+    if (ngrp >= 8) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) fetch(j < blocks ? j : blocks - 1, e[j]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            e[0].s[k] = load_short(scales[k], ngrp);
+            e[0].b[k] = load_short(biases[k], ngrp);
+        }
+#pragma unroll
+        for (int j = 1; j < AHEAD; ++j) e[j] = e[0];
+    }
+    wait_loads<0>();
+    // the compiler's own wait for these stands here, where it is none
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) asm volatile("" : "+v"(e[j].s[k]), "+v"(e[j].b[k]));
+    asm volatile("" : "+v"(my_down));
+    meet();
     issue_weights(0);
     issue_x(0);
-    if (tid < TM) s_down[tid] = *(global_i32_ptr)(notes + (size_t)s_row[tid] * (size_t)(2 * C));
 
     // ---- bias term of the tile, acc[tok][row] = sum_g (b[row][g] + 8 s[row][g]) * X[tok][g], and the rows' exponents
     const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     f32x16 acc[2][2] = {{zero, zero}, {zero, zero}};
     int top[2] = {0, 0};                            // row block nb: the scales of this lane's row are below 2^top[nb]
     int windows = 1;
+    auto more_sums = [&](int first) {               // the workgroup is done with the blocks in LDS: the next ones
+        meet();
+        issue_sums(first);
+        wait_loads<0>();
+        meet();
+    };
+    if (!live)                                      // the other waves meet here
+        for (int first = SUM_BLOCKS; first < blocks; first += SUM_BLOCKS) more_sums(first);
     if (live) {
-        const int padded = padded_groups(ngrp);
-        global_u8_ptr sums[2];
-        global_u16_ptr biases[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            sums[k] = notes + (size_t)s_row[k * 32 + l32] * (size_t)(2 * C) + 16 + half * 16;
-            biases[k] = (global_u16_ptr)(uintptr_t)(job.biases ? job.biases : job.scales) + (size_t)row[k] * (size_t)ngrp;
-        }
-        struct Eights { u32x4 s[2], b[2]; };
         const uint32_t keep = job.biases ? 0xffffffffu : 0u;        // without biases the scales stand in, masked
-        auto fetch = [&](int g0, bool whole, Eights &e) {           // sixteen groups, eight per lane half
-            const int first = eight_start((g0 >> 3) + half, ngrp);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                if (whole) {
-                    e.s[k] = *(global_u128_any_ptr)(scales[k] + first);
-                    e.b[k] = *(global_u128_any_ptr)(biases[k] + first);
-                } else {
-                    e.s[k] = load_short(scales[k], ngrp);
-                    e.b[k] = load_short(biases[k], ngrp);
-                }
-            }
-        };
         f32x16 tb[2][2] = {{zero, zero}, {zero, zero}}, ts[2][2] = {{zero, zero}, {zero, zero}};
         uint32_t s_max[2] = {0, 0}, b_max[2] = {0, 0}, s_min[2] = {0xffffffffu, 0xffffffffu};
-        Eights e;
-        if (ngrp >= 8) fetch(0, true, e); else fetch(0, false, e);
-        for (int g0 = 0; g0 < ngrp; g0 += 16) {
-            Eights c = e;
+        typedef const u32x4 __attribute__((address_space(3))) *sums_ptr;
+        auto add_block = [&](int slot, Eights &c) {
             u32x4 x[3][2];
+            const sums_ptr at = (sums_ptr)(stage + sum_place(slot) + l32 * 96 + half * 16);
 #pragma unroll
             for (int plane = 0; plane < 3; ++plane)
 #pragma unroll
-                for (int mb = 0; mb < 2; ++mb) x[plane][mb] = *(global_u128_ptr)(sums[mb] + (plane * padded + g0) * 2);
-            if (g0 + 16 < ngrp) fetch(g0 + 16, true, e);
+                for (int mb = 0; mb < 2; ++mb) x[plane][mb] = at[mb * (32 * 6) + plane * 2];
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
@@ -404,6 +445,15 @@ void q4_mfma_kernel(const MfmaLaunch L) {
                     s_min[nb] = pk_min(s_min[nb], pk_less_one(sa));
                     b_max[nb] = pk_max(b_max[nb], c.b[nb][j] & 0x7fff7fffu);
                 }
+        };
+        for (int block = 0; block < blocks; block += AHEAD) {
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j) {
+                if (block + j >= blocks) break;
+                if (j == 0 && block > 0) more_sums(block);
+                add_block(j, e[j]);
+                if (block + j + AHEAD < blocks) fetch(block + j + AHEAD, e[j]);
+            }
         }
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
@@ -435,6 +485,7 @@ void q4_mfma_kernel(const MfmaLaunch L) {
         }
     }
     if (lane == 0) s_windows[wave] = windows;
+    if (tid < TM) s_down[tid] = my_down;
     wait_loads<0>();
     __syncthreads();                                // the first stage and chunk are there as well
     windows = s_windows[0];
@@ -575,9 +626,10 @@ void q4_mfma_kernel(const MfmaLaunch L) {
         else walk(std::integral_constant<int, 1>{});
 
         if (live) {
-#pragma unroll
-            for (int mb = 0; mb < 2; ++mb) {
-                if (mb == 1 && !wide) break;
+            // WHOLE: the wave's block of rows and tokens is inside the output and new, and nothing is asked about a value (with a
+            // test for each the stores took 6700 to 8000 clocks of a tile's 50000 to 130000, without 4000 to 5000)
+            auto store = [&](auto all, int mb) {
+                constexpr bool WHOLE = decltype(all)::value;
                 int tok_base = mb * 32 + half * 4;
                 asm volatile("" : "+v"(tok_base));      // the output addresses are made here, not kept through the loop
                 global_f32_out line = (global_f32_out)(uintptr_t)job.y + (size_t)(tok0 + tok_base) * job.rows + row0 + l32;
@@ -587,15 +639,19 @@ void q4_mfma_kernel(const MfmaLaunch L) {
                     const int down = s_down[tok];
 #pragma unroll
                     for (int nb = 0; nb < 2; ++nb) {
-                        if (tok < toks_here && row0 + nb * 32 + l32 < job.rows) {
-                            float v = __builtin_amdgcn_ldexpf(acc[mb][nb][i], down - raise[nb]);
-                            if (window != 0) v = line[nb * 32] + v;
+                        if (WHOLE || (tok < toks_here && row0 + nb * 32 + l32 < job.rows)) {
+                            float v = __builtin_amdgcn_ldexpf(mb ? acc[1][nb][i] : acc[0][nb][i], down - raise[nb]);
+                            if (!WHOLE && window != 0) v = line[nb * 32] + v;
                             line[nb * 32] = v;
                         }
                     }
                     line += (size_t)job.rows * ((i & 3) == 3 ? 5 : 1);
                 }
-            }
+            };
+            const bool rows_inside = row0 + 64 <= job.rows && window == 0;
+            if (rows_inside && toks_here >= 32) store(std::true_type{}, 0); else store(std::false_type{}, 0);
+            if (rows_inside && toks_here == TM) store(std::true_type{}, 1);
+            else if (wide) store(std::false_type{}, 1);
         }
         if (++window >= windows) break;             // uniform over the workgroup
         __syncthreads();                            // the last group has been read by every wave
@@ -681,7 +737,7 @@ __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ 
     for (int at = 8 * tail + tid; at < padded; at += THREADS)
         if (at < 8 * tail + shift || at >= ngrp + shift)
 #pragma unroll
-            for (int plane = 0; plane < 3; ++plane) notes[8 + plane * padded + at] = 0;
+            for (int plane = 0; plane < 3; ++plane) notes[sum_entry(at, plane)] = 0;
 #pragma unroll
     for (int it = 0; it < SPLIT_MAX_ITEMS; ++it) {
         const int c0 = (it * THREADS + tid) * 8;
@@ -711,8 +767,8 @@ __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ 
                 uint32_t h, m, l;
                 split3(sum, h, m, l);
                 const int g = c0 >> 6;
-                uint16_t *at = notes + 8 + (g < 8 * tail ? g : g + shift);
-                at[0] = (uint16_t)h; at[padded] = (uint16_t)m; at[2 * padded] = (uint16_t)l;
+                uint16_t *const at = notes + sum_entry(g < 8 * tail ? g : g + shift, 0);
+                at[0] = (uint16_t)h; at[16] = (uint16_t)m; at[32] = (uint16_t)l;
             }
         }
     }
