@@ -24,9 +24,11 @@
 // and no second kernel.  Smaller ones are also split over workgroups, whose
 // partials a second kernel adds in split order.
 //
-// 8192 x 8192, 256 tokens: 64.2 -> 50.3 us with the activation pass, the kernel alone 51 + 9 (partial sums) -> 46.
+// 8192 x 8192, 256 tokens: 64.2 -> 45.7 us with the activation pass (48.1 with a wait for all loads at every stage, by
+// __syncthreads and by the compiler, see lds_load.h).
 // Bound: lines from the cache to the compute unit (64 KB per stage of two rounds of matrix work, of which the planes
 // are half), then the matrix cores.
+#include "lds_load.h"
 #include "mi355_internal.h"
 
 #include <stddef.h>
@@ -41,9 +43,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef const uint8_t __attribute__((address_space(1))) *global_u8_ptr;
-typedef const void __attribute__((address_space(1))) *global_void_ptr;
 typedef float __attribute__((address_space(1))) *global_f32_out;
-typedef void __attribute__((address_space(3))) *lds_void_ptr;
 typedef const u32x4 __attribute__((address_space(3))) *lds_u128_ptr;
 typedef const uint32_t __attribute__((address_space(3))) *lds_u32_ptr;
 
@@ -73,6 +73,13 @@ __device__ __forceinline__ int place_mask(int row) { return (row >> 1) & 7; }
 
 template <int N> __device__ __forceinline__ void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// The workgroup meets; a wave's LDS reads are done, its loads on their way stay there (__syncthreads waits for them).
+__device__ __forceinline__ void meet() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 }
 
 // Whether the activation pass rejected its input: the launch's status word, or the OR of the pass's per-workgroup
@@ -158,8 +165,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
         for (int i = 0; i < S::XT; ++i) {
             if (i * RW * 8 >= 32 && !wide) break;
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(plane + (x_src[i] + at)), (lds_void_ptr)(x + i * (RW * 1024)),
-                                             16, 0, 0);
+            load_to_lds<16>(plane, x_src[i] + at, x + i * (RW * 1024));
         }
     };
     // A row's scales of a chunk are 16 bytes.  They come in one load where addresses allow it: 64 rows are 64 cache
@@ -177,20 +183,17 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
             byte = byte < last ? byte : last;
             r = r < (uint32_t)rows_left ? r : (uint32_t)rows_left - 1u;
             const Offset line = FAR ? (Offset)r * (uint32_t)(C >> 1) : (Offset)__umul24(r, (uint32_t)(C >> 1));
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(codes + (line + byte)),
-                                             (lds_void_ptr)(stage + S::W_OFF + wave * S::W_BYTES + j * 1024), 16, 0, 0);
+            load_to_lds<16>(codes, line + byte, stage + S::W_OFF + wave * S::W_BYTES + j * 1024);
         }
         if (whole_scales) {                          // a chunk's scales of a row at once, from the row's end backwards
             const uint32_t s_at = (uint32_t)(first + it) * 4u, s_last = (uint32_t)G.chunks * 4u - 16u;
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(scale_rows + (scale_at + (s_at < s_last ? s_at : s_last))),
-                                             (lds_void_ptr)(stage + S::S_OFF + wave * S::S_BYTES), 16, 0, 0);
+            load_to_lds<16>(scale_rows, scale_at + (s_at < s_last ? s_at : s_last), stage + S::S_OFF + wave * S::S_BYTES);
             return;
         }
 #pragma unroll
         for (int k = 0; k < 2 * CH; ++k) {           // the two scales of each half of each stage
             const int g = first + it + (k >> 1) < G.chunks ? first + it + (k >> 1) : last_chunk;
-            __builtin_amdgcn_global_load_lds((global_void_ptr)(scale_rows + (scale_at + (uint32_t)(g * 4 + (k & 1) * 2))),
-                                             (lds_void_ptr)(stage + S::S_OFF + wave * S::S_BYTES + k * 256), 2, 0, 0);
+            load_to_lds<2>(scale_rows, scale_at + (uint32_t)(g * 4 + (k & 1) * 2), stage + S::S_OFF + wave * S::S_BYTES + k * 256);
         }
     };
     struct Weights { u32x4 w[CH][2]; uint32_t s[CH][2]; };
@@ -265,6 +268,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
         };
         take_weights(0, now);
         if (CH < iterations) issue_weights(CH);
+        asm volatile("" ::: "memory");
         read(0, 0, a[0]);
         decode(now.w[0], now.s[0], 0, first < end, b[0]);
         __builtin_amdgcn_sched_barrier(0);
@@ -287,7 +291,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
                 } else {
                     wait_loads<0>();
                 }
-                __syncthreads();
+                meet();
                 if (it + 2 < iterations) issue_x(it + 2);
                 if (gi == CH - 1) {
                     take_weights(it + 1, now);
@@ -303,7 +307,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
     } else {
         for (int it = 0; it < iterations; ++it) {    // a wave without rows helps to stage
             wait_loads<0>();
-            __syncthreads();
+            meet();
             if (it + 2 < iterations) issue_x(it + 2);
         }
     }
