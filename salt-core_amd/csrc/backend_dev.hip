@@ -26,7 +26,7 @@ int salt_mi355_q4_matmul_dev(const void *vals, const void *scales, const void *b
     }
     uint16_t *planes = (uint16_t *)workspace;
     const size_t plane_stride = (size_t)B * C;
-    if (x_split_launch(xs, nullptr, nullptr, 1, C, B, C, planes, plane_stride, (hipStream_t)stream) != 0) {
+    if (x_split_launch(xs, nullptr, nullptr, 1, C, B, C, planes, plane_stride, nullptr, 0, (hipStream_t)stream) != 0) {
         set_error("q4 matmul: activation split launch failed");
         return -1;
     }

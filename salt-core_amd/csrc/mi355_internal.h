@@ -172,13 +172,17 @@ struct MfmaLaunch {
     const int *row_map;       // optional gather: token t of a job reads plane row row_map[row_base + t] / map_divisor
     int map_divisor;
     int tile_tokens;          // tokens per tile: MFMA_TM or half of it; the launcher chooses for a single job
+    // optional, for a table whose jobs all have row_tiles tiles of rows: the job of the tiles i * row_tiles .. + row_tiles - 1
+    const int *tile_jobs;
+    int row_tiles;
 };
 
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream);
 // rows of fp32 -> two fp16 planes + a plane of notes; output row r reads input row row_map[r] / map_divisor when a map is
-// given; with a gate the value split is gelu_tanh(gate) * x (gate has the layout of x)
+// given; with a gate the value split is gelu_tanh(gate) * x (gate has the layout of x); `clear_words` words at `clear` are
+// set to zero on the way (a launch of its own for a few counters takes as long as the counting).
 int x_split_launch(const float *x, const float *gate, const int *row_map, int map_divisor, int x_stride, int rows,
-                   int cols, uint16_t *planes, size_t plane_stride, hipStream_t stream);
+                   int cols, uint16_t *planes, size_t plane_stride, uint32_t *clear, int clear_words, hipStream_t stream);
 
 // ---------------------------------------------------------------- NVFP4
 

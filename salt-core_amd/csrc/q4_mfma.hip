@@ -56,7 +56,7 @@
 //
 // Bound: the matrix cores, which execute twice the useful operations, at the
 // clock that their power leaves them: 44 % busy at 1.6 to 2.1 GHz in the grouped
-// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 590 us a layer);
+// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 585 us a layer);
 // one 16384 x 2816 matrix, 333 tokens: 101 -> 78 us, 384 tiles on 256 compute
 // units.  Before, every scale group cost 16 multiply-adds per block and a
 // conversion in each of two waves, and each 32 bytes of codes and each scale
@@ -157,9 +157,13 @@ __device__ __forceinline__ MfmaJob find_job(const MfmaLaunch &L, int tile) {
     const uniform_u64_ptr words = (uniform_u64_ptr)(uintptr_t)L.table;
     const int njobs = L.njobs_dev ? *(const int __attribute__((address_space(4))) *)(uintptr_t)L.njobs_dev : L.njobs;
     int lo = 0, hi = njobs - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if ((int)(uint32_t)words[7 * mid + 6] <= tile) lo = mid; else hi = mid - 1;
+    if (L.tile_jobs) {                          // a chain of dependent loads less at every tile's start
+        lo = ((const int __attribute__((address_space(4))) *)(uintptr_t)L.tile_jobs)[tile / L.row_tiles];
+    } else {
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if ((int)(uint32_t)words[7 * mid + 6] <= tile) lo = mid; else hi = mid - 1;
+        }
     }
     const uniform_u64_ptr rec = words + 7 * lo;
     MfmaJob job;
@@ -680,11 +684,12 @@ template <bool GATED, int ROW_WAVES>
 __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ x, const float *__restrict__ gate,
                                                       const int *__restrict__ row_map, int map_divisor, int x_stride,
                                                       int rows, int cols, uint16_t *__restrict__ planes,
-                                                      size_t plane_stride) {
+                                                      size_t plane_stride, uint32_t *__restrict__ clear, int clear_words) {
     __shared__ uint32_t wave_top[4];
     constexpr int THREADS = 64 * ROW_WAVES;
     const int tid = threadIdx.x & (THREADS - 1);
     const int row = ROW_WAVES == 4 ? (int)blockIdx.x : (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < clear_words; i += gridDim.x * 256) clear[i] = 0u;
     if (row >= rows) return;                        // whole waves, and only where no barrier follows
     const int src_row = row_map ? row_map[row] / map_divisor : row;
     float v[SPLIT_MAX_ITEMS][8];
@@ -800,7 +805,7 @@ int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream) {
 }
 
 int x_split_launch(const float *x, const float *gate, const int *row_map, int map_divisor, int x_stride, int rows,
-                   int cols, uint16_t *planes, size_t plane_stride, hipStream_t stream) {
+                   int cols, uint16_t *planes, size_t plane_stride, uint32_t *clear, int clear_words, hipStream_t stream) {
     if (rows < 1 || cols < 64 || (cols & 63) || cols > SPLIT_MAX_ITEMS * 256 * 8) return -1;
     // A wave per row leaves no thread of a short row idle (gelu_tanh(gate) * up, 16384 rows of 704: 50 -> 41 us), a
     // workgroup per row shortens the chain of a call with few rows (900 rows of 704: 5.9 against 7.2 us).
@@ -809,7 +814,7 @@ int x_split_launch(const float *x, const float *gate, const int *row_map, int ma
     auto kernel = gate ? (one_wave ? x_split_kernel<true, 1> : x_split_kernel<true, 4>)
                        : (one_wave ? x_split_kernel<false, 1> : x_split_kernel<false, 4>);
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, gate, row_map, map_divisor, x_stride, rows, cols, planes,
-                       plane_stride);
+                       plane_stride, clear, clear_words);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
