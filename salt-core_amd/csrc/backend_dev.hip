@@ -36,7 +36,7 @@ int salt_mi355_q4_matmul_dev(const void *vals, const void *scales, const void *b
     launch.one.biases = (const uint8_t *)biases;
     launch.one.planes = planes; launch.one.y = ys;
     launch.one.tokens = B; launch.one.rows = R;
-    launch.njobs = 1; launch.cols = C; launch.plane_stride = plane_stride;
+    launch.cols = C; launch.plane_stride = plane_stride;
     if (q4_mfma_launch(launch, (hipStream_t)stream) != 0) { set_error("q4 matmul: launch failed"); return -1; }
     return 0;
 }
@@ -235,7 +235,7 @@ int salt_mi355_nvfp4_matvec_qdq_dev(const void *packed, const void *scales, floa
     launch.one.weight_global_scale = 1.0f / stored_divisor;
     launch.one.rows = R;
     launch.one.x_stride = C;
-    launch.njobs = 1; launch.cols = C; launch.tokens = 1;
+    launch.cols = C; launch.tokens = 1;
     launch.total_tiles = (R + 63) / 64;
     launch.qdq = 1; launch.input_global_scale = input_global_scale; launch.status = status_dev;
     if (fp4_launch(launch, chains, (hipStream_t)stream) != 0) { set_error("nvfp4 matvec: launch failed"); return -1; }

@@ -160,21 +160,24 @@ struct MfmaJob {
     int row_base;             // with a row map: index of this job's first token in the map
 };
 
+// Tiles are numbered with those of MFMA_TM tokens first, then those of half as many.
 struct MfmaLaunch {
     MfmaJob one;
-    const MfmaJob *table;
-    int njobs;
     int cols;
-    int total_tiles;          // grid size; an upper bound when the counts below live on the device
     size_t plane_stride;      // elements between planes
-    const int *njobs_dev;     // optional: job and tile counts produced by an earlier kernel;
-    const int *total_tiles_dev;   // workgroups past *total_tiles_dev exit at once
     const int *row_map;       // optional gather: token t of a job reads plane row row_map[row_base + t] / map_divisor
     int map_divisor;
-    int tile_tokens;          // tokens per tile: MFMA_TM or half of it; the launcher chooses for a single job
-    // optional, for a table whose jobs all have row_tiles tiles of rows: the job of the tiles i * row_tiles .. + row_tiles - 1
+    // one job (no table): blocks of MFMA_TM and of half as many tokens, and the tiles of each; the launcher chooses
+    int wide_blocks, narrow_blocks;
+    int wide_tiles, narrow_tiles;
+    // A table of jobs that an earlier kernel filled, all with row_tiles tiles of rows: the numbers of tiles of both sizes
+    // (surplus workgroups leave at once), the job of the tiles i * row_tiles .. + row_tiles - 1, and a bound on their sum.
+    // A job's tokens lie in blocks of MFMA_TM as long as more than half a block is left, the rest in one of half; tile0
+    // is its first tile of MFMA_TM tokens.
+    const MfmaJob *table;
+    const int *tiles_dev;
     const int *tile_jobs;
-    int row_tiles;
+    int row_tiles, most_tiles;
 };
 
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream);

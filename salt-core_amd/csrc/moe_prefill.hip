@@ -21,8 +21,7 @@ constexpr int MAX_EXPERTS = 1024;
 
 struct PrefillPlan {            // device ints produced by the count and scan kernels
     int status;                 // 0 ok, -1 the selection is invalid
-    int gate_up_jobs, down_jobs;
-    int gate_up_tiles, down_tiles;
+    int gate_up_tiles[2], down_tiles[2];        // of 64 and of 32 tokens
 };
 
 // Exclusive prefix sum over the threads of a workgroup (blockDim a multiple of 64, at most 1024).
@@ -110,7 +109,7 @@ struct ScanArgs {
     PrefillPlan *plan;
     int *status_out;                     // optional
     MfmaJob *gate_up_jobs, *down_jobs;
-    int *gate_up_tile_jobs, *down_tile_jobs;     // job of every tile of tokens of a launch
+    int *gate_up_tile_jobs, *down_tile_jobs;     // job of every block of tokens of a launch, those of 64 tokens first
     const uint16_t *planes_in;           // split of the inputs, one row per token  [tokens][hidden]
     const uint16_t *planes_act;          // split of the activations, grouped rows   [rows][routed]
     float *gate, *up, *down;
@@ -121,11 +120,16 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
     __shared__ int s_wave[MAX_EXPERTS / 64];
     const int e = threadIdx.x;
     const int n = e < a.n_experts ? a.counts[e] : 0;
-    const int mt = (n + MFMA_TM - 1) / MFMA_TM;
-    int rows_total, mt_total, used_total;
+    const int wide = (n + MFMA_TM / 2 - 1) / MFMA_TM, narrow = n > wide * MFMA_TM;     // blocks of 64 and of 32 tokens
+    int rows_total, blocks_total;
     const int row0 = block_exclusive_scan(n, s_wave, &rows_total);
-    const int mt0 = block_exclusive_scan(mt, s_wave, &mt_total);
-    const int job = block_exclusive_scan(n > 0, s_wave, &used_total);
+    // both counts in one scan: at most MAX_EXPERTS narrow blocks, and 2^18 wide ones
+    constexpr int BITS = 11;
+    static_assert(MAX_EXPERTS < 1 << BITS && MFMA_TM == 64, "the sums stay below 2^30");
+    const int blocks0 = block_exclusive_scan(wide << BITS | narrow, s_wave, &blocks_total);
+    const int wide0 = blocks0 >> BITS, narrow0 = blocks0 & ((1 << BITS) - 1);
+    const int wide_total = blocks_total >> BITS, narrow_total = blocks_total & ((1 << BITS) - 1);
+    const int job = block_exclusive_scan(n > 0, s_wave, nullptr);
     if (e < a.n_experts) {
         a.offsets[e] = row0;
         if (a.group_rows) a.group_rows[e] = n;
@@ -134,10 +138,10 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
     const bool valid = a.plan->status == 0;          // written by the previous kernel on this stream
     if (e == 0) {
         a.offsets[a.n_experts] = rows_total;
-        a.plan->gate_up_jobs = valid ? 2 * used_total : 0;
-        a.plan->down_jobs = valid ? used_total : 0;
-        a.plan->gate_up_tiles = valid ? 2 * mt_total * nt_up : 0;
-        a.plan->down_tiles = valid ? mt_total * nt_down : 0;
+        a.plan->gate_up_tiles[0] = valid ? 2 * wide_total * nt_up : 0;
+        a.plan->gate_up_tiles[1] = valid ? 2 * narrow_total * nt_up : 0;
+        a.plan->down_tiles[0] = valid ? wide_total * nt_down : 0;
+        a.plan->down_tiles[1] = valid ? narrow_total * nt_down : 0;
         if (a.status_out) *a.status_out = a.plan->status;
     }
     if (valid && e < a.n_experts && n > 0) {
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
             j.planes = a.planes_in;                           // gathered through the row map
             j.y = (p == 0 ? a.gate : a.up) + (size_t)row0 * a.routed;
             j.tokens = n; j.rows = a.routed;
-            j.tile0 = (2 * mt0 + p * mt) * nt_up;
+            j.tile0 = (2 * wide0 + p * wide) * nt_up;
             j.row_base = row0;
             a.gate_up_jobs[2 * job + p] = j;
         }
@@ -159,13 +163,18 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
         d.planes = a.planes_act + (size_t)row0 * a.routed;
         d.y = a.down + (size_t)row0 * a.hidden;
         d.tokens = n; d.rows = a.hidden;
-        d.tile0 = mt0 * nt_down;
+        d.tile0 = wide0 * nt_down;
         d.row_base = 0;
         a.down_jobs[job] = d;
-        for (int i = 0; i < mt; ++i) {
-            a.gate_up_tile_jobs[2 * mt0 + i] = 2 * job;
-            a.gate_up_tile_jobs[2 * mt0 + mt + i] = 2 * job + 1;
-            a.down_tile_jobs[mt0 + i] = job;
+        for (int i = 0; i < wide; ++i) {
+            a.gate_up_tile_jobs[2 * wide0 + i] = 2 * job;
+            a.gate_up_tile_jobs[2 * wide0 + wide + i] = 2 * job + 1;
+            a.down_tile_jobs[wide0 + i] = job;
+        }
+        if (narrow) {
+            a.gate_up_tile_jobs[2 * (wide_total + narrow0)] = 2 * job;
+            a.gate_up_tile_jobs[2 * (wide_total + narrow0) + 1] = 2 * job + 1;
+            a.down_tile_jobs[wide_total + narrow0] = job;
         }
     }
 }
@@ -331,11 +340,11 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
     // ceil(n_e / 64) <= rows / 64 + experts) and surplus workgroups leave at once.
     MfmaLaunch gu;
     memset(&gu, 0, sizeof gu);
-    gu.table = w.gate_up_jobs; gu.cols = g.hidden; gu.total_tiles = 2 * m_upper * nt_up;
+    gu.table = w.gate_up_jobs; gu.cols = g.hidden; gu.most_tiles = 2 * m_upper * nt_up;
     gu.plane_stride = (size_t)tokens * g.hidden;
-    gu.row_map = rp; gu.map_divisor = g.topk; gu.tile_tokens = MFMA_TM;
+    gu.row_map = rp; gu.map_divisor = g.topk;
     gu.tile_jobs = w.gate_up_tile_jobs; gu.row_tiles = nt_up;
-    gu.njobs_dev = &w.plan->gate_up_jobs; gu.total_tiles_dev = &w.plan->gate_up_tiles;
+    gu.tiles_dev = w.plan->gate_up_tiles;
     if (q4_mfma_launch(gu, stream) != 0) return -1;
     // gelu(gate) * up, split for the down projection
     if (x_split_launch(w.up, w.gate, nullptr, 1, g.routed, rows, g.routed, w.planes_act, (size_t)rows * g.routed, nullptr, 0,
@@ -343,11 +352,10 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
         return -1;
     MfmaLaunch dn;
     memset(&dn, 0, sizeof dn);
-    dn.table = w.down_jobs; dn.cols = g.routed; dn.total_tiles = m_upper * nt_down;
+    dn.table = w.down_jobs; dn.cols = g.routed; dn.most_tiles = m_upper * nt_down;
     dn.plane_stride = (size_t)rows * g.routed;
-    dn.tile_tokens = MFMA_TM;
     dn.tile_jobs = w.down_tile_jobs; dn.row_tiles = nt_down;
-    dn.njobs_dev = &w.plan->down_jobs; dn.total_tiles_dev = &w.plan->down_tiles;
+    dn.tiles_dev = w.plan->down_tiles;
     if (q4_mfma_launch(dn, stream) != 0) return -1;
     hipLaunchKernelGGL(prefill_reduce_kernel, dim3(tokens, (g.hidden + 1023) / 1024), dim3(256), 0, stream, w.down,
                        w.pair_rows, weights, g.topk, g.hidden, w.plan, outputs);

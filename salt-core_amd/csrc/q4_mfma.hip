@@ -56,15 +56,15 @@
 //
 // Bound: the matrix cores, which execute twice the useful operations, at the
 // clock that their power leaves them: 44 % busy at 1.6 to 2.1 GHz in the grouped
-// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 585 us a layer);
-// one 16384 x 2816 matrix, 333 tokens: 101 -> 78 us, 384 tiles on 256 compute
-// units.  Before, every scale group cost 16 multiply-adds per block and a
-// conversion in each of two waves, and each 32 bytes of codes and each scale
-// fetched a cache line of its own.  Calls of few tiles are bound by one wave per
-// SIMD that issues an instruction every eight clocks: 33 tokens, 8192 x 2816
-// 39.5 -> 34.1 us and 8192 x 8192 98.7 -> 84.9, 64 tokens, 4096 x 4096 54.3 ->
-// 46.2 once nothing in the walk waits but what has to (lds_load.h).  Four
-// stages of planes instead of two gained nothing there.
+// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 581 us a layer);
+// one 16384 x 2816 matrix, 333 tokens: 101 -> 75 us (256 tokens, one tile of 64
+// for each compute unit, 55 us: 1.1 PFLOP/s of both planes).  Before, every scale
+// group cost 16 multiply-adds per block and a conversion in each of two waves,
+// and each 32 bytes of codes and each scale fetched a cache line of its own.
+// Calls of few tiles are bound by one wave per SIMD, whose dependent vector
+// instructions issue eight clocks apart: 33 tokens, 8192 x 2816 39.5 -> 34.1 us
+// and 8192 x 8192 98.7 -> 84.9, 64 tokens, 4096 x 4096 54.3 -> 46.2 once nothing
+// in the walk waits but what has to (lds_load.h).
 //
 // Inside every aligned run of eight columns the planes are stored in the order
 // 0,4,1,5,2,6,3,7, which is the order the pair extraction yields the codes in;
@@ -95,7 +95,8 @@ typedef const uint8_t __attribute__((address_space(1))) *global_u8_ptr;
 typedef const int __attribute__((address_space(1))) *global_i32_ptr;
 typedef float __attribute__((address_space(1))) *global_f32_out;
 
-constexpr int TM = MFMA_TM;                 // tokens per workgroup
+constexpr int TM = MFMA_TM;                 // tokens per workgroup, or half of it
+constexpr int CUS = 256;
 constexpr int X_PLANES = 2;                 // fp16 planes of the scaled activation
 constexpr int WINDOW = 28;                  // binades of scale that are exact fp16 operands at a time
 constexpr int MAX_WINDOWS = 10;             // all of a bf16's binades
@@ -152,20 +153,11 @@ __device__ __forceinline__ void meet() {
 
 static_assert(sizeof(MfmaJob) == 56, "find_job reads a job record as seven 64-bit words");
 
+// In a table every job has L.row_tiles tiles of rows: the job follows from the tile's number by one load.
 __device__ __forceinline__ MfmaJob find_job(const MfmaLaunch &L, int tile) {
     if (L.table == nullptr) return L.one;
-    const uniform_u64_ptr words = (uniform_u64_ptr)(uintptr_t)L.table;
-    const int njobs = L.njobs_dev ? *(const int __attribute__((address_space(4))) *)(uintptr_t)L.njobs_dev : L.njobs;
-    int lo = 0, hi = njobs - 1;
-    if (L.tile_jobs) {                          // a chain of dependent loads less at every tile's start
-        lo = ((const int __attribute__((address_space(4))) *)(uintptr_t)L.tile_jobs)[tile / L.row_tiles];
-    } else {
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if ((int)(uint32_t)words[7 * mid + 6] <= tile) lo = mid; else hi = mid - 1;
-        }
-    }
-    const uniform_u64_ptr rec = words + 7 * lo;
+    const int at = ((const int __attribute__((address_space(4))) *)(uintptr_t)L.tile_jobs)[tile / L.row_tiles];
+    const uniform_u64_ptr rec = (uniform_u64_ptr)(uintptr_t)L.table + 7 * at;
     MfmaJob job;
     job.vals = (const uint8_t *)rec[0];
     job.scales = (const uint8_t *)rec[1];
@@ -240,19 +232,40 @@ void q4_mfma_kernel(const MfmaLaunch L) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
 
-    // Workgroups go round the eight partitions of the device in turn; a partition takes one run of consecutive tiles,
-    // so that the tiles of one weight matrix, or of one expert, meet in one partition's cache.
-    const int total = L.total_tiles_dev ? *(const int __attribute__((address_space(4))) *)(uintptr_t)L.total_tiles_dev
-                                        : L.total_tiles;
-    const int run = (total + 7) >> 3;
-    const int tile = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= run || tile >= total) return;      // uniform: the whole workgroup leaves
-    const MfmaJob job = find_job(L, tile);
+    // Workgroups go round the eight partitions of the device in turn; a partition takes one run of consecutive tiles of 64
+    // tokens, so that the tiles of one weight matrix, or of one expert, meet in one partition's cache, and then one of the
+    // tiles of 32: no partition is left with the longer tiles, and the shorter ones fill the end
+    // (all tiles in one run each: grouped prefill of 256 tokens over 128 experts 225 -> 234 us, 512 over 32 79 -> 82; one
+    // matrix of 65500 x 2816, 96 tokens, 80 -> 86).
+    int wide_tiles = L.wide_tiles, narrow_tiles = L.narrow_tiles;
+    if (L.table) {
+        const int __attribute__((address_space(4))) *counts = (const int __attribute__((address_space(4))) *)(uintptr_t)L.tiles_dev;
+        wide_tiles = counts[0];
+        narrow_tiles = counts[1];
+    }
+    const int wide_run = (wide_tiles + 7) >> 3, narrow_run = (narrow_tiles + 7) >> 3;
+    const int part = (int)(blockIdx.x & 7), turn = (int)(blockIdx.x >> 3);
+    const bool first = turn < wide_run;
+    const int nth = first ? part * wide_run + turn : part * narrow_run + turn - wide_run;
+    if (nth >= (first ? wide_tiles : narrow_tiles) || turn >= wide_run + narrow_run) return;  // uniform: the whole workgroup leaves
+    const MfmaJob job = find_job(L, first ? nth : wide_tiles + nth);
     const int C = L.cols, ngrp = C >> 6;
-    const int tm = L.tile_tokens;                   // TM, or half of it
-    const int mtiles = (job.tokens + tm - 1) / tm;
-    const int t = tile - job.tile0;
-    const int tok0 = (t % mtiles) * tm, row0 = (t / mtiles) * MFMA_TN + wave * 64;
+    // Blocks of tokens: in a table as many of 64 as hold more than 32, and one of 32 for the rest.
+    const int wide_blocks = L.table ? (job.tokens + 31) >> 6 : L.wide_blocks;
+    int tok0, row_tile;
+    if (first) {
+        const int t = nth - job.tile0;
+        row_tile = t / wide_blocks;
+        tok0 = (t - row_tile * wide_blocks) * TM;
+    } else if (L.table) {
+        row_tile = nth % L.row_tiles;
+        tok0 = wide_blocks * TM;
+    } else {
+        row_tile = nth / L.narrow_blocks;
+        tok0 = wide_blocks * TM + (nth - row_tile * L.narrow_blocks) * (TM / 2);
+    }
+    const int row0 = row_tile * MFMA_TN + wave * 64;
+    const int tm = first ? TM : TM / 2;
     const int toks_here = job.tokens - tok0 < tm ? job.tokens - tok0 : tm;
     const bool wide = toks_here > 32;               // both token blocks hold tokens
     const bool live = row0 < job.rows;              // this wave has rows; the others only help to stage
@@ -781,26 +794,41 @@ __global__ __launch_bounds__(256) void x_split_kernel(const float *__restrict__ 
 
 }  // namespace
 
-namespace {
-int mfma_tiles(int tokens, int tile_tokens, int rows) {
-    return ((tokens + tile_tokens - 1) / tile_tokens) * ((rows + MFMA_TN - 1) / MFMA_TN);
-}
-}  // namespace
-
 int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream) {
     MfmaLaunch L = launch;
     if (L.cols < 64 || (L.cols & 63)) return -1;
+    int turns;                                  // of the eight partitions
     if (L.table == nullptr) {                   // one job: the tiling is chosen here
+        const int halves = (L.one.tokens + TM / 2 - 1) / (TM / 2), row_tiles = (L.one.rows + MFMA_TN - 1) / MFMA_TN;
         // Tiles of half the tokens where each still finds a compute unit of its own: half the matrix work per step of a
-        // walk that is bound by its waits (4096 x 4096, 64 tokens: 67 us in 64-token tiles, 54 in these).
-        L.tile_tokens = mfma_tiles(L.one.tokens, TM / 2, L.one.rows) <= 256 ? TM / 2 : TM;
+        // walk that is bound by its waits (4096 x 4096, 64 tokens: 67 us in 64-token tiles, 54 in these).  Else tiles of 64
+        // and, for what is left, one of 32; but between two and three halves per compute unit no unit gets two tiles of 64
+        // while others have one: as many of those as there are units, then tiles of 32, as long as all of them are at work
+        // at once (2816 columns, us with the cap and without: 16384 rows, 333 tokens 74.6 and 79.1; 2816, 1600 74.7 and
+        // 83.3; 25600, 224 77.2 and 80.5; with four tiles left over for a third turn, 33000, 150, 88.3 and 79.1).
+        const long long work = (long long)halves * row_tiles;
+        L.wide_blocks = halves / 2;
+        if (work <= CUS) L.wide_blocks = 0;
+        else if (work > 2 * CUS && work <= 3 * CUS) {
+            const int cap = CUS / row_tiles;
+            if (cap < L.wide_blocks && work - (long long)cap * row_tiles <= 2 * CUS) L.wide_blocks = cap;
+        }
+        L.narrow_blocks = halves - 2 * L.wide_blocks;
         L.one.tile0 = 0;
-        L.total_tiles = mfma_tiles(L.one.tokens, L.tile_tokens, L.one.rows);
+        L.row_tiles = row_tiles;
+        if (L.one.tokens < 1 || L.one.rows < 1 || work > (1 << 30)) return -1;
+        L.wide_tiles = L.wide_blocks * row_tiles;
+        L.narrow_tiles = L.narrow_blocks * row_tiles;
+        turns = (L.wide_tiles + 7) / 8 + (L.narrow_tiles + 7) / 8;
+        note_kernel("q4_mfma_kernel, tiles of %d tokens", work <= CUS ? TM / 2 : TM);
+    } else {
+        if (L.most_tiles < 1 || L.row_tiles < 1 || !L.tile_jobs || !L.tiles_dev) return -1;
+        turns = (L.most_tiles + 14) / 8;        // both runs, each rounded up
+        note_kernel("q4_mfma_kernel, tiles of %d tokens", TM);
     }
     if (3 * (unsigned long long)L.plane_stride >= (1ull << 32)) return -1;      // 32-bit byte offsets inside a plane
-    if (L.total_tiles < 1 || (L.tile_tokens != TM && L.tile_tokens != TM / 2) || (L.row_map && L.map_divisor < 1)) return -1;
-    note_kernel("q4_mfma_kernel, tiles of %d tokens", L.tile_tokens);
-    hipLaunchKernelGGL(q4_mfma_kernel, dim3((L.total_tiles + 7) / 8 * 8), dim3(256), 0, stream, L);
+    if (L.row_map && L.map_divisor < 1) return -1;
+    hipLaunchKernelGGL(q4_mfma_kernel, dim3(turns * 8), dim3(256), 0, stream, L);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
