@@ -124,9 +124,10 @@ __device__ __forceinline__ float add_staged(const float *mine, int count, float 
 // the result.
 // (Subnormals and the lowest normal binade share their unit; a zero accumulator is even; infinities and NaN are walked.)
 //
-// 2816 squares of a normal vector: 9 of 235 parts are walked, 3.0 us instead of 10.1 for the chain (a lone wave issues a
-// vector instruction every eight clocks, 3.6 ns, which is what counts here).  The feed-forward block of 2816/2112/704
-// with 128 experts, three such sums deep: 90.1 -> 63.8 us; its first cell 13.5 -> 6.2 us, its last 30.6 -> 11.2.
+// 2816 squares of a normal vector: 9 of 235 parts are walked, 3.0 us instead of 10.1 for the chain (a lone wave's dependent
+// vector instructions issue eight clocks apart, 3.6 ns, independent ones four, which is what counts here).  The
+// feed-forward block of 2816/2112/704 with 128 experts, three such sums deep: 90.1 -> 63.8 us (57.5 since its branches
+// share their launches); its first cell 13.5 -> 6.2 us, its last 30.6 -> 11.2.
 constexpr int ORDERED_MIN = 512;      // below, the chain is as quick
 constexpr int PARTS = 4;              // of a lane
 constexpr int ORDERED_FLOATS = 64 * (SQ_CHUNK / 64 + 4);     // LDS of SQ_CHUNK addends; a lane's block is 4 floats apart
@@ -247,7 +248,7 @@ __device__ __forceinline__ float ordered_sum(const float *addends, float acc, Or
 
     // From here on every lane does the same: the parts between two walked ones in one addition to the bit pattern, the
     // walked ones addend by addend.  Lane l holds where the l-th walked part of a round of 64 lies; its record and its
-    // addends are read one walked part ahead.  Few instructions matter here: a lone wave issues one every eight clocks.
+    // addends are read one walked part ahead.  Few instructions matter here: a lone wave issues one in four to eight clocks.
     auto words_of = [&](int part) { return (words_ptr)(addends + (part >> 2) * PITCH + (part & 3) * 4 * WORDS); };
     auto add = [&](const float4 &v) {
         acc = acc + v.x;

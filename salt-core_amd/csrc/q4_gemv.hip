@@ -170,7 +170,8 @@ constexpr int x_batch_groups(int S, int NB) {
 // workgroup has 1 / SPLIT of the waves and a wave the same work.  The chain order leaves rows as the only axis to cut
 // along, and a wave's instruction count does not shrink with idle lanes.  The slice differs inside a wave, so the
 // activations come from LDS as in the prologues above.  One chain per lane (S = 1) leaves a wave with fewer than half of
-// the instructions of two and doubles the waves: a lone wave issues one every eight clocks, two on a SIMD fill it.
+// the instructions of two and doubles the waves: a lone wave's dependent instructions issue eight clocks apart,
+// two waves on a SIMD fill the gaps.
 // One token, 2816 x 2816 (44 tiles): 10.8 us whole, 6.9 in quarters with two chains per lane, 5.9 with one.
 template <int S, int NB, int CB, int PRO, int SPLIT>
 struct TileKernel {
