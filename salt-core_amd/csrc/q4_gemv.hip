@@ -208,23 +208,27 @@ struct TileKernel {
     // the router prologue borrows memory that is used later, and one thread per expert (q4_moe_gate_up_launch sees to that)
     static_assert(PRO != 1 || sizeof(RouterShared) <= (SPLIT > 1 && !STEP_X ? sizeof(Lds::x) : sizeof(Lds::w)), "the router fits");
 
-    // `block` numbers the launch's workgroups from 0
-    static __device__ __forceinline__ void run(const Q4Launch &L, int block, Lds &lds);
+    // `block` numbers the launch's workgroups from 0.  A kernel of one body declares each of the pieces by itself: where they
+    // are members of one object the compiler leaves LDS reads of activations single (three tokens, 264 tiles: 22.7 us), and
+    // joined by hand it waits for them one by one (20.0 to 20.2; so 19.8).
+    static __device__ __forceinline__ void run(const Q4Launch &L, int block, uint8_t *w_lds, float *m_lds, float *x_lds, int &slow_flag);
+    static __device__ __forceinline__ void run(const Q4Launch &L, int block, Lds &lds) { run(L, block, lds.w, lds.m, lds.x, lds.slow); }
 };
 
 template <int S, int NB, int CB, int PRO = 0, int SPLIT = 1>
 __global__ __launch_bounds__((TileKernel<S, NB, CB, PRO, SPLIT>::THREADS), (TileKernel<S, NB, CB, PRO, SPLIT>::MIN_WAVES))
 void q4_tile_kernel(const Q4Launch L) {
-    __shared__ typename TileKernel<S, NB, CB, PRO, SPLIT>::Lds lds;
-    TileKernel<S, NB, CB, PRO, SPLIT>::run(L, (int)blockIdx.x, lds);
+    using Tile = TileKernel<S, NB, CB, PRO, SPLIT>;
+    __shared__ __attribute__((aligned(16))) uint8_t w[Tile::W_BYTES];
+    __shared__ __attribute__((aligned(16))) float m[2 * Tile::M_STAGE];
+    __shared__ __attribute__((aligned(16))) float x[Tile::X_FLOATS];
+    __shared__ int slow;
+    Tile::run(L, (int)blockIdx.x, w, m, x, slow);
 }
 
 template <int S, int NB, int CB, int PRO, int SPLIT>
-__device__ __forceinline__ void TileKernel<S, NB, CB, PRO, SPLIT>::run(const Q4Launch &L, const int block, Lds &lds) {
-    auto &w_lds = lds.w;
-    auto &m_lds = lds.m;
-    auto &x_lds = lds.x;
-    int &slow_flag = lds.slow;
+__device__ __forceinline__ void TileKernel<S, NB, CB, PRO, SPLIT>::run(const Q4Launch &L, const int block, uint8_t *const w_lds,
+                                                                           float *const m_lds, float *const x_lds, int &slow_flag) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -439,17 +443,13 @@ __device__ __forceinline__ void TileKernel<S, NB, CB, PRO, SPLIT>::run(const Q4L
     // x of `groups` consecutive scale groups starting at group g0 of the row
     auto load_x = [&](int g0, float (&xq)[NB][XN], int groups) {
         if (LDS_X) {                      // every lane of a slice reads the same LDS words: the activations travel in vector registers
-            typedef float f32xS __attribute__((ext_vector_type(S)));        // a slice's activations of one block, one LDS read
-            const float *xl = x_step + g0 * 64 + S * slice;
+            // aligned: a slice's activations of one block are one LDS read
+            const float *xl = (const float *)__builtin_assume_aligned(x_step + g0 * 64 + S * slice, 4 * S < 16 ? 4 * S : 16);
 #pragma unroll
             for (int t = 0; t < NB; ++t)
 #pragma unroll
-                for (int b = 0; b < XN / S; ++b)
-                    if (b < groups * 2) {
-                        const f32xS v = *reinterpret_cast<const f32xS *>(xl + t * X_STEP + b * 32);
-#pragma unroll
-                        for (int k = 0; k < S; ++k) xq[t][b * S + k] = v[k];
-                    }
+                for (int k = 0; k < XN; ++k)
+                    if (k < groups * 2 * S) xq[t][k] = xl[t * X_STEP + (k / S) * 32 + (k % S)];
             return;
         }
         const uniform_f32_ptr xg = xbase + (size_t)g0 * 64;
