@@ -29,12 +29,18 @@ __device__ __forceinline__ lds_load_from uniform_address(lds_load_from p) {
 }
 
 // sixteen or two bytes per lane, from a uniform address and a lane's 32-bit offset
+//
+// A memory instruction may read a scalar register five wait states after a vector instruction has written it (a
+// readfirstlane, or the readlane of a spilled one) and no sooner, which the compiler sees to for instructions that it knows.
+// Here the load's base is a copy that a scalar instruction makes: that one waits for vector writes by itself, and nobody has
+// to wait for what it writes.  It is also the one wait state that a load into LDS wants after the write of m0.
 template <int SIZE> __device__ __forceinline__ void load_to_lds(lds_load_from base, uint32_t offset, const void *to) {
     static_assert(SIZE == 16 || SIZE == 2, "");
+    uint64_t copy;
     if (SIZE == 16)
-        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds_load_place(to)), "v"(offset), "s"(base) : "memory");
+        asm volatile("s_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(copy) : "{m0}"(lds_load_place(to)), "v"(offset), "s"(base) : "memory");
     else
-        asm volatile("s_nop 0\n\tglobal_load_lds_ushort %1, %2" ::"{m0}"(lds_load_place(to)), "v"(offset), "s"(base) : "memory");
+        asm volatile("s_mov_b64 %0, %3\n\tglobal_load_lds_ushort %2, %0" : "=&s"(copy) : "{m0}"(lds_load_place(to)), "v"(offset), "s"(base) : "memory");
 }
 
 // the same with a 64-bit offset
