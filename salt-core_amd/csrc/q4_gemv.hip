@@ -727,9 +727,9 @@ constexpr int shape_key(int chains, int blocks, int split) { return (chains * 64
 
 template <int S, int NB, int CB, int PRO, int SPLIT>
 int launch_as(const Q4Launch &L, int extra, hipStream_t stream) {
-    if (PRO == 0) {
-        if (SPLIT == 1) note_kernel("q4_tile_kernel<%d,%d,%d,0>", S, NB, CB);
-        else note_kernel("q4_tile_kernel<%d,%d,%d,0,%d>", S, NB, CB, SPLIT);
+    if (PRO == 0 || PRO == 3) {                 // the MoE launches are noted in pairs
+        if (SPLIT == 1) note_kernel("q4_tile_kernel<%d,%d,%d,%d>", S, NB, CB, PRO);
+        else note_kernel("q4_tile_kernel<%d,%d,%d,%d,%d>", S, NB, CB, PRO, SPLIT);
     }
     hipLaunchKernelGGL((q4_tile_kernel<S, NB, CB, PRO, SPLIT>), dim3(SPLIT * L.total_tiles + extra), dim3(64 * 32 / (S * SPLIT)),
                        0, stream, L);
@@ -802,7 +802,9 @@ namespace {
 // 18.5 / 18.2 / quarters 18.9; 176 of 1024 17.0 / 16.7 / quarters 18.8, of 1536 17.5 / 17.2 / 16.5, of 2816 24.3 / 22.7 /
 // 21.4; 192 of 2816 (four quarters a compute unit, with the publisher) 23.5 / 21.9 / 23.4; 256 of 1024 21.1 / 18.8 / halves
 // <4> 16.3, of 2048 24.9 / 23.0 / 19.9, 208 of 2816 24.0 / 22.5 / 22.7.
-TileShape gate_up_shape(const MoeFuse &m, int tiles) {
+int gate_up_tiles(const MoeFuse &m) { return 2 * m.topk * ((m.routed + TILE_ROWS - 1) / TILE_ROWS); }
+TileShape gate_up_shape(const MoeFuse &m) {
+    const int tiles = gate_up_tiles(m);
     TileShape shape = open_shape(tiles, m.hidden, 1);
     if (shape.split > 1 && tiles <= COMPUTE_UNITS) {
         if (tiles <= COMPUTE_UNITS / 2) {
@@ -826,7 +828,7 @@ bool prepare_gate_up(Q4Launch &L) {
         m.topk > ROUTER_MAX_TOPK || m.hidden < 64 || (m.hidden & 63) || m.routed < 64 || (m.routed & 63))
         return false;
     L.table = nullptr; L.njobs = 1; L.cols = m.hidden; L.tokens = 1;
-    L.total_tiles = 2 * m.topk * ((m.routed + TILE_ROWS - 1) / TILE_ROWS);
+    L.total_tiles = gate_up_tiles(m);
     return true;
 }
 }  // namespace
@@ -835,7 +837,7 @@ int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream) {
     Q4Launch L = launch;
     if (!prepare_gate_up(L)) return -1;
     // one more workgroup, the first, publishes the router's outputs
-    return launch_one<1>(L, gate_up_shape(L.moe, L.total_tiles), 1, stream);
+    return launch_one<1>(L, gate_up_shape(L.moe), 1, stream);
 }
 
 namespace {
@@ -876,7 +878,11 @@ bool prepare_down(Q4Launch &L) {
 int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream) {
     Q4Launch L = launch;
     if (!prepare_down(L)) return -1;
-    return launch_one<2>(L, down_shape(L.moe), 0, stream);
+    const TileShape up = gate_up_shape(L.moe), down = down_shape(L.moe);
+    if (L.moe.arrivals)                         // a step by itself; in a block on two streams the dense branch's name stays
+        note_kernel("q4_tile_kernel<%d,1,%d,1,%d> + q4_tile_kernel<%d,1,%d,2,%d>", up.chains, up.blocks, up.split, down.chains,
+                    down.blocks, down.split);
+    return launch_one<2>(L, down, 0, stream);
 }
 
 int q4_activated_launch(const Q4Launch &L, hipStream_t stream) {
@@ -951,7 +957,9 @@ int q4_ffn_down_launch(const Q4Launch &launch, const Q4Launch &dense, hipStream_
     if (!prepare_down(moe) || dense.total_tiles < 1 || dense.tokens != 1 || dense.cols < 64 || (dense.cols & 63) ||
         dense.cols > MOE_FUSE_MAX_ROUTED)
         return -1;
-    const TileShape shape = down_shape(moe.moe);
+    const TileShape shape = down_shape(moe.moe), up = gate_up_shape(moe.moe);
+    note_kernel("ffn_gate_kernel + q4_tile_kernel<%d,1,%d,1,%d> + ffn_down_kernel<%d,%d,%d>", up.chains, up.blocks, up.split,
+                shape.chains, shape.blocks, shape.split);
     switch (shape_key(shape.chains, shape.blocks, shape.split)) {
         case shape_key(1, 32, 4): return launch_downs<1, 32, 4>(moe, dense, stream);
         case shape_key(2, 32, 2): return launch_downs<2, 32, 2>(moe, dense, stream);

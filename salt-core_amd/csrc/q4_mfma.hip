@@ -820,11 +820,14 @@ int q4_mfma_launch(const MfmaLaunch &launch, hipStream_t stream) {
         L.wide_tiles = L.wide_blocks * row_tiles;
         L.narrow_tiles = L.narrow_blocks * row_tiles;
         turns = (L.wide_tiles + 7) / 8 + (L.narrow_tiles + 7) / 8;
-        note_kernel("q4_mfma_kernel, tiles of %d tokens", work <= CUS ? TM / 2 : TM);
+        if (L.wide_blocks && L.narrow_blocks)
+            note_kernel("q4_mfma_kernel, %d blocks of %d tokens and %d of %d", L.wide_blocks, TM, L.narrow_blocks, TM / 2);
+        else
+            note_kernel("q4_mfma_kernel, tiles of %d tokens", L.wide_blocks ? TM : TM / 2);
     } else {
         if (L.most_tiles < 1 || L.row_tiles < 1 || !L.tile_jobs || !L.tiles_dev) return -1;
         turns = (L.most_tiles + 14) / 8;        // both runs, each rounded up
-        note_kernel("q4_mfma_kernel, tiles of %d tokens", TM);
+        note_kernel("q4_mfma_kernel, blocks of %d and of %d tokens by table", TM, TM / 2);
     }
     if (3 * (unsigned long long)L.plane_stride >= (1ull << 32)) return -1;      // 32-bit byte offsets inside a plane
     if (L.row_map && L.map_divisor < 1) return -1;

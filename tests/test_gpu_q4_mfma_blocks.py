@@ -12,19 +12,10 @@ from golden import cases
 from moe_bounds import group_term_magnitudes
 from oracle_lib import ExpertGeometry, host_threads, ptr
 from test_gpu_moe_prefill import check_values, expected_grouping
-from test_gpu_q4_mfma_shapes import check
+from test_gpu_q4_mfma_shapes import check, name_of
 
 pytestmark = pytest.mark.gpu
 synth = cases.synth
-
-
-def blocks(R, B):
-    """Blocks of 64 and of 32 tokens per 256 rows."""
-    halves, row_tiles = -(-B // 32), -(-R // 256)
-    work, wide = halves * row_tiles, halves // 2
-    if work <= 256: wide = 0
-    elif 512 < work <= 768 and work - 256 // row_tiles * row_tiles <= 512: wide = min(wide, 256 // row_tiles)
-    return wide, halves - 2 * wide
 
 
 @pytest.mark.parametrize("R,C_,B,form", [
@@ -40,10 +31,10 @@ def blocks(R, B):
 ])
 def test_mixed_blocks(pkg, oracle, R, C_, B, form):
     print(f"mfma blocks R={R} C={C_} B={B}", flush=True)
-    assert blocks(R, B) == form
     vals, scales, biases = synth.q4_tensor(R, C_, R + B)
     xs = synth.activations(C_, B, 31)
     got = pkg.lib.q4_matmul(vals, scales, biases, R, C_, xs).view(np.uint32)
+    assert pkg.lib.load().salt_mi355_last_kernel().decode() == name_of(*form)
     step = 32 * max(1, 256 // -(-R // 256))
     for first in range(0, B, step):
         piece = pkg.lib.q4_matmul(vals, scales, biases, R, C_, xs[first:first + step])

@@ -18,10 +18,24 @@ def tile_tokens(R, B):
     return 32 if -(-B // 32) * -(-R // 256) <= 256 else 64
 
 
+def blocks(R, B):
+    """Blocks of 64 and of 32 tokens per 256 rows."""
+    halves, row_tiles = -(-B // 32), -(-R // 256)
+    work, wide = halves * row_tiles, halves // 2
+    if tile_tokens(R, B) == 32: wide = 0
+    elif 512 < work <= 768 and work - 256 // row_tiles * row_tiles <= 512: wide = min(wide, 256 // row_tiles)
+    return wide, halves - 2 * wide
+
+
+def name_of(wide, narrow):
+    """What a launch of so many blocks reports."""
+    if wide and narrow: return f"q4_mfma_kernel, {wide} blocks of 64 tokens and {narrow} of 32"
+    return f"q4_mfma_kernel, tiles of {64 if wide else 32} tokens"
+
+
 def matmul(pkg, vals, scales, biases, R, C, xs):
     got = pkg.lib.q4_matmul(vals, scales, biases, R, C, xs)
-    form = f"q4_mfma_kernel, tiles of {tile_tokens(R, xs.shape[0])} tokens"
-    assert pkg.lib.load().salt_mi355_last_kernel().decode() == form
+    assert pkg.lib.load().salt_mi355_last_kernel().decode() == name_of(*blocks(R, xs.shape[0]))
     return got
 
 

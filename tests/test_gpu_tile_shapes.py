@@ -63,20 +63,20 @@ def test_every_open_shape(pkg, oracle, rows, C, tokens, kernel):
         assert np.array_equal(bits(bufs[4].to_host(np.float32).reshape(y.shape)), bits(y))
 
 
-@pytest.mark.parametrize("E,K,H,F", [
-    (16, 1, 1088, 576),          # gate/up 18 tiles: halves; down 17: quarters
-    (32, 2, 2112, 1024),         # 64: quarters with one chain; 66: halves
-    (32, 3, 1984, 704),          # 66: halves; 93: halves
-    (16, 8, 1280, 640),          # 160: quarters; 160: whole
-    (16, 8, 1024, 640),          # 160 of narrow rows: halves; 128: halves
-    (20, 6, 1920, 1216),         # 228: halves with four chains; 180: whole
-    (24, 8, 2112, 1344),         # 336: halves with four chains; 264: whole with four
-    (16, 1, 4160, 64),           # counters of halves do not fit: whole tiles
-    (300, 8, 1280, 640),         # a router of more than 256 experts: no workgroups of 256 threads
-    (300, 8, 512, 1152),
-    (16, 1, 8256, 128),          # too wide a row for parts
+@pytest.mark.parametrize("E,K,H,F,gate_up,down", [
+    (16, 1, 1088, 576, "2,1,32,1,2", "1,1,32,2,4"),      # gate/up 18 tiles: halves; down 17: quarters
+    (32, 2, 2112, 1024, "1,1,32,1,4", "2,1,32,2,2"),     # 64: quarters with one chain; 66: halves
+    (32, 3, 1984, 704, "2,1,32,1,2", "2,1,32,2,2"),      # 66: halves; 93: halves
+    (16, 8, 1280, 640, "2,1,16,1,4", "2,1,32,2,1"),      # 160: quarters; 160: whole
+    (16, 8, 1024, 640, "2,1,16,1,2", "2,1,32,2,2"),      # 160 of narrow rows: halves; 128: halves
+    (20, 6, 1920, 1216, "4,1,16,1,2", "2,1,32,2,1"),     # 228: halves with four chains; 180: whole
+    (24, 8, 2112, 1344, "4,1,16,1,2", "4,1,16,2,1"),     # 336: halves with four chains; 264: whole with four
+    (16, 1, 4160, 64, "1,1,32,1,4", "2,1,32,2,1"),       # counters of halves do not fit: whole tiles
+    (300, 8, 1280, 640, "2,1,16,1,2", "2,1,32,2,1"),     # a router of more than 256 experts: no workgroups of 256 threads
+    (300, 8, 512, 1152, "4,1,16,1,1", "1,1,32,2,4"),
+    (16, 1, 8256, 128, "2,1,32,1,1", "2,1,32,2,1"),      # too wide a row for parts
 ])
-def test_moe_step_in_parts(pkg, oracle, E, K, H, F):
+def test_moe_step_in_parts(pkg, oracle, E, K, H, F, gate_up, down):
     print(f"moe parts E={E} K={K} H={H} F={F}", flush=True)
     pool = synth.expert_pool(E, H, F, 1)
     logits, scale = synth.router_logits(E, 2), np.linspace(0.5, 2.0, E).astype(np.float32)
@@ -84,6 +84,7 @@ def test_moe_step_in_parts(pkg, oracle, E, K, H, F):
     for seed in (3, 4, 5):                       # the counters start from zero in every step
         x = synth.activations(H, 1, seed)[0]
         status, sel, w, eo, y = layer.step(logits, scale, x)
+        assert pkg.lib.load().salt_mi355_last_kernel().decode() == f"q4_tile_kernel<{gate_up}> + q4_tile_kernel<{down}>"
         osel, ow, oeo, oy = np.zeros(K, np.int32), np.zeros(K, np.float32), np.zeros((K, H), np.float32), np.zeros(H, np.float32)
         assert oracle.orc_moe_decode_step(ct.byref(ExpertGeometry(H, F)), ptr(pool), E, K, ptr(logits), ptr(scale), ptr(x),
                                           ptr(osel), ptr(ow), ptr(oeo), ptr(oy), 2) == 0
