@@ -7,12 +7,14 @@
 // expert's position is its rank: the number of larger logits plus the number
 // of equal logits with a smaller index.  Ranks are computed in parallel; the
 // two fp32 sums whose order the reference fixes (over all experts ascending,
-// over the selected experts in list order) are done by one lane, in order.
+// over the selected experts in list order) are done by one wave, in order.
 #pragma once
 
 #include "device_math.h"
 
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 namespace mi355 {
 
@@ -20,7 +22,7 @@ constexpr int ROUTER_MAX_EXPERTS = 1024;
 constexpr int ROUTER_MAX_TOPK = 64;
 
 struct RouterShared {
-    float logit[ROUTER_MAX_EXPERTS];
+    __attribute__((aligned(16))) float logit[ROUTER_MAX_EXPERTS];       // up to the next multiple of 64 behind the last: -inf
     float expv[ROUTER_MAX_EXPERTS];
     float wave_max[ROUTER_MAX_EXPERTS / 64];
     int rank[ROUTER_MAX_EXPERTS];
@@ -51,8 +53,9 @@ __device__ __forceinline__ void router_topk_block(const float *__restrict__ logi
         mine = logits[e];
         const float sc = per_expert_scale[e];
         if (!(__builtin_fabsf(mine) < __builtin_inff()) || !(__builtin_fabsf(sc) < __builtin_inff())) sh.bad = 1;
-        sh.logit[e] = mine;
     }
+    const int padded = (n_experts + 63) & ~63;
+    if (e < padded) sh.logit[e] = mine;
     // max over finite values is exact in any order
     float m = mine;
 #pragma unroll
@@ -70,21 +73,44 @@ __device__ __forceinline__ void router_topk_block(const float *__restrict__ logi
     const float peak = sh.peak;
     // Ranks: the comparisons of one expert are spread over as many threads as
     // the workgroup has to spare (integer counts, so the split changes nothing).
-    const int padded = (n_experts + 63) & ~63;
+    // A thread compares sixteen logits per wait for LDS, with one instruction for
+    // the ones that lie wholly before or behind its wave's own.  Bound: the ordered
+    // sum, one dependent addition per expert.  As a launch of its own, 128 experts,
+    // top-8: 6.4 us (11.8 with a wait for every logit and the weights' divisions in
+    // one lane), 512: 13.7 (35.8), 16: 4.4 (4.6).  It matters most where 256 threads
+    // publish for a launch of many short workgroups, and beyond 256 experts, where
+    // every workgroup of the exact step runs it.
     const int parts = (int)blockDim.x / padded > 0 ? (int)blockDim.x / padded : 1;
     if (live) sh.rank[e] = 0;
     __syncthreads();
-    if (!bad && e < padded * parts) {
-        const int who = e % padded, part = e / padded;
+    // a wave's 64 experts, the same part of the others for all of them: whole batches lie before, behind or among its own
+    const int base = __builtin_amdgcn_readfirstlane(e & ~63), part = base / padded, own = base % padded;
+    if (!bad && base < padded * parts) {
+        const int who = own + (e & 63);
         if (who < n_experts) {
             const float self = sh.logit[who];
-            const int span = (n_experts + parts - 1) / parts;
-            const int first = part * span, last = first + span < n_experts ? first + span : n_experts;
+            const int all = (n_experts + 3) & ~3, span = ((all + parts - 1) / parts + 3) & ~3;
+            const int first = part * span, last = first + span < all ? first + span : all;
             int count = 0;
-            for (int j = first; j < last; ++j) {
-                const float other = sh.logit[j];
-                count += (other > self) || (other == self && j < who);
-            }
+            auto batch = [&](int j, auto size) {
+                constexpr int N = decltype(size)::value;
+                float other[N];
+#pragma unroll
+                for (int k = 0; k < N; k += 4) *(float4 *)&other[k] = *(const float4 *)&sh.logit[j + k];
+                if (j + N <= own) {
+#pragma unroll
+                    for (int k = 0; k < N; ++k) count += other[k] >= self;
+                } else if (j >= own + 64) {
+#pragma unroll
+                    for (int k = 0; k < N; ++k) count += other[k] > self;
+                } else {
+#pragma unroll
+                    for (int k = 0; k < N; ++k) count += (int)(other[k] > self) | ((int)(other[k] == self) & (int)(j + k < who));
+                }
+            };
+            int j = first;
+            for (; j + 16 <= last; j += 16) batch(j, std::integral_constant<int, 16>{});
+            for (; j < last; j += 4) batch(j, std::integral_constant<int, 4>{});
             if (parts > 1) atomicAdd(&sh.rank[who], count); else sh.rank[who] = count;
         }
     }
@@ -94,7 +120,10 @@ __device__ __forceinline__ void router_topk_block(const float *__restrict__ logi
         if (sh.rank[e] < topk) sh.sel[sh.rank[e]] = e;
     }
     __syncthreads();
-    if (want_weights && e == 0 && !bad) {
+    if (want_weights && e < 64 && !bad) {       // one wave: the sums in order, a lane per chosen expert
+        const bool mine_chosen = e < topk;
+        const int expert = mine_chosen ? sh.sel[e] : 0;
+        const float scale = per_expert_scale[expert], value = sh.expv[expert];
         float all = 0.0f;
         int j0 = 0;
         for (; j0 + 16 <= n_experts; j0 += 16) {       // batches of LDS reads, then the ordered adds
@@ -106,20 +135,13 @@ __device__ __forceinline__ void router_topk_block(const float *__restrict__ logi
         }
         for (int j = j0; j < n_experts; ++j) all = all + sh.expv[j];
         if (!(all > 0.0f) || !(all < __builtin_inff())) bad = 1;
+        const float w = value / all;
         float chosen = 0.0f;
-        if (!bad) {
-            for (int j = 0; j < topk; ++j) {
-                sh.w[j] = sh.expv[sh.sel[j]] / all;
-                chosen = chosen + sh.w[j];
-            }
-            if (!(chosen > 0.0f) || !(chosen < __builtin_inff())) bad = 1;
-        }
-        if (!bad)
-            for (int j = 0; j < topk; ++j) {
-                const float share = sh.w[j] / chosen;
-                sh.w[j] = share * per_expert_scale[sh.sel[j]];
-            }
-        sh.bad = bad;
+        for (int j = 0; j < topk; ++j) chosen = chosen + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
+        if (!(chosen > 0.0f) || !(chosen < __builtin_inff())) bad = 1;
+        const float share = w / chosen;
+        if (mine_chosen) sh.w[e] = share * scale;
+        if (e == 0) sh.bad = bad;
     }
     __syncthreads();
     bad = sh.bad;
