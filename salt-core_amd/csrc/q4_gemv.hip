@@ -796,28 +796,33 @@ int q4_uniform_tiles(const Q4Job *table, int njobs) {
 }
 
 namespace {
-// Every wave of the MoE step's gate/up launch first finds its expert, so that more and shorter workgroups cost more than in
-// a plain launch.  us per decode step, whole / halves <2> / quarters <2> or halves <4>: 40 tiles of 2048 columns 17.2 / 14.1
-// (quarters <1> 14.0), 64 of 2048 16.9 / 14.1 (14.7), 64 of 2816 20.3 / 16.1 (15.1), 120 of 2816 21.2 / 17.2; 144 of 1600
-// 18.5 / 18.2 / quarters 18.9; 176 of 1024 17.0 / 16.7 / quarters 18.8, of 1536 17.5 / 17.2 / 16.5, of 2816 24.3 / 22.7 /
-// 21.4; 192 of 2816 (four quarters a compute unit, with the publisher) 23.5 / 21.9 / 23.4; 256 of 1024 21.1 / 18.8 / halves
-// <4> 16.3, of 2048 24.9 / 23.0 / 19.9, 208 of 2816 24.0 / 22.5 / 22.7.
 int gate_up_tiles(const MoeFuse &m) { return 2 * m.topk * ((m.routed + TILE_ROWS - 1) / TILE_ROWS); }
+
+// Every wave of the MoE step's gate/up launch first finds its expert, and workgroup 0 publishes the router's outputs with as
+// many threads as the others have, so that more and shorter workgroups cost more than in a plain launch.  us per decode step
+// with 16 / 128 / 256 experts:
+//   tiles      columns    halves <2>          quarters <1>        quarters <2>         halves <4>
+//   44 - 64    1536       13.4 / 13.8         12.5 / 14.0
+//              2048       14.1 / 14.1 / 15.7  13.4 / 13.6 / 15.9
+//              2816       16.1 / 16.3 / 17.4  15.1 / 15.3 / 16.8
+//   112 - 128  2816       17.0 / 18.2 / 20.4  17.3 / 18.6 / 20.9  17.3 / 18.3 / 20.1
+//   140        1024       14.9 / 15.6 / 17.3                      14.1 / 15.9 / 18.4   14.4 / 15.7 / 18.3
+//              2816       20.7 / 21.7 / 23.0                      19.7 / 20.7 / 22.0   20.7 / 21.6 / 22.6
+//   176        1024       15.7 / 16.3 / 18.1                      15.3 / 16.1 / 18.7   15.0 / 15.9 / 18.5
+//              2816       22.1 / 23.1 / 24.6                      21.3 / 21.5 / 24.2   22.0 / 23.1 / 24.2
+//   192        2816       21.9 / 22.6 / 24.9                      23.2 / 25.4 / 28.8   21.8 / 22.6 / 24.6
+//   256        2816       25.1 / 26.4 / 31.1                      28.0 / 29.0 / 31.3   23.7 / 24.7 / 26.6
+// (192 tiles in quarters are four workgroups for some compute unit, the publisher being one more.)  A router of more than 256
+// experts takes a thread per expert and is run by every workgroup: 257 and 512 experts, 2816 columns, us in halves <2> / whole
+// <2> / whole <4>: 176 tiles 29.2, 33.8 / 27.9, 30.6 / 30.5, 31.8; 256 tiles 38.1, 44.2 / 35.6, 42.3 / 32.1, 35.3.
 TileShape gate_up_shape(const MoeFuse &m) {
     const int tiles = gate_up_tiles(m);
-    TileShape shape = open_shape(tiles, m.hidden, 1);
-    if (shape.split > 1 && tiles <= COMPUTE_UNITS) {
-        if (tiles <= COMPUTE_UNITS / 2) {
-            if (shape.chains == 2 || shape.split == 8 || m.hidden <= 2048) shape = {2, 32, 2};
-        } else if (tiles <= COMPUTE_UNITS * 3 / 4) {
-            if (tiles <= COMPUTE_UNITS * 3 / 5 || 4 * tiles + 1 > 3 * COMPUTE_UNITS || m.hidden < 1280) shape = {2, 16, 2};
-        } else {
-            shape = {4, 16, 2};
-        }
-    }
-    if (shape.threads() >= m.n_experts) return shape;            // the router wants a thread per expert
-    if (tiles > COMPUTE_UNITS) return whole_shape(4, tiles, 1);
-    return {2, tiles <= COMPUTE_UNITS / 2 ? 32 : 16, 2};         // open_shape gave parts: the row fits in LDS
+    const TileShape shape = open_shape(tiles, m.hidden, 1);
+    if (shape.split == 1) return shape;
+    if (tiles <= COMPUTE_UNITS / 2) return shape.chains == 2 || shape.split == 8 || m.hidden < 2048 ? TileShape{2, 32, 2} : shape;
+    const bool few = 4 * tiles + 1 <= 3 * COMPUTE_UNITS;
+    if (m.n_experts > ROUTER_WAVE_MAX_EXPERTS) return few ? TileShape{2, 32, 1} : TileShape{4, 16, 1};
+    return few ? TileShape{2, 16, 4} : TileShape{4, 16, 2};
 }
 }  // namespace
 

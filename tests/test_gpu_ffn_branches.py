@@ -26,10 +26,10 @@ SECOND_STREAM = "q4_tile_kernel<2,1,32,0>"          # the dense down projection 
     (1088, 1024, 576, 16, 1, together("2,1,32,1,2", "1,32,4")),         # 18 tiles: halves; down 17: quarters, one chain per lane
     (2112, 1216, 1024, 32, 2, together("1,1,32,1,4", "2,32,2")),        # 64: quarters, one chain per lane
     (1280, 4096, 640, 16, 8, together("2,1,16,1,4", "2,32,1")),         # 160: quarters; the widest dense branch; down 160: whole
-    (1024, 128, 640, 16, 8, together("2,1,16,1,2", "2,32,2")),          # 160 of narrow rows: halves; down 128: halves
+    (1024, 128, 640, 16, 8, together("2,1,16,1,4", "2,32,2")),          # 160; down 128: halves
     (1920, 704, 1216, 20, 6, together("4,1,16,1,2", "2,32,1")),         # 228: halves, four chains
     (512, 320, 1600, 24, 8, together("4,1,16,1,1", "1,32,4")),          # 400: whole tiles, four chains
-    (512, 192, 640, 300, 8, together("2,1,16,1,2", "1,32,4")),          # more than 256 experts
+    (512, 192, 640, 300, 8, together("2,1,32,1,1", "1,32,4")),          # more than 256 experts: whole
     (4096, 192, 64, 8, 2, together("1,1,32,1,4", "2,32,2")),            # the widest gate
     (256, 4160, 128, 16, 4, SECOND_STREAM),                             # a dense branch too wide
     (4160, 192, 64, 8, 2, SECOND_STREAM),                               # a gate too wide

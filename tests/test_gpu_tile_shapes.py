@@ -68,12 +68,19 @@ def test_every_open_shape(pkg, oracle, rows, C, tokens, kernel):
     (32, 2, 2112, 1024, "1,1,32,1,4", "2,1,32,2,2"),     # 64: quarters with one chain; 66: halves
     (32, 3, 1984, 704, "2,1,32,1,2", "2,1,32,2,2"),      # 66: halves; 93: halves
     (16, 8, 1280, 640, "2,1,16,1,4", "2,1,32,2,1"),      # 160: quarters; 160: whole
-    (16, 8, 1024, 640, "2,1,16,1,2", "2,1,32,2,2"),      # 160 of narrow rows: halves; 128: halves
+    (16, 8, 1024, 640, "2,1,16,1,4", "2,1,32,2,2"),      # 160; 128: halves
+    (16, 2, 1984, 704, "2,1,32,1,2", "1,1,32,2,4"),      # 44 tiles of rows just too narrow for one chain per lane
+    (16, 2, 2048, 704, "1,1,32,1,4", "1,1,32,2,4"),
+    (256, 8, 128, 704, "2,1,16,1,4", "1,1,32,2,4"),      # as many experts as threads; 176 tiles
+    (16, 6, 256, 1024, "4,1,16,1,2", "1,1,32,2,4"),      # 192: four quarters and the publisher would be one too many
     (20, 6, 1920, 1216, "4,1,16,1,2", "2,1,32,2,1"),     # 228: halves with four chains; 180: whole
     (24, 8, 2112, 1344, "4,1,16,1,2", "4,1,16,2,1"),     # 336: halves with four chains; 264: whole with four
     (16, 1, 4160, 64, "1,1,32,1,4", "2,1,32,2,1"),       # counters of halves do not fit: whole tiles
-    (300, 8, 1280, 640, "2,1,16,1,2", "2,1,32,2,1"),     # a router of more than 256 experts: no workgroups of 256 threads
-    (300, 8, 512, 1152, "4,1,16,1,1", "1,1,32,2,4"),
+    (300, 3, 1984, 704, "2,1,32,1,2", "2,1,32,2,2"),     # a router of more than 256 experts: no workgroups of 256 threads
+    (300, 8, 1280, 640, "2,1,32,1,1", "2,1,32,2,1"),
+    (300, 6, 256, 1024, "4,1,16,1,1", "1,1,32,2,4"),     # 192 tiles
+    (512, 8, 128, 1024, "4,1,16,1,1", "1,1,32,2,4"),     # 256
+    (300, 8, 512, 1152, "4,1,16,1,1", "1,1,32,2,4"),     # 288
     (16, 1, 8256, 128, "2,1,32,1,1", "2,1,32,2,1"),      # too wide a row for parts
 ])
 def test_moe_step_in_parts(pkg, oracle, E, K, H, F, gate_up, down):
