@@ -688,9 +688,11 @@ constexpr int COMPUTE_UNITS = 256;
 // Whole tiles: up to one per compute unit, sixteen waves per tile (two chains per lane) hide more of the LDS and
 // scalar-load latency, and a single token's workgroup, alone on its compute unit, stages twice as much per step; beyond
 // that four chains per lane win (one token, 2816 columns: 10.4 against 10.8 us at 256 tiles, 14.2 against 20.3 at 264;
-// eight chains per lane never do).
+// eight chains per lane never do).  Four chains per lane do not gain from the longer steps, which leave too few scalar
+// registers (one token, 128 tiles of 2816 / 8192 columns: 10.4 / 28.5 us in steps of sixteen blocks, 13.2 / 46.4 in steps of
+// thirty-two with all activations of half a step in registers, 10.3 / 33.4 with an eighth).
 TileShape whole_shape(int chains, int tiles, int tokens) {
-    return {chains, tokens == 1 && chains <= 4 && tiles <= COMPUTE_UNITS ? 32 : 16, 1};
+    return {chains, tokens == 1 && chains == 2 && tiles <= COMPUTE_UNITS ? 32 : 16, 1};
 }
 
 // The shape of a launch whose caller leaves it open.  A compute unit's time follows the rows of the fullest one, so parts
@@ -752,7 +754,6 @@ int launch_one(const Q4Launch &L, const TileShape &shape, int extra, hipStream_t
     }
     if (PRO == 0) switch (shape_key(shape.chains, shape.blocks, shape.split)) {         // as the caller asked
         case shape_key(2, 16, 1): return launch_as<2, 1, 16, 0, 1>(L, extra, stream);
-        case shape_key(4, 32, 1): return launch_as<4, 1, 32, 0, 1>(L, extra, stream);
         case shape_key(8, 16, 1): return launch_as<8, 1, 16, 0, 1>(L, extra, stream);
     }
     return -1;

@@ -37,9 +37,21 @@ SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("rows,C,tokens,kernel", [(r, c, t, k) for r, c, ts, k in SHAPES for t in ts])
-def test_every_open_shape(pkg, oracle, rows, C, tokens, kernel):
-    print(f"q4 shape {kernel} rows={rows} C={C} tokens={tokens}", flush=True)
+# the same where the caller states the chains per lane: whole tiles
+STATED = [
+    ((70, 1, 1033, 333), 1088, (1,), 4, "q4_tile_kernel<4,1,16,0>"),                     # 25 tiles
+    ((16384,), 64, (1,), 4, "q4_tile_kernel<4,1,16,0>"),                                 # 256
+    ((16385,), 64, (1, 2, 3, 4), 4, "q4_tile_kernel<4,{},16,0>"),
+    ((70, 1033), 1088, (1,), 2, "q4_tile_kernel<2,1,32,0>"),
+    ((16385,), 64, (1, 2, 3, 4), 2, "q4_tile_kernel<2,{},16,0>"),
+    ((70, 1033), 1088, (1, 2, 3, 4), 8, "q4_tile_kernel<8,{},16,0>"),
+]
+
+
+@pytest.mark.parametrize("rows,C,tokens,chains,kernel", [(r, c, t, 0, k) for r, c, ts, k in SHAPES for t in ts] +
+                         [(r, c, t, n, k) for r, c, ts, n, k in STATED for t in ts])
+def test_every_shape(pkg, oracle, rows, C, tokens, chains, kernel):
+    print(f"q4 shape {kernel} rows={rows} C={C} tokens={tokens} chains={chains}", flush=True)
     lib = pkg.lib.init()
     stream = lib.salt_mi355_stream()
     hold, jobs, want = [], (pkg.lib.Q4Job * len(rows))(), []
@@ -56,7 +68,7 @@ def test_every_open_shape(pkg, oracle, rows, C, tokens, kernel):
         jobs[j] = pkg.lib.Q4Job(*[b.ptr for b in bufs], R)
         hold.append(bufs)
         want.append(y)
-    pkg.lib.check(lib.salt_mi355_q4_jobs_dev(jobs, len(rows), C, tokens, 0, stream), "q4_jobs_dev")
+    pkg.lib.check(lib.salt_mi355_q4_jobs_dev(jobs, len(rows), C, tokens, chains, stream), "q4_jobs_dev")
     pkg.lib.check(lib.salt_mi355_stream_sync(stream), "sync")
     assert lib.salt_mi355_last_kernel().decode() == kernel.format(tokens)
     for bufs, y in zip(hold, want):
