@@ -128,7 +128,8 @@ __device__ __forceinline__ float add_staged(const float *mine, int count, float 
 // vector instructions issue eight clocks apart, 3.6 ns, independent ones four, which is what counts here).  The
 // feed-forward block of 2816/2112/704 with 128 experts, three such sums deep: 90.1 -> 63.8 us (57.5 since its branches
 // share their launches); its first cell 13.5 -> 6.2 us, its last 30.6 -> 11.2.
-constexpr int ORDERED_MIN = 512;      // below, the chain is as quick
+constexpr int ORDERED_MIN = 736;      // below, the chain is quicker (a norm of 512 / 704 / 736 / 768 values 5.2 / 5.85 / 5.86 / 6.0 us,
+                                      // 5.8 to 5.9 with ordered_sum)
 constexpr int PARTS = 4;              // of a lane
 constexpr int ORDERED_FLOATS = 64 * (SQ_CHUNK / 64 + 4);     // LDS of SQ_CHUNK addends; a lane's block is 4 floats apart
                                                              // from the next, so that 16-byte reads hit all banks
@@ -311,16 +312,18 @@ template <int V> struct SumScratch {
 };
 static_assert(ORDERED_FLOATS >= SQ_CHUNK && ORDERED_MIN <= SQ_CHUNK, "both layouts fit");
 
-// Sums of at most SQ_CHUNK staged squares: place(i) is where the square of element i of a vector of ORDERED_FLOATS goes;
-// add(v, acc) is called by the whole wave v.
-struct Staged {
+// Sums of at most SQ_CHUNK staged squares: place(i) is where the square of element i of a vector of ORDERED_FLOATS goes, and
+// zeros follow up to end(), which add nothing to a sum that is never negative; add(v, acc) is called by the whole wave v.
+// LONG: whether a vector of ORDERED_MIN elements and more can come.  A kernel for shorter ones does not carry the code of
+// ordered_sum (one norm of 64 values 3.8 us with it, 3.5 without).
+template <bool LONG> struct Staged {
     int count, words;
     bool chain;
-    __device__ explicit Staged(int n) : count(n), words(part_words(n)), chain(n < ORDERED_MIN) {}
-    __device__ int end() const { return chain ? count : 1024 * words; }
+    __device__ explicit Staged(int n) : count(n), words(part_words(n)), chain(!LONG || n < ORDERED_MIN) {}
+    __device__ int end() const { return chain ? (count + 31) & ~31 : 1024 * words; }
     __device__ int place(int i) const { return chain ? i : ordered_place(i, words); }
     __device__ __forceinline__ float add(const float *sq, float acc, OrderedScratch &scratch) const {
-        if (chain) return add_staged(sq, count, acc);
+        if (chain) return add_staged(sq, end(), acc);
         switch (words) {
         case 1: return ordered_sum<1>(sq, acc, scratch);
         case 2: return ordered_sum<2>(sq, acc, scratch);
@@ -330,20 +333,21 @@ struct Staged {
     }
 };
 
-// The sums of squares of `vectors` (at most V) vectors of at most SQ_CHUNK elements, a multiple of SLOTS, that the
-// threads already hold: val[v][k] is element SLOTS * tid + k of vector v (any value past the end).
-template <int V>
+// The sums of squares of `vectors` (at most V) vectors of at most SQ_CHUNK elements that the threads already hold: val[v][k]
+// is element SLOTS * tid + k of vector v (any value past the end).  RAGGED: n need not be a multiple of SLOTS.
+template <int V, bool RAGGED>
 __device__ __forceinline__ void chains_from_registers(const float (&val)[V][SLOTS], int vectors, int n,
                                                       SumScratch<V> &scratch, float (&ss)[V]) {
     static_assert(SLOTS == 4, "a thread's elements are 16 bytes");
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = SLOTS * tid;
-    const Staged staged(n);
+    const Staged<true> staged(n);
     if (i < staged.end())
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-            const float4 square = make_float4(val[v][0] * val[v][0], val[v][1] * val[v][1], val[v][2] * val[v][2],
-                                              val[v][3] * val[v][3]);
-            *(float4 *)&scratch.sq[v * ORDERED_FLOATS + staged.place(i)] = i < n ? square : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            float square[SLOTS];
+#pragma unroll
+            for (int k = 0; k < SLOTS; ++k) square[k] = (RAGGED ? i + k : i) < n ? val[v][k] * val[v][k] : 0.0f;
+            *(float4 *)&scratch.sq[v * ORDERED_FLOATS + staged.place(i)] = make_float4(square[0], square[1], square[2], square[3]);
         }
     __syncthreads();
     if (wave < vectors) {
@@ -355,25 +359,37 @@ __device__ __forceinline__ void chains_from_registers(const float (&val)[V][SLOT
     for (int v = 0; v < V; ++v) ss[v] = scratch.ss[v];
 }
 
-// SLOTS consecutive floats on any four-byte boundary
+// A thread's elements i .. i + SLOTS - 1 of n, on any four-byte boundary; past the end the last elements again (n a multiple
+// of SLOTS) or the last one (RAGGED, where the threads at the end ask for one at a time)
 typedef float any_float4 __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ void load_slots(const float *from, float (&to)[SLOTS]) {
-    const any_float4 v = *(const any_float4 *)from;
-    to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
+template <bool RAGGED> __device__ __forceinline__ void load_slots(const float *from, int i, int n, float (&to)[SLOTS]) {
+    if (RAGGED && i + SLOTS > n) {
+#pragma unroll
+        for (int k = 0; k < SLOTS; ++k) to[k] = from[i + k < n ? i + k : n - 1];
+    } else {
+        const any_float4 v = *(const any_float4 *)(from + (RAGGED || i < n ? i : n - SLOTS));
+        to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
+    }
 }
-__device__ __forceinline__ void store_slots(float *to, const float (&from)[SLOTS]) {
-    *(any_float4 *)to = any_float4{from[0], from[1], from[2], from[3]};
+template <bool RAGGED> __device__ __forceinline__ void store_slots(float *to, int i, int n, const float (&from)[SLOTS]) {
+    if (RAGGED && i + SLOTS > n) {
+#pragma unroll
+        for (int k = 0; k < SLOTS; ++k)
+            if (i + k < n) to[i + k] = from[k];
+    } else if (i < n) {
+        *(any_float4 *)(to + i) = any_float4{from[0], from[1], from[2], from[3]};
+    }
 }
 
 // Serial sums of squares of V vectors of n floats: wave v adds vector v's squares left to right.  Returns the sums in
 // ss_out[] on every thread; `bad` collects non-finite elements.
-template <int V>
+template <int V, bool LONG>
 __device__ __forceinline__ void serial_square_sums(const float *const (&x)[V], int n, SumScratch<V> &scratch, float (&ss_out)[V],
                                    unsigned &bad) {
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     float acc = 0.0f;
     for (int base = 0; base < n; base += SQ_CHUNK) {
-        const Staged staged(n - base < SQ_CHUNK ? n - base : SQ_CHUNK);
+        const Staged<LONG> staged(n - base < SQ_CHUNK ? n - base : SQ_CHUNK);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             const float *src = x[v] + base;
@@ -412,13 +428,13 @@ struct NormArgs {
     int *status;
 };
 
-__global__ __launch_bounds__(THREADS) void norm_cell_kernel(NormArgs a) {
+template <bool LONG> __global__ __launch_bounds__(THREADS) void norm_cell_kernel(NormArgs a) {
     __shared__ SumScratch<1> scratch;
     if (*a.status != 0) return;
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps);
     const float *const vec[1] = {a.x};
     float ss[1];
-    serial_square_sums<1>(vec, a.n, scratch, ss, bad);
+    serial_square_sums<1, LONG>(vec, a.n, scratch, ss, bad);
     const float inv = inverse_from_sum(ss[0], a.n, a.eps);
     bad |= nonfinite(inv);
     float root = a.root;
@@ -459,16 +475,16 @@ struct PreArgs {
 __global__ __launch_bounds__(THREADS) void ffn_pre_small_kernel(PreArgs a) {
     __shared__ SumScratch<1> scratch;
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps);
-    const int i = SLOTS * (int)threadIdx.x, at = i < a.n ? i : a.n - SLOTS;       // past the end the last elements again
+    const int i = SLOTS * (int)threadIdx.x;
     float r[1][SLOTS], w1[SLOTS], w2[SLOTS], rs[SLOTS];
-    load_slots(a.residual + at, r[0]);
-    load_slots(a.w1 + at, w1);
-    load_slots(a.w2 + at, w2);
-    load_slots(a.router_scale + at, rs);
+    load_slots<false>(a.residual, i, a.n, r[0]);
+    load_slots<false>(a.w1, i, a.n, w1);
+    load_slots<false>(a.w2, i, a.n, w2);
+    load_slots<false>(a.router_scale, i, a.n, rs);
 #pragma unroll
     for (int k = 0; k < SLOTS; ++k) bad |= nonfinite(r[0][k]) | nonfinite(w1[k]) | nonfinite(w2[k]) | nonfinite(rs[k]);
     float ss[1];
-    chains_from_registers<1>(r, 1, a.n, scratch, ss);
+    chains_from_registers<1, false>(r, 1, a.n, scratch, ss);
     const float inv = inverse_from_sum(ss[0], a.n, a.eps);
     bad |= nonfinite(inv);
     const float root = 1.0f / det_sqrtf((float)a.n);
@@ -483,10 +499,10 @@ __global__ __launch_bounds__(THREADS) void ffn_pre_small_kernel(PreArgs a) {
     }
     const bool failed = __syncthreads_or((int)bad);
     if (threadIdx.x == 0) *a.status = failed ? -1 : 0;
-    if (failed || i >= a.n) return;
-    store_slots(a.norm_a + i, na);
-    store_slots(a.norm_b + i, nb);
-    store_slots(a.router_in + i, ri);
+    if (failed) return;
+    store_slots<false>(a.norm_a, i, a.n, na);
+    store_slots<false>(a.norm_b, i, a.n, nb);
+    store_slots<false>(a.router_in, i, a.n, ri);
 }
 
 __global__ __launch_bounds__(THREADS) void ffn_pre_kernel(PreArgs a) {
@@ -494,7 +510,7 @@ __global__ __launch_bounds__(THREADS) void ffn_pre_kernel(PreArgs a) {
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps);
     const float *const vec[1] = {a.residual};
     float ss[1];
-    serial_square_sums<1>(vec, a.n, scratch, ss, bad);
+    serial_square_sums<1, true>(vec, a.n, scratch, ss, bad);
     const float inv = inverse_from_sum(ss[0], a.n, a.eps);
     bad |= nonfinite(inv);
     const float root = 1.0f / det_sqrtf((float)a.n);
@@ -528,19 +544,19 @@ struct CombineArgs {
     int topk;
 };
 
-// n <= SQ_CHUNK, a multiple of SLOTS: one load phase, everything else in registers and LDS; a thread has SLOTS consecutive
-// elements.  Bound by what one compute unit can fetch (six vectors and topk expert outputs, 158 KB at 2816 and eight, in
+// n <= SQ_CHUNK: one load phase, everything else in registers and LDS; a thread has SLOTS consecutive elements (RAGGED: n need not be
+// a multiple of them).  Bound by what one compute unit can fetch (six vectors and topk expert outputs, 158 KB at 2816 and eight, in
 // 2 us; a wait for each expert and four bytes per load took 7), then by the two rounds of sums, 3 us each.
-__global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
+template <bool RAGGED> __global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
     __shared__ SumScratch<2> scratch;
     unsigned bad = !(a.eps >= 0.0f) || nonfinite(a.eps) || nonfinite(a.scalar);
     // Every input is asked for before anything is waited for, the status words among them; the experts' outputs eight
     // at a time.
     const int status = *a.status, other = a.other ? *a.other : 0;
-    const int i = SLOTS * (int)threadIdx.x, at = i < a.n ? i : a.n - SLOTS;       // past the end the last elements again
+    const int i = SLOTS * (int)threadIdx.x;
     float dr[2][SLOTS], res[SLOTS], wd[SLOTS], wr[SLOTS], wf[SLOTS];
-    load_slots(a.dense + at, dr[0]);
-    if (!a.expert_out) load_slots(a.routed + at, dr[1]);
+    load_slots<RAGGED>(a.dense, i, a.n, dr[0]);
+    if (!a.expert_out) load_slots<RAGGED>(a.routed, i, a.n, dr[1]);
     else {
 #pragma unroll
         for (int k = 0; k < SLOTS; ++k) dr[1][k] = 0.0f;
@@ -550,7 +566,7 @@ __global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
             for (int e = 0; e < 8; ++e) {
                 if (e0 + e >= a.topk) break;
                 w[e] = a.weights[e0 + e];
-                load_slots(a.expert_out + (size_t)(e0 + e) * a.n + at, term[e]);
+                load_slots<RAGGED>(a.expert_out + (size_t)(e0 + e) * a.n, i, a.n, term[e]);
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -563,10 +579,10 @@ __global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
             }
         }
     }
-    load_slots(a.residual + at, res);
-    load_slots(a.wd + at, wd);
-    load_slots(a.wr + at, wr);
-    load_slots(a.wf + at, wf);
+    load_slots<RAGGED>(a.residual, i, a.n, res);
+    load_slots<RAGGED>(a.wd, i, a.n, wd);
+    load_slots<RAGGED>(a.wr, i, a.n, wr);
+    load_slots<RAGGED>(a.wf, i, a.n, wf);
     if (status != 0) return;
     if (other != 0) {
         if (threadIdx.x == 0) *a.status = -1;
@@ -582,7 +598,7 @@ __global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
 #pragma unroll 1
     for (int vectors = 2; vectors >= 1; --vectors) {
         float ss[2];
-        chains_from_registers<2>(dr, vectors, a.n, scratch, ss);
+        chains_from_registers<2, RAGGED>(dr, vectors, a.n, scratch, ss);
         // odd lanes see to the routed branch
         const bool odd = (threadIdx.x & 1) != 0 && vectors == 2;
         inv = inverse_from_sum(odd ? ss[1] : ss[0], a.n, a.eps);
@@ -610,7 +626,7 @@ __global__ __launch_bounds__(THREADS) void combine_small_kernel(CombineArgs a) {
         if (threadIdx.x == 0) *a.status = -1;
         return;
     }
-    if (i < a.n) store_slots(a.out + i, y);
+    store_slots<RAGGED>(a.out, i, a.n, y);
 }
 
 __global__ __launch_bounds__(THREADS) void combine_cell_kernel(CombineArgs a) {
@@ -648,7 +664,7 @@ __global__ __launch_bounds__(THREADS) void combine_cell_kernel(CombineArgs a) {
     }
     const float *const vec[2] = {a.dense, a.routed};
     float ss[2];
-    serial_square_sums<2>(vec, a.n, scratch, ss, bad);
+    serial_square_sums<2, true>(vec, a.n, scratch, ss, bad);
     const float inv_d = inverse_from_sum(ss[0], a.n, a.eps), inv_r = inverse_from_sum(ss[1], a.n, a.eps);
     bad |= nonfinite(inv_d) | nonfinite(inv_r);
     each_element(a.n, [&](int i) {
@@ -662,7 +678,7 @@ __global__ __launch_bounds__(THREADS) void combine_cell_kernel(CombineArgs a) {
     });
     const float *const vec2[1] = {a.sum};               // a thread reads back the elements it wrote itself
     float ss_sum[1];
-    serial_square_sums<1>(vec2, a.n, scratch_sum, ss_sum, bad);
+    serial_square_sums<1, true>(vec2, a.n, scratch_sum, ss_sum, bad);
     const float inv_f = inverse_from_sum(ss_sum[0], a.n, a.eps);
     bad |= nonfinite(inv_f);
     each_element(a.n, [&](int i) {
@@ -708,7 +724,8 @@ int norm_cell_launch(int kind, const float *x, const float *weight, const float 
     if (!x || !out || !status || n < 1 || kind < 0 || kind > 2 || (kind != 0 && !weight) || (kind == 2 && !residual))
         return -1;
     NormArgs a = {x, weight, residual, out, n, kind, eps, root, status};
-    norm_cell_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
+    if (n < ORDERED_MIN) norm_cell_kernel<false><<<dim3(1), dim3(THREADS), 0, stream>>>(a);
+    else norm_cell_kernel<true><<<dim3(1), dim3(THREADS), 0, stream>>>(a);
     return launched() ? 0 : -1;
 }
 
@@ -730,8 +747,9 @@ int combine_cell_launch(const float *residual, const float *dense, const float *
         return -1;
     CombineArgs a = {residual, dense, routed, wd, wr, wf, sum_scratch, out, n, eps, scalar, status, other_status,
                      expert_out, weights, topk};
-    if (n <= SQ_CHUNK && n % SLOTS == 0) combine_small_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
-    else combine_cell_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
+    if (n > SQ_CHUNK) combine_cell_kernel<<<dim3(1), dim3(THREADS), 0, stream>>>(a);
+    else if (n % SLOTS == 0) combine_small_kernel<false><<<dim3(1), dim3(THREADS), 0, stream>>>(a);
+    else combine_small_kernel<true><<<dim3(1), dim3(THREADS), 0, stream>>>(a);
     return launched() ? 0 : -1;
 }
 

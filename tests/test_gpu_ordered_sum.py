@@ -45,7 +45,7 @@ def vector(kind, n, g):
 KINDS = ["normal", "ties", "ones", "growing", "falling", "outliers", "zeros", "subnormal", "edge", "overflow"]
 
 
-@pytest.mark.parametrize("n", [511, 512, 513, 1024, 1025, 2047, 2049, 2816, 3072, 3073, 4095, 4096, 4097, 4608, 9000])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 31, 33, 64, 511, 512, 513, 735, 736, 737, 1024, 1025, 2047, 2049, 2816, 3072, 3073, 4095, 4096, 4097, 4608, 9000])
 def test_sum_of_squares_is_the_chain(gpu, oracle, n):
     eps = f32(1e-6)
     for at, kind in enumerate(KINDS):
