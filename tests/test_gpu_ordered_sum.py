@@ -1,10 +1,12 @@
 """The sum of squares of a norm is the left-to-right fp32 chain whatever its values do to the accumulator: ties to even,
 jumps over many powers of two, subnormals, overflow, sizes around every layout's edge."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from golden import cases
-from oracle_lib import bits, ptr
+from oracle_lib import bits, ffn_layer_struct, host_threads, ptr
 
 pytestmark = pytest.mark.gpu
 synth = cases.synth
@@ -39,10 +41,16 @@ def vector(kind, n, g):
         x = np.where(np.arange(n) % 12 == 11, np.sqrt(np.exp2(np.arange(n) // 48 - 20.0)), 1e-4 * x)
     elif kind == "overflow":
         x = x * 1e18
+    elif kind == "stagnant":                # squares of less than half a unit leave the chain below two, a plain sum passes it
+        x = np.full(n, 2.0 ** -12.5)
+        x[0] = np.sqrt(2 - 2.0 ** -15)
+    elif kind == "overtaking":              # squares that the chain rounds up to a unit each: it passes two before a plain sum
+        x = np.full(n, np.sqrt(0.6) * 2.0 ** -11.5)
+        x[0] = np.sqrt(2 - 200 * 2.0 ** -23)
     return x.astype(f32)
 
 
-KINDS = ["normal", "ties", "ones", "growing", "falling", "outliers", "zeros", "subnormal", "edge", "overflow"]
+KINDS = ["normal", "ties", "ones", "growing", "falling", "outliers", "zeros", "subnormal", "edge", "overflow", "stagnant", "overtaking"]
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 31, 33, 64, 511, 512, 513, 735, 736, 737, 1024, 1025, 2047, 2049, 2816, 3072, 3073, 4095, 4096, 4097, 4608, 9000])
@@ -70,3 +78,20 @@ def test_sum_of_squares_is_the_chain(gpu, oracle, n):
         assert st == rc
         if rc == 0:
             assert np.array_equal(bits(got["out"]), bits(want))
+
+
+@pytest.mark.parametrize("H", [704, 768, 2816, 4096, 4160])
+def test_first_norm_of_a_block(gpu, oracle, H):
+    """The same vectors as the residual of a feed-forward block, whose first launch has a kernel of its own."""
+    D, F, E, K = 64, 64, 2, 1
+    w = synth.ffn_layer(H, D, F, E, K, 3)
+    block, layer = gpu.FfnBlock(w), ffn_layer_struct(w)
+    for at, kind in enumerate(KINDS):
+        print("ordered sum, block", H, kind, flush=True)
+        residual = vector(kind, H, synth.rng(50 * H + at))
+        want, sel, wt = np.zeros(H, f32), np.zeros(K, np.int32), np.zeros(K, f32)
+        rc = oracle.orc_ffn_block(C.byref(layer), ptr(residual), ptr(want), ptr(sel), ptr(wt), host_threads())
+        st, gsel, gwt, out = block.step(residual)
+        assert st == rc
+        if rc == 0:
+            assert np.array_equal(gsel, sel) and np.array_equal(bits(gwt), bits(wt)) and np.array_equal(bits(out), bits(want))
