@@ -54,6 +54,8 @@ def check(pkg, oracle, vals, scales, biases, R, C, xs):
     (257, 512, 70), (130, 576, 33),             # eight and nine groups
     (200, 4096, 100), (70, 1088, 64),           # sixty-four and seventeen
     (16640, 192, 130), (16448, 704, 129),       # 64-token tiles; a last tile of one token
+    # waves without rows beside two and three rounds of group sums (49, 97 and 128 groups, 48 to a round)
+    (65, 3136, 33), (65, 6208, 40), (300, 8192, 70), (16449, 3136, 70),
 ])
 def test_tile_forms(pkg, oracle, R, C, B):
     print(f"mfma forms R={R} C={C} B={B}", flush=True)
@@ -61,7 +63,8 @@ def test_tile_forms(pkg, oracle, R, C, B):
     check(pkg, oracle, vals, scales, biases, R, C, synth.activations(C, B, 23))
 
 
-@pytest.mark.parametrize("R,C,B", [(130, 576, 33), (300, 448, 65), (16640, 192, 130), (16448, 704, 129)])
+@pytest.mark.parametrize("R,C,B", [(130, 576, 33), (300, 448, 65), (16640, 192, 130), (16448, 704, 129),
+                                   (65, 6208, 33), (130, 3136, 65)])
 def test_without_biases(pkg, oracle, R, C, B):
     print(f"mfma no biases R={R} C={C} B={B}", flush=True)
     vals, scales, _ = synth.q4_tensor(R, C, R + C + B)
