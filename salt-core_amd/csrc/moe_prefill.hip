@@ -46,6 +46,9 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *wave_totals, int
     return before + incl - v;
 }
 
+// Blocks of 64 of an expert's n tokens; what they leave, at most 32, is one more block of that many.
+__device__ __forceinline__ int wide_blocks(int n) { return (n + MFMA_TM / 2 - 1) / MFMA_TM; }
+
 // One thread per token: validate, count per expert in LDS, then one global add per expert and workgroup.  With up to
 // MAXK experts per token the whole selection of a token is sent for at once and checked in registers: the launch is a
 // chain of load latencies, not of work (2048 tokens, top-8: 9.1 -> 5.0 us).  MAXK = 0: any number.
@@ -109,18 +112,20 @@ struct ScanArgs {
     PrefillPlan *plan;
     int *status_out;                     // optional
     MfmaJob *gate_up_jobs, *down_jobs;
-    int *gate_up_tile_jobs, *down_tile_jobs;     // job of every block of tokens of a launch, those of 64 tokens first
+    int4 *places;                        // of every expert with tokens: its job, its first blocks of 64 and of 32 tokens
     const uint16_t *planes_in;           // split of the inputs, one row per token  [tokens][hidden]
     const uint16_t *planes_act;          // split of the activations, grouped rows   [rows][routed]
     float *gate, *up, *down;
 };
 
-// one workgroup: exclusive scans over the experts, job tables for both launches
+// One workgroup: exclusive scans over the experts, job tables for both launches.  The jobs of the blocks of tokens are left to
+// the fill, which has a workgroup per expert (2048 tokens, 128 experts: 8.1 us with them, 6.6 without; 65536 tokens, sixteen
+// experts, 34.5 and 5.0).
 __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs a) {
     __shared__ int s_wave[MAX_EXPERTS / 64];
     const int e = threadIdx.x;
     const int n = e < a.n_experts ? a.counts[e] : 0;
-    const int wide = (n + MFMA_TM / 2 - 1) / MFMA_TM, narrow = n > wide * MFMA_TM;     // blocks of 64 and of 32 tokens
+    const int wide = wide_blocks(n), narrow = n > wide * MFMA_TM;
     int rows_total, blocks_total;
     const int row0 = block_exclusive_scan(n, s_wave, &rows_total);
     // both counts in one scan: at most MAX_EXPERTS narrow blocks, and 2^18 wide ones
@@ -166,32 +171,28 @@ __global__ __launch_bounds__(MAX_EXPERTS) void group_scan_kernel(const ScanArgs 
         d.tile0 = wide0 * nt_down;
         d.row_base = 0;
         a.down_jobs[job] = d;
-        for (int i = 0; i < wide; ++i) {
-            a.gate_up_tile_jobs[2 * wide0 + i] = 2 * job;
-            a.gate_up_tile_jobs[2 * wide0 + wide + i] = 2 * job + 1;
-            a.down_tile_jobs[wide0 + i] = job;
-        }
-        if (narrow) {
-            a.gate_up_tile_jobs[2 * (wide_total + narrow0)] = 2 * job;
-            a.gate_up_tile_jobs[2 * (wide_total + narrow0) + 1] = 2 * job + 1;
-            a.down_tile_jobs[wide_total + narrow0] = job;
-        }
+        a.places[e] = make_int4(job, wide0, wide_total + narrow0, 0);
     }
 }
 
 // One workgroup of sixteen waves per expert: its (token, rank) pairs in token-major order.  Each wave owns a
 // contiguous run of the selection and walks it 64 pairs at a time (one coalesced load), twice: first to count its
 // matches, then, knowing how many matches the waves before it hold, to place them.  A match's place inside a chunk
-// is the number of matching lanes below it, so the order is the selection's own.  The launch is a chain of load
-// latencies: FILL_AHEAD chunks are sent for at once, and a run that short is not read again (2048 tokens, top-8:
-// 14.5 -> 7.0 us).
+// is the number of matching lanes below it, so the order is the selection's own.  On the way it writes the job of each of its
+// expert's blocks of tokens, those of 64 tokens first, which a lane per expert of the scan would have to do one by one.
+// The launch is a chain of load latencies: FILL_AHEAD chunks are sent for at once (as many as a lane has registers to spare),
+// and a run that short, 16384 pairs over the sixteen waves, is not read again: 2048 tokens, top-8, 14.5 -> 7.2 us; 2304
+// tokens, read twice, 9.3.
 constexpr int FILL_WAVES = 16, FILL_AHEAD = 16;
 
 __global__ __launch_bounds__(FILL_WAVES * 64) void group_fill_kernel(const int *__restrict__ selected, int pairs, int topk,
                                                                      const int *__restrict__ offsets, int n_experts,
                                                                      const PrefillPlan *__restrict__ plan,
+                                                                     const int4 *__restrict__ places,
                                                                      int *__restrict__ row_pairs,
-                                                                     int *__restrict__ pair_rows) {
+                                                                     int *__restrict__ pair_rows,
+                                                                     int *__restrict__ gate_up_tile_jobs,
+                                                                     int *__restrict__ down_tile_jobs) {
     __shared__ int wave_count[FILL_WAVES];
     if (plan->status != 0) {            // keep the gather in range: every grouped row reads token 0
         for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < pairs; p += gridDim.x * blockDim.x) row_pairs[p] = 0;
@@ -219,6 +220,18 @@ __global__ __launch_bounds__(FILL_WAVES * 64) void group_fill_kernel(const int *
         for (int i = 0; i < FILL_AHEAD; ++i) mine += __popcll(__ballot(held[i] == e));
     }
     if (lane == 0) wave_count[wave] = mine;
+    const int4 place = places[e];
+    const int n = offsets[e + 1] - offsets[e], wide = wide_blocks(n);
+    for (int i = threadIdx.x; i < wide; i += FILL_WAVES * 64) {
+        gate_up_tile_jobs[2 * place.y + i] = 2 * place.x;
+        gate_up_tile_jobs[2 * place.y + wide + i] = 2 * place.x + 1;
+        down_tile_jobs[place.y + i] = place.x;
+    }
+    if (threadIdx.x == 0 && n > wide * MFMA_TM) {
+        gate_up_tile_jobs[2 * place.z] = 2 * place.x;
+        gate_up_tile_jobs[2 * place.z + 1] = 2 * place.x + 1;
+        down_tile_jobs[place.z] = place.x;
+    }
     __syncthreads();
     int at = offsets[e];
     for (int w = 0; w < wave; ++w) at += wave_count[w];
@@ -267,6 +280,7 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 struct PrefillWorkspace {
     PrefillPlan *plan; int *counts, *offsets, *pair_rows, *row_pairs;
     MfmaJob *gate_up_jobs, *down_jobs;
+    int4 *places;
     int *gate_up_tile_jobs, *down_tile_jobs;
     uint16_t *planes_in, *planes_act;
     float *gate, *up, *down;
@@ -285,6 +299,7 @@ PrefillWorkspace carve(const MoeGeometry &g, int tokens, void *base) {
     w.row_pairs = (int *)take(rows * 4);
     w.gate_up_jobs = (MfmaJob *)take(2 * E * sizeof(MfmaJob));
     w.down_jobs = (MfmaJob *)take(E * sizeof(MfmaJob));
+    w.places = (int4 *)take(E * sizeof(int4));
     const size_t tiles = rows / MFMA_TM + (E < rows ? E : rows);          // of tokens, at most
     w.gate_up_tile_jobs = (int *)take(2 * tiles * 4);
     w.down_tile_jobs = (int *)take(tiles * 4);
@@ -327,13 +342,13 @@ int moe_prefill_launch(const MoeGeometry &g, const uint8_t *pool, size_t expert_
     a.pool = pool; a.expert_stride = expert_stride; a.n_experts = g.n_experts; a.hidden = g.hidden; a.routed = g.routed;
     a.counts = w.counts; a.offsets = w.offsets; a.group_rows = group_rows; a.plan = w.plan; a.status_out = status_dev;
     a.gate_up_jobs = w.gate_up_jobs; a.down_jobs = w.down_jobs;
-    a.gate_up_tile_jobs = w.gate_up_tile_jobs; a.down_tile_jobs = w.down_tile_jobs;
+    a.places = w.places;
     a.planes_in = w.planes_in; a.planes_act = w.planes_act;
     a.gate = w.gate; a.up = w.up; a.down = w.down;
     hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(MAX_EXPERTS), 0, stream, a);
     int *rp = row_pairs ? row_pairs : w.row_pairs;
     hipLaunchKernelGGL(group_fill_kernel, dim3(g.n_experts), dim3(FILL_WAVES * 64), 0, stream, selected, rows, g.topk,
-                       w.offsets, g.n_experts, w.plan, rp, w.pair_rows);
+                       w.offsets, g.n_experts, w.plan, w.places, rp, w.pair_rows, w.gate_up_tile_jobs, w.down_tile_jobs);
     if (hipGetLastError() != hipSuccess) return -1;
 
     // The number of 64-token tiles is known only on the device; the grid covers its upper bound (sum over experts of

@@ -43,9 +43,12 @@ def test_mixed_blocks(pkg, oracle, R, C_, B, form):
     check(pkg, oracle, vals[:rows * C_ // 8], scales[:rows * C_ // 64], biases[:rows * C_ // 64], rows, C_, xs[:70])
 
 
-@pytest.mark.parametrize("H,F", [(128, 320), (320, 128)])
-def test_experts_around_the_block_sizes(pkg, oracle, H, F):
-    counts = [0, 1, 31, 32, 33, 0, 63, 64, 65, 95, 96, 97, 128, 129, 0]
+EDGES = [0, 1, 31, 32, 33, 0, 63, 64, 65, 95, 96, 97, 128, 129, 0]
+LONG = [33, 65568, 0, 40]               # one expert with 1025 blocks of 64 tokens, more than a workgroup has threads
+
+
+@pytest.mark.parametrize("H,F,counts", [(128, 320, EDGES), (320, 128, EDGES), (64, 64, LONG)])
+def test_experts_around_the_block_sizes(pkg, oracle, H, F, counts):
     print(f"prefill blocks H={H} F={F}", flush=True)
     E, T, K = len(counts), sum(counts), 1
     sel = np.random.default_rng(3).permutation(np.repeat(np.arange(E, dtype=np.int32), counts)).reshape(T, K)
