@@ -72,7 +72,7 @@ struct Q4Launch {
 };
 int q4_moe_gate_up_launch(const Q4Launch &launch, hipStream_t stream);   // fills tiles and jobs from launch.moe
 int q4_moe_down_launch(const Q4Launch &launch, hipStream_t stream);
-int q4_moe_arrival_rows(int hidden, int routed, int topk);     // as the down launch prefers; 64 is always possible
+int q4_moe_arrival_rows(int hidden, int topk);     // as the down launch prefers; 64 is always possible
 
 // chains_per_lane: 8, 4 or 2; 0 lets the launcher choose from the tile count.
 int q4_launch(const Q4Launch &launch, int chains_per_lane, hipStream_t stream);

@@ -190,7 +190,7 @@ int moe_decode_step_launch(const MoeGeometry &g, const uint8_t *pool, size_t exp
         m.out = out;
         if (out) {
             // counters of parts of a tile lie where this plan keeps nothing else, or the down launch runs whole tiles
-            m.arrival_rows = q4_moe_arrival_rows(g.hidden, g.routed, g.topk);
+            m.arrival_rows = q4_moe_arrival_rows(g.hidden, g.topk);
             m.arrivals = (int *)ws.act;
             if (m.arrival_rows == 64 || (long long)(g.hidden + m.arrival_rows - 1) / m.arrival_rows > (long long)g.topk * g.routed) {
                 m.arrival_rows = 64;

@@ -738,23 +738,26 @@ int launch_as(const Q4Launch &L, int extra, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// One token.  `extra` workgroups follow those of the tiles.
+// One token, in the shapes that the rule of its prologue can choose.  `extra` workgroups follow those of the tiles.
 template <int PRO>
 int launch_one(const Q4Launch &L, const TileShape &shape, int extra, hipStream_t stream) {
-    switch (shape_key(shape.chains, shape.blocks, shape.split)) {
+    const int key = shape_key(shape.chains, shape.blocks, shape.split);
+    switch (key) {
         case shape_key(1, 32, 4): return launch_as<1, 1, 32, PRO, 4>(L, extra, stream);
-        case shape_key(1, 32, 8): return launch_as<1, 1, 32, PRO, 8>(L, extra, stream);
         case shape_key(2, 32, 1): return launch_as<2, 1, 32, PRO, 1>(L, extra, stream);
         case shape_key(2, 32, 2): return launch_as<2, 1, 32, PRO, 2>(L, extra, stream);
-        case shape_key(2, 32, 4): return launch_as<2, 1, 32, PRO, 4>(L, extra, stream);
-        case shape_key(2, 16, 2): return launch_as<2, 1, 16, PRO, 2>(L, extra, stream);
-        case shape_key(2, 16, 4): return launch_as<2, 1, 16, PRO, 4>(L, extra, stream);
         case shape_key(4, 16, 1): return launch_as<4, 1, 16, PRO, 1>(L, extra, stream);
+    }
+    if constexpr (PRO <= 1) switch (key) {
+        case shape_key(2, 16, 4): return launch_as<2, 1, 16, PRO, 4>(L, extra, stream);
         case shape_key(4, 16, 2): return launch_as<4, 1, 16, PRO, 2>(L, extra, stream);
     }
-    if (PRO == 0) switch (shape_key(shape.chains, shape.blocks, shape.split)) {         // as the caller asked
-        case shape_key(2, 16, 1): return launch_as<2, 1, 16, 0, 1>(L, extra, stream);
-        case shape_key(8, 16, 1): return launch_as<8, 1, 16, 0, 1>(L, extra, stream);
+    if constexpr (PRO == 0) switch (key) {
+        case shape_key(1, 32, 8): return launch_as<1, 1, 32, 0, 8>(L, extra, stream);
+        case shape_key(2, 32, 4): return launch_as<2, 1, 32, 0, 4>(L, extra, stream);
+        case shape_key(2, 16, 2): return launch_as<2, 1, 16, 0, 2>(L, extra, stream);
+        case shape_key(2, 16, 1): return launch_as<2, 1, 16, 0, 1>(L, extra, stream);      // as the caller asked, this and
+        case shape_key(8, 16, 1): return launch_as<8, 1, 16, 0, 1>(L, extra, stream);      // this
     }
     return -1;
 }
@@ -863,9 +866,9 @@ TileShape down_shape(const MoeFuse &m) {
 }
 }  // namespace
 
-int q4_moe_arrival_rows(int hidden, int routed, int topk) {
+int q4_moe_arrival_rows(int hidden, int topk) {
     MoeFuse m = {};
-    m.hidden = hidden; m.routed = routed; m.topk = topk;
+    m.hidden = hidden; m.topk = topk;
     return TILE_ROWS / down_shape(m).split;
 }
 
