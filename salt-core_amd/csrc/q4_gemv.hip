@@ -696,19 +696,24 @@ TileShape whole_shape(int chains, int tiles, int tokens) {
 }
 
 // The shape of a launch whose caller leaves it open.  A compute unit's time follows the rows of the fullest one, so parts
-// pay where whole tiles leave some idle or some with one tile more than the rest.  us, 2816 columns:
-//   tiles      one token                                      three tokens
-//   16 - 64    quarters <1> 5.9, <2> 7.0, halves 7.4, whole 10.8   8.7 / 10.9 / 10.6 / 16.4
-//   65 - 96    eighths <1> 6.9, quarters <1> 7.5, halves 7.4      quarters <1> 10.9, halves 10.5, quarters <2> 11.7
-//   97 - 128   halves 7.4, quarters <1> 7.6                       halves 10.6, quarters <1> 11.2
-//   129 - 192  quarters <2> 8.9, halves 9.7, whole 10.2            14.3 / 15.7 / 16.4
-//   193 - 256  halves 10.0, quarters <2> 13.7, whole 10.3           15.7 / 16.6 / 16.4
-//   257 - 384  halves <4> 12.3, quarters <2> 14.7, whole <4> 14.2  20.3 / 19.7 / 22.8
-//   385 - 512  whole <4> 14.9, halves <4> 15.7                    22.8 / 27.6
-//   513 - 640  whole <4> 19.1, halves <4> 19.2                    35.0 / 31.3
-// (<n>: chains per lane.  257 - 384 with three or four tokens: three waves a SIMD need 168 registers or fewer; without
-// that bound halves took 26.9 and 32.2 us.)  Two and four tokens as three.  Below 1024 columns one chain per lane gives
-// nothing (a launch of any shape takes 4.2 to 4.6 us), and at 513 - 640 tiles 5 to 7 % as everywhere.
+// pay where whole tiles leave some idle or some with one tile more than the rest.  us, 2816 columns, first and last of a range:
+//   tiles      one token                                                   three tokens
+//   16 - 64    quarters <1> 5.8, 6.0; <2> 6.8, 7.1; halves 7.2, 7.4;       8.4, 9.0; 10.6, 11.1; 10.4, 10.7;
+//              whole 10.7                                                  16.3
+//   72 - 96    eighths <1> 6.9, 7.0; quarters <1> 7.5; halves 7.4          quarters <1> 11.1, 11.5; halves 10.4, 10.8
+//   112 - 128  halves 7.5; quarters <1> 7.7                                halves 11.0; quarters <1> 11.7
+//   144 - 192  quarters <2> 8.8, 9.0; halves 9.8; whole 10.7               13.8, 14.4; 15.5; 16.3
+//   208 - 256  halves 9.8, 10.1; quarters <2> 13.9, 14.2; whole 11.3       15.4, 15.5; 16.6; 16.3
+//   264 - 384  halves <4> 12.4, 13.4; quarters <2> 15.1, 17.6;             20.5, 21.1; 19.5, 26.2;
+//              whole <4> 14.2, 14.6                                        22.8, 23.3
+//   400 - 512  whole <4> 14.6, 14.9; halves <4> 15.6, 16.3                 23.2, 23.4; 27.8, 28.9
+//   520 - 640  whole <4> 18.9, 19.7; halves <4> 17.9, 19.0                 35.1, 35.5; 31.3, 32.1
+// (<n>: chains per lane, two where none is given.  257 - 384 with three or four tokens: three waves a SIMD need 168 registers
+// or fewer; without that bound halves took 26.9 and 32.2 us.)  Two and four tokens as three, except at 257 - 384: one line
+// serves all numbers of tokens there, although up to 320 tiles quarters <2> would be quicker for two (16.0 against 18.0 us at
+// 264; 20.2 against 19.0 at 384) and, in rows of 2816 columns and more, for three (1024 columns 9.2 against 8.9); for four they
+// are not (26.1 against 24.1).  Below 1024 columns one chain per lane gives nothing (a launch of any shape takes 4.2 to 4.6
+// us).  At 513 - 640 one token's halves would be 3 to 6 % quicker.
 // A single token's parts keep its whole row in LDS, except <4>, which stages activations with each step's weights.
 TileShape open_shape(int tiles, int cols, int tokens) {
     const int wide = tokens == 1 ? 32 : 16;
