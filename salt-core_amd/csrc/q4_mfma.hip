@@ -55,9 +55,10 @@
 // eight waves 102.
 //
 // Bound: the matrix cores, which execute twice the useful operations, at the
-// clock that their power leaves them: 44 % busy at 1.6 to 2.1 GHz in the grouped
-// prefill (2048 tokens, 128 experts, top-8, 2816/704: 946 -> 581 us a layer);
-// one 16384 x 2816 matrix, 333 tokens: 101 -> 75 us (256 tokens, one tile of 64
+// clock that their power leaves them: in the grouped prefill (2048 tokens, 128
+// experts, top-8, 2816/704: 946 -> 592 us a layer) 51 % busy in gate and up, 37 % in
+// down, at 1.6 to 2.1 GHz;
+// one 16384 x 2816 matrix, 333 tokens: 101 -> 76 us (256 tokens, one tile of 64
 // for each compute unit, 55 us: 1.1 PFLOP/s of both planes).  Before, every scale
 // group cost 16 multiply-adds per block and a conversion in each of two waves,
 // and each 32 bytes of codes and each scale fetched a cache line of its own.
