@@ -952,7 +952,7 @@ int launch_downs(const Q4Launch &moe, const Q4Launch &dense, hipStream_t stream)
 }  // namespace
 
 bool q4_ffn_serves(const FfnShape &f, const Q8Launch &gate) {
-    // (a chain's width, 4096, also lets every shape of gate_up_shape but the whole tiles of wider rows through)
+    // (a chain's width, 4096, is also within what parts of a tile hold of a row)
     return q8_chain_takes(gate) && f.dense <= MOE_FUSE_MAX_ROUTED && f.routed <= MOE_FUSE_MAX_ROUTED &&
            f.n_experts <= MOE_FUSE_MAX_EXPERTS && f.topk <= ROUTER_MAX_TOPK;
 }
