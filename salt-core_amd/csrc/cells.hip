@@ -80,11 +80,11 @@ __device__ __forceinline__ void each_element(int n, F f) {
     }
 }
 
-// acc + mine[0] + mine[1] + ... + mine[count - 1], left to right.  32 values per batch; the next batch is read from
-// LDS while the current one is added, unconditionally one batch ahead (what is read past the end is dropped, the
-// staging buffers have a tail for it).
+// acc + mine[0] + mine[1] + ... + mine[count - 1], left to right; count is a multiple of 32.  32 values per batch; the next
+// batch is read from LDS while the current one is added, unconditionally one batch ahead (what is read past the end is
+// dropped, the staging buffers have a tail for it).
 __device__ __forceinline__ float add_staged(const float *mine, int count, float acc) {
-    const int full = count & ~31, pairs = full & ~63;
+    const int pairs = count & ~63;
     float4 a[8], b[8];
     auto fetch = [&](float4 (&dst)[8], int at) {
 #pragma unroll
@@ -106,8 +106,7 @@ __device__ __forceinline__ float add_staged(const float *mine, int count, float 
         fetch(a, i + 64);
         add(b);
     }
-    if (full != pairs) add(a);
-    for (int i = full; i < count; ++i) acc = acc + mine[i];
+    if (count != pairs) add(a);
     return acc;
 }
 
